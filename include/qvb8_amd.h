@@ -276,6 +276,8 @@ int64_t qvb8_moe_workspace_bytes(int64_t tokens, int64_t topk, int64_t n_experts
  *     tokens chose it.  An expert's pairs are the rows of one operand, as many as there are tokens: an expert with more
  *     pairs than that (only possible when a token lists it twice) makes the whole output NaN instead of a sum with pairs
  *     missing; the other paths take such lists.
+ * More than 16 tokens, any x_dtype, P_up and P_dn multiples of 128: four launches as well, on the matrix cores with H handed over
+ * in fp32 (used as fp16 hi + lo of a row scaled by a power of two); an expert is read once for up to 64 of its pairs.
  * Everything else takes the general path (four launches, H in fp32, an expert read once for up to 8 of its tokens).
  * Replaces: ext.moe_experts  qvb8_moe_experts_forward qvb8_cuda.cu:937-992 (kernels qvb8_moe_gemv :860-907,
  * qvb8_moe_act :910-918, qvb8_moe_combine :924-935) with act QVB8_MOE_SILU_GATED, and ext.moe_experts_relu2

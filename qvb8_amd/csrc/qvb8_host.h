@@ -4,6 +4,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 #include <stdlib.h>
+#include <atomic>
 #include <string>
 
 namespace qvb8 {
@@ -41,6 +42,21 @@ inline int device_cus() {
         cached[dev] = n;
     }
     return cached[dev];
+}
+
+// Lets a kernel be launched with `bytes` of dynamic LDS (more than the default 64 KB); asked of the runtime once per
+// kernel and device.
+template <auto Kernel>
+inline int raise_lds_limit(size_t bytes, const char* who) {
+    static std::atomic<bool> done[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(-3, "%s: no current device", who);
+    if (!done[dev].load(std::memory_order_acquire)) {
+        if (hipFuncSetAttribute((const void*)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
+            return fail(-3, "%s: cannot raise the kernel's LDS limit", who);
+        done[dev].store(true, std::memory_order_release);
+    }
+    return 0;
 }
 
 // Integer knob from the environment, read on every call (cheap; lets a test change it between calls).

@@ -23,83 +23,133 @@
 #include "qvb8_device.h"
 #include "qvb8_host.h"
 #include "qvb8_mma_device.h"
+#include "qvb8_moe_plan.h"
 
 namespace qvb8 {
 
 constexpr int kMoeMB = 8;              // pairs that share one pass over an expert's rows
 constexpr int kMoeThreads = 256;
 
-// Workspace layout (bytes from the start): plan | H | Yd
-//   plan: i32 n_bad, i32 slots in use (+2 pad), int4 slot[n_slots] = {expert, first pair, end pair, 0} for the experts that have pairs
-//   (end == first for unused slots), i32 order[npairs] (pair numbers grouped by expert)
-struct MoePlan {
-    int32_t* n_bad; int4* slot; int32_t* order;
-};
-__host__ __device__ inline int64_t moe_slots(int64_t E, int64_t npairs) { return E < npairs ? E : npairs; }
-__host__ __device__ inline size_t moe_plan_bytes(int64_t E, int64_t npairs) {
-    return (size_t)(16 + moe_slots(E, npairs) * 16 + npairs * 4 + 255) & ~(size_t)255;
-}
-__host__ __device__ inline MoePlan moe_plan_at(void* ws, int64_t E, int64_t npairs) {
-    unsigned char* p = reinterpret_cast<unsigned char*>(ws);
-    return MoePlan{reinterpret_cast<int32_t*>(p), reinterpret_cast<int4*>(p + 16),
-                   reinterpret_cast<int32_t*>(p + 16 + moe_slots(E, npairs) * 16)};
-}
+constexpr int kPlanMaxThreads = 1024;
+constexpr int kPlanTableExperts = 512;
+constexpr int kPlanKept = 4;           // pairs per thread kept in registers from the count to the placement
 
-// One workgroup: pairs grouped by expert (counting sort), table of the experts that have pairs.  The two running
-// sums over the experts (pairs before expert e, selected experts before e) are a workgroup scan, 256 experts per round.
+// One workgroup: pairs grouped by expert (a stable counting sort: an expert's pairs keep their order, so that the plan, and
+// with it every sum that depends on how an expert's pairs are cut into blocks, is the same run to run), table of the experts
+// that have pairs.  The running sums over the experts (pairs, selected experts and token blocks before expert e) are a
+// workgroup scan, blockDim experts per round.
 // `cap`: the most pairs one expert may have for the path that follows (the grouped walk takes an expert's pairs as the token
 // rows of ONE operand: at most one per token); an expert with more counts as a bad entry, so the results come out as NaN
 // instead of sums with pairs missing.
-__global__ void __launch_bounds__(kMoeThreads) moe_plan_kernel(const int64_t* __restrict__ idx, int npairs, int E, MoePlan pl, int cap) {
-    extern __shared__ int32_t s_cnt[];                        // [E] counts, then cursors; [E .. E + 8) scan scratch
+// Placement (`ordered`; the paths whose results do not depend on the order let every pair move its expert's cursor), blockDim
+// pairs at a time: every wave counts its pairs per expert in a table [wave][expert], a thread per expert
+// turns the counts into places, the pairs take them; with more than kPlanTableExperts experts the waves take turns at the
+// experts' cursors instead.  Bound by its chain of barriers and LDS trips (4072 pairs, 128 experts: 13.2 us; turns only
+// 19.1; cursors moved by atomics 15.4).
+__global__ void __launch_bounds__(kPlanMaxThreads) moe_plan_kernel(const int64_t* __restrict__ idx, int npairs, int E, MoePlan pl, int cap, int ordered) {
+    extern __shared__ int32_t s_cnt[];                        // [E] counts, then cursors; [48] scan scratch; [waves][E] where E allows
     int32_t* s_scan = s_cnt + E;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int32_t* s_wave = s_scan + 48;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n_waves = (int)blockDim.x >> 6;
+    // the thread's first pairs, asked for together and kept for both passes (-1: no such pair, -2: outside the stack)
+    int mine[kPlanKept];
+#pragma unroll
+    for (int k = 0; k < kPlanKept; ++k) {
+        const int p = tid + k * (int)blockDim.x;
+        const int64_t e = idx[min(p, npairs - 1)];
+        mine[k] = p >= npairs ? -1 : (e >= 0 && e < E) ? (int)e : -2;
+    }
+    auto expert_of = [&](int p, int k) {
+        if (k < kPlanKept) return mine[k];
+        const int64_t e = p < npairs ? idx[p] : -1;
+        return p >= npairs ? -1 : (e >= 0 && e < E) ? (int)e : -2;
+    };
     for (int e = tid; e < E; e += blockDim.x) s_cnt[e] = 0;
     if (tid == 0) *pl.n_bad = 0;
     __syncthreads();
     int bad = 0;
-    for (int p = tid; p < npairs; p += blockDim.x) {
-        const int64_t e = idx[p];
-        if (e >= 0 && e < E) atomicAdd(&s_cnt[(int)e], 1); else ++bad;
-    }
+    auto count = [&](int e) { if (e >= 0) atomicAdd(&s_cnt[e], 1); else if (e == -2) ++bad; };
+#pragma unroll
+    for (int k = 0; k < kPlanKept; ++k) count(mine[k]);
+    for (int p = tid + kPlanKept * blockDim.x; p < npairs; p += blockDim.x) count(expert_of(p, kPlanKept));
     if (bad) atomicAdd(pl.n_bad, bad);
     __syncthreads();
     const int n_slots = E < npairs ? E : npairs;
-    int run_pairs = 0, run_active = 0;                        // totals of the rounds before this one (same in every thread)
+    int run_pairs = 0, run_active = 0, run_blocks = 0;        // totals of the rounds before this one (same in every thread)
     for (int e0 = 0; e0 < E; e0 += blockDim.x) {
         const int e = e0 + tid;
         const int c = e < E ? s_cnt[e] : 0;
         if (c > cap) atomicAdd(pl.n_bad, 1);
-        // inclusive scan of (c, c > 0) packed as pairs * 2^16 + active: both stay below 2^15 per round... pairs can be
-        // larger, so scan them separately
-        int sc = c, sa = c > 0 ? 1 : 0;
+        const int blocks = (c + kGroupTokens - 1) / kGroupTokens;
+        int sc = c, sa = c > 0 ? 1 : 0, sb = blocks;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
-            const int tc = __shfl_up(sc, o, 64), ta = __shfl_up(sa, o, 64);
-            if (lane >= o) { sc += tc; sa += ta; }
+            const int tc = __shfl_up(sc, o, 64), ta = __shfl_up(sa, o, 64), tb = __shfl_up(sb, o, 64);
+            if (lane >= o) { sc += tc; sa += ta; sb += tb; }
         }
-        if (lane == 63) { s_scan[wave] = sc; s_scan[4 + wave] = sa; }
+        if (lane == 63) { s_scan[wave] = sc; s_scan[16 + wave] = sa; s_scan[32 + wave] = sb; }
         __syncthreads();
-        int base_c = run_pairs, base_a = run_active, tot_c = 0, tot_a = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-            if (w < wave) { base_c += s_scan[w]; base_a += s_scan[4 + w]; }
-            tot_c += s_scan[w]; tot_a += s_scan[4 + w];
+        int base_c = run_pairs, base_a = run_active, base_b = run_blocks, tot_c = 0, tot_a = 0, tot_b = 0;
+        for (int w = 0; w < n_waves; ++w) {
+            if (w < wave) { base_c += s_scan[w]; base_a += s_scan[16 + w]; base_b += s_scan[32 + w]; }
+            tot_c += s_scan[w]; tot_a += s_scan[16 + w]; tot_b += s_scan[32 + w];
         }
         const int first = base_c + sc - c;                    // pairs before expert e
         if (e < E) {
-            if (c > 0) pl.slot[base_a + sa - 1] = int4{e, first, first + c, 0};
+            if (c > 0) pl.slot[base_a + sa - 1] = int4{e, first, first + c, base_b + sb - blocks};
             s_cnt[e] = first;                                 // becomes the expert's cursor
         }
-        run_pairs += tot_c; run_active += tot_a;
+        run_pairs += tot_c; run_active += tot_a; run_blocks += tot_b;
         __syncthreads();
     }
     for (int i = run_active + tid; i < n_slots; i += blockDim.x) pl.slot[i] = int4{0, 0, 0, 0};
-    if (tid == 0) pl.n_bad[1] = run_active;                   // slots in use
-    __syncthreads();
-    for (int p = tid; p < npairs; p += blockDim.x) {
-        const int64_t e = idx[p];
-        if (e >= 0 && e < E) pl.order[atomicAdd(&s_cnt[(int)e], 1)] = p;
-    }
+    if (tid == 0) { pl.n_bad[1] = run_active; pl.n_bad[2] = run_blocks; }      // slots in use, token blocks of all of them
+    const int e_bits = 32 - __builtin_clz(E > 1 ? E - 1 : 1);
+    auto place = [&](int p0, int mine_e) {
+        const int p = p0 + tid;
+        const bool has = mine_e >= 0;
+        const int e = has ? mine_e : 0;
+        if (!ordered) {
+            if (has) pl.order[atomicAdd(&s_cnt[e], 1)] = p;
+            return;
+        }
+        // the lanes of this wave with the same expert: by the bits of its number
+        uint64_t same = __builtin_amdgcn_ballot_w64(has);
+        for (int b = 0; b < e_bits; ++b) {
+            const uint64_t m = __builtin_amdgcn_ballot_w64(has && ((e >> b) & 1));
+            same &= ((e >> b) & 1) ? m : ~m;
+        }
+        const int rank = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+        int at = 0;
+        if (E <= kPlanTableExperts) {
+            for (int i = tid; i < n_waves * E; i += blockDim.x) s_wave[i] = 0;
+            __syncthreads();
+            if (has && rank == 0) s_wave[wave * E + e] = __builtin_popcountll(same);
+            __syncthreads();
+            for (int i = tid; i < E; i += blockDim.x) {
+                int run = s_cnt[i];
+                for (int w = 0; w < n_waves; ++w) { const int c = s_wave[w * E + i]; s_wave[w * E + i] = run; run += c; }
+                s_cnt[i] = run;
+            }
+            __syncthreads();
+            if (has) at = s_wave[wave * E + e] + rank;
+            __syncthreads();
+        } else {
+            const int turns = min(n_waves, (npairs - p0 + 63) / 64);
+            for (int w = 0; w < turns; ++w) {
+                if (w == wave && has) {
+                    at = s_cnt[e] + rank;                     // every lane reads before the group's first lane moves the cursor
+                    if (rank == 0) s_cnt[e] = at + __builtin_popcountll(same);
+                }
+                __syncthreads();
+            }
+        }
+        if (has) pl.order[at] = p;
+    };
+#pragma unroll
+    for (int k = 0; k < kPlanKept; ++k)
+        if (k * (int)blockDim.x < npairs) place(k * (int)blockDim.x, mine[k]);          // the same in every thread: place() has barriers
+    for (int p0 = kPlanKept * (int)blockDim.x; p0 < npairs; p0 += blockDim.x) place(p0, expert_of(p0 + tid, kPlanKept));
 }
 
 struct MoeGemvArgs {
@@ -947,6 +997,13 @@ int launch_moe_gemv(int stage, MoeGemvArgs a, int64_t slots, hipStream_t s) {
     else hipLaunchKernelGGL(moe_gemv_kernel<1>, grid, dim3(kMoeThreads), lds, s, a);
     return host::check_launch("qvb8_moe_experts");
 }
+int launch_moe_combine(const float* Yd, const float* w, void* out, int out_dtype, int64_t topk, int64_t D, int64_t tokens, const MoePlan& pl, hipStream_t s) {
+    dim3 grid((unsigned)((D + 255) / 256), (unsigned)tokens);
+    if (out_dtype == QVB8_F32) hipLaunchKernelGGL(moe_combine_kernel<0>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)D, (int)tokens, pl.n_bad);
+    else if (out_dtype == QVB8_F16) hipLaunchKernelGGL(moe_combine_kernel<1>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)D, (int)tokens, pl.n_bad);
+    else hipLaunchKernelGGL(moe_combine_kernel<2>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)D, (int)tokens, pl.n_bad);
+    return host::check_launch("qvb8_moe_experts combine");
+}
 // The matrix-core walk: what it needs.  H (fp16) takes the place of the fp32 H in the workspace.
 bool moe_walk_shapes_ok(int64_t topk, int x_dtype, int64_t P_up, int64_t Q_dn, int64_t P_dn) {
     if (x_dtype != QVB8_F16 && x_dtype != QVB8_BF16) return false;
@@ -1095,8 +1152,11 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
         return launch_moe_one<true, false, 2>(o, dn_regular, dn_blocks, tk, s);
     }
 
-    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(kMoeThreads), (size_t)(n_experts + 8) * 4, s, idx, (int)np, (int)n_experts, pl,
-                       grouped ? (int)(tokens < 16 ? tokens : 16) : (int)np);
+    // a thread per pair (or per expert, when they are more) up to the most a workgroup has
+    const int64_t plan_threads = std::min<int64_t>(kPlanMaxThreads, (std::max(np, n_experts) + 255) / 256 * 256);
+    const size_t plan_lds = (size_t)(n_experts + 48 + (n_experts <= kPlanTableExperts ? n_experts * (plan_threads / 64) : 0)) * 4;
+    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3((unsigned)plan_threads), plan_lds, s, idx, (int)np, (int)n_experts, pl,
+                       grouped ? (int)(tokens < 16 ? tokens : 16) : (int)np, grouped ? 0 : 1);
     if (int rc = host::check_launch("qvb8_moe_experts plan")) return rc;
     const int64_t slots = moe_slots(n_experts, np);
     if (grouped) {
@@ -1110,11 +1170,20 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
         wa.min_s = dn_min; wa.tau_s = dn_tau; wa.nbits = dn_nb; wa.bit_off = dn_off; wa.out = Yd;
         wa.Q = (int)Q_dn; wa.P = (int)P_dn; wa.units = (int)Q_dn; wa.gated = 0;
         if (int rc = launch_moe_walk<true, false>(wa, dn_regular, slots, tokens, s)) return rc;
-        dim3 cgrid((unsigned)((Q_dn + 255) / 256), (unsigned)tokens);
-        if (out_dtype == QVB8_F32) hipLaunchKernelGGL(moe_combine_kernel<0>, cgrid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)Q_dn, (int)tokens, pl.n_bad);
-        else if (out_dtype == QVB8_F16) hipLaunchKernelGGL(moe_combine_kernel<1>, cgrid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)Q_dn, (int)tokens, pl.n_bad);
-        else hipLaunchKernelGGL(moe_combine_kernel<2>, cgrid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)Q_dn, (int)tokens, pl.n_bad);
-        return host::check_launch("qvb8_moe_experts combine");
+        return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
+    }
+    if (tokens > 16 && moe_group_shapes_ok(P_up, Q_dn, P_dn)) {
+        MoeGroupArgs ga;
+        ga.X = X; ga.plan = pl; ga.ids = up_ids; ga.ids_bytes = up_ids_bytes;
+        ga.min_s = up_min; ga.tau_s = up_tau; ga.nbits = up_nb; ga.bit_off = up_off; ga.out = H;
+        ga.E = (int)n_experts; ga.Q = (int)Q_up; ga.P = (int)P_up; ga.topk = (int)topk; ga.units = (int)P_dn; ga.gated = act == 0 ? 1 : 0;
+        ga.row_blocks = ga.items = 0;
+        if (int rc = launch_moe_group(false, x_dtype, ga, np, s)) return rc;
+        ga.X = H; ga.ids = dn_ids; ga.ids_bytes = dn_ids_bytes;
+        ga.min_s = dn_min; ga.tau_s = dn_tau; ga.nbits = dn_nb; ga.bit_off = dn_off; ga.out = Yd;
+        ga.Q = (int)Q_dn; ga.P = (int)P_dn; ga.units = (int)Q_dn; ga.gated = 0;
+        if (int rc = launch_moe_group(true, QVB8_F32, ga, np, s)) return rc;
+        return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
     }
 
     MoeGemvArgs a;
@@ -1126,11 +1195,7 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
     a.out = Yd; a.Q = (int)Q_dn; a.P = (int)P_dn; a.x_dtype = QVB8_F32; a.units = (int)Q_dn;
     if (int rc = launch_moe_gemv(1, a, slots, s)) return rc;
 
-    dim3 grid((unsigned)((Q_dn + 255) / 256), (unsigned)tokens);
-    if (out_dtype == QVB8_F32) hipLaunchKernelGGL(moe_combine_kernel<0>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)Q_dn, (int)tokens, pl.n_bad);
-    else if (out_dtype == QVB8_F16) hipLaunchKernelGGL(moe_combine_kernel<1>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)Q_dn, (int)tokens, pl.n_bad);
-    else hipLaunchKernelGGL(moe_combine_kernel<2>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)Q_dn, (int)tokens, pl.n_bad);
-    return host::check_launch("qvb8_moe_experts combine");
+    return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
 }
 
 // ---- the same call for callers that cannot allocate ------------------------------------------------------------------

@@ -2,9 +2,10 @@
 
 Same class name, constructor, `from_packfiles`, `build_stack` layout and `forward(hidden_states, top_k_index,
 top_k_weights)` as the reference (src/qv_band/formats/qvb8/backends_experts.py:91-272).  The routed decode path is
-ext.moe_experts (four launches, no host round trip, each selected expert read once for all the tokens that chose it);
-larger token counts, stacks with escapes, other activations or shapes take the per-expert loop over QVBandLinearV8
-modules, which still runs on the GPU library.  There is no CPU reader here (the reference's QVBandLinearCPUV8 is its
+ext.moe_experts (four launches, no host round trip, each selected expert read once for all the tokens that chose it), for
+any number of tokens when the rows are whole 128-column steps; stacks with escapes, other activations, and more than
+FUSED_MAX_TOKENS tokens of other shapes take the per-expert loop over QVBandLinearV8 modules, which still runs on the GPU
+library.  There is no CPU reader here (the reference's QVBandLinearCPUV8 is its
 CPU-only dense path; this build's CPU restatement lives with the tests and is not a product path).
 """
 from __future__ import annotations
@@ -90,7 +91,8 @@ def _stackable(mods) -> bool:
 
 
 class QVBandExpertsV8(nn.Module):
-    # Up to this many tokens the routed kernels run; above it the per-expert loop (its GEMMs amortise the restore).
+    # Up to this many tokens the routed kernels run whatever the shape; above it only stacks whose rows are whole 128-column
+    # steps (the matrix-core kernels), the others take the per-expert loop.
     FUSED_MAX_TOKENS = 64
 
     def __init__(self, gate_up_experts, down_experts, *, num_experts: int, act_fn=None):
@@ -132,6 +134,9 @@ class QVBandExpertsV8(nn.Module):
             self._stk = (stack_projection(gu), stack_projection(dn)) if ok else False
         return self._stk is not False
 
+    def _whole_steps(self) -> bool:
+        return self.gate_up_experts[0].in_features % 128 == 0 and self.down_experts[0].in_features % 128 == 0
+
     def prepare(self) -> "QVBandExpertsV8":
         """Builds the stacks now (at load) instead of on the first routed call: the experts' rows are re-stored then, so
         footprints read afterwards are the ones that stay, and a first call inside a graph capture finds them built.
@@ -142,7 +147,7 @@ class QVBandExpertsV8(nn.Module):
 
     def forward(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:
         n_tok = top_k_index.shape[0]
-        if hidden_states.is_cuda and n_tok <= self.FUSED_MAX_TOKENS and self.build_stack():
+        if hidden_states.is_cuda and (n_tok <= self.FUSED_MAX_TOKENS or self._whole_steps()) and self.build_stack():
             g, d = self._stk
             return ext.moe_experts(hidden_states.contiguous(), top_k_index.contiguous(), top_k_weights.float(),
                                    g["ids"], g["min_s"], g["tau_s"], g["nbits"], g["bit_off"], g["Q"], g["P"],

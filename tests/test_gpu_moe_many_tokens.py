@@ -1,0 +1,38 @@
+"""GPU parity of the many-token expert kernels (more than 16 tokens, rows of whole 128-column steps): the sizes at which their
+tiles change -- 16, 32, 48, 64 and 65 pairs of an expert, one step and several chunks of columns -- with every width of
+row, against the oracle and run to run."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import qvb8_oracle as O
+from qvb8_amd import ext_qvb8 as ext
+from tests.test_gpu_moe import _check, _hand_made_stack
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("T,pairs,hidden,inter,gated,dtype", [
+    (17, 16, 128, 128, True, torch.bfloat16), (17, 17, 384, 256, False, torch.float16), (40, 33, 1152, 128, True, torch.float32),
+    (70, 48, 256, 640, False, torch.bfloat16), (70, 65, 640, 384, True, torch.float16), (140, 129, 2176, 128, True, torch.bfloat16)])
+def test_many_tokens(T, pairs, hidden, inter, gated, dtype):
+    """Expert 1 is chosen by `pairs` of the T tokens, the rest is spread; one expert is chosen by nobody."""
+    E, k = 6, 2
+    Qup = 2 * inter if gated else inter
+    up, Wup = _hand_made_stack(E, Qup, hidden, [6] * 16 + [7, 5, 6] + [4] * 13 + list(range(1, 15)) + [8] * 18, seed=40)
+    dn, Wdn = _hand_made_stack(E, hidden, inter, [5] * 16 + [4, 5, 6, 7, 8, 11, 3], seed=80)
+    rng = np.random.default_rng(T)
+    idx = np.stack([rng.permutation([0, 2, 3, 4])[:k] for _ in range(T)]).astype(np.int64)          # 5 is never chosen
+    idx[rng.permutation(T)[:pairs], 0] = 1
+    w = rng.uniform(0.1, 1.0, (T, k)).astype(np.float32)
+    x = torch.randn(T, hidden, generator=torch.Generator().manual_seed(T)).to(dtype)
+    fn = ext.moe_experts if gated else ext.moe_experts_relu2
+    args = (x.to(DEV), torch.from_numpy(idx).to(DEV), torch.from_numpy(w).to(DEV), *up, Qup, hidden, *dn, hidden, inter)
+    out = fn(*args)
+    assert out.dtype == dtype and out.shape == (T, hidden)
+    _check(out, O.moe_reference(x.float().numpy(), idx, w, Wup, Wdn, act="silu" if gated else "relu2"), dtype)
+    assert torch.equal(out, fn(*args))
+    bad = args[1].clone()
+    bad[3, 1] = E
+    assert bool(torch.isnan(fn(args[0], bad, *args[2:]).float()).all())
