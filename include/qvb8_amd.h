@@ -52,9 +52,9 @@ enum qvb8_status {
 
 /* Library identification: ABI version, bumped on any signature change or new entry point (3: row lookup, attention over
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
- * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe).  A binding compares the loaded library's answer
+ * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
-#define QVB8_ABI_VERSION 7
+#define QVB8_ABI_VERSION 8
 int qvb8_abi_version(void);
 /* Message of the calling thread's most recent failure ("" if none). Valid until that thread's next call. */
 const char* qvb8_last_error(void);
@@ -403,6 +403,45 @@ int qvb8_attn_fwd(const void* q, int64_t sq_r, int64_t sq_h, const void* ki, con
  * Replaces the torch expressions of attend  kv/fused_attn.py:302-316. */
 int qvb8_attn_combine(const float* o, const float* m, const float* l, int64_t n_splits, int64_t n_kv_heads,
                       int64_t n_rows, int64_t head_dim, int64_t G, float* out, float* lse, void* stream);
+
+/* ---- the banded KV cache's codec -------------------------------------------------------------------------------------- */
+
+/* A segment of keys or values x (heads, seq, dim), contiguous, in x_dtype, becomes per head ids of a fixed width and per channel
+ * (min, step):  step = max((max - min) / (2^w - 1), 1e-12),  id = clamp(round_to_even((x - min) / step), 0, 2^w - 1), fp32, each
+ * operation rounded by itself; non-finite values count as 0.  1 <= heads <= QVB8_KV_MAX_HEADS per call, dim <= 2048.
+ *   qvb8_kv_chunks  chunks of rows the calls below should use for this shape (their number is the caller's to keep);
+ *   qvb8_kv_range   partial[heads][chunks][2][dim] f32: every chunk's minima, then maxima;
+ *   qvb8_kv_check   lo, span (heads, dim) from the partial results (with `widths`: as an earlier call left them), and report[heads][2 + chunks] f32: the head's largest span, its
+ *                   width, and per chunk the largest |decoded - x|, the decoder's min + id * step rounded to orig_dtype.  Width =
+ *                   widths[head] (host array), or with widths null the smallest w in bits..16 with 2^w >= span / (2 tau) + 1.
+ *                   report null: lo and span only;
+ *   qvb8_kv_pack    step (heads, dim) and the ids at the given widths: packed[head] (host array of device pointers, 4-byte aligned,
+ *                   (seq * dim * width + 7) / 8 bytes each), fields LSB first, row-major.
+ * Replaces the torch expressions of band_kv_heads and pack_ids  kv/codec.py:53-68, 175-241. */
+#define QVB8_KV_MAX_HEADS 32
+int64_t qvb8_kv_chunks(int64_t heads, int64_t seq);
+int qvb8_kv_range(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, float* partial, int64_t chunks, void* stream);
+int qvb8_kv_check(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, const float* partial, int64_t chunks,
+                  int orig_dtype, int bits, double tau, const uint8_t* widths, float* lo, float* span, float* report, void* stream);
+int qvb8_kv_pack(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, const float* lo, const float* span,
+                 const uint8_t* widths, float* step, uint8_t* const* packed, void* stream);
+
+/* Packed heads into the id layout of qvb8_attn_fwd: per entry seq x dim ids to ids_out (u8 or u16 by id_bytes; keys row_stride ids
+ * apart), mid_out[dim] = min + step * c, step_out[dim] = step, *centre_out = c = (2^bits - 1) / 2.  `list`: host array, any number
+ * of entries.  With dim % 32 == 0, ids_out and row_stride must be 16-byte aligned.
+ * Replaces the loops of layout_from_segments  kv/fused_attn.py:189-216. */
+typedef struct qvb8_kv_head {
+    const uint8_t* packed; const float* min; const float* step;
+    void* ids_out; float* mid_out; float* step_out; float* centre_out;
+    int64_t seq; int32_t bits; int32_t reserved;
+} qvb8_kv_head;
+int qvb8_kv_unpack(const qvb8_kv_head* list, int64_t n_list, int64_t dim, int id_bytes, int64_t row_stride, void* stream);
+
+/* The tile table of qvb8_attn_fwd for segments of seg_len[0 .. n_seg) keys (host array) that follow each other: tiles of block_n
+ * keys inside each segment, the last of a segment shorter.  table i32[3][n_tiles] = first keys, lengths, segments; n_tiles must be
+ * the sum of ceil(seg_len / block_n).
+ * Replaces the loops of QVLayout  kv/fused_attn.py:155-186. */
+int qvb8_kv_tiles(const int64_t* seg_len, int64_t n_seg, int64_t block_n, int32_t* table, int64_t n_tiles, void* stream);
 
 #ifdef __cplusplus
 }

@@ -4,15 +4,17 @@ stream.  A failed call raises RuntimeError with the library's message; a missing
 library raises NativeLibraryError.  Nothing here computes anything."""
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
+import struct
 
 import torch
 
 from .common.errors import NativeLibraryError
 
 _LIB = None
-EXPECTED_ABI = 7            # QVB8_ABI_VERSION of include/qvb8_amd.h that the argument lists below were written for
+EXPECTED_ABI = 8            # QVB8_ABI_VERSION of include/qvb8_amd.h that the argument lists below were written for
 F32, F16, BF16 = 0, 1, 2
 _DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
@@ -20,7 +22,8 @@ _DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 SYMBOLS = ("qvb8_abi_version", "qvb8_last_error", "qvb8_decode", "qvb8_lookup_rows", "qvb8_scatter_escapes", "qvb8_certify",
            "qvb8_sat_half", "qvb8_scale_sat_half", "qvb8_gemv_workspace_bytes", "qvb8_gemv", "qvb8_mma_rowinfo_bytes", "qvb8_mma_prepare", "qvb8_mma_workspace_bytes", "qvb8_mma", "qvb8_launch_probe", "qvb8_mlp_workspace_bytes", "qvb8_mlp_init", "qvb8_mlp",
            "qvb8_moe_workspace_bytes", "qvb8_moe_experts", "qvb8_moe_experts_static",
-           "qvb8r_decode", "qvb8r_decode_blocks", "qvb8r_gemv_workspace_bytes", "qvb8r_gemv", "qvb8r_walk_probe", "qvb8r_fix_escapes", "qvb8_attn_fwd", "qvb8_attn_combine")
+           "qvb8r_decode", "qvb8r_decode_blocks", "qvb8r_gemv_workspace_bytes", "qvb8r_gemv", "qvb8r_walk_probe", "qvb8r_fix_escapes", "qvb8_attn_fwd", "qvb8_attn_combine",
+           "qvb8_kv_chunks", "qvb8_kv_range", "qvb8_kv_check", "qvb8_kv_pack", "qvb8_kv_unpack", "qvb8_kv_tiles")
 
 
 def lib_path() -> str:
@@ -103,6 +106,13 @@ def load(build_if_missing: bool = True):
     lib.qvb8_attn_fwd.argtypes = ([vp, i64, i64, vp, vp, i32, i64, i64] + [vp] * 9 + [i64, vp, vp, vp] + [i64] * 6
                                   + [ctypes.c_double, i64, vp])
     lib.qvb8_attn_combine.argtypes = [vp, vp, vp, i64, i64, i64, i64, i64, vp, vp, vp]
+    lib.qvb8_kv_chunks.argtypes = [i64, i64]
+    lib.qvb8_kv_chunks.restype = i64
+    lib.qvb8_kv_range.argtypes = [vp, i32, i64, i64, i64, vp, i64, vp]
+    lib.qvb8_kv_check.argtypes = [vp, i32, i64, i64, i64, vp, i64, i32, i32, ctypes.c_double, vp, vp, vp, vp, vp]
+    lib.qvb8_kv_pack.argtypes = [vp, i32, i64, i64, i64, vp, vp, vp, vp, vp, vp]
+    lib.qvb8_kv_unpack.argtypes = [vp, i64, i64, i32, i64, vp]
+    lib.qvb8_kv_tiles.argtypes = [vp, i64, i64, vp, i64, vp]
     for name in SYMBOLS:
         getattr(lib, name)                           # every declared symbol must be exported
     _LIB = lib
@@ -121,6 +131,12 @@ class MmaLayout(ctypes.Structure):
 class MlpPlan(ctypes.Structure):
     """qvb8_mlp_plan of include/qvb8_amd.h."""
     _fields_ = [("hidden", ctypes.c_int64), ("inter", ctypes.c_int64), ("out_features", ctypes.c_int64), ("magic", ctypes.c_int64)]
+
+
+KV_MAX_HEADS = 32
+
+
+KV_HEAD = struct.Struct("=7Qqii")         # qvb8_kv_head of include/qvb8_amd.h
 
 
 class RCore(ctypes.Structure):
@@ -150,7 +166,17 @@ def ptr(t) -> int | None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream's handle on t's device, without making a Stream object of it (2.9 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device_of(t: torch.Tensor):
+    """`with torch.cuda.device(t.device)`, for nothing when that device is the current one already."""
+    index = t.get_device()
+    return _HERE if index == torch._C._cuda_getDevice() else torch.cuda.device(index)
 
 
 def require_cuda(*ts):

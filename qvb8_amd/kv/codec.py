@@ -3,15 +3,19 @@ segment of one kv head, one (min_s, tau_s) per channel,
 
     id = round((x - min_c) / step_c),  step_c = (max_c - min_c) / (2^B - 1),  recon = min_c + id * step_c,
 
-no escapes (minimum and maximum cover every value).  The encoder runs as torch ops on the tensor's device; the ids are
-kept bit-packed, LSB first, row-major (codec.py:53-82), as the cache stores them between attention calls.
+no escapes (minimum and maximum cover every value).  On the GPU the encoder is three launches of the HIP library (four when
+a head's width has to rise), on the CPU torch ops; both give the same bits.  The ids are kept bit-packed, LSB first,
+row-major (codec.py:53-82), as the cache stores them between attention calls.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 
 import torch
+
+from qvb8_amd import _lib
 
 STEP_FLOOR = 1e-12
 MAX_BITS = 16
@@ -120,12 +124,72 @@ def _channel_grid(x, lo, span, widths):
     return torch.minimum(torch.round((x - lo) / step).clamp_(min=0), levels), step
 
 
+def _first_width(widest: float, bits: int, tau: float) -> int:
+    """The least width that puts half a step of the widest channel within tau, `bits` at least."""
+    return min(MAX_BITS, max(bits, math.ceil(math.log2(widest / (2.0 * tau) + 1.0)))) if widest > 0 else bits
+
+
+def _next_width(head: int, width: int, off: float, tau: float, orig_dtype) -> int:
+    if width >= MAX_BITS:
+        raise KVCertificateError(f"head {head}: at {MAX_BITS} bits the per-channel grid is still {off:.4g} off, "
+                                 f"tau = {tau:g} cannot be certified for values stored as {orig_dtype}")
+    return width + 1
+
+
+_KV_MAX_DIM = 2048                         # channels per head the kernels take
+_STORED_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+
+
+def _band_on_gpu(t, orig_dtype, bits: int, tau: float, certify: bool) -> list:
+    """band_kv_heads on the HIP library: ranges, widths with the error they leave (one host read; a head that still misses tau
+    is checked again one bit wider), then the ids at their final widths straight into their packed streams."""
+    heads, seq, dim = t.shape
+    x = t.detach()
+    x = (x if x.dtype in _STORED_DTYPES else x.to(torch.float32)).contiguous()
+    lib, dev, dt = _lib.load(), x.device, _lib.dtype_code(x.dtype)
+    certifying = bool(certify and tau > 0)
+    with _lib.on_device_of(x):
+        stream = _lib.stream_of(x)
+        chunks = lib.qvb8_kv_chunks(heads, seq)
+        partial = torch.empty(heads * chunks * 2 * dim, dtype=torch.float32, device=dev)
+        lo, span, step = torch.empty((3, heads, dim), dtype=torch.float32, device=dev).unbind(0)
+        # the kernel writes its report where the host reads it: pinned memory, no copy behind it
+        report = torch.empty((heads, 2 + chunks), dtype=torch.float32, pin_memory=True) if certifying else None
+        _lib._check(lib.qvb8_kv_range(x.data_ptr(), dt, heads, seq, dim, partial.data_ptr(), chunks, stream), lib)
+
+        def check(widths):
+            given = None if widths is None else bytes(widths)
+            _lib._check(lib.qvb8_kv_check(x.data_ptr(), dt, heads, seq, dim, partial.data_ptr(), chunks, _lib.dtype_code(orig_dtype), bits,
+                                          float(tau), given, lo.data_ptr(), span.data_ptr(), report.data_ptr() if certifying else None, stream), lib)
+            if not certifying:
+                return None
+            torch.cuda.current_stream().synchronize()
+            return torch.cat([report[:, :2], report[:, 2:].amax(1, keepdim=True)], 1).tolist()        # span, width, largest error
+
+        found = check(None)
+        widths = [bits] * heads
+        if certifying:
+            widths = [_first_width(r[0], bits, tau) for r in found]
+            if widths != [int(r[1]) for r in found]:         # a span on the edge of a power of two: the host's logarithm decides
+                found = check(widths)
+            while not all(r[2] <= tau for r in found):
+                widths = [w if r[2] <= tau else _next_width(i, w, r[2], tau, orig_dtype) for i, (w, r) in enumerate(zip(widths, found))]
+                found = check(widths)
+        packed = [torch.empty((seq * dim * w + 7) // 8, dtype=torch.uint8, device=dev) for w in widths]
+        where = (ctypes.c_void_p * heads)(*[p.data_ptr() for p in packed])
+        _lib._check(lib.qvb8_kv_pack(x.data_ptr(), dt, heads, seq, dim, lo.data_ptr(), span.data_ptr(), bytes(widths), step.data_ptr(), where, stream), lib)
+    return [BandedKV(packed[i], lo[i], step[i], widths[i], (seq, dim), orig_dtype, tau) for i in range(heads)]
+
+
 def band_kv_heads(t: torch.Tensor, orig_dtype: torch.dtype, bits: int, tau: float = 0.0, certify: bool = True) -> list:
     """(heads, seq, head_dim) -> one BandedKV per head (codec.py:175-241).  With certify and tau > 0, `bits` is a floor:
     a head's width rises (to 16 at most) until the decoder's own expression, rounded to `orig_dtype`, is within tau of
     every element; KVCertificateError when 16 bits do not reach it.  Heads are independent: only the heads that still
     miss tau are quantised again, one host read per round."""
     heads, seq, dim = t.shape
+    if t.is_cuda and 0 < heads <= _lib.KV_MAX_HEADS and seq > 0 and 0 < dim <= _KV_MAX_DIM and seq * dim < 1 << 31 and 1 <= bits <= MAX_BITS \
+            and orig_dtype in _STORED_DTYPES:
+        return _band_on_gpu(t, orig_dtype, bits, tau, certify)
     x = torch.nan_to_num(t.detach().to(torch.float32), nan=0.0, posinf=0.0, neginf=0.0)
     lo = x.amin(1, keepdim=True)
     span = x.amax(1, keepdim=True) - lo
@@ -134,8 +198,7 @@ def band_kv_heads(t: torch.Tensor, orig_dtype: torch.dtype, bits: int, tau: floa
     if certify and tau > 0:
         open_heads = list(range(heads))
         for i, widest in enumerate(span.amax((1, 2)).cpu().tolist()):     # first guess: half a step within tau
-            if widest > 0:
-                widths[i] = min(MAX_BITS, max(bits, math.ceil(math.log2(widest / (2.0 * tau) + 1.0))))
+            widths[i] = _first_width(widest, bits, tau)
     ids, step = _channel_grid(x, lo, span, widths)
     while open_heads:
         sel = torch.tensor(open_heads, device=x.device)
@@ -146,10 +209,7 @@ def band_kv_heads(t: torch.Tensor, orig_dtype: torch.dtype, bits: int, tau: floa
             break
         worst = dict(zip(sel.tolist(), miss))
         for i in open_heads:
-            if widths[i] >= MAX_BITS:
-                raise KVCertificateError(f"head {i}: at {MAX_BITS} bits the per-channel grid is still {worst[i]:.4g} off, "
-                                         f"tau = {tau:g} cannot be certified for values stored as {orig_dtype}")
-            widths[i] += 1
+            widths[i] = _next_width(i, widths[i], worst[i], tau, orig_dtype)
         sel = torch.tensor(open_heads, device=x.device)
         ids[sel], step[sel] = _channel_grid(x[sel], lo[sel], span[sel], [widths[i] for i in open_heads])
     return [BandedKV(pack_ids(ids[i].to(torch.int64).reshape(-1), widths[i]), lo[i, 0].contiguous(), step[i, 0].contiguous(),

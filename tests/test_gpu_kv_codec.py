@@ -1,0 +1,49 @@
+"""The banded KV codec's kernels against the same codec on the CPU (torch operations, pinned by the oracle): streams, constants
+and widths bit for bit, and the id layout built from them."""
+import pytest
+import torch
+
+from qvb8_amd.kv import codec as C
+from qvb8_amd.kv import fused_attn as FA
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _values(heads, seq, dim, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(heads, seq, dim, generator=g) * torch.exp(torch.randn(heads, 1, dim, generator=g)) + torch.randn(heads, 1, dim, generator=g)
+    x[:, :, dim // 2] = 0.75                                     # a constant channel
+    if seq > 3:
+        x[0, 1, 0], x[0, 2, 1], x[0, 3, 0] = float("nan"), float("inf"), float("-inf")
+    return x.to(dtype)
+
+
+# tau small enough for bf16 that the first width leaves a rounding too much and has to rise; none at all; and wide fp32 ids: the
+# widest channel spans about 72, so 16 bits reach 72 / 65535 / 2 = 5.5e-4 and a bound of 1e-3 is within them
+@pytest.mark.parametrize("heads,seq,dim,dtype,bits,tau", [
+    (1, 1, 8, torch.float32, 1, 0.0), (3, 17, 64, torch.bfloat16, 5, 0.03), (2, 70, 100, torch.float16, 6, 0.01), (5, 9, 33, torch.bfloat16, 7, 0.5),
+    (4, 513, 256, torch.bfloat16, 6, 0.25), (2, 1025, 128, torch.float32, 4, 0.001), (3, 31, 2048, torch.float16, 16, 0.0), (32, 40, 96, torch.bfloat16, 3, 0.1)])
+def test_bands_are_those_of_the_cpu_codec(heads, seq, dim, dtype, bits, tau):
+    x = _values(heads, seq, dim, dtype, seed=seq + dim)
+    if tau and dtype == torch.bfloat16:
+        x = x.clamp(-12, 12)                                     # what bf16 can certify
+    want = C.band_kv_heads(x, dtype, bits, tau=tau)
+    got = C.band_kv_heads(x.to(DEV), dtype, bits, tau=tau)
+    for w, g in zip(want, got):
+        assert g.bits == w.bits and g.orig_shape == w.orig_shape and g.orig_dtype == w.orig_dtype
+        for name in ("min_s", "tau_s", "packed"):
+            assert torch.equal(getattr(g, name).cpu(), getattr(w, name)), name
+    wide = any(b.bits > 8 for b in want)
+    want_lay = FA.layout_from_segments([want, want], [want, want], [seq, seq], "cpu", allow_wide=True)
+    got_lay = FA.layout_from_segments([got, got], [got, got], [seq, seq], DEV, allow_wide=True)
+    assert got_lay.ki.dtype == (torch.int16 if wide else torch.uint8)
+    for name in ("ki", "vi", "kmin", "kstep", "vmin", "vstep", "kc", "vc", "t_start", "t_len", "t_seg"):
+        assert torch.equal(getattr(got_lay, name).cpu(), getattr(want_lay, name)), name
+
+
+def test_a_bound_that_sixteen_bits_miss_is_refused():
+    x = torch.tensor([[[0.0], [1.1], [3e4]]])
+    for dev in ("cpu", DEV):
+        with pytest.raises(C.KVCertificateError):
+            C.band_kv_heads(x.to(dev), torch.float32, 6, tau=1e-9)
