@@ -363,6 +363,256 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
     }
 }
 
+// ---- many query rows (a prompt chunk, a wide draft): 128 rows per workgroup -----------------------------------------------
+// With hundreds of rows the products bound the work, and what has to be shared is the restored tile: 4 waves x 32 query
+// rows share one, in two LDS buffers (tile t is multiplied while tile t + 1 is restored; one barrier per tile).  The
+// products run transposed, S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_f16: a lane then holds the scores of ONE
+// query (column lane % 32), so
+//   * the softmax needs one exchange between the two halves of the wave and no LDS: a lane's sixteen scores per tile are
+//     its own, its running maximum and sum are scalars of the lane, and rescaling O is a multiply by a lane's own factor;
+//   * with K's rows read in the order `swap bits 2 and 3`, the scores a lane holds are of eight consecutive keys per half
+//     and 16-key step, which is the B operand of the second product as it stands: P never leaves the registers.
+// Q stays in registers (B operands), V is restored as [channel % 4][channel / 4][key]: a thread's four channels then lie a
+// plane apart and its 16-byte stores, 80 bytes from lane to lane, meet no bank twice; the operand reads are 80 bytes apart too.
+// O is rescaled only where a row's maximum has risen by more than 2^8 since the last time (p stays below 256, in fp16 as
+// exact as below 1); the true maximum is kept beside it and settled at the end.
+// Two workgroups per CU (78 KB of LDS, at most 256 registers): one restores while the other one's products run.
+// Bound by what a CU issues beside its products (restoring, exp2, conversions): 720 rows x 4 kv heads over 16001 keys of 256
+// channels 251.6 us in the row-block kernel (32 rows share a tile), 100.7 us here = 0.47 PFLOP/s; one workgroup per CU 133.  The
+// ids of tile t + 2 are asked for between the two products: asked for before the first one, the sixteen registers they come back to are
+// spilled away from Q (118 us against 133 for the whole call).
+constexpr int kWideRows = 128, kWaveRows = 32;
+constexpr int kWideFrom = 33;                                 // fewest rows that take it: fused_attn.py has the measurements
+constexpr int kVRow = kKeys + 8;                              // halfs per row of V in LDS
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef float f16_t __attribute__((ext_vector_type(16)));
+constexpr int krow_wide(int D) { return D + 8; }              // halfs per key of K in LDS
+constexpr size_t wide_lds(int D) { return (size_t)2 * kKeys * krow_wide(D) * 2 + (size_t)2 * D * kVRow * 2 + (size_t)4 * D * 4; }
+constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f, kRescaleFrom = 8.0f;
+
+// The lane's number, worked out anew where it is asked for: the addresses made from it then need no registers between their
+// uses (kept across the loop they are spilled, and waiting for a spilled one also waits for the ids in flight).
+__device__ __forceinline__ int lane_now() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+
+template <int D, typename T>
+__global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2) void attn_wide_kernel(const AttnArgs a) {
+    constexpr int CG = D / 4;                  // channel groups (four channels each) of a key
+    constexpr int KPT = kKeys * CG / kAttnThreads;            // consecutive keys a thread restores: 8 (D = 256) or 4
+    constexpr int KROW = krow_wide(D), NKS = D / 16, NF = D / 32, NFC = NF / 4;
+    using QD = Quad<T>;
+    using U = typename QD::type;
+    extern __shared__ __align__(16) unsigned char smem[];
+    _Float16* const Ks = reinterpret_cast<_Float16*>(smem);                     // [2][kKeys][KROW]
+    _Float16* const Vt = Ks + 2 * kKeys * KROW;                                 // [2][4][CG][kVRow]
+    float* const Cs = reinterpret_cast<float*>(Vt + 2 * D * kVRow);             // [4][D]: kmid, kstep, vmid, vstep of the segment
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n32 = lane & 31, hf = lane >> 5;
+    // Workgroups go to the XCDs in turn.  The row blocks of one (head, split) read the same ids: where the pairs divide by
+    // eight, a pair's row blocks go to one XCD one after the other and its L2 serves all but the first.
+    int h = blockIdx.x, sp = blockIdx.y, z = blockIdx.z;
+    {
+        const int nx = gridDim.x, nz = gridDim.z, pairs = nx * (int)gridDim.y;
+        if (nz > 1 && (pairs & 7) == 0) {
+            const int flat = h + nx * (sp + (int)gridDim.y * z), k = flat >> 3;
+            const int pair = (k / nz) * 8 + (flat & 7);
+            z = k % nz; h = pair % nx; sp = pair / nx;
+        }
+    }
+    const int row0 = z * kWideRows, wrow0 = row0 + wave * kWaveRows, myrow = wrow0 + n32;
+    const int per_wave = 64 / CG;                             // key groups a wave restores: 1 (D = 256) or 2
+    const bool row_ok = myrow < a.n_rows;
+    const bool wave_ok = wrow0 < a.n_rows;                                      // uniform
+
+    h8_t qb[NKS];
+    {
+        const int rr = row_ok ? myrow : 0;
+        const uint16_t* qp = a.q + (int64_t)(rr / a.G) * a.sq_r + (int64_t)(h * a.G + rr % a.G) * a.sq_h + 8 * hf;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const h4_t lo = *reinterpret_cast<const h4_t*>(qp + 16 * ks), hi = *reinterpret_cast<const h4_t*>(qp + 16 * ks + 4);
+            const h8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            qb[ks] = row_ok ? v : h8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+    }
+    const int qpos = a.q_pos0 + (row_ok ? myrow / a.G : 0);
+    const int wqmin = a.q_pos0 + wrow0 / a.G;                                   // of the wave's rows: first position,
+    const int wqmax = a.q_pos0 + (min(wrow0 + kWaveRows, a.n_rows) - 1) / a.G;  // last
+    const int qmax = a.q_pos0 + (min(row0 + kWideRows, a.n_rows) - 1) / a.G;    // last position any row of the workgroup sees
+
+    const int t0 = (int)min((int64_t)sp * a.tps, (int64_t)a.n_tiles), t1 = (int)min((int64_t)t0 + a.tps, (int64_t)a.n_tiles);
+    const uint32_t key_stride = (uint32_t)a.s_n * (uint32_t)sizeof(T);
+    const unsigned char* const kbytes = reinterpret_cast<const unsigned char*>(reinterpret_cast<const T*>(a.ki) + (int64_t)h * a.s_h);
+    const unsigned char* const vbytes = reinterpret_cast<const unsigned char*>(reinterpret_cast<const T*>(a.vi) + (int64_t)h * a.s_h);
+    U rk[KPT], rv[KPT];
+    // ids of tile t; a tile that is not wanted (past the split's end or behind the last visible position) re-reads key 0
+    auto fetch = [&](int t, TileRef& ref) __attribute__((always_inline)) {
+        tile_entry(a.ts, a.tl, a.tseg, min(t, t1 - 1), ref);
+        ref.ok = __builtin_amdgcn_readfirstlane((int)(t < t1 && ref.start <= qmax)) != 0;
+        const int start = ref.ok ? ref.start : 0, nlen = ref.ok ? ref.nlen : 1;
+        const int64_t tile_byte = (int64_t)start * a.s_n * (int64_t)sizeof(T);
+        const uint32_t last_off = (uint32_t)max(nlen - 1, 0) * key_stride;
+        const int ln = lane_now();
+        const uint32_t cg_off = (uint32_t)(4 * (ln % CG)) * (uint32_t)sizeof(T), key_off0 = (uint32_t)((wave * per_wave + ln / CG) * KPT) * key_stride;
+        const unsigned char* kb = kbytes + tile_byte;
+        const unsigned char* vb = vbytes + tile_byte;
+#pragma unroll
+        for (int j = 0; j < KPT; ++j) {
+            const uint32_t off = min(key_off0 + (uint32_t)j * key_stride, last_off) + cg_off;
+            rk[j] = *reinterpret_cast<const U*>(kb + off);
+            rv[j] = *reinterpret_cast<const U*>(vb + off);
+        }
+    };
+
+    int cur_seg = -1;
+    float kc = 0.f, vc = 0.f;
+    // the ids in the registers -> keys and values of LDS buffer `buf`
+    auto restore = [&](int buf, const TileRef& ref) __attribute__((always_inline)) {
+        const int ln = lane_now(), cg = ln % CG, key0 = (wave * per_wave + ln / CG) * KPT;
+        if (ref.seg != cur_seg) {
+            // a new segment: its constants for this thread's channels.  Threads of the same channels write the same values,
+            // all in the interval between two barriers in which this tile is restored; each reads back what it wrote.
+            const int64_t pb = ((int64_t)ref.seg * a.nhkv + h) * D + 4 * cg;
+            *reinterpret_cast<float4*>(Cs + 4 * cg) = *reinterpret_cast<const float4*>(a.kmid + pb);
+            *reinterpret_cast<float4*>(Cs + D + 4 * cg) = *reinterpret_cast<const float4*>(a.kstep + pb);
+            *reinterpret_cast<float4*>(Cs + 2 * D + 4 * cg) = *reinterpret_cast<const float4*>(a.vmid + pb);
+            *reinterpret_cast<float4*>(Cs + 3 * D + 4 * cg) = *reinterpret_cast<const float4*>(a.vstep + pb);
+            kc = a.kc[ref.seg * a.nhkv + h]; vc = a.vc[ref.seg * a.nhkv + h];
+            cur_seg = ref.seg;
+        }
+        {
+            const float4 mid = *reinterpret_cast<const float4*>(Cs + 4 * cg), st = *reinterpret_cast<const float4*>(Cs + D + 4 * cg);
+#pragma unroll
+            for (int j = 0; j < KPT; ++j) {
+                uint2 kv;
+                kv.x = restore_pair(st.x, QD::id(rk[j], 0) - kc, mid.x, st.y, QD::id(rk[j], 1) - kc, mid.y);
+                kv.y = restore_pair(st.z, QD::id(rk[j], 2) - kc, mid.z, st.w, QD::id(rk[j], 3) - kc, mid.w);
+                *reinterpret_cast<uint2*>(Ks + (buf * kKeys + key0 + j) * KROW + 4 * cg) = kv;
+            }
+        }
+        const float4 mid4 = *reinterpret_cast<const float4*>(Cs + 2 * D + 4 * cg), st4 = *reinterpret_cast<const float4*>(Cs + 3 * D + 4 * cg);
+        const float mid[4] = {mid4.x, mid4.y, mid4.z, mid4.w}, st[4] = {st4.x, st4.y, st4.z, st4.w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            uint32_t w[KPT / 2];
+#pragma unroll
+            for (int j = 0; j < KPT; j += 2) w[j / 2] = restore_pair(st[c], QD::id(rv[j], c) - vc, mid[c], st[c], QD::id(rv[j + 1], c) - vc, mid[c]);
+            if (ref.nlen != kKeys) {                          // keys past the tile's length: zero (0 * inf would poison the sums)
+#pragma unroll
+                for (int j = 0; j < KPT; j += 2) w[j / 2] &= (key0 + j < ref.nlen ? 0x0000FFFFu : 0u) | (key0 + j + 1 < ref.nlen ? 0xFFFF0000u : 0u);
+            }
+            _Float16* dst = Vt + ((buf * 4 + c) * CG + cg) * kVRow + key0;
+            if constexpr (KPT == 8) *reinterpret_cast<uint4*>(dst) = uint4{w[0], w[1], w[2], w[3]};
+            else *reinterpret_cast<uint2*>(dst) = uint2{w[0], w[1]};
+        }
+    };
+
+    float m_true = -INFINITY, m_ref = -INFINITY, l_run = 0.f;                    // in powers of two; l: this half's keys
+    f16_t acc[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[f][i] = 0.f;
+    const float to_log2 = a.scale * kLog2e;
+
+    // register i of a lane: the score of key 16 (i / 8) + 8 hf + i % 8
+    auto scores = [&](int buf, const TileRef& ref, h8_t (&p)[2]) __attribute__((always_inline)) {
+        f16_t s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.f;
+        const int ln = lane_now(), half8 = 8 * (ln >> 5);
+        const int key = (ln & 19) | ((ln & 4) << 1) | ((ln & 8) >> 1);                   // A row ln % 32 of S^T is this key of the tile
+        const _Float16* const ka = Ks + (buf * kKeys + key) * KROW + half8;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t*>(ka + 16 * ks), qb[ks], s, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] *= to_log2;
+        if (!(ref.nlen == kKeys && ref.start + kKeys - 1 <= wqmin)) {
+            const int seen = row_ok ? min(ref.nlen, qpos - ref.start + 1) - half8 : 0;      // keys of the tile this row sees
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = 16 * (i >> 3) + (i & 7) < seen ? s[i] : -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        m_true = fmaxf(m_true, mx);
+        const bool rises = mx > m_ref + kRescaleFrom;         // also the first visible key: m_ref is -inf
+        if (__builtin_amdgcn_ballot_w64(rises)) {
+            const float m_new = rises ? mx : m_ref;
+            const float alpha = m_ref == -INFINITY ? 0.f : (m_new == m_ref ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new));
+            m_ref = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[f][i] *= alpha;
+        }
+        const float m_safe = m_ref == -INFINITY ? 0.f : m_ref;
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+            const h2_t pp = {(_Float16)__builtin_amdgcn_exp2f(s[i] - m_safe), (_Float16)__builtin_amdgcn_exp2f(s[i + 1] - m_safe)};
+            l_run = __builtin_amdgcn_fdot2(pp, h2_t{(_Float16)1.f, (_Float16)1.f}, l_run, false);    // the rounded p, as the product sees it
+            p[i >> 3][i & 7] = pp[0];
+            p[i >> 3][(i & 7) + 1] = pp[1];
+        }
+    };
+    auto values = [&](int buf, const h8_t (&p)[2]) __attribute__((always_inline)) {
+        const int ln = lane_now();
+        const _Float16* const va = Vt + (buf * D + (ln & 31)) * kVRow + 8 * (ln >> 5);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+                acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t*>(va + 32 * f * kVRow + 16 * k), p[k], acc[f], 0, 0, 0);
+    };
+
+    if (t0 < t1) {
+        TileRef cur, next;
+        fetch(t0, cur);
+        if (cur.ok) restore(0, cur);
+        fetch(t0 + 1, next);
+        __syncthreads();
+        int buf = 0;
+        for (int t = t0; cur.ok; ++t) {
+            const TileRef now = cur;
+            cur = next;
+            if (cur.ok) restore(buf ^ 1, cur);
+            const bool mine = wave_ok && now.start <= wqmax;
+            h8_t p[2] = {};
+            if (mine) scores(buf, now, p);
+            fetch(t + 2, next);
+            __builtin_amdgcn_sched_barrier(0);
+            if (mine) values(buf, p);
+            __syncthreads();                                  // buffer buf ^ 1 is filled, buffer buf is free
+            buf ^= 1;
+        }
+    }
+    if (!row_ok) return;
+    // register i of fragment c NFC + fi: channel 4 (32 fi + 8 (i / 4) + 4 hf + i % 4) + c of the lane's row
+    const float settle = m_true == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_true);
+    const int ln = lane_now(), hf_e = ln >> 5;
+    const int64_t at = ((int64_t)sp * a.nhkv + h) * a.n_rows + wrow0 + (ln & 31);
+#pragma unroll
+    for (int fi = 0; fi < NFC; ++fi)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            *reinterpret_cast<float4*>(a.o + at * D + 4 * (32 * fi + 8 * (i >> 2) + 4 * hf_e + (i & 3))) =
+                make_float4(acc[fi][i] * settle, acc[NFC + fi][i] * settle, acc[2 * NFC + fi][i] * settle, acc[3 * NFC + fi][i] * settle);
+    const float l = (l_run + __shfl_xor(l_run, 32)) * settle;
+    if (hf_e == 0) {
+        a.m[at] = m_true == -INFINITY ? -INFINITY : m_true * kLn2;
+        a.l[at] = l;
+    }
+}
+
 // Splits -> the normalised result and the log-sum-exp.  One workgroup per (kv head, row, 16 channels): 64 groups of 4
 // threads share the splits (group g takes splits g, g + 64, ...), a thread holds four channels; the groups' maxima,
 // sums and partial results meet in LDS.  A thread has a few independent loads, so the launch costs a few trips to
@@ -407,12 +657,50 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
     }
 }
 
+// The same for many rows: a thread holds four channels of one row and takes the splits in ascending order.  (The kernel above
+// spreads the splits over a workgroup, for launches of few rows; with thousands of rows and a few splits most of its
+// threads have nothing to do: 2880 rows of 256 channels from 21 splits 58.7 us there, 16.5 us here.)  Taken from 65536 threads on.
+__global__ __launch_bounds__(256) void attn_combine_rows_kernel(const float* __restrict__ o, const float* __restrict__ m, const float* __restrict__ l,
+                                                                int n_splits, int nhkv, int n_rows, int D, int G,
+                                                                float* __restrict__ out, float* __restrict__ lse) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)nhkv * n_rows;
+    const int per_row = D / 4;
+    const int64_t hr = i / per_row;
+    if (hr >= stride) return;
+    const int ch = (int)(i - hr * per_row) * 4;
+    float top = -INFINITY;
+    for (int s = 0; s < n_splits; ++s) top = fmaxf(top, m[s * stride + hr]);
+    if (top == -INFINITY) top = 0.f;
+    float total = 0.f;
+    f4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int s = 0; s < n_splits; ++s) {
+        const float w = expf(m[s * stride + hr] - top);
+        total += (l ? l[s * stride + hr] : 1.f) * w;
+        acc += *reinterpret_cast<const f4_t*>(o + (s * stride + hr) * D + ch) * w;
+    }
+    const int h = (int)(hr / n_rows), r = (int)(hr - (int64_t)h * n_rows);
+    const int64_t dst = (int64_t)(r / G) * (nhkv * G) + h * G + r % G;
+    *reinterpret_cast<f4_t*>(out + dst * D + ch) = acc * (1.f / fmaxf(total, 1e-30f));
+    if (ch == 0) lse[dst] = total > 0.f ? top + logf(fmaxf(total, 1e-30f)) : -INFINITY;
+}
+
+template <int D, typename T>
+int launch_attn_wide(const AttnArgs& a, int64_t n_splits, hipStream_t s) {
+    if (int rc = host::raise_lds_limit<attn_wide_kernel<D, T>>(wide_lds(D), "qvb8_attn_fwd")) return rc;
+    const dim3 grid((unsigned)a.nhkv, (unsigned)n_splits, (unsigned)((a.n_rows + kWideRows - 1) / kWideRows));
+    if (grid.z > 65535u) return host::fail(-1, "qvb8_attn_fwd: %d rows are more than one launch takes", a.n_rows);
+    hipLaunchKernelGGL((attn_wide_kernel<D, T>), grid, dim3(kAttnThreads), wide_lds(D), s, a);
+    return host::check_launch("qvb8_attn_fwd");
+}
+
 template <int D, typename T>
 int launch_attn(const AttnArgs& a, int64_t n_splits, hipStream_t s) {
-    // up to 16 rows: one block per workgroup; up to 32: two; beyond: four with 128 channels, two with 256 (four blocks'
-    // accumulators and Q do not fit the registers there).  QVB8_ATTN_ROW_BLOCKS forces 1, 2 or 4.
+    // up to 16 rows: one block per workgroup; up to 32: two; beyond: the kernel of 128 rows.  QVB8_ATTN_ROW_BLOCKS forces this
+    // kernel with 1, 2 or 4 blocks (256 channels: at most 2, four blocks' accumulators and Q do not fit the registers).
     int rb = a.n_rows <= kRows ? 1 : a.n_rows <= 2 * kRows ? 2 : 4;
     const int forced = host::env_int("QVB8_ATTN_ROW_BLOCKS", 0);
+    if (forced == 0 && a.n_rows >= kWideFrom) return launch_attn_wide<D, T>(a, n_splits, s);
     if (forced == 1 || forced == 2 || forced == 4) rb = forced;
     if (D == 256 && rb > 2) rb = 2;
     const dim3 grid((unsigned)a.nhkv, (unsigned)n_splits, (unsigned)((a.n_rows + rb * kRows - 1) / (rb * kRows)));
@@ -482,6 +770,13 @@ extern "C" int qvb8_attn_combine(const float* o, const float* m, const float* l,
     if (!o || !m || !out || !lse) return host::fail(-1, "%s: null pointer", who);
     if (!aligned(o, 16) || !aligned(out, 16)) return host::fail(-1, "%s: o and out must be 16-byte aligned", who);
     if (n_kv_heads * n_rows > INT32_MAX || n_splits > INT32_MAX) return host::fail(-1, "%s: size beyond what one launch takes", who);
+    const int64_t quads = n_kv_heads * n_rows * (head_dim / 4);
+    if (quads >= 65536 && n_splits <= 64) {
+        if (quads > (int64_t)INT32_MAX * 256) return host::fail(-1, "%s: size beyond what one launch takes", who);
+        hipLaunchKernelGGL(attn_combine_rows_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
+                           o, m, l, (int)n_splits, (int)n_kv_heads, (int)n_rows, (int)head_dim, (int)G, out, lse);
+        return host::check_launch(who);
+    }
     hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)(n_kv_heads * n_rows), (unsigned)((head_dim + 15) / 16)), dim3(256), 0, static_cast<hipStream_t>(stream),
                        o, m, l, (int)n_splits, (int)n_kv_heads, (int)n_rows, (int)head_dim, (int)G, out, lse);
     return host::check_launch(who);

@@ -1,0 +1,47 @@
+"""Attention of many query rows over the banded KV cache (the kernel of 128 rows per workgroup) against the oracle, at the sizes
+where its tiles change: the fewest rows it takes, one row more than a wave and a workgroup hold, tokens cut across both, key
+tiles of one key and of none a row sees, segment changes, 16-bit ids, scores that keep rising (the lazy rescale) or jump."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import kv_attn_oracle as A
+from tests.test_gpu_kv_attn import DEV, check_split_outputs, run_fwd, to_device, vmax
+from tests.test_oracle_kv_attn import make_layout
+from qvb8_amd.kv import fused_attn as FA
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,Hkv,G,MQ,seg_len,q_pos0,bits,tps,amp", [
+    (256, 2, 6, 6, [33, 1, 70], 98, 6, 2, 1.0), (128, 1, 3, 11, [40], 5, 8, 1, 1.0), (256, 1, 8, 16, [300], 284, 7, 4, 1.0),
+    (128, 2, 1, 129, [200, 31], 102, 6, 3, 1.0), (256, 1, 6, 43, [500, 17], -3, 6, 100, 1.0), (128, 3, 8, 33, [64, 64, 3], 98, 11, 2, 1.0),
+    (256, 1, 4, 40, [130], 90, 10, 3, 1.0), (128, 4, 6, 24, [321], 297, 7, 2, 40.0), (256, 1, 5, 30, [257], 227, 6, 9, 40.0)])
+def test_wide_rows_match_the_oracle(D, Hkv, G, MQ, seg_len, q_pos0, bits, tps, amp):
+    lay = make_layout(D + MQ + G, seg_len, Hkv, D, bits=bits)
+    rng = np.random.default_rng(MQ)
+    q = (rng.normal(0, amp, (MQ, Hkv * G, D)) * D ** -0.5).astype(np.float16)
+    want = A.fwd_split(q, lay["ki"], lay["vi"], lay["kmid"], lay["kstep"], lay["vmid"], lay["vstep"], lay["kc"], lay["vc"],
+                       lay["ts"], lay["tl"], lay["tseg"], q_pos0, tps, 1.0, G)
+    dl = to_device(lay, wide=bits > 8, slack=MQ % 3)
+    got = run_fwd(lay, dl, torch.from_numpy(q).to(DEV), q_pos0, tps, G)
+    check_split_outputs(got, want, lay)
+    ref, ref_lse = A.combine(*want, MQ, G)
+    out, lse = (t.cpu().numpy() for t in FA.combine_splits(*[torch.from_numpy(t).to(DEV) for t in got], G))
+    assert np.all(np.abs(out - ref) <= 1e-3 * vmax(lay) + 1e-6)
+    assert np.array_equal(np.isneginf(lse), np.isneginf(ref_lse))
+    seen = np.isfinite(ref_lse)
+    assert np.all(np.abs(lse[seen] - ref_lse[seen]) <= 1e-3 * np.abs(ref_lse[seen]) + 1e-3)
+
+
+def test_combining_many_rows_is_combining_few():
+    """3 splits of 300 rows x 4 heads (a thread per four channels) against the CPU's combination, rows without a key among them."""
+    g = torch.Generator().manual_seed(2)
+    S, h, rows, d, G = 3, 4, 300, 256, 6
+    o, m = torch.randn(S, h, rows, d, generator=g), 3 * torch.randn(S, h, rows, generator=g)
+    l = torch.rand(S, h, rows, generator=g) + 0.5
+    m[0, 1], l[0, 1], o[0, 1] = -float("inf"), 0, 0
+    m[:, 2, 7:19], l[:, 2, 7:19], o[:, 2, 7:19] = -float("inf"), 0, 0
+    out, lse = FA.combine_splits(o.to(DEV), m.to(DEV), l.to(DEV), G)
+    ref, ref_lse = A.combine(o.numpy(), m.numpy(), l.numpy(), rows // G, G)
+    assert np.allclose(out.cpu().numpy(), ref, rtol=1e-5, atol=1e-5) and np.allclose(lse.cpu().numpy(), ref_lse, rtol=1e-5, atol=1e-5)
