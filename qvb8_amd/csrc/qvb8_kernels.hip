@@ -215,16 +215,33 @@ __global__ void __launch_bounds__(256) certify_kernel(const void* __restrict__ a
 // ===========================================================================================================
 // activation narrowing
 // ===========================================================================================================
-template <int DT>
-__global__ void __launch_bounds__(256) sat_half_kernel(const void* __restrict__ x, uint16_t* __restrict__ out, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = (uint16_t)sat_half_bits(load_as_f32<DT>(x, i));
-}
-
-template <int DT>
-__global__ void __launch_bounds__(256) scale_sat_half_kernel(const void* __restrict__ x, float scale, uint16_t* __restrict__ out, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = (uint16_t)sat_half_bits(load_as_f32<DT>(x, i) * scale);
+// Eight values a thread, as 16-byte loads and stores where both arrays start on 16 bytes (`vec`): bound by memory.  One value a
+// thread moved 2 bytes per request: 1999 x 12288 bf16 values (98 MB moved) 46.7 us, so 17.2 us = 5.7 TB/s.  SCALED: x is multiplied in fp32 first.
+template <int DT, bool SCALED>
+__global__ void __launch_bounds__(256) sat_half_kernel(const void* __restrict__ x, float scale, uint16_t* __restrict__ out, int64_t n, bool vec) {
+    const int64_t i = 8 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    auto narrow = [scale](float v) { return sat_half_bits(SCALED ? v * scale : v); };
+    if (vec && i + 8 <= n) {
+        float v[8];
+        if constexpr (DT == 0) {
+            const float4 a = reinterpret_cast<const float4*>((const float*)x + i)[0], b = reinterpret_cast<const float4*>((const float*)x + i)[1];
+            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        } else {
+            const uint4 a = *reinterpret_cast<const uint4*>((const uint16_t*)x + i);
+            const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const uint32_t bits = (w[k / 2] >> (16 * (k & 1))) & 0xFFFFu;
+                v[k] = DT == 1 ? f16_bits_to_f32(bits) : bf16_bits_to_f32(bits);
+            }
+        }
+        uint32_t o[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = narrow(v[2 * k]) | (narrow(v[2 * k + 1]) << 16);
+        *reinterpret_cast<uint4*>(out + i) = make_uint4(o[0], o[1], o[2], o[3]);
+    } else {
+        for (int64_t k = i; k < n && k < i + 8; ++k) out[k] = (uint16_t)narrow(load_as_f32<DT>(x, k));
+    }
 }
 
 // ===========================================================================================================
@@ -644,34 +661,29 @@ extern "C" int qvb8_certify(const void* restored, int restored_dtype, const void
     return host::check_launch("qvb8_certify");
 }
 
-extern "C" int qvb8_sat_half(const void* x, int x_dtype, int64_t n, void* out_f16, void* stream) {
-    if (x_dtype < 0 || x_dtype > 2 || n < 0) return host::fail(QVB8_ERR_ARG, "qvb8_sat_half: bad argument");
+template <bool SCALED>
+static int launch_sat_half(const char* who, const void* x, int x_dtype, int64_t n, float scale, void* out_f16, hipStream_t s) {
+    if (x_dtype < 0 || x_dtype > 2 || n < 0) return host::fail(QVB8_ERR_ARG, "%s: bad argument", who);
     if (n == 0) return QVB8_OK;
-    if (!x || !out_f16) return host::fail(QVB8_ERR_ARG, "qvb8_sat_half: null pointer");
-    const int64_t blocks = (n + 255) / 256;
-    if (blocks > 0x7fffffff) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_sat_half: too large");
-    hipStream_t s = (hipStream_t)stream;
+    if (!x || !out_f16) return host::fail(QVB8_ERR_ARG, "%s: null pointer", who);
+    const int64_t blocks = (n + 2047) / 2048;
+    if (blocks > 0x7fffffff / 8) return host::fail(QVB8_ERR_UNSUPPORTED, "%s: too large", who);
+    const bool vec = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out_f16)) & 15u) == 0;
+    const dim3 grid((unsigned)blocks), block(256);
     switch (x_dtype) {
-        case QVB8_F32: hipLaunchKernelGGL(sat_half_kernel<0>, dim3((unsigned)blocks), dim3(256), 0, s, x, (uint16_t*)out_f16, n); break;
-        case QVB8_F16: hipLaunchKernelGGL(sat_half_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, s, x, (uint16_t*)out_f16, n); break;
-        default: hipLaunchKernelGGL(sat_half_kernel<2>, dim3((unsigned)blocks), dim3(256), 0, s, x, (uint16_t*)out_f16, n); break;
+        case QVB8_F32: hipLaunchKernelGGL((sat_half_kernel<0, SCALED>), grid, block, 0, s, x, scale, (uint16_t*)out_f16, n, vec); break;
+        case QVB8_F16: hipLaunchKernelGGL((sat_half_kernel<1, SCALED>), grid, block, 0, s, x, scale, (uint16_t*)out_f16, n, vec); break;
+        default: hipLaunchKernelGGL((sat_half_kernel<2, SCALED>), grid, block, 0, s, x, scale, (uint16_t*)out_f16, n, vec); break;
     }
-    return host::check_launch("qvb8_sat_half");
+    return host::check_launch(who);
+}
+
+extern "C" int qvb8_sat_half(const void* x, int x_dtype, int64_t n, void* out_f16, void* stream) {
+    return launch_sat_half<false>("qvb8_sat_half", x, x_dtype, n, 1.f, out_f16, (hipStream_t)stream);
 }
 
 extern "C" int qvb8_scale_sat_half(const void* x, int x_dtype, int64_t n, float scale, void* out_f16, void* stream) {
-    if (x_dtype < 0 || x_dtype > 2 || n < 0) return host::fail(QVB8_ERR_ARG, "qvb8_scale_sat_half: bad argument");
-    if (n == 0) return QVB8_OK;
-    if (!x || !out_f16) return host::fail(QVB8_ERR_ARG, "qvb8_scale_sat_half: null pointer");
-    const int64_t blocks = (n + 255) / 256;
-    if (blocks > 0x7fffffff) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_scale_sat_half: too large");
-    hipStream_t s = (hipStream_t)stream;
-    switch (x_dtype) {
-        case QVB8_F32: hipLaunchKernelGGL(scale_sat_half_kernel<0>, dim3((unsigned)blocks), dim3(256), 0, s, x, scale, (uint16_t*)out_f16, n); break;
-        case QVB8_F16: hipLaunchKernelGGL(scale_sat_half_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, s, x, scale, (uint16_t*)out_f16, n); break;
-        default: hipLaunchKernelGGL(scale_sat_half_kernel<2>, dim3((unsigned)blocks), dim3(256), 0, s, x, scale, (uint16_t*)out_f16, n); break;
-    }
-    return host::check_launch("qvb8_scale_sat_half");
+    return launch_sat_half<true>("qvb8_scale_sat_half", x, x_dtype, n, scale, out_f16, (hipStream_t)stream);
 }
 
 // ---- GEMV launch plan --------------------------------------------------------------------------------------

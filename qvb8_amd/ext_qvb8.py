@@ -44,7 +44,7 @@ def _check_escapes(esc_idx, esc_vals):
     return n
 
 
-def _decode_to(code, dtype, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals):
+def _decode_to(code, dtype, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo=None):
     lib = _lib.load()
     Q = _check_pack(ids, min_s, row_nbits, row_bit_off, tau_s)
     n_esc = _check_escapes(esc_idx, esc_vals)
@@ -53,22 +53,28 @@ def _decode_to(code, dtype, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_id
     with torch.cuda.device(ids.device):
         out = torch.empty((Q, int(P)), dtype=dtype, device=ids.device)
         st = _lib.stream_of(ids)
-        _lib._check(lib.qvb8_decode(_lib.ptr(ids), ids.numel(), _lib.ptr(min_s), _lib.ptr(tau_s), _lib.ptr(row_nbits),
-                                    _lib.ptr(row_bit_off), Q, int(P), code, _lib.ptr(out), st), lib)
+        if rowinfo is not None:
+            if rowinfo.dtype != torch.int64 or rowinfo.numel() * 8 != lib.qvb8_mma_rowinfo_bytes(Q) or not rowinfo.is_cuda:
+                raise RuntimeError("rowinfo must be the int64 GPU tensor mma_prepare returned")
+            _lib._check(lib.qvb8_decode_tiles(_lib.ptr(ids), ids.numel(), rowinfo.contiguous().data_ptr(), Q, int(P), code, _lib.ptr(out), st), lib)
+        else:
+            _lib._check(lib.qvb8_decode(_lib.ptr(ids), ids.numel(), _lib.ptr(min_s), _lib.ptr(tau_s), _lib.ptr(row_nbits),
+                                        _lib.ptr(row_bit_off), Q, int(P), code, _lib.ptr(out), st), lib)
         if n_esc:
             ei, ev = esc_idx.contiguous(), esc_vals.contiguous()
             _lib._check(lib.qvb8_scatter_escapes(_lib.ptr(out), code, out.numel(), _lib.ptr(ei), _lib.ptr(ev), n_esc, st), lib)
     return out
 
 
-def decode(ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals):
-    """Dense (Q, P) fp16 weight: fp16(fma(id, tau_s, min_s)), escapes written over it."""
-    return _decode_to(_lib.F16, torch.float16, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals)
+def decode(ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo=None):
+    """Dense (Q, P) fp16 weight: fp16(fma(id, tau_s, min_s)), escapes written over it.  `rowinfo` (mma_prepare's, of these
+    rows): the same values read tile by tile, for rows stored in planes."""
+    return _decode_to(_lib.F16, torch.float16, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo)
 
 
-def decode_bf16(ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals):
+def decode_bf16(ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo=None):
     """Dense (Q, P) bf16 weight, the band value rounded once to bf16."""
-    return _decode_to(_lib.BF16, torch.bfloat16, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals)
+    return _decode_to(_lib.BF16, torch.bfloat16, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo)
 
 
 def decode_f32(ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals):
@@ -534,21 +540,21 @@ def mma_multi(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
     return mma_tiles(Xk, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, perm, saturate=True)
 
 
-def _forward(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, out_half):
+def _forward(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, out_half, rowinfo=None):
     M = 1 if X.dim() == 1 else X.shape[0]
     if M <= 8:
         return gemv_multi(X.reshape(M, int(P)), ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals)
     # M > 8: certified fp16 weight once, then a library GEMM with fp32 accumulate
-    W = decode(ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals)
+    W = decode(ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo)
     Xh = saturating_half(X)
     if out_half:
         return torch.mm(Xh, W.t())
     return torch.mm(Xh, W.t(), out_dtype=torch.float32)
 
 
-def forward(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals):
-    """Any M.  M <= 8: fused GEMV, fp32 (M, Q).  M > 8: fp16 restore + GEMM, fp32 result."""
-    return _forward(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, False)
+def forward(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo=None):
+    """Any M.  M <= 8: fused GEMV, fp32 (M, Q).  M > 8: fp16 restore + GEMM, fp32 result.  `rowinfo`: as decode's."""
+    return _forward(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, False, rowinfo)
 
 
 def forward_half(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals):

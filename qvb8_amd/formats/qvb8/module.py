@@ -350,18 +350,21 @@ class QVBandLinearV8(nn.Module):
             y = ext.gemv_multi(xk, self.ids, self.min_s, self.nbits, self.bit_off, self.in_features, self.tau_s,
                                self.esc_idx, self.esc_vals)
             return self._finish(y, orig, out_dtype)
+        # a weight whose rows lie in planes is restored tile by tile, through the row records built with them
+        built = self.__dict__.get("_mma_cache")
+        rowinfo = built[1] if built and self._planes else None
         if xk.dtype == torch.bfloat16 and self.bf16_gemm and self.bf16_certified:
             W = ext.decode_bf16(self.ids, self.min_s, self.nbits, self.bit_off, self.in_features, self.tau_s,
-                                self.esc_idx_bf16, self.esc_vals_bf16)
+                                self.esc_idx_bf16, self.esc_vals_bf16, rowinfo)
             b = None if self.bias is None else self.bias.to(torch.bfloat16)
             return F.linear(xk, W, b).reshape(*orig[:-1], self.out_features)
         if xk.dtype == torch.float16:
             W = ext.decode(self.ids, self.min_s, self.nbits, self.bit_off, self.in_features, self.tau_s,
-                           self.esc_idx, self.esc_vals)
+                           self.esc_idx, self.esc_vals, rowinfo)
             b16 = None if self.bias is None else self.bias.to(torch.float16)
             return F.linear(xk, W, b16).reshape(*orig[:-1], self.out_features)
         y = ext.forward(xk, self.ids, self.min_s, self.nbits, self.bit_off, self.in_features, self.tau_s,
-                        self.esc_idx, self.esc_vals)
+                        self.esc_idx, self.esc_vals, rowinfo)
         return self._finish(y, orig, out_dtype)
 
 
