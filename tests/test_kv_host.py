@@ -102,3 +102,22 @@ def test_take_rows_and_unband_keep_every_value():
     with pytest.raises(ValueError):
         heads[0].take_rows(torch.tensor([30]))
     assert C.unband_kv_4d([], 1, 2).shape == (1, 2, 0, 0)
+
+
+def test_only_whole_heads_go_to_the_unpacking_kernel():
+    """The kernel reads seq * dim * bits bits and dim constants without looking at lengths: a head that holds fewer, or in
+    another type, must not reach it (the general path refuses a short stream)."""
+    import dataclasses
+    import types
+    g = torch.Generator().manual_seed(3)
+    bk = C.band_kv_heads(torch.randn(1, 40, 32, generator=g), torch.float32, 6)[0]
+    here = types.SimpleNamespace(index=-1)                       # what get_device() says of a CPU tensor
+    reads = lambda **change: FA._kernel_reads(dataclasses.replace(bk, **change), 40, 32, here)       # noqa: E731
+    assert reads()
+    assert not reads(packed=bk.packed[:-1].clone()) and not reads(bits=7) and not reads(bits=0)
+    assert not reads(packed=bk.packed.to(torch.int32)) and not reads(packed=torch.cat([bk.packed] * 2)[::2])
+    assert not reads(min_s=bk.min_s[:-1].clone()) and not reads(tau_s=bk.tau_s.double()) and not reads(tau_s=bk.tau_s[:1].expand(32))
+    assert not FA._kernel_reads(bk, 41, 32, here) and not FA._kernel_reads(bk, 40, 33, here)
+    short = dataclasses.replace(bk, packed=bk.packed[:-1].clone())
+    with pytest.raises(RuntimeError):
+        FA.layout_from_segments([[short]], [[bk]], [40], "cpu")
