@@ -1172,7 +1172,7 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
         if (int rc = launch_moe_walk<true, false>(wa, dn_regular, slots, tokens, s)) return rc;
         return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
     }
-    if (tokens > 16 && moe_group_shapes_ok(P_up, Q_dn, P_dn)) {
+    if (tokens > 16 && (reinterpret_cast<uintptr_t>(X) & 15u) == 0 && moe_group_shapes_ok(P_up, Q_dn, P_dn)) {
         MoeGroupArgs ga;
         ga.X = X; ga.plan = pl; ga.ids = up_ids; ga.ids_bytes = up_ids_bytes;
         ga.min_s = up_min; ga.tau_s = up_tau; ga.nbits = up_nb; ga.bit_off = up_off; ga.out = H;

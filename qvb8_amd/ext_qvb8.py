@@ -581,6 +581,8 @@ def _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids
             raise RuntimeError(f"moe: expected {dt}, got {t.dtype}")
     T, k, E = X.shape[0], idx.shape[1], up_min.shape[0]
     Xc, idxc, wc = X.contiguous(), idx.contiguous(), w.contiguous()
+    if Xc.data_ptr() % 16:                      # a view into the middle of a buffer: the kernels load 16 bytes of a row at a time
+        Xc = Xc.clone()
     tens = [t.contiguous() for t in (up_ids, up_min, up_tau, up_nb, up_off, dn_ids, dn_min, dn_tau, dn_nb, dn_off)]
     with torch.cuda.device(Xc.device):
         out = torch.empty((T, int(Qdn)), dtype=Xc.dtype, device=Xc.device)

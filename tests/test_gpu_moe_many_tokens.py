@@ -36,3 +36,18 @@ def test_many_tokens(T, pairs, hidden, inter, gated, dtype):
     bad = args[1].clone()
     bad[3, 1] = E
     assert bool(torch.isnan(fn(args[0], bad, *args[2:]).float()).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_tokens_that_start_off_a_16_byte_line(dtype):
+    """Activations that are a view one element into a buffer: the same bits as from a buffer of their own."""
+    E, k, T, hidden, inter = 3, 2, 37, 256, 128
+    up, _ = _hand_made_stack(E, 2 * inter, hidden, [6, 7, 5, 8], seed=4)
+    dn, _ = _hand_made_stack(E, hidden, inter, [5, 6], seed=8)
+    g = torch.Generator().manual_seed(1)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).to(DEV)
+    w = torch.rand(T, k, generator=g).to(DEV)
+    buf = torch.randn(T * hidden + 1, generator=g).to(dtype).to(DEV)
+    x = buf[1:].view(T, hidden)
+    rest = (idx, w, *up, 2 * inter, hidden, *dn, hidden, inter)
+    assert torch.equal(ext.moe_experts(x, *rest), ext.moe_experts(x.clone(), *rest))
