@@ -374,8 +374,10 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
 //     and 16-key step, which is the B operand of the second product as it stands: P never leaves the registers.
 // Q stays in registers (B operands), V is restored as [channel % 4][channel / 4][key]: a thread's four channels then lie a
 // plane apart and its 16-byte stores, 80 bytes from lane to lane, meet no bank twice; the operand reads are 80 bytes apart too.
-// O is rescaled only where a row's maximum has risen by more than 2^8 since the last time (p stays below 256, in fp16 as
-// exact as below 1); the true maximum is kept beside it and settled at the end.
+// O is rescaled whenever a row's maximum rises, as in the row-block kernel: p is then rounded to fp16 with the row's largest at
+// 1, and the keys that matter most lie just below it, where fp16 is finest for their size.  (A reference that lags behind
+// the maximum by up to 2^8 saves the multiplications but puts them anywhere in their binade: 1 .. 2.5 % more error against
+// 64 bits over 33 .. 1024 rows.)
 // Two workgroups per CU (78 KB of LDS, at most 256 registers): one restores while the other one's products run.
 // Bound by what a CU issues beside its products (restoring, exp2, conversions): 720 rows x 4 kv heads over 16001 keys of 256
 // channels 251.6 us in the row-block kernel (32 rows share a tile), 100.7 us here = 0.47 PFLOP/s; one workgroup per CU 133.  The
@@ -389,7 +391,7 @@ typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef float f16_t __attribute__((ext_vector_type(16)));
 constexpr int krow_wide(int D) { return D + 8; }              // halfs per key of K in LDS
 constexpr size_t wide_lds(int D) { return (size_t)2 * kKeys * krow_wide(D) * 2 + (size_t)2 * D * kVRow * 2 + (size_t)4 * D * 4; }
-constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f, kRescaleFrom = 8.0f;
+constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
 
 // The lane's number, worked out anew where it is asked for: the addresses made from it then need no registers between their
 // uses (kept across the loop they are spilled, and waiting for a spilled one also waits for the ids in flight).
@@ -513,7 +515,7 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
         }
     };
 
-    float m_true = -INFINITY, m_ref = -INFINITY, l_run = 0.f;                    // in powers of two; l: this half's keys
+    float m_run = -INFINITY, l_run = 0.f;                    // m: in powers of two; l: this half's keys
     f16_t acc[NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f)
@@ -543,19 +545,17 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
 #pragma unroll
         for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        m_true = fmaxf(m_true, mx);
-        const bool rises = mx > m_ref + kRescaleFrom;         // also the first visible key: m_ref is -inf
+        const bool rises = mx > m_run;                        // also the first visible key: m_run is -inf
         if (__builtin_amdgcn_ballot_w64(rises)) {
-            const float m_new = rises ? mx : m_ref;
-            const float alpha = m_ref == -INFINITY ? 0.f : (m_new == m_ref ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new));
-            m_ref = m_new;
+            const float alpha = rises ? (m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - mx)) : 1.f;
+            m_run = rises ? mx : m_run;
             l_run *= alpha;
 #pragma unroll
             for (int f = 0; f < NF; ++f)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[f][i] *= alpha;
         }
-        const float m_safe = m_ref == -INFINITY ? 0.f : m_ref;
+        const float m_safe = m_run == -INFINITY ? 0.f : m_run;
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
             const h2_t pp = {(_Float16)__builtin_amdgcn_exp2f(s[i] - m_safe), (_Float16)__builtin_amdgcn_exp2f(s[i + 1] - m_safe)};
@@ -597,7 +597,6 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
     }
     if (!row_ok) return;
     // register i of fragment c NFC + fi: channel 4 (32 fi + 8 (i / 4) + 4 hf + i % 4) + c of the lane's row
-    const float settle = m_true == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_true);
     const int ln = lane_now(), hf_e = ln >> 5;
     const int64_t at = ((int64_t)sp * a.nhkv + h) * a.n_rows + wrow0 + (ln & 31);
 #pragma unroll
@@ -605,10 +604,10 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
             *reinterpret_cast<float4*>(a.o + at * D + 4 * (32 * fi + 8 * (i >> 2) + 4 * hf_e + (i & 3))) =
-                make_float4(acc[fi][i] * settle, acc[NFC + fi][i] * settle, acc[2 * NFC + fi][i] * settle, acc[3 * NFC + fi][i] * settle);
-    const float l = (l_run + __shfl_xor(l_run, 32)) * settle;
+                make_float4(acc[fi][i], acc[NFC + fi][i], acc[2 * NFC + fi][i], acc[3 * NFC + fi][i]);
+    const float l = l_run + __shfl_xor(l_run, 32);
     if (hf_e == 0) {
-        a.m[at] = m_true == -INFINITY ? -INFINITY : m_true * kLn2;
+        a.m[at] = m_run == -INFINITY ? -INFINITY : m_run * kLn2;
         a.l[at] = l;
     }
 }

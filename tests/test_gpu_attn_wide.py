@@ -45,3 +45,31 @@ def test_combining_many_rows_is_combining_few():
     out, lse = FA.combine_splits(o.to(DEV), m.to(DEV), l.to(DEV), G)
     ref, ref_lse = A.combine(o.numpy(), m.numpy(), l.numpy(), rows // G, G)
     assert np.allclose(out.cpu().numpy(), ref, rtol=1e-5, atol=1e-5) and np.allclose(lse.cpu().numpy(), ref_lse, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("D,Hkv,G,MQ,n,bits", [(256, 2, 6, 40, 4000, 7), (128, 2, 8, 32, 3000, 6), (256, 1, 6, 6, 2500, 10)])
+def test_no_further_from_64_bits_than_the_row_block_kernel(D, Hkv, G, MQ, n, bits, monkeypatch):
+    """One long split, so that the running maximum keeps rising.  Both kernels round keys, values and probabilities to fp16 and
+    sum in fp32; with every probability rounded relative to the same running maximum their errors (5.6e-4 here) differ by the fp32
+    order of sums only, 1e-6 of the result = 2e-3 of the error at most.  A maximum that lags behind costs 1 .. 2.5 % of it."""
+    lay = make_layout(7 * D + MQ, [n], Hkv, D, bits=bits)
+    rng = np.random.default_rng(n)
+    q = (rng.normal(0, 1, (MQ, Hkv * G, D)) * D ** -0.5).astype(np.float16)
+    dl = to_device(lay, wide=bits > 8)
+    K, V = ((lay[m][0][None].astype(np.float64) + lay[s][0][None] * (lay[i].astype(np.float64) - lay[c][0][None, :, None]))
+            for i, m, s, c in (("ki", "kmid", "kstep", "kc"), ("vi", "vmid", "vstep", "vc")))
+    exact = np.empty((MQ, Hkv * G, D))
+    for h in range(Hkv * G):
+        s = q[:, h].astype(np.float64) @ K[:, h // G].T
+        s[np.arange(n)[None] > n - MQ + np.arange(MQ)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        exact[:, h] = p @ V[:, h // G] / p.sum(1, keepdims=True)
+
+    def error():
+        got = run_fwd(lay, dl, torch.from_numpy(q).to(DEV), n - MQ, 1 << 20, G)
+        out, _ = FA.combine_splits(*[torch.from_numpy(t).to(DEV) for t in got], G)
+        return np.linalg.norm(out.cpu().numpy() - exact) / np.linalg.norm(exact)
+
+    wide = error()
+    monkeypatch.setenv("QVB8_ATTN_ROW_BLOCKS", "1")
+    assert wide <= 1.002 * error()
