@@ -7,6 +7,9 @@ import torch
 
 from oracle import qvb8_oracle as O
 from qvb8_amd import ext_qvb8 as ext
+from qvb8_amd.formats.qvb8 import pack as PK
+from qvb8_amd.formats.qvb8.backends_experts import stack_projection
+from qvb8_amd.formats.qvb8.module import QVBandLinearV8
 from tests.test_gpu_moe import _check, _hand_made_stack
 
 pytestmark = pytest.mark.gpu
@@ -51,3 +54,43 @@ def test_tokens_that_start_off_a_16_byte_line(dtype):
     x = buf[1:].view(T, hidden)
     rest = (idx, w, *up, 2 * inter, hidden, *dn, hidden, inter)
     assert torch.equal(ext.moe_experts(x, *rest), ext.moe_experts(x.clone(), *rest))
+
+
+@pytest.mark.parametrize("T,E,hidden,inter,gated", [(17, 4, 2048, 768, True), (64, 6, 1152, 512, True), (40, 3, 640, 896, False)])
+def test_no_further_from_64_bits_than_the_general_path(T, E, hidden, inter, gated, monkeypatch):
+    """fp32 activations that fp16 holds exactly and fp32 results: what is left is the arithmetic.  The general path multiplies
+    and adds in fp32; the matrix-core kernels have to be as exact on weights whose rows lie unevenly around zero in their width."""
+    k, Qup = 2, 2 * inter if gated else inter
+    up, dn = (_packed_stack(E, Q, P, seed) for Q, P, seed in ((Qup, hidden, 1), (hidden, inter, 2)))
+    g = torch.Generator().manual_seed(T)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)])
+    w = torch.rand(T, k, generator=g).half().float()
+    x = torch.randn(T, hidden, generator=g).half().float()
+    exact = torch.zeros(T, hidden, dtype=torch.float64)
+    for e in range(E):
+        t, c = (idx == e).nonzero(as_tuple=True)
+        h = x[t].double() @ up[1][e].T
+        h = torch.relu(h) ** 2 if not gated else h[:, :inter] * torch.sigmoid(h[:, :inter]) * h[:, inter:]
+        exact.index_add_(0, t, (h @ dn[1][e].T) * w[t, c, None].double())
+    fn = ext.moe_experts if gated else ext.moe_experts_relu2
+
+    def error():
+        out = fn(x.to(DEV), idx.to(DEV), w.to(DEV), *up[0], Qup, hidden, *dn[0], hidden, inter)
+        return float((out.cpu().double() - exact).norm() / exact.norm())
+
+    grouped = error()
+    monkeypatch.setenv("QVB8_MOE_GROUPED", "0")
+    assert grouped <= error()
+
+
+def _packed_stack(E, Q, P, seed):
+    """E packed experts of N(0.003, 0.02) weights (several widths, no row centred in its own) and what they stand for in 64 bits."""
+    gen = torch.Generator().manual_seed(seed)
+    enc = [PK.encode_tensor((0.02 * torch.randn(Q, P, generator=gen) + 0.003).to(torch.bfloat16).to(DEV), 2e-3) for _ in range(E)]
+    stk = stack_projection([QVBandLinearV8.from_encoded(e) for e in enc])
+    exact = []
+    for e in range(E):
+        row = [stk[n][e] for n in ("nbits", "bit_off", "min_s", "tau_s")]
+        ids = ext.decode_f32(stk["ids"], torch.zeros_like(row[2]), row[0], row[1], P, torch.ones_like(row[3]), *(enc[0][n] for n in ("esc_idx", "esc_vals")))
+        exact.append((ids.double() * row[3].double()[:, None] + row[2].double()[:, None]).cpu())
+    return tuple(stk[n] for n in ("ids", "min_s", "tau_s", "nbits", "bit_off")), exact
