@@ -260,7 +260,10 @@ enum qvb8_moe_act {
      * are then read id by id, as without the flag).  A stack for which the statement is false gives wrong results (never
      * an access outside the ids buffer). */
     QVB8_MOE_UP_REGULAR = 0x100,
-    QVB8_MOE_DOWN_REGULAR = 0x200
+    QVB8_MOE_DOWN_REGULAR = 0x200,
+    /* More than 16 tokens: an infinity among fp16 activations stays one.  Without the flag it becomes +-65504, as every value beyond
+     * fp16's range does in the other activation types (up to 16 tokens fp16 activations are always taken as they are). */
+    QVB8_MOE_KEEP_INF = 0x400
 };
 
 /* Bytes of workspace qvb8_moe_experts needs (routing plan + fp32 H (pairs, P_dn) + fp32 Yd (pairs, Q_dn)). */

@@ -161,6 +161,7 @@ struct MoeGemvArgs {
     int Q, P, topk, x_dtype, act;  // act: 0 gated silu, 1 relu2 (stage 0 only)
     int units;                     // output columns per pair: stage 0 gated Q/2, relu2 Q; stage 1 Q
     int units_per_block;
+    int keep_inf;                  // QVB8_MOE_KEEP_INF
     int x_rows;                    // activation rows a workgroup stages at a time: min(kMoeMB, tokens)
 };
 
@@ -282,7 +283,8 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
             for (int c = tid; c < a.P; c += blockDim.x) {
                 float v;
                 if constexpr (STAGE == 0) {
-                    const uint32_t hb = sat_half_bits(load_as_f32(a.X, (int64_t)(p / a.topk) * a.P + c, a.x_dtype));
+                    const int64_t at = (int64_t)(p / a.topk) * a.P + c;
+                    const uint32_t hb = a.keep_inf && a.x_dtype == QVB8_F16 ? reinterpret_cast<const uint16_t*>(a.X)[at] : sat_half_bits(load_as_f32(a.X, at, a.x_dtype));
                     v = f16_bits_to_f32(hb);
                     xs[(size_t)mb * a.P + c] = __builtin_bit_cast(XT, (uint16_t)hb);
                 } else {
@@ -1097,9 +1099,10 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
                                 const uint8_t* dn_nb, const int64_t* dn_off, int64_t Q_dn, int64_t P_dn,
                                 int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
     if (tokens < 0 || topk < 1 || n_experts < 1 || n_experts > 8192) return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: bad token / top-k / expert count");
-    if ((act & ~(QVB8_MOE_UP_REGULAR | QVB8_MOE_DOWN_REGULAR)) != 0 && (act & ~(QVB8_MOE_UP_REGULAR | QVB8_MOE_DOWN_REGULAR)) != 1)
-        return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: act must be 0 (gated SiLU) or 1 (ReLU squared), with the QVB8_MOE_*_REGULAR flags at most");
-    const bool up_regular = (act & QVB8_MOE_UP_REGULAR) != 0, dn_regular = (act & QVB8_MOE_DOWN_REGULAR) != 0;
+    constexpr int kActFlags = QVB8_MOE_UP_REGULAR | QVB8_MOE_DOWN_REGULAR | QVB8_MOE_KEEP_INF;
+    if ((act & ~kActFlags) != 0 && (act & ~kActFlags) != 1)
+        return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: act must be 0 (gated SiLU) or 1 (ReLU squared), with the QVB8_MOE_* flags at most");
+    const bool up_regular = (act & QVB8_MOE_UP_REGULAR) != 0, dn_regular = (act & QVB8_MOE_DOWN_REGULAR) != 0, keep_inf = (act & QVB8_MOE_KEEP_INF) != 0;
     act &= 0xFF;
     if (Q_up <= 0 || P_up <= 0 || Q_dn <= 0 || P_dn <= 0 || Q_up > 0x7fffffff || P_up > 0x7fffffff || Q_dn > 0x7fffffff || P_dn > 0x7fffffff)
         return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: bad shape");
@@ -1177,7 +1180,7 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
         ga.X = X; ga.plan = pl; ga.ids = up_ids; ga.ids_bytes = up_ids_bytes;
         ga.min_s = up_min; ga.tau_s = up_tau; ga.nbits = up_nb; ga.bit_off = up_off; ga.out = H;
         ga.E = (int)n_experts; ga.Q = (int)Q_up; ga.P = (int)P_up; ga.topk = (int)topk; ga.units = (int)P_dn; ga.gated = act == 0 ? 1 : 0;
-        ga.row_blocks = ga.items = 0;
+        ga.row_blocks = ga.items = 0; ga.keep_inf = keep_inf ? 1 : 0;
         if (int rc = launch_moe_group(false, x_dtype, ga, np, s)) return rc;
         ga.X = H; ga.ids = dn_ids; ga.ids_bytes = dn_ids_bytes;
         ga.min_s = dn_min; ga.tau_s = dn_tau; ga.nbits = dn_nb; ga.bit_off = dn_off; ga.out = Yd;
@@ -1189,7 +1192,7 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
     MoeGemvArgs a;
     a.X = X; a.ids = up_ids; a.ids_bytes = up_ids_bytes; a.min_s = up_min; a.tau_s = up_tau; a.nbits = up_nb; a.bit_off = up_off;
     a.out = H; a.plan = pl; a.Q = (int)Q_up; a.P = (int)P_up; a.topk = (int)topk; a.x_dtype = x_dtype; a.act = act;
-    a.units = (int)P_dn; a.units_per_block = 0; a.x_rows = (int)(tokens < kMoeMB ? tokens : kMoeMB);
+    a.units = (int)P_dn; a.keep_inf = keep_inf ? 1 : 0; a.units_per_block = 0; a.x_rows = (int)(tokens < kMoeMB ? tokens : kMoeMB);
     if (int rc = launch_moe_gemv(0, a, slots, s)) return rc;
     a.X = H; a.ids = dn_ids; a.ids_bytes = dn_ids_bytes; a.min_s = dn_min; a.tau_s = dn_tau; a.nbits = dn_nb; a.bit_off = dn_off;
     a.out = Yd; a.Q = (int)Q_dn; a.P = (int)P_dn; a.x_dtype = QVB8_F32; a.units = (int)Q_dn;

@@ -75,20 +75,23 @@ __device__ __forceinline__ Piece<XDT> load_piece(const void* row, int col) {
 __device__ __forceinline__ uint32_t pack_half2(_Float16 a, _Float16 b) {
     return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
 }
-// ... as fp16, narrowed like saturating_half
+// (by value: a bit cast straight from a vector's element reads the vector's first element with this compiler)
+__device__ __forceinline__ half2_t as_half2(uint32_t w) { return __builtin_bit_cast(half2_t, w); }
+// ... as fp16 within its finite range (NaN kept); `keep_inf`: fp16 as it is
 template <int XDT>
-__device__ __forceinline__ v4u_t narrow_piece(const Piece<XDT>& p) {
+__device__ __forceinline__ v4u_t narrow_piece(const Piece<XDT>& p, bool keep_inf) {
     v4u_t o;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        if constexpr (XDT == QVB8_F16) o[k] = p.v[0][k];
+        if constexpr (XDT == QVB8_F16) {
+            const half2_t top = {(_Float16)65504.0f, (_Float16)65504.0f}, h = as_half2(p.v[0][k]);
+            o[k] = keep_inf ? p.v[0][k] : __builtin_bit_cast(uint32_t, (half2_t)__builtin_elementwise_maximum(__builtin_elementwise_minimum(h, top), -top));
+        }
         else if constexpr (XDT == QVB8_BF16) o[k] = XIn<false, true>::pair(p.v[0][k]);
         else o[k] = sat_half_bits(__uint_as_float(p.v[k / 2][(2 * k) % 4])) | (sat_half_bits(__uint_as_float(p.v[k / 2][(2 * k + 1) % 4])) << 16);
     }
     return o;
 }
-// (by value: a bit cast straight from a vector's element reads the vector's first element with this compiler)
-__device__ __forceinline__ half2_t as_half2(uint32_t w) { return __builtin_bit_cast(half2_t, w); }
 __device__ __forceinline__ float sum_piece(const v4u_t& h, float s) {
     const half2_t one = {(_Float16)1.0f, (_Float16)1.0f};
 #pragma unroll
@@ -177,7 +180,7 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
                     *reinterpret_cast<v4u_t*>(to + L::plane + 2 * c) = lo;
                 }
             } else {
-                const v4u_t h = narrow_piece<XDT>(px[i]);
+                const v4u_t h = narrow_piece<XDT>(px[i], a.keep_inf != 0);
                 if (in) {
                     xsum = sum_piece(h, xsum);
                     *reinterpret_cast<v4u_t*>(to + 2 * c) = h;
@@ -314,7 +317,10 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
                 for (int c = lane; c < a.P; c += kWave) {
                     float x;
                     if constexpr (DOWN) x = reinterpret_cast<const float*>(a.X)[(size_t)p * a.P + c] * (1.0f / s_inv[tok]);
-                    else x = f16_bits_to_f32(sat_half_bits(load_as_f32<XDT>(a.X, (int64_t)(p / a.topk) * a.P + c)));
+                    else {
+                        x = load_as_f32<XDT>(a.X, (int64_t)(p / a.topk) * a.P + c);
+                        if (XDT != QVB8_F16 || !a.keep_inf) x = f16_bits_to_f32(sat_half_bits(x));
+                    }
                     part = __builtin_fmaf(x, (float)row_field(a.ids, off, nb, c, clamp_byte), part);
                 }
                 const float tot = wave_sum(part);

@@ -35,6 +35,7 @@ struct MoeGroupArgs {
     float* out;                    // up: H (pairs, units); down: Yd (pairs, Q)
     int E, Q, P, topk;
     int units, gated;              // up: outputs per expert; whether the rows come as (gate, up) halves
+    int keep_inf;                  // up: an infinity among fp16 activations stays one
     int row_blocks, items;         // set by the launcher
 };
 bool moe_group_shapes_ok(int64_t P_up, int64_t Q_dn, int64_t P_dn);

@@ -600,6 +600,7 @@ def _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids
 
 
 MOE_UP_REGULAR, MOE_DOWN_REGULAR = 0x100, 0x200      # qvb8_moe_act flags: one width per stack, rows at regular places
+MOE_KEEP_INF = 0x400                                 # ... an infinity among fp16 activations stays one (more than 16 tokens)
 
 
 def stack_is_regular(nbits, bit_off, P) -> bool:
@@ -614,10 +615,11 @@ def stack_is_regular(nbits, bit_off, P) -> bool:
 
 
 def moe_experts(X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn,
-                regular=(False, False)):
+                regular=(False, False), keep_inf=False):
     """Routed gated-SiLU expert stack on the stacked layout (reference: qvb8_cuda.cu:937-992); returns (tokens, Qdn)
-    in X's dtype.  `regular` = (up, down): the caller states that the stack is regular (stack_is_regular)."""
-    act = 0 | (MOE_UP_REGULAR if regular[0] else 0) | (MOE_DOWN_REGULAR if regular[1] else 0)
+    in X's dtype.  `regular` = (up, down): the caller states that the stack is regular (stack_is_regular).  `keep_inf`: fp16
+    activations beyond 16 tokens are taken as they are, infinities too (else they become +-65504)."""
+    act = 0 | (MOE_UP_REGULAR if regular[0] else 0) | (MOE_DOWN_REGULAR if regular[1] else 0) | (MOE_KEEP_INF if keep_inf else 0)
     return _moe(act, X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn)
 
 

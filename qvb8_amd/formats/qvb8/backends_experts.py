@@ -152,7 +152,7 @@ class QVBandExpertsV8(nn.Module):
             return ext.moe_experts(hidden_states.contiguous(), top_k_index.contiguous(), top_k_weights.float(),
                                    g["ids"], g["min_s"], g["tau_s"], g["nbits"], g["bit_off"], g["Q"], g["P"],
                                    d["ids"], d["min_s"], d["tau_s"], d["nbits"], d["bit_off"], d["Q"], d["P"],
-                                   regular=(g["regular"], d["regular"]))
+                                   regular=(g["regular"], d["regular"]), keep_inf=n_tok > self.FUSED_MAX_TOKENS)
         return self._forward_loop(hidden_states, top_k_index, top_k_weights)
 
     def _forward_loop(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:

@@ -94,3 +94,22 @@ def _packed_stack(E, Q, P, seed):
         ids = ext.decode_f32(stk["ids"], torch.zeros_like(row[2]), row[0], row[1], P, torch.ones_like(row[3]), *(enc[0][n] for n in ("esc_idx", "esc_vals")))
         exact.append((ids.double() * row[3].double()[:, None] + row[2].double()[:, None]).cpu())
     return tuple(stk[n] for n in ("ids", "min_s", "tau_s", "nbits", "bit_off")), exact
+
+
+@pytest.mark.parametrize("T", [17, 40, 70])
+def test_infinities_among_fp16_activations(T):
+    """Narrowed to +-65504 like every value fp16 cannot hold (what O.moe_reference does); on request they stay, and only the
+    tokens that hold one are lost."""
+    E, k, hidden, inter = 3, 2, 256, 128
+    up, Wup = _hand_made_stack(E, 2 * inter, hidden, [6, 7, 5, 8, 11], seed=4)
+    dn, Wdn = _hand_made_stack(E, hidden, inter, [5, 6, 3], seed=8)
+    g = torch.Generator().manual_seed(T)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)])
+    w = torch.rand(T, k, generator=g)
+    x = (1e-3 * torch.randn(T, hidden, generator=g)).half()
+    x[3, 5], x[T - 1, 200] = float("inf"), -float("inf")
+    args = (x.to(DEV), idx.to(DEV), w.to(DEV), *up, 2 * inter, hidden, *dn, hidden, inter)
+    clamped = torch.equal(ext.moe_experts(*args), ext.moe_experts(x.clamp(-65504, 65504).to(DEV), *args[1:]))
+    assert clamped
+    kept = ext.moe_experts(*args, keep_inf=True).isfinite().all(1).cpu()
+    assert kept.tolist() == [t not in (3, T - 1) for t in range(T)]
