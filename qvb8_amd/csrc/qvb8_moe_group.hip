@@ -195,16 +195,13 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         GroupRow& q = g[t];
-        q.ok = row_in_bounds(off[t], q.nb, a.P, a.ids_bytes);
-        const bool plane = off_is_plane(off[t]);
-        const uint64_t base = (uint64_t)((off[t] & kOffBitsMask) >> 3);
+        q.ok = !off_is_plane(off[t]) && row_in_bounds(off[t], q.nb, a.P, a.ids_bytes);        // stacks hold rows back to back only
         const uint32_t nb = (uint32_t)q.nb;
         q.sliced = q.ok && nb >= 4 && nb <= 8 && (off[t] & 31) == 0;
         if (q.sliced) {
-            const uint32_t entry = (uint32_t)off_plane_row(off[t]) + 16u * (uint32_t)kg;
-            q.at = base + (plane ? entry * 16u : (uint32_t)kg * 4u * nb);
-            q.tail = plane ? 1008u + (entry + 1u) * 4u * (nb - 4u) - entry * 16u : 4u * (nb - 4u);
-            q.stride = (plane ? 256u : 16u) * nb;
+            q.at = (uint64_t)(off[t] >> 3) + (uint32_t)kg * 4u * nb;
+            q.tail = 4u * (nb - 4u);
+            q.stride = 16u * nb;
         } else { q.at = 0; q.tail = 16; q.stride = 0; }
         const float zero = rintf(-a.min_s[row_at + row0[t]] / a.tau_s[row_at + row0[t]]);
         const int c = q.sliced ? (int)fminf(fmaxf(zero, 0.f), (float)((1 << q.nb) - 1)) : 0;          // (NaN: 0)
@@ -321,7 +318,7 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
                         x = load_as_f32<XDT>(a.X, (int64_t)(p / a.topk) * a.P + c);
                         if (XDT != QVB8_F16 || !a.keep_inf) x = f16_bits_to_f32(sat_half_bits(x));
                     }
-                    part = __builtin_fmaf(x, (float)row_field(a.ids, off, nb, c, clamp_byte), part);
+                    part = __builtin_fmaf(x, (float)load_field(a.ids, off + (int64_t)c * nb, nb, clamp_byte), part);
                 }
                 const float tot = wave_sum(part);
 #pragma unroll

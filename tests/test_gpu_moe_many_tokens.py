@@ -113,3 +113,18 @@ def test_infinities_among_fp16_activations(T):
     assert clamped
     kept = ext.moe_experts(*args, keep_inf=True).isfinite().all(1).cpu()
     assert kept.tolist() == [t not in (3, T - 1) for t in range(T)]
+
+
+@pytest.mark.parametrize("T", [17, 70])
+def test_rows_that_claim_to_lie_in_planes_are_nan(T):
+    """Stacks hold their rows back to back; a plane mark (bit 62 of the offset) puts a row outside the buffer on every path."""
+    E, k, hidden, inter = 4, 2, 256, 128
+    up, _ = _hand_made_stack(E, 2 * inter, hidden, [6] * 16 + [7, 5], seed=4)
+    dn, _ = _hand_made_stack(E, hidden, inter, [5, 6], seed=8)
+    g = torch.Generator().manual_seed(T)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)])
+    marked = up[4].clone()
+    marked[2, 5] |= 1 << 62
+    out = ext.moe_experts(torch.randn(T, hidden, generator=g).to(DEV), idx.to(DEV), torch.rand(T, k, generator=g).to(DEV), *up[:4], marked,
+                          2 * inter, hidden, *dn, hidden, inter)
+    assert torch.equal(out.isnan().all(1).cpu(), (idx == 2).any(1)) and torch.equal(out.isnan().any(1).cpu(), (idx == 2).any(1))
