@@ -53,9 +53,9 @@ enum qvb8_status {
 /* Library identification: ABI version, bumped on any signature change or new entry point (3: row lookup, attention over
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
  * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*;
- * 9: qvb8_decode_tiles).  A binding compares the loaded library's answer
+ * 9: qvb8_decode_tiles; 10: its constants).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
-#define QVB8_ABI_VERSION 9
+#define QVB8_ABI_VERSION 10
 int qvb8_abi_version(void);
 /* Message of the calling thread's most recent failure ("" if none). Valid until that thread's next call. */
 const char* qvb8_last_error(void);
@@ -148,10 +148,11 @@ enum qvb8_mma_flags {
 int64_t qvb8_mma_rowinfo_bytes(int64_t Q);
 int qvb8_mma_prepare(const uint8_t* nbits, const int64_t* bit_off, const float* tau_s, const float* min_s,
                      const int32_t* perm, int64_t Q, int64_t P, int64_t ids_bytes, uint64_t* rowinfo, void* stream);
-/* The dense (Q, P) weight as fp16 or bf16, every row through its record of qvb8_mma_prepare (bit for bit what qvb8_decode
- * gives; escapes are not written): for rows stored in tiles, which it reads and writes in whole runs.  P % 128 == 0. */
-int qvb8_decode_tiles(const uint8_t* ids, int64_t ids_bytes, const uint64_t* rowinfo, int64_t Q, int64_t P, int out_dtype,
-                      void* out, void* stream);
+/* The dense (Q, P) weight as fp16 or bf16 (bit for bit what qvb8_decode gives; escapes are not written): for rows stored in
+ * tiles, which it reads and writes in whole runs.  `rowinfo` (qvb8_mma_prepare) gives the order of the rows and nothing
+ * else: widths, offsets and constants are read from the four row vectors.  P % 128 == 0. */
+int qvb8_decode_tiles(const uint8_t* ids, int64_t ids_bytes, const float* min_s, const float* tau_s, const uint8_t* nbits,
+                      const int64_t* bit_off, const uint64_t* rowinfo, int64_t Q, int64_t P, int out_dtype, void* out, void* stream);
 
 /* Optional description of a pack whose rows are STORED in tile order from bit 0 of `ids`, back to back, one run per
  * width (what a loader gets by copying the rows once, sorted by width): positions [first_pos[c], first_pos[c+1]) have

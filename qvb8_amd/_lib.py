@@ -14,7 +14,7 @@ import torch
 from .common.errors import NativeLibraryError
 
 _LIB = None
-EXPECTED_ABI = 9            # QVB8_ABI_VERSION of include/qvb8_amd.h that the argument lists below were written for
+EXPECTED_ABI = 10           # QVB8_ABI_VERSION of include/qvb8_amd.h that the argument lists below were written for
 F32, F16, BF16 = 0, 1, 2
 _DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
@@ -103,7 +103,7 @@ def load(build_if_missing: bool = True):
     lib.qvb8r_gemv.argtypes = [vp, i32, i64, vp, i64, vp, vp, i64, vp]
     lib.qvb8r_walk_probe.argtypes = [vp, i64, vp, vp]
     lib.qvb8r_fix_escapes.argtypes = [vp, i32, i64, vp, vp, vp, vp, i64, vp, i64, i64, vp]
-    lib.qvb8_decode_tiles.argtypes = [vp, i64, vp, i64, i64, i32, vp, vp]
+    lib.qvb8_decode_tiles.argtypes = [vp, i64, vp, vp, vp, vp, vp, i64, i64, i32, vp, vp]
     lib.qvb8_attn_fwd.argtypes = ([vp, i64, i64, vp, vp, i32, i64, i64] + [vp] * 9 + [i64, vp, vp, vp] + [i64] * 6
                                   + [ctypes.c_double, i64, vp])
     lib.qvb8_attn_combine.argtypes = [vp, vp, vp, i64, i64, i64, i64, i64, vp, vp, vp]

@@ -61,6 +61,15 @@ struct TileArgs {
     int planes;                   // rows of whole 16-row tiles of one sliceable width are stored in planes (see qvb8_device.h)
 };
 
+// where the row's ids are, its width, and how they are read: bits 0..47 the bit offset, 48..55 the width, 56..57 the kind
+// (0: outside the buffer, 1: sliced, 2: id by id), bit 58 and 59..62 a row stored in planes and its number in the tile
+__device__ __forceinline__ uint64_t row_record(int nb, int64_t bit0, int P, int64_t ids_bytes) {
+    const bool ok = row_in_bounds(bit0, nb, P, ids_bytes);
+    if (ok && off_is_plane(bit0))
+        return (uint64_t)(bit0 & kOffBitsMask) | ((uint64_t)nb << 48) | (1ull << 56) | (1ull << 58) | ((uint64_t)off_plane_row(bit0) << 59);
+    const uint64_t kind = !ok ? 0 : ((bit0 & 31) == 0 && nb >= 4 && nb <= 8) ? 1 : 2;
+    return (ok ? (uint64_t)bit0 : 0) | ((uint64_t)nb << 48) | (kind << 56);
+}
 __global__ void __launch_bounds__(256) rowinfo_kernel(const uint8_t* __restrict__ nbits, const int64_t* __restrict__ bit_off,
                                                       const float* __restrict__ tau_s, const float* __restrict__ min_s,
                                                       const int32_t* __restrict__ perm, int Q, int P, int64_t ids_bytes,
@@ -72,15 +81,7 @@ __global__ void __launch_bounds__(256) rowinfo_kernel(const uint8_t* __restrict_
     uint4 f = {0u, 0u, 0xffffffffu, 0u};
     if (q >= 0 && q < Q) {
         f = uint4{__float_as_uint(tau_s[q]), __float_as_uint(min_s[q]), (uint32_t)q, 0u};
-        const int nb = nbits[q];
-        const int64_t bit0 = bit_off[q];
-        const bool ok = row_in_bounds(bit0, nb, P, ids_bytes);
-        if (ok && off_is_plane(bit0)) {
-            rec = (uint64_t)(bit0 & kOffBitsMask) | ((uint64_t)nb << 48) | (1ull << 56) | (1ull << 58) | ((uint64_t)off_plane_row(bit0) << 59);
-        } else {
-            const uint64_t kind = !ok ? 0 : ((bit0 & 31) == 0 && nb >= 4 && nb <= 8) ? 1 : 2;
-            rec = (ok ? (uint64_t)bit0 : 0) | ((uint64_t)nb << 48) | (kind << 56);
-        }
+        rec = row_record(nbits[q], bit_off[q], P, ids_bytes);
     }
     loc[i] = rec;
     fin[i] = f;
@@ -609,12 +610,13 @@ __global__ void __launch_bounds__(256) tile_fix_escapes_kernel(const uint16_t* _
     Y[(size_t)t * Q + q] += acc;
 }
 
-// ---- dense restore along the row records ------------------------------------------------------------------------------
+// ---- dense restore in tile order ------------------------------------------------------------------------------
 // The rows of a 16-row tile stored in planes lie together in memory but far apart in the weight: a wave that restores one
 // output row picks 16 bytes out of every 256 of its tile, and the lines it leaves are fetched again by whoever restores the
 // next row (measured at 4096 x 12288 of 7 bits into fp16: 68.0 us).  Here a wave takes the 16 positions of a tile, a 128-column
 // step at a time -- lane l the 32 ids of position l % 16, column group l / 16, which for a tile in planes is one contiguous
-// run -- and turns the step round in LDS, so that its stores are 16 rows of 256 contiguous bytes.  Any other row is read by its own record.
+// run -- and turns the step round in LDS, so that its stores are 16 rows of 256 contiguous bytes.  Any other row is read where it lies.
+// The row records say only which rows make a tile: widths, places and constants are the weight's own at the time of the call.
 // Bound by memory: 25.2 us there, 144 MB at 5.7 TB/s.
 constexpr int kRestoreWaves = 4, kRestoreRow = kStepCols * 2 + 16;       // bytes per row of a step in LDS
 constexpr int kRestoreSteps = 4;                                          // steps a wave takes
@@ -637,17 +639,20 @@ __device__ __forceinline__ void restore_slice(const uint8_t* __restrict__ ids, u
 }
 
 template <int DT>
-__global__ void __launch_bounds__(64 * kRestoreWaves) restore_tiles_kernel(const uint8_t* __restrict__ ids, int64_t ids_bytes, const uint64_t* __restrict__ loc,
-                                                                          const uint4* __restrict__ fin, int Q, int P, uint16_t* __restrict__ out) {
+__global__ void __launch_bounds__(64 * kRestoreWaves) restore_tiles_kernel(const uint8_t* __restrict__ ids, int64_t ids_bytes, const float* __restrict__ min_s,
+                                                                          const float* __restrict__ tau_s, const uint8_t* __restrict__ nbits,
+                                                                          const int64_t* __restrict__ bit_off, const uint4* __restrict__ fin,
+                                                                          int Q, int P, uint16_t* __restrict__ out) {
     __shared__ __align__(16) unsigned char turn_all[kRestoreWaves][16 * kRestoreRow];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     unsigned char* const turn = turn_all[wave];
     const int pos = 16 * (int)blockIdx.x + (lane & 15), g = lane >> 4;
     const int n_steps = P / kStepCols, first = ((int)blockIdx.y * kRestoreWaves + wave) * kRestoreSteps;
     if (first >= n_steps) return;                              // no barrier follows: each wave works in its own part of LDS
-    const uint64_t rec = pos < Q ? loc[pos] : 0;
-    const uint4 f = pos < Q ? fin[pos] : uint4{0u, 0u, 0xffffffffu, 0u};
-    const float ts = __uint_as_float(f.x), mn = __uint_as_float(f.y);
+    const uint32_t row = pos < Q ? fin[pos].z : 0xffffffffu;
+    const bool has = row < (uint32_t)Q;
+    const uint64_t rec = has ? row_record(nbits[row], bit_off[row], P, ids_bytes) : 0;
+    const float ts = has ? tau_s[row] : 0.f, mn = has ? min_s[row] : 0.f;
     const int nb = (int)(rec >> 48) & 255, kind = (int)(rec >> 56) & 3;
     const int64_t clamp_byte = (ids_bytes - 8) & ~(int64_t)3;
     for (int st = first; st < min(n_steps, first + kRestoreSteps); ++st) {
@@ -681,7 +686,7 @@ __global__ void __launch_bounds__(64 * kRestoreWaves) restore_tiles_kernel(const
         for (int k = 0; k < 4; ++k) {
             const int r = 4 * k + g;
             const uint4 v = *reinterpret_cast<const uint4*>(turn + r * kRestoreRow + 16 * (lane & 15));
-            const uint32_t q = (uint32_t)__shfl((int)f.z, r);
+            const uint32_t q = (uint32_t)__shfl((int)row, r);
             if (q < (uint32_t)Q) *reinterpret_cast<uint4*>(out + (size_t)q * P + st * kStepCols + 8 * (lane & 15)) = v;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1488,12 +1493,13 @@ extern "C" int qvb8_mma_prepare(const uint8_t* nbits, const int64_t* bit_off, co
     return host::check_launch("qvb8_mma_prepare");
 }
 
-extern "C" int qvb8_decode_tiles(const uint8_t* ids, int64_t ids_bytes, const uint64_t* rowinfo, int64_t Q, int64_t P, int out_dtype, void* out, void* stream) {
+extern "C" int qvb8_decode_tiles(const uint8_t* ids, int64_t ids_bytes, const float* min_s, const float* tau_s, const uint8_t* nbits,
+                                 const int64_t* bit_off, const uint64_t* rowinfo, int64_t Q, int64_t P, int out_dtype, void* out, void* stream) {
     if (Q < 0 || P < 0 || Q > 0x7fffffff || P > 0x7fffffff) return host::fail(QVB8_ERR_ARG, "qvb8_decode_tiles: Q or P out of range");
     if (out_dtype != QVB8_F16 && out_dtype != QVB8_BF16) return host::fail(QVB8_ERR_ARG, "qvb8_decode_tiles: out_dtype %d (fp16 or bf16)", out_dtype);
     if (P % kStepCols) return host::fail(QVB8_ERR_ARG, "qvb8_decode_tiles: needs P%%128==0");
     if (Q == 0 || P == 0) return QVB8_OK;
-    if (!ids || !rowinfo || !out) return host::fail(QVB8_ERR_ARG, "qvb8_decode_tiles: null pointer");
+    if (!ids || !min_s || !tau_s || !nbits || !bit_off || !rowinfo || !out) return host::fail(QVB8_ERR_ARG, "qvb8_decode_tiles: null pointer");
     if (ids_bytes < 8 || (reinterpret_cast<uintptr_t>(ids) & 3u)) return host::fail(QVB8_ERR_ARG, "qvb8_decode_tiles: ids must be 4-byte aligned and hold their 8 pad bytes");
     if ((reinterpret_cast<uintptr_t>(out) & 15u) || (reinterpret_cast<uintptr_t>(rowinfo) & 7u)) return host::fail(QVB8_ERR_ARG, "qvb8_decode_tiles: out must be 16-byte aligned");
     const int64_t steps_y = (P / kStepCols + kRestoreWaves * kRestoreSteps - 1) / (kRestoreWaves * kRestoreSteps);
@@ -1501,8 +1507,8 @@ extern "C" int qvb8_decode_tiles(const uint8_t* ids, int64_t ids_bytes, const ui
     const dim3 grid((unsigned)((Q + 15) / 16), (unsigned)steps_y), block(64 * kRestoreWaves);
     const uint4* fin = reinterpret_cast<const uint4*>(rowinfo + rowinfo_loc_words(Q));
     hipStream_t s = (hipStream_t)stream;
-    if (out_dtype == QVB8_F16) hipLaunchKernelGGL((restore_tiles_kernel<1>), grid, block, 0, s, ids, ids_bytes, rowinfo, fin, (int)Q, (int)P, (uint16_t*)out);
-    else hipLaunchKernelGGL((restore_tiles_kernel<2>), grid, block, 0, s, ids, ids_bytes, rowinfo, fin, (int)Q, (int)P, (uint16_t*)out);
+    if (out_dtype == QVB8_F16) hipLaunchKernelGGL((restore_tiles_kernel<1>), grid, block, 0, s, ids, ids_bytes, min_s, tau_s, nbits, bit_off, fin, (int)Q, (int)P, (uint16_t*)out);
+    else hipLaunchKernelGGL((restore_tiles_kernel<2>), grid, block, 0, s, ids, ids_bytes, min_s, tau_s, nbits, bit_off, fin, (int)Q, (int)P, (uint16_t*)out);
     return host::check_launch("qvb8_decode_tiles");
 }
 

@@ -56,7 +56,8 @@ def _decode_to(code, dtype, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_id
         if rowinfo is not None:
             if rowinfo.dtype != torch.int64 or rowinfo.numel() * 8 != lib.qvb8_mma_rowinfo_bytes(Q) or not rowinfo.is_cuda:
                 raise RuntimeError("rowinfo must be the int64 GPU tensor mma_prepare returned")
-            _lib._check(lib.qvb8_decode_tiles(_lib.ptr(ids), ids.numel(), rowinfo.contiguous().data_ptr(), Q, int(P), code, _lib.ptr(out), st), lib)
+            _lib._check(lib.qvb8_decode_tiles(_lib.ptr(ids), ids.numel(), _lib.ptr(min_s), _lib.ptr(tau_s), _lib.ptr(row_nbits),
+                                              _lib.ptr(row_bit_off), rowinfo.contiguous().data_ptr(), Q, int(P), code, _lib.ptr(out), st), lib)
         else:
             _lib._check(lib.qvb8_decode(_lib.ptr(ids), ids.numel(), _lib.ptr(min_s), _lib.ptr(tau_s), _lib.ptr(row_nbits),
                                         _lib.ptr(row_bit_off), Q, int(P), code, _lib.ptr(out), st), lib)
@@ -68,7 +69,7 @@ def _decode_to(code, dtype, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_id
 
 def decode(ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo=None):
     """Dense (Q, P) fp16 weight: fp16(fma(id, tau_s, min_s)), escapes written over it.  `rowinfo` (mma_prepare's, of these
-    rows): the same values read tile by tile, for rows stored in planes."""
+    rows): the same values read tile by tile, for rows stored in planes; only the order of the rows is taken from it."""
     return _decode_to(_lib.F16, torch.float16, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, rowinfo)
 
 

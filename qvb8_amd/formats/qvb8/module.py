@@ -350,7 +350,7 @@ class QVBandLinearV8(nn.Module):
             y = ext.gemv_multi(xk, self.ids, self.min_s, self.nbits, self.bit_off, self.in_features, self.tau_s,
                                self.esc_idx, self.esc_vals)
             return self._finish(y, orig, out_dtype)
-        # a weight whose rows lie in planes is restored tile by tile, through the row records built with them
+        # a weight whose rows lie in planes is restored tile by tile, in the order of the row records built with them
         built = self.__dict__.get("_mma_cache")
         rowinfo = built[1] if built and self._planes else None
         if xk.dtype == torch.bfloat16 and self.bf16_gemm and self.bf16_certified:

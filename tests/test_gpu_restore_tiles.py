@@ -5,6 +5,8 @@ import torch
 
 from oracle import qvb8_oracle as O
 from qvb8_amd import ext_qvb8 as ext
+from qvb8_amd.formats.qvb8 import pack as PK
+from qvb8_amd.formats.qvb8.module import QVBandLinearV8
 from tests.helpers import mixed_width_pack, oracle_ids, to_device_args
 
 pytestmark = pytest.mark.gpu
@@ -41,3 +43,21 @@ def test_narrowing_of_any_length_and_alignment(n, skip, dtype):
     got = ext.saturating_half(x.to(DEV)[skip:]).cpu()
     want = x[skip:] if dtype == torch.float16 else x[skip:].float().clamp(-65504, 65504).half()
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("x", [torch.float16, torch.bfloat16])
+def test_constants_rewritten_after_prepare_are_honoured(x):
+    """More than 256 rows restore the weight: row constants changed in place since prepare() count, as they do when the
+    weight has no row records."""
+    Q, P, M = 272, 1024, 300
+    enc = PK.encode_tensor((0.02 * torch.randn(Q, P, generator=torch.Generator().manual_seed(1))).to(torch.bfloat16).to(DEV), 1e-3)
+    mod = QVBandLinearV8.from_encoded(enc).prepare()
+    assert mod._planes
+    X = torch.randn(M, P, generator=torch.Generator().manual_seed(2)).to(x).to(DEV)
+    other = QVBandLinearV8.from_encoded(dict(enc, min_s=enc["min_s"] - 0.01, tau_s=enc["tau_s"] * 1.5))
+    assert other.__dict__.get("_mma_cache") is None              # restored row by row
+    before = mod(X)
+    with torch.no_grad():
+        mod.min_s.sub_(0.01), mod.tau_s.mul_(1.5)
+    now = mod(X)
+    assert not torch.equal(now, before) and torch.equal(now, other(X))
