@@ -4,8 +4,8 @@ Same class name, constructor, `from_packfiles`, `build_stack` layout and `forwar
 top_k_weights)` as the reference (src/qv_band/formats/qvb8/backends_experts.py:91-272).  The routed decode path is
 ext.moe_experts (four launches, no host round trip, each selected expert read once for all the tokens that chose it), for
 any number of tokens when the rows are whole 128-column steps; stacks with escapes, other activations, and more than
-FUSED_MAX_TOKENS tokens of other shapes take the per-expert loop over QVBandLinearV8 modules, which still runs on the GPU
-library.  There is no CPU reader here (the reference's QVBandLinearCPUV8 is its
+FUSED_MAX_TOKENS tokens of other shapes, or of calls that need what only the loop does (_many_as_the_loop), take the
+per-expert loop over QVBandLinearV8 modules, which still runs on the GPU library.  There is no CPU reader here (the reference's QVBandLinearCPUV8 is its
 CPU-only dense path; this build's CPU restatement lives with the tests and is not a product path).
 """
 from __future__ import annotations
@@ -14,9 +14,13 @@ import os
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from qvb8_amd import ext_qvb8 as ext
 from .module import QVBandLinearV8
+
+_KERNEL_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+_INDEX_DTYPES = (torch.int64, torch.int32, torch.int16, torch.int8, torch.uint8)
 
 
 def stack_projection(mods) -> dict:
@@ -145,14 +149,38 @@ class QVBandExpertsV8(nn.Module):
             self.build_stack()
         return self
 
+    def _many_as_the_loop(self, x: torch.Tensor, idx: torch.Tensor, w: torch.Tensor) -> bool:
+        """Whether the routed kernels do for more than FUSED_MAX_TOKENS tokens what the per-expert loop does.  They see neither
+        autograd nor the experts' hooks; activations are narrowed to fp16, which the loop does not do to bf16 ones of packs
+        certified for it; and calls of other types or layouts are the loop's, to answer or to refuse."""
+        if x.dtype not in _KERNEL_DTYPES or idx.dtype not in _INDEX_DTYPES or not w.is_floating_point():
+            return False
+        if x.dim() != 2 or idx.dim() != 2 or w.shape != idx.shape or x.shape != (idx.shape[0], self.gate_up_experts[0].in_features):
+            return False
+        if idx.device != x.device or w.device != x.device or not self._whole_steps():
+            return False
+        if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+            return False
+        if _has_any_global_hook() or getattr(self.act_fn, "_forward_hooks", None) or getattr(self.act_fn, "_forward_pre_hooks", None):
+            return False
+        bf16, fp16 = x.dtype == torch.bfloat16, x.dtype == torch.float16
+        for stack in (self.gate_up_experts, self.down_experts):
+            for m in stack._modules.values():
+                if m._forward_hooks or m._forward_pre_hooks or (bf16 and m.bf16_certified) or (fp16 and m.fp16_table_missing):
+                    return False
+        return True
+
     def forward(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:
         n_tok = top_k_index.shape[0]
-        if hidden_states.is_cuda and (n_tok <= self.FUSED_MAX_TOKENS or self._whole_steps()) and self.build_stack():
+        many = n_tok > self.FUSED_MAX_TOKENS
+        if hidden_states.is_cuda and (not many or self._many_as_the_loop(hidden_states, top_k_index, top_k_weights)) and self.build_stack():
+            if many:
+                top_k_index = top_k_index.to(torch.int64)
             g, d = self._stk
             return ext.moe_experts(hidden_states.contiguous(), top_k_index.contiguous(), top_k_weights.float(),
                                    g["ids"], g["min_s"], g["tau_s"], g["nbits"], g["bit_off"], g["Q"], g["P"],
                                    d["ids"], d["min_s"], d["tau_s"], d["nbits"], d["bit_off"], d["Q"], d["P"],
-                                   regular=(g["regular"], d["regular"]), keep_inf=n_tok > self.FUSED_MAX_TOKENS)
+                                   regular=(g["regular"], d["regular"]), keep_inf=many)
         return self._forward_loop(hidden_states, top_k_index, top_k_weights)
 
     def _forward_loop(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:

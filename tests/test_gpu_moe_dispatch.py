@@ -1,0 +1,83 @@
+"""QVBandExpertsV8 with more than FUSED_MAX_TOKENS tokens: the routed kernels where they do what the per-expert loop does, the loop
+for every other call."""
+import pytest
+import torch
+
+from oracle import qvb8_oracle as O
+from qvb8_amd.formats.qvb8 import pack as PK
+from qvb8_amd.formats.qvb8.backends_experts import QVBandExpertsV8
+from qvb8_amd.formats.qvb8.module import QVBandLinearV8
+from tests import helpers as H
+from tests.test_gpu_moe import _check, _experts
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+E, K, HIDDEN, INTER = 4, 2, 256, 128
+
+
+def _module(tau=2e-3, restore="fp16", hidden=HIDDEN, inter=INTER):
+    made = lambda Q, P, seed: QVBandLinearV8.from_encoded(PK.encode_tensor(H.synth_weight(Q, P, seed=seed).to(DEV), tau, restore=restore))     # noqa: E731
+    return QVBandExpertsV8([made(2 * inter, hidden, 2 * e) for e in range(E)], [made(hidden, inter, 2 * e + 1) for e in range(E)], num_experts=E)
+
+
+def _call(T, dtype=torch.bfloat16, seed=0, hidden=HIDDEN):
+    g = torch.Generator().manual_seed(seed + T)
+    idx = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(T)])
+    return torch.randn(T, hidden, generator=g).to(dtype).to(DEV), idx.to(DEV), torch.rand(T, K, generator=g).to(DEV)
+
+
+def _spy(mod, monkeypatch):
+    """Counts the calls the loop answers."""
+    calls, loop = [], mod._forward_loop
+    monkeypatch.setattr(mod, "_forward_loop", lambda *a: (calls.append(1), loop(*a))[1], raising=False)
+    return calls
+
+
+@pytest.mark.parametrize("T", [65, 300])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_many_tokens_match_the_oracle(T, dtype, monkeypatch):
+    gu, dn, Wgu, Wdn = _experts(E, HIDDEN, INTER, 2e-3, seed=7)
+    mod = QVBandExpertsV8(gu, dn, num_experts=E)
+    calls = _spy(mod, monkeypatch)
+    x, idx, w = _call(T, dtype)
+    out = mod(x, idx, w)
+    assert not calls and out.dtype == dtype
+    _check(out, O.moe_reference(x.float().cpu().numpy(), idx.cpu().numpy(), w.cpu().numpy(), Wgu, Wdn), dtype)
+    assert torch.equal(mod(x, idx.to(torch.int32), w), out)                     # any integer routing, as the loop takes it
+    assert torch.equal(mod(x, idx.to(torch.uint8), w.to(torch.float64)), out) and not calls
+
+
+def test_calls_the_loop_answers(monkeypatch):
+    mod, T = _module(), 70
+    x, idx, w = _call(T)
+    mod(x, idx, w)
+    calls = _spy(mod, monkeypatch)
+    w.requires_grad_()
+    out = mod(x, idx, w)                                                         # routing weights that want a gradient
+    out.float().pow(2).sum().backward()
+    assert len(calls) == 1 and w.grad is not None and bool((w.grad != 0).any())
+    with torch.no_grad():
+        mod(x, idx, w)
+    assert len(calls) == 1
+    w = w.detach()
+    fired = []
+    hook = mod.down_experts[2].register_forward_hook(lambda *a: fired.append(1))
+    mod(x, idx, w)
+    assert len(calls) == 2 and fired
+    hook.remove()
+    more = torch.cat([x, x[:3]])                                                 # rows that no routing row names give zeros
+    assert torch.equal(mod(more, idx, w)[:T], mod._forward_loop(x, idx, w)) and len(calls) == 4
+    mod(x, idx, w)
+    assert len(calls) == 4
+
+
+def test_bf16_certified_experts_multiply_bf16_activations_as_they_are(monkeypatch):
+    mod = _module(restore="fp16+bf16")
+    if any(m.esc_idx_bf16.numel() for m in [*mod.gate_up_experts, *mod.down_experts]):
+        pytest.skip("this pack has bf16 escapes: never stacked")
+    x, idx, w = _call(80)
+    x[5, 7] = 1e6                                                                # beyond fp16, within bf16
+    assert torch.equal(mod(x, idx, w), mod._forward_loop(x, idx, w))
+    calls = _spy(mod, monkeypatch)
+    mod(x.clamp(-1e4, 1e4).half(), idx, w)
+    assert not calls
