@@ -53,7 +53,7 @@ enum qvb8_status {
 /* Library identification: ABI version, bumped on any signature change or new entry point (3: row lookup, attention over
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
  * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*;
- * 9: qvb8_decode_tiles; 10: its constants).  A binding compares the loaded library's answer
+ * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
 #define QVB8_ABI_VERSION 10
 int qvb8_abi_version(void);
@@ -298,6 +298,17 @@ int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* 
                      const uint8_t* dn_ids, int64_t dn_ids_bytes, const float* dn_min, const float* dn_tau,
                      const uint8_t* dn_nb, const int64_t* dn_off, int64_t Q_dn, int64_t P_dn,
                      int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+/* The same from 17 tokens on, for callers that want to know whether the routing was sound: returns when the routing plan has
+ * run (the products are queued behind it and not waited for), with the number of routing entries outside the stack -- each
+ * of which makes the whole output NaN -- in *bad_pairs, host memory the device can write (pinned, coherent).  Not inside a
+ * stream capture. */
+int qvb8_moe_experts_checked(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, const float* w, int64_t topk,
+                             int64_t n_experts,
+                             const uint8_t* up_ids, int64_t up_ids_bytes, const float* up_min, const float* up_tau,
+                             const uint8_t* up_nb, const int64_t* up_off, int64_t Q_up, int64_t P_up,
+                             const uint8_t* dn_ids, int64_t dn_ids_bytes, const float* dn_min, const float* dn_tau,
+                             const uint8_t* dn_nb, const int64_t* dn_off, int64_t Q_dn, int64_t P_dn,
+                             int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes, int32_t* bad_pairs, void* stream);
 
 /* qvb8_moe_experts for callers that cannot allocate device memory or bring a workspace: code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc.  Same operands, same kernels and the same results bit for bit; the

@@ -32,6 +32,7 @@ constexpr int kMoeThreads = 256;
 
 constexpr int kPlanMaxThreads = 1024;
 constexpr int kPlanTableExperts = 512;
+constexpr int kPlanScratch = 49;       // running sums of 16 waves x 3, entries outside the stack
 constexpr int kPlanKept = 4;           // pairs per thread kept in registers from the count to the placement
 
 // One workgroup: pairs grouped by expert (a stable counting sort: an expert's pairs keep their order, so that the plan, and
@@ -41,15 +42,17 @@ constexpr int kPlanKept = 4;           // pairs per thread kept in registers fro
 // `cap`: the most pairs one expert may have for the path that follows (the grouped walk takes an expert's pairs as the token
 // rows of ONE operand: at most one per token); an expert with more counts as a bad entry, so the results come out as NaN
 // instead of sums with pairs missing.
+// `bad_out`: where the number of entries outside the stack goes, or null.
 // Placement (`ordered`; the paths whose results do not depend on the order let every pair move its expert's cursor), blockDim
 // pairs at a time: every wave counts its pairs per expert in a table [wave][expert], a thread per expert
 // turns the counts into places, the pairs take them; with more than kPlanTableExperts experts the waves take turns at the
 // experts' cursors instead.  Bound by its chain of barriers and LDS trips (4072 pairs, 128 experts: 13.2 us; turns only
 // 19.1; cursors moved by atomics 15.4).
-__global__ void __launch_bounds__(kPlanMaxThreads) moe_plan_kernel(const int64_t* __restrict__ idx, int npairs, int E, MoePlan pl, int cap, int ordered) {
-    extern __shared__ int32_t s_cnt[];                        // [E] counts, then cursors; [48] scan scratch; [waves][E] where E allows
+__global__ void __launch_bounds__(kPlanMaxThreads) moe_plan_kernel(const int64_t* __restrict__ idx, int npairs, int E, MoePlan pl, int cap, int ordered, int32_t* bad_out) {
+    extern __shared__ int32_t s_cnt[];                        // [E] counts, then cursors; scan scratch; [waves][E] where E allows
     int32_t* s_scan = s_cnt + E;
-    int32_t* s_wave = s_scan + 48;
+    int32_t* s_bad = s_scan + 48;
+    int32_t* s_wave = s_scan + kPlanScratch;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n_waves = (int)blockDim.x >> 6;
     // the thread's first pairs, asked for together and kept for both passes (-1: no such pair, -2: outside the stack)
     int mine[kPlanKept];
@@ -65,14 +68,14 @@ __global__ void __launch_bounds__(kPlanMaxThreads) moe_plan_kernel(const int64_t
         return p >= npairs ? -1 : (e >= 0 && e < E) ? (int)e : -2;
     };
     for (int e = tid; e < E; e += blockDim.x) s_cnt[e] = 0;
-    if (tid == 0) *pl.n_bad = 0;
+    if (tid == 0) { *pl.n_bad = 0; *s_bad = 0; }
     __syncthreads();
     int bad = 0;
     auto count = [&](int e) { if (e >= 0) atomicAdd(&s_cnt[e], 1); else if (e == -2) ++bad; };
 #pragma unroll
     for (int k = 0; k < kPlanKept; ++k) count(mine[k]);
     for (int p = tid + kPlanKept * blockDim.x; p < npairs; p += blockDim.x) count(expert_of(p, kPlanKept));
-    if (bad) atomicAdd(pl.n_bad, bad);
+    if (bad) { atomicAdd(pl.n_bad, bad); atomicAdd(s_bad, bad); }
     __syncthreads();
     const int n_slots = E < npairs ? E : npairs;
     int run_pairs = 0, run_active = 0, run_blocks = 0;        // totals of the rounds before this one (same in every thread)
@@ -103,7 +106,10 @@ __global__ void __launch_bounds__(kPlanMaxThreads) moe_plan_kernel(const int64_t
         __syncthreads();
     }
     for (int i = run_active + tid; i < n_slots; i += blockDim.x) pl.slot[i] = int4{0, 0, 0, 0};
-    if (tid == 0) { pl.n_bad[1] = run_active; pl.n_bad[2] = run_blocks; }      // slots in use, token blocks of all of them
+    if (tid == 0) {
+        pl.n_bad[1] = run_active; pl.n_bad[2] = run_blocks;   // slots in use, token blocks of all of them
+        if (bad_out) __hip_atomic_store(bad_out, *s_bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);        // the host waits for this word alone
+    }
     const int e_bits = 32 - __builtin_clz(E > 1 ? E - 1 : 1);
     auto place = [&](int p0, int mine_e) {
         const int p = p0 + tid;
@@ -1092,12 +1098,13 @@ extern "C" int64_t qvb8_moe_workspace_bytes(int64_t tokens, int64_t topk, int64_
     return (int64_t)(moe_plan_bytes(n_experts, np) + align256((size_t)np * P_dn * 4) + align256((size_t)np * Q_dn * 4));
 }
 
-extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, const float* w, int64_t topk, int64_t n_experts,
-                                const uint8_t* up_ids, int64_t up_ids_bytes, const float* up_min, const float* up_tau,
-                                const uint8_t* up_nb, const int64_t* up_off, int64_t Q_up, int64_t P_up,
-                                const uint8_t* dn_ids, int64_t dn_ids_bytes, const float* dn_min, const float* dn_tau,
-                                const uint8_t* dn_nb, const int64_t* dn_off, int64_t Q_dn, int64_t P_dn,
-                                int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+namespace {
+int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, const float* w, int64_t topk, int64_t n_experts,
+                const uint8_t* up_ids, int64_t up_ids_bytes, const float* up_min, const float* up_tau,
+                const uint8_t* up_nb, const int64_t* up_off, int64_t Q_up, int64_t P_up,
+                const uint8_t* dn_ids, int64_t dn_ids_bytes, const float* dn_min, const float* dn_tau,
+                const uint8_t* dn_nb, const int64_t* dn_off, int64_t Q_dn, int64_t P_dn,
+                int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes, int32_t* bad_out, void* stream) {
     if (tokens < 0 || topk < 1 || n_experts < 1 || n_experts > 8192) return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: bad token / top-k / expert count");
     constexpr int kActFlags = QVB8_MOE_UP_REGULAR | QVB8_MOE_DOWN_REGULAR | QVB8_MOE_KEEP_INF;
     if ((act & ~kActFlags) != 0 && (act & ~kActFlags) != 1)
@@ -1157,9 +1164,9 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
 
     // a thread per pair (or per expert, when they are more) up to the most a workgroup has
     const int64_t plan_threads = std::min<int64_t>(kPlanMaxThreads, (std::max(np, n_experts) + 255) / 256 * 256);
-    const size_t plan_lds = (size_t)(n_experts + 48 + (n_experts <= kPlanTableExperts ? n_experts * (plan_threads / 64) : 0)) * 4;
+    const size_t plan_lds = (size_t)(n_experts + kPlanScratch + (n_experts <= kPlanTableExperts ? n_experts * (plan_threads / 64) : 0)) * 4;
     hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3((unsigned)plan_threads), plan_lds, s, idx, (int)np, (int)n_experts, pl,
-                       grouped ? (int)(tokens < 16 ? tokens : 16) : (int)np, grouped ? 0 : 1);
+                       grouped ? (int)(tokens < 16 ? tokens : 16) : (int)np, grouped ? 0 : 1, bad_out);
     if (int rc = host::check_launch("qvb8_moe_experts plan")) return rc;
     const int64_t slots = moe_slots(n_experts, np);
     if (grouped) {
@@ -1199,6 +1206,42 @@ extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, cons
     if (int rc = launch_moe_gemv(1, a, slots, s)) return rc;
 
     return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
+}
+
+}  // namespace
+
+extern "C" int qvb8_moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, const float* w, int64_t topk, int64_t n_experts,
+                                const uint8_t* up_ids, int64_t up_ids_bytes, const float* up_min, const float* up_tau,
+                                const uint8_t* up_nb, const int64_t* up_off, int64_t Q_up, int64_t P_up,
+                                const uint8_t* dn_ids, int64_t dn_ids_bytes, const float* dn_min, const float* dn_tau,
+                                const uint8_t* dn_nb, const int64_t* dn_off, int64_t Q_dn, int64_t P_dn,
+                                int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+    return moe_experts(X, x_dtype, tokens, idx, w, topk, n_experts, up_ids, up_ids_bytes, up_min, up_tau, up_nb, up_off, Q_up, P_up,
+                       dn_ids, dn_ids_bytes, dn_min, dn_tau, dn_nb, dn_off, Q_dn, P_dn, act, out, out_dtype, workspace, workspace_bytes, nullptr, stream);
+}
+
+extern "C" int qvb8_moe_experts_checked(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, const float* w, int64_t topk, int64_t n_experts,
+                                        const uint8_t* up_ids, int64_t up_ids_bytes, const float* up_min, const float* up_tau,
+                                        const uint8_t* up_nb, const int64_t* up_off, int64_t Q_up, int64_t P_up,
+                                        const uint8_t* dn_ids, int64_t dn_ids_bytes, const float* dn_min, const float* dn_tau,
+                                        const uint8_t* dn_nb, const int64_t* dn_off, int64_t Q_dn, int64_t P_dn,
+                                        int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes, int32_t* bad_pairs, void* stream) {
+    if (!bad_pairs || (reinterpret_cast<uintptr_t>(bad_pairs) & 3u)) return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts_checked: needs a counter");
+    if (tokens <= 16) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_moe_experts_checked: 17 tokens or more");
+    __atomic_store_n(bad_pairs, -1, __ATOMIC_RELEASE);
+    if (int rc = moe_experts(X, x_dtype, tokens, idx, w, topk, n_experts, up_ids, up_ids_bytes, up_min, up_tau, up_nb, up_off, Q_up, P_up,
+                             dn_ids, dn_ids_bytes, dn_min, dn_tau, dn_nb, dn_off, Q_dn, P_dn, act, out, out_dtype, workspace, workspace_bytes, bad_pairs, stream))
+        return rc;
+    // The plan kernel writes the counter in the middle of its work; the products are queued behind it by now.  (An event between
+    // the two, waited for instead, put 8 us of idle GPU there.)  The wait ends with the stream at the latest.
+    for (int64_t spins = 1; __atomic_load_n(bad_pairs, __ATOMIC_ACQUIRE) < 0; ++spins) {
+        if (spins % 4096) continue;
+        const hipError_t e = hipStreamQuery((hipStream_t)stream);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess || __atomic_load_n(bad_pairs, __ATOMIC_ACQUIRE) < 0)
+            return host::fail(QVB8_ERR_LAUNCH, "qvb8_moe_experts_checked: the routing plan did not run: %s", hipGetErrorString(e));
+    }
+    return QVB8_OK;
 }
 
 // ---- the same call for callers that cannot allocate ------------------------------------------------------------------

@@ -563,7 +563,7 @@ def forward_half(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_v
     return _forward(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, True)
 
 
-def _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn):
+def _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn, checked=False):
     lib = _lib.load()
     _lib.require_cuda(X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, dn_ids, dn_min, dn_tau, dn_nb, dn_off)
     if X.dim() != 2 or X.shape[1] != int(Pup):
@@ -592,11 +592,17 @@ def _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids
         nws = lib.qvb8_moe_workspace_bytes(T, k, E, int(Qup), int(Pdn), int(Qdn))
         ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=Xc.device)
         u, d = tens[:5], tens[5:]
-        _lib._check(lib.qvb8_moe_experts(
+        entry, extra = lib.qvb8_moe_experts, ()
+        if checked:
+            bad = torch.empty(1, dtype=torch.int32, pin_memory=True)
+            entry, extra = lib.qvb8_moe_experts_checked, (bad.data_ptr(),)
+        _lib._check(entry(
             _lib.ptr(Xc), _lib.dtype_code(Xc.dtype), T, _lib.ptr(idxc), _lib.ptr(wc), k, E,
             _lib.ptr(u[0]), u[0].numel(), _lib.ptr(u[1]), _lib.ptr(u[2]), _lib.ptr(u[3]), _lib.ptr(u[4]), int(Qup), int(Pup),
             _lib.ptr(d[0]), d[0].numel(), _lib.ptr(d[1]), _lib.ptr(d[2]), _lib.ptr(d[3]), _lib.ptr(d[4]), int(Qdn), int(Pdn),
-            act, _lib.ptr(out), _lib.dtype_code(out.dtype), _lib.ptr(ws), ws.numel(), _lib.stream_of(Xc)), lib)
+            act, _lib.ptr(out), _lib.dtype_code(out.dtype), _lib.ptr(ws), ws.numel(), *extra, _lib.stream_of(Xc)), lib)
+        if checked and int(bad[0]):
+            return None
     return out
 
 
@@ -616,12 +622,14 @@ def stack_is_regular(nbits, bit_off, P) -> bool:
 
 
 def moe_experts(X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn,
-                regular=(False, False), keep_inf=False):
+                regular=(False, False), keep_inf=False, checked=False):
     """Routed gated-SiLU expert stack on the stacked layout (reference: qvb8_cuda.cu:937-992); returns (tokens, Qdn)
     in X's dtype.  `regular` = (up, down): the caller states that the stack is regular (stack_is_regular).  `keep_inf`: fp16
-    activations beyond 16 tokens are taken as they are, infinities too (else they become +-65504)."""
+    activations beyond 16 tokens are taken as they are, infinities too (else they become +-65504).  `checked` (17 tokens
+    or more): the host waits for the routing plan, not for the products, and gets None where an entry lies outside the
+    stack (else such an entry makes the whole result NaN)."""
     act = 0 | (MOE_UP_REGULAR if regular[0] else 0) | (MOE_DOWN_REGULAR if regular[1] else 0) | (MOE_KEEP_INF if keep_inf else 0)
-    return _moe(act, X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn)
+    return _moe(act, X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn, checked)
 
 
 def moe_experts_relu2(X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn,

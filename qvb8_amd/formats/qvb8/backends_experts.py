@@ -171,17 +171,21 @@ class QVBandExpertsV8(nn.Module):
         return True
 
     def forward(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:
-        n_tok = top_k_index.shape[0]
-        many = n_tok > self.FUSED_MAX_TOKENS
+        many = top_k_index.shape[0] > self.FUSED_MAX_TOKENS
         if hidden_states.is_cuda and (not many or self._many_as_the_loop(hidden_states, top_k_index, top_k_weights)) and self.build_stack():
-            if many:
-                top_k_index = top_k_index.to(torch.int64)
-            g, d = self._stk
-            return ext.moe_experts(hidden_states.contiguous(), top_k_index.contiguous(), top_k_weights.float(),
-                                   g["ids"], g["min_s"], g["tau_s"], g["nbits"], g["bit_off"], g["Q"], g["P"],
-                                   d["ids"], d["min_s"], d["tau_s"], d["nbits"], d["bit_off"], d["Q"], d["P"],
-                                   regular=(g["regular"], d["regular"]), keep_inf=many)
+            out = self._routed(hidden_states, top_k_index.to(torch.int64) if many else top_k_index, top_k_weights, many)
+            if out is not None:
+                return out
         return self._forward_loop(hidden_states, top_k_index, top_k_weights)
+
+    def _routed(self, x: torch.Tensor, idx: torch.Tensor, w: torch.Tensor, many: bool):
+        """The routed kernels.  With more than FUSED_MAX_TOKENS tokens, None where an expert number lies outside 0..E-1: the loop
+        counts negative ones from the end and refuses the others (inside a graph capture nothing can be read back: NaN)."""
+        g, d = self._stk
+        return ext.moe_experts(x.contiguous(), idx.contiguous(), w.float(),
+                               g["ids"], g["min_s"], g["tau_s"], g["nbits"], g["bit_off"], g["Q"], g["P"],
+                               d["ids"], d["min_s"], d["tau_s"], d["nbits"], d["bit_off"], d["Q"], d["P"],
+                               regular=(g["regular"], d["regular"]), keep_inf=many, checked=many and not torch.cuda.is_current_stream_capturing())
 
     def _forward_loop(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:
         """The (token, choice) pairs sorted by expert once, then one pass per expert that was chosen: its tokens through

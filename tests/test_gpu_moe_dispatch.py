@@ -81,3 +81,36 @@ def test_bf16_certified_experts_multiply_bf16_activations_as_they_are(monkeypatc
     calls = _spy(mod, monkeypatch)
     mod(x.clamp(-1e4, 1e4).half(), idx, w)
     assert not calls
+
+
+@pytest.mark.parametrize("T", [65, 300])
+def test_expert_numbers_outside_the_stack(T):
+    """Past the end: refused, by the call that has them.  Negative ones count from the end, as in any list."""
+    mod = _module()
+    x, idx, w = _call(T)
+    want = mod(x, idx, w)
+    for at, bad in (((T - 1, 1), E), ((0, 0), 1 << 40), ((T // 2, 0), -E - 1)):
+        wrong = idx.clone()
+        wrong[at] = bad
+        with pytest.raises(IndexError):
+            mod(x, wrong, w)
+    back = torch.where(torch.arange(T, device=DEV)[:, None] % 3 == 0, idx - E, idx)
+    assert torch.equal(mod(x, back, w), mod._forward_loop(x, back, w))
+    assert torch.equal(mod(x, idx, w), want)
+
+
+def test_many_tokens_inside_a_graph():
+    """Captured and replayed with other inputs in the same buffers, eager calls between the replays."""
+    mod = _module()
+    x, idx, w = _call(90)
+    mod(x, idx, w)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        out = mod(x, idx, w)
+    for seed in range(3):
+        nx, nidx, nw = _call(90, seed=10 + seed)
+        x.copy_(nx), idx.copy_(nidx), w.copy_(nw)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, mod(nx, nidx, nw))
