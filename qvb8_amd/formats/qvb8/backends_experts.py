@@ -78,7 +78,8 @@ def stack_projection(mods) -> dict:
         m.__dict__.pop("_sorted_layout", None)
     table = {name: torch.stack([getattr(m, name) for m in mods]).contiguous() for name in ("min_s", "tau_s", "nbits", "bit_off")}
     regular = uniform and ext.stack_is_regular(table["nbits"], table["bit_off"], mods[0].in_features)
-    return dict(ids=shared, Q=int(mods[0].out_features), P=int(mods[0].in_features), regular=regular, **table)
+    sliced = bool(((table["nbits"] >= 4) & (table["nbits"] <= 8) & (table["bit_off"] % 32 == 0)).all())       # no row is read id by id
+    return dict(ids=shared, Q=int(mods[0].out_features), P=int(mods[0].in_features), regular=regular, sliced=sliced, **table)
 
 
 def _stackable(mods) -> bool:
@@ -98,6 +99,19 @@ class QVBandExpertsV8(nn.Module):
     # Up to this many tokens the routed kernels run whatever the shape; above it only stacks whose rows are whole 128-column
     # steps (the matrix-core kernels), the others take the per-expert loop.
     FUSED_MAX_TOKENS = 64
+    # Above it the loop also takes calls it is faster at.  It restores an expert once and multiplies with a library GEMM, where the
+    # routed kernels decode it again for every 64 of its pairs: that pays from 512 pairs per expert on, if the expert is large
+    # enough for its product to outlast the ten or so launches it costs (products of pairs and weights per expert; measured,
+    # us, routed / loop).  8 experts of 4096/14336 (176 M weights): 256 pairs 2239 / 2855, 512 pairs 3591 / 3583, 1024 pairs
+    # 6609 / 4886, 2048 pairs 12697 / 8312.  50 M weights: 512 pairs 2137 / 2897 (16 experts of 4096/4096) and 653 / 883 (4 of
+    # 2048/8192), 1024 pairs 3874 / 3826 and 1157 / 1182, 2048 pairs 7558 / 5945 and 2082 / 1716.  2048/768 (4.7 M weights): 8192 pairs
+    # 3531 / 4634 (16 experts), 512 pairs 1996 / 19906 (128 experts).
+    LOOP_FROM_PAIRS, LOOP_FROM_PRODUCTS = 512, 5e10
+    # Rows the kernels read id by id (width outside 4..8 or off a dword): for each pair again, while the loop restores them once
+    # from 97 rows of activations on and is slow below that only where experts are small.  32 experts of 2048/768, a third of
+    # the rows 9 bits wide: 16 pairs 4049 / 17287, 75 pairs 15259 / 81750, 150 pairs 19489 / 5636; 8 of 4096/4096, three quarters:
+    # 16 pairs 24125 / 14425, 64 pairs 73024 / 48029, 150 pairs 104639 / 1548.
+    ODD_ROWS_MAX_PAIRS, ODD_ROWS_MAX_WEIGHTS = 75, 2 ** 23
 
     def __init__(self, gate_up_experts, down_experts, *, num_experts: int, act_fn=None):
         super().__init__()
@@ -149,6 +163,16 @@ class QVBandExpertsV8(nn.Module):
             self.build_stack()
         return self
 
+    def _loop_is_faster(self, n_pairs: int) -> bool:
+        """Whether a call of so many (token, choice) pairs is the loop's, going by the pairs an expert gets on average."""
+        g, d = self._stk
+        pairs, weights = n_pairs / self.num_experts, g["Q"] * g["P"] + d["Q"] * d["P"]
+        if os.environ.get("QVB8_MOE_GROUPED", "1") == "0":           # the kernels are switched off
+            return True
+        if not (g["sliced"] and d["sliced"]) and (pairs > self.ODD_ROWS_MAX_PAIRS or weights > self.ODD_ROWS_MAX_WEIGHTS):
+            return True
+        return pairs >= self.LOOP_FROM_PAIRS and pairs * weights >= self.LOOP_FROM_PRODUCTS
+
     def _many_as_the_loop(self, x: torch.Tensor, idx: torch.Tensor, w: torch.Tensor) -> bool:
         """Whether the routed kernels do for more than FUSED_MAX_TOKENS tokens what the per-expert loop does.  They see neither
         autograd nor the experts' hooks; activations are narrowed to fp16, which the loop does not do to bf16 ones of packs
@@ -173,9 +197,12 @@ class QVBandExpertsV8(nn.Module):
     def forward(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:
         many = top_k_index.shape[0] > self.FUSED_MAX_TOKENS
         if hidden_states.is_cuda and (not many or self._many_as_the_loop(hidden_states, top_k_index, top_k_weights)) and self.build_stack():
-            out = self._routed(hidden_states, top_k_index.to(torch.int64) if many else top_k_index, top_k_weights, many)
-            if out is not None:
-                return out
+            if not many:
+                return self._routed(hidden_states, top_k_index, top_k_weights, False)
+            if not self._loop_is_faster(top_k_index.numel()):
+                out = self._routed(hidden_states, top_k_index.to(torch.int64), top_k_weights, True)
+                if out is not None:
+                    return out
         return self._forward_loop(hidden_states, top_k_index, top_k_weights)
 
     def _routed(self, x: torch.Tensor, idx: torch.Tensor, w: torch.Tensor, many: bool):

@@ -114,3 +114,41 @@ def test_many_tokens_inside_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, mod(nx, nidx, nw))
+
+
+def test_the_loop_takes_what_it_is_faster_at(monkeypatch):
+    """The rule by pairs per expert and weights per expert, at its edges; and that a call follows it."""
+    mod = _module()
+    x, idx, w = _call(100)
+    mod(x, idx, w)
+    weights = 3 * HIDDEN * INTER
+    monkeypatch.setattr(QVBandExpertsV8, "LOOP_FROM_PRODUCTS", 50 * weights)
+    assert not mod._loop_is_faster(512 * E - 1) and mod._loop_is_faster(512 * E)
+    monkeypatch.setattr(QVBandExpertsV8, "LOOP_FROM_PRODUCTS", 600 * weights)
+    assert not mod._loop_is_faster(600 * E - 1) and mod._loop_is_faster(600 * E)
+    monkeypatch.setattr(QVBandExpertsV8, "LOOP_FROM_PAIRS", 100)
+    monkeypatch.setattr(QVBandExpertsV8, "LOOP_FROM_PRODUCTS", 0)
+    calls = _spy(mod, monkeypatch)
+    mod(x, idx, w)                                                               # 50 pairs per expert
+    assert not calls
+    mod(x.repeat(2, 1), idx.repeat(2, 1), w.repeat(2, 1))
+    assert len(calls) == 1
+    monkeypatch.setenv("QVB8_MOE_GROUPED", "0")
+    mod(x, idx, w)
+    assert len(calls) == 2
+
+
+def test_stacks_with_rows_read_id_by_id(monkeypatch):
+    mod = _module(tau=2e-4)
+    x, idx, w = _call(100)
+    mod.prepare()
+    assert int(mod._stk[0]["nbits"].max()) > 8 and not mod._stk[0]["sliced"]
+    calls = _spy(mod, monkeypatch)
+    out = mod(x, idx, w)                                                         # 50 pairs per expert of 98304 weights
+    assert not calls
+    monkeypatch.setattr(QVBandExpertsV8, "ODD_ROWS_MAX_PAIRS", 49)
+    loop = mod(x, idx, w)
+    monkeypatch.setattr(QVBandExpertsV8, "ODD_ROWS_MAX_PAIRS", 75)
+    monkeypatch.setattr(QVBandExpertsV8, "ODD_ROWS_MAX_WEIGHTS", 98303)
+    assert torch.equal(mod(x, idx, w), loop) and len(calls) == 2
+    assert float((out.float() - loop.float()).norm() / loop.float().norm()) <= 1e-2      # (the loop rounds to bf16 four times)
