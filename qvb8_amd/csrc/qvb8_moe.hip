@@ -962,7 +962,7 @@ __global__ void __launch_bounds__(64 * kWalkWaves) moe_walk_wide_kernel(MoeWalkA
 template <int DT>
 __global__ void __launch_bounds__(256) moe_combine_kernel(const float* __restrict__ Yd, const float* __restrict__ w, void* __restrict__ out,
                                                           int topk, int D, int tokens, const int32_t* __restrict__ n_bad) {
-    const int t = blockIdx.y;
+    const int t = (int)(blockIdx.z * gridDim.y + blockIdx.y);
     const int d = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= tokens || d >= D) return;
     float acc = 0.f;
@@ -1006,7 +1006,9 @@ int launch_moe_gemv(int stage, MoeGemvArgs a, int64_t slots, hipStream_t s) {
     return host::check_launch("qvb8_moe_experts");
 }
 int launch_moe_combine(const float* Yd, const float* w, void* out, int out_dtype, int64_t topk, int64_t D, int64_t tokens, const MoePlan& pl, hipStream_t s) {
-    dim3 grid((unsigned)((D + 255) / 256), (unsigned)tokens);
+    const int64_t rows = std::min<int64_t>(tokens, 65535), layers = (tokens + rows - 1) / rows;       // a grid's y and z end at 65535
+    if (layers > 65535) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_moe_experts: too many tokens for one launch");
+    const dim3 grid((unsigned)((D + 255) / 256), (unsigned)rows, (unsigned)layers);
     if (out_dtype == QVB8_F32) hipLaunchKernelGGL(moe_combine_kernel<0>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)D, (int)tokens, pl.n_bad);
     else if (out_dtype == QVB8_F16) hipLaunchKernelGGL(moe_combine_kernel<1>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)D, (int)tokens, pl.n_bad);
     else hipLaunchKernelGGL(moe_combine_kernel<2>, grid, dim3(256), 0, s, Yd, w, out, (int)topk, (int)D, (int)tokens, pl.n_bad);

@@ -112,6 +112,9 @@ class QVBandExpertsV8(nn.Module):
     # the rows 9 bits wide: 16 pairs 4049 / 17287, 75 pairs 15259 / 81750, 150 pairs 19489 / 5636; 8 of 4096/4096, three quarters:
     # 16 pairs 24125 / 14425, 64 pairs 73024 / 48029, 150 pairs 104639 / 1548.
     ODD_ROWS_MAX_PAIRS, ODD_ROWS_MAX_WEIGHTS = 75, 2 ** 23
+    # The routed kernels keep H and the down results of all pairs of a call in fp32: tokens go through them in slices whose
+    # share stays below this (5957 tokens of a 2048/768 layer with 8 experts each).
+    SCRATCH_BYTES = 512 << 20
 
     def __init__(self, gate_up_experts, down_experts, *, num_experts: int, act_fn=None):
         super().__init__()
@@ -200,10 +203,29 @@ class QVBandExpertsV8(nn.Module):
             if not many:
                 return self._routed(hidden_states, top_k_index, top_k_weights, False)
             if not self._loop_is_faster(top_k_index.numel()):
-                out = self._routed(hidden_states, top_k_index.to(torch.int64), top_k_weights, True)
+                out = self._routed_in_slices(hidden_states, top_k_index.to(torch.int64), top_k_weights)
                 if out is not None:
                     return out
         return self._forward_loop(hidden_states, top_k_index, top_k_weights)
+
+    def _routed_in_slices(self, x: torch.Tensor, idx: torch.Tensor, w: torch.Tensor):
+        """_routed of many tokens, in equal slices of at most SCRATCH_BYTES of fp32 results (never as few tokens as the other
+        kernels take)."""
+        n_tok, per_token = idx.shape[0], 4 * idx.shape[1] * (self._stk[1]["P"] + self._stk[1]["Q"])
+        n = -(-n_tok // max(self.FUSED_MAX_TOKENS + 1, self.SCRATCH_BYTES // per_token))
+        while n > 1 and n_tok // n <= self.FUSED_MAX_TOKENS:
+            n -= 1
+        if n == 1:
+            return self._routed(x, idx, w, True)
+        out, at = [], 0
+        for i in range(n):
+            end = n_tok * (i + 1) // n
+            part = self._routed(x[at:end], idx[at:end], w[at:end], True)
+            if part is None:
+                return None
+            out.append(part)
+            at = end
+        return torch.cat(out)
 
     def _routed(self, x: torch.Tensor, idx: torch.Tensor, w: torch.Tensor, many: bool):
         """The routed kernels.  With more than FUSED_MAX_TOKENS tokens, None where an expert number lies outside 0..E-1: the loop
