@@ -5,6 +5,7 @@ import torch
 
 from qvb8_amd.kv import codec as C
 from qvb8_amd.kv import fused_attn as FA
+from tests.test_kv_host import lengths_and_segments_must_match
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -47,3 +48,8 @@ def test_a_bound_that_sixteen_bits_miss_is_refused():
     for dev in ("cpu", DEV):
         with pytest.raises(C.KVCertificateError):
             C.band_kv_heads(x.to(dev), torch.float32, 6, tau=1e-9)
+
+
+def test_lengths_and_segments_must_match_on_the_gpu():
+    """The kernel path paired segments with lengths until one of the two ran out: the rest was dropped without a word."""
+    lengths_and_segments_must_match(DEV)

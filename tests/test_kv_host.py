@@ -121,3 +121,18 @@ def test_only_whole_heads_go_to_the_unpacking_kernel():
     short = dataclasses.replace(bk, packed=bk.packed[:-1].clone())
     with pytest.raises(RuntimeError):
         FA.layout_from_segments([[short]], [[bk]], [40], "cpu")
+
+
+def lengths_and_segments_must_match(device):
+    seg = C.band_kv_heads(torch.randn(2, 40, 32, generator=torch.Generator().manual_seed(3)).to(device), torch.float32, 6)
+    two = [seg, seg]
+    for k, v, lens in ((two, two, [40]), (two, [seg], [40, 40]), ([seg], [seg], [40, 40]), (two, two, [])):
+        with pytest.raises(IndexError):
+            FA.layout_from_segments(k, v, lens, device)
+    whole = FA.layout_from_segments(two, two, [40, 40], device)
+    padded = FA.layout_from_segments(two, two, [40, 40, 0], device)              # an empty segment more: no tiles
+    assert whole.n == 80 and torch.equal(padded.ki, whole.ki) and torch.equal(padded.t_seg, whole.t_seg) and padded.n_tiles == whole.n_tiles
+
+
+def test_lengths_and_segments_must_match():
+    lengths_and_segments_must_match("cpu")
