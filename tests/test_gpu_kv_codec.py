@@ -53,3 +53,14 @@ def test_a_bound_that_sixteen_bits_miss_is_refused():
 def test_lengths_and_segments_must_match_on_the_gpu():
     """The kernel path paired segments with lengths until one of the two ran out: the rest was dropped without a word."""
     lengths_and_segments_must_match(DEV)
+
+
+@pytest.mark.parametrize("n_seg", [1, 256, 257, 600])
+def test_tile_tables_of_many_segments(n_seg):
+    """The table is filled 256 segments a launch: empty segments and ones of a single key among them."""
+    lens = [(7 * i) % 90 for i in range(n_seg - 1)] + [33]
+    parts = [torch.zeros(n_seg, 1, 128) for _ in range(4)]
+    ids = torch.zeros(sum(lens), 1, 128, dtype=torch.uint8)
+    want, got = (FA.QVLayout(ids.to(d), ids.to(d), *[p.to(d) for p in parts], lens, d) for d in ("cpu", DEV))
+    for name in ("t_start", "t_len", "t_seg"):
+        assert torch.equal(getattr(got, name).cpu(), getattr(want, name)), name

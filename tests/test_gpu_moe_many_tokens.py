@@ -128,3 +128,21 @@ def test_rows_that_claim_to_lie_in_planes_are_nan(T):
     out = ext.moe_experts(torch.randn(T, hidden, generator=g).to(DEV), idx.to(DEV), torch.rand(T, k, generator=g).to(DEV), *up[:4], marked,
                           2 * inter, hidden, *dn, hidden, inter)
     assert torch.equal(out.isnan().all(1).cpu(), (idx == 2).any(1)) and torch.equal(out.isnan().any(1).cpu(), (idx == 2).any(1))
+
+
+# 1024 threads place the pairs: one round of them and a ragged second one, more than the four rounds that are kept in registers,
+# more experts than the table of counts takes (turns), with more than a round of pairs there too, and one expert that gets all
+@pytest.mark.parametrize("T,E,k", [(550, 6, 2), (2100, 6, 2), (2049, 3, 2), (40, 513, 3), (700, 520, 2), (2100, 600, 2), (1100, 1, 1)])
+def test_routing_plans_of_many_pairs(T, E, k):
+    hidden = inter = 128
+    made = min(E, 8)
+    up, Wup = _hand_made_stack(made, 2 * inter, hidden, [6, 7, 5, 8], seed=4)
+    dn, Wdn = _hand_made_stack(made, hidden, inter, [5, 6], seed=8)
+    same = torch.arange(E, device=DEV) % made                    # expert e holds the rows of expert e % 8
+    up, dn = ((s[0], *[t[same].contiguous() for t in s[1:]]) for s in (up, dn))
+    g = torch.Generator().manual_seed(T + E)
+    idx = torch.rand(T, E, generator=g).topk(k, 1).indices
+    w = torch.rand(T, k, generator=g) + 0.1
+    x = torch.randn(T, hidden, generator=g).half()
+    out = ext.moe_experts(x.to(DEV), idx.to(DEV), w.to(DEV), *up, 2 * inter, hidden, *dn, hidden, inter, checked=True)
+    _check(out, O.moe_reference(x.float().numpy(), (idx % made).numpy(), w.numpy(), Wup, Wdn), torch.float16)
