@@ -380,9 +380,10 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
 // 64 bits over 33 .. 1024 rows.)
 // Two workgroups per CU (78 KB of LDS, at most 256 registers): one restores while the other one's products run.
 // Bound by what a CU issues beside its products (restoring, exp2, conversions): 720 rows x 4 kv heads over 16001 keys of 256
-// channels 251.6 us in the row-block kernel (32 rows share a tile), 100.7 us here = 0.47 PFLOP/s; one workgroup per CU 133.  The
-// ids of tile t + 2 are asked for between the two products: asked for before the first one, the sixteen registers they come back to are
-// spilled away from Q (118 us against 133 for the whole call).
+// channels 251.6 us in the row-block kernel (32 rows share a tile), 108.7 us here = 0.43 PFLOP/s, of which rescaling O takes 4.7.  Two
+// workgroups per CU against one, and the ids of tile t + 2 asked for between the two products against before the first one (the
+// sixteen registers they come back to are then spilled away from Q): 100.7 against 133 and 118 against 133 for the whole
+// call, measured with the lagging reference.
 constexpr int kWideRows = 128, kWaveRows = 32;
 constexpr int kWideFrom = 33;                                 // fewest rows that take it: fused_attn.py has the measurements
 constexpr int kVRow = kKeys + 8;                              // halfs per row of V in LDS

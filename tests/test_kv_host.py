@@ -136,3 +136,20 @@ def lengths_and_segments_must_match(device):
 
 def test_lengths_and_segments_must_match():
     lengths_and_segments_must_match("cpu")
+
+
+def test_split_plans(monkeypatch):
+    """As many splits as workgroups fit the card at once, by the kernel that takes the rows; a forced row-block kernel is planned
+    for as such."""
+    import types
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda device: types.SimpleNamespace(multi_processor_count=256))
+    monkeypatch.delenv("QVB8_ATTN_WG_PER_CU", raising=False)
+    monkeypatch.delenv("QVB8_ATTN_ROW_BLOCKS", raising=False)
+    plan = lambda rows, **kw: FA.plan_splits(4096, 4, rows, "cuda", **kw)                  # noqa: E731
+    assert plan(16) == (22, 187) and plan(32) == (32, 128)                       # 3 and 2 workgroups on each of 256 CUs, over 4 heads
+    assert plan(33) == plan(128) == (32, 128) and plan(129) == (64, 64)          # 128 rows share a workgroup
+    assert plan(33, d=128) == (22, 187) and plan(33, wide=True) == (64, 64)
+    monkeypatch.setenv("QVB8_ATTN_ROW_BLOCKS", "1")
+    assert plan(33) == (64, 64) and plan(96) == (128, 32)                        # 16 rows: 3 and 6 row blocks
+    monkeypatch.setenv("QVB8_ATTN_ROW_BLOCKS", "4")
+    assert plan(33, d=128) == (32, 128) and plan(33) == (64, 64)                 # 64 rows; 256 channels: 32 at most
