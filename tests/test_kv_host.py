@@ -149,6 +149,8 @@ def test_split_plans(monkeypatch):
     assert plan(16) == (22, 187) and plan(32) == (32, 128)                       # 3 and 2 workgroups on each of 256 CUs, over 4 heads
     assert plan(33) == plan(128) == (32, 128) and plan(129) == (64, 64)          # 128 rows share a workgroup
     assert plan(33, d=128) == (22, 187) and plan(33, wide=True) == (64, 64)
+    short = lambda rows: FA.plan_splits(188, 2, rows, "cuda")[0]                 # noqa: E731
+    assert short(512) == short(520) == 8 and short(120) == 3                     # short splits: no step where a fifth row block begins
     monkeypatch.setenv("QVB8_ATTN_ROW_BLOCKS", "1")
     assert plan(33) == (64, 64) and plan(96) == (128, 32)                        # 16 rows: 3 and 6 row blocks
     monkeypatch.setenv("QVB8_ATTN_ROW_BLOCKS", "4")
