@@ -689,7 +689,6 @@ template <int D, typename T>
 int launch_attn_wide(const AttnArgs& a, int64_t n_splits, hipStream_t s) {
     if (int rc = host::raise_lds_limit<attn_wide_kernel<D, T>>(wide_lds(D), "qvb8_attn_fwd")) return rc;
     const dim3 grid((unsigned)a.nhkv, (unsigned)n_splits, (unsigned)((a.n_rows + kWideRows - 1) / kWideRows));
-    if (grid.z > 65535u) return host::fail(-1, "qvb8_attn_fwd: %d rows are more than one launch takes", a.n_rows);
     hipLaunchKernelGGL((attn_wide_kernel<D, T>), grid, dim3(kAttnThreads), wide_lds(D), s, a);
     return host::check_launch("qvb8_attn_fwd");
 }

@@ -184,7 +184,7 @@ class QVBandExpertsV8(nn.Module):
             return False
         if x.dim() != 2 or idx.dim() != 2 or w.shape != idx.shape or x.shape != (idx.shape[0], self.gate_up_experts[0].in_features):
             return False
-        if idx.device != x.device or w.device != x.device or not self._whole_steps():
+        if idx.device != x.device or w.device != x.device or self.gate_up_experts[0].ids.device != x.device or not self._whole_steps():
             return False
         if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
             return False
