@@ -1232,8 +1232,10 @@ extern "C" int qvb8_moe_experts_checked(const void* X, int x_dtype, int64_t toke
     if (tokens <= 16) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_moe_experts_checked: 17 tokens or more");
     __atomic_store_n(bad_pairs, -1, __ATOMIC_RELEASE);
     if (int rc = moe_experts(X, x_dtype, tokens, idx, w, topk, n_experts, up_ids, up_ids_bytes, up_min, up_tau, up_nb, up_off, Q_up, P_up,
-                             dn_ids, dn_ids_bytes, dn_min, dn_tau, dn_nb, dn_off, Q_dn, P_dn, act, out, out_dtype, workspace, workspace_bytes, bad_pairs, stream))
+                             dn_ids, dn_ids_bytes, dn_min, dn_tau, dn_nb, dn_off, Q_dn, P_dn, act, out, out_dtype, workspace, workspace_bytes, bad_pairs, stream)) {
+        (void)hipStreamSynchronize((hipStream_t)stream);       // a plan launched before the failure still writes the counter
         return rc;
+    }
     // The plan kernel writes the counter in the middle of its work; the products are queued behind it by now.  (An event between
     // the two, waited for instead, put 8 us of idle GPU there.)  The wait ends with the stream at the latest.
     for (int64_t spins = 1; __atomic_load_n(bad_pairs, __ATOMIC_ACQUIRE) < 0; ++spins) {
