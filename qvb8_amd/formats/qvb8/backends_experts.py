@@ -167,7 +167,10 @@ class QVBandExpertsV8(nn.Module):
         return self
 
     def _loop_is_faster(self, n_pairs: int) -> bool:
-        """Whether a call of so many (token, choice) pairs is the loop's, going by the pairs an expert gets on average."""
+        """Whether a call of so many (token, choice) pairs is the loop's, going by the pairs an expert gets on average.  Never
+        inside a graph capture: the loop reads the routing back."""
+        if torch.cuda.is_current_stream_capturing():
+            return False
         g, d = self._stk
         pairs, weights = n_pairs / self.num_experts, g["Q"] * g["P"] + d["Q"] * d["P"]
         if os.environ.get("QVB8_MOE_GROUPED", "1") == "0":           # the kernels are switched off

@@ -105,15 +105,22 @@ def test_expert_numbers_outside_the_stack(T):
     assert torch.equal(mod(x, idx, w), want)
 
 
-def test_many_tokens_inside_a_graph():
-    """Captured and replayed with other inputs in the same buffers, eager calls between the replays."""
+@pytest.mark.parametrize("loop_is_faster", [False, True])
+def test_many_tokens_inside_a_graph(loop_is_faster, monkeypatch):
+    """Captured and replayed with other inputs in the same buffers, eager calls between the replays -- also where the loop, which
+    cannot be captured, would be the faster one."""
     mod = _module()
     x, idx, w = _call(90)
     mod(x, idx, w)
     torch.cuda.synchronize()
+    limit = QVBandExpertsV8.LOOP_FROM_PAIRS
+    if loop_is_faster:
+        monkeypatch.setattr(QVBandExpertsV8, "LOOP_FROM_PAIRS", 1)
+        monkeypatch.setattr(QVBandExpertsV8, "LOOP_FROM_PRODUCTS", 0)
     graph = torch.cuda.CUDAGraph()
     with torch.no_grad(), torch.cuda.graph(graph):
         out = mod(x, idx, w)
+    monkeypatch.setattr(QVBandExpertsV8, "LOOP_FROM_PAIRS", limit)
     for seed in range(3):
         nx, nidx, nw = _call(90, seed=10 + seed)
         x.copy_(nx), idx.copy_(nidx), w.copy_(nw)
