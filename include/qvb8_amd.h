@@ -53,9 +53,9 @@ enum qvb8_status {
 /* Library identification: ABI version, bumped on any signature change or new entry point (3: row lookup, attention over
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
  * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*;
- * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked).  A binding compares the loaded library's answer
+ * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
-#define QVB8_ABI_VERSION 10
+#define QVB8_ABI_VERSION 11
 int qvb8_abi_version(void);
 /* Message of the calling thread's most recent failure ("" if none). Valid until that thread's next call. */
 const char* qvb8_last_error(void);
@@ -134,10 +134,16 @@ enum qvb8_mma_flags {
     QVB8_MMA_Y_BF16 = 4,      /* otherwise store; likewise bf16.  Only for a weight without escapes (n_esc == 0): the escape
                                  correction adds to fp32 results.  Saves the caller's cast pass over Y (the reference's
                                  operator casts the extension's fp32 result, formats/qvb8/module.py:430-441). */
-    QVB8_MMA_PLANES = 8       /* the pack has rows stored in planes (bit 62 of their bit_off, see "rows stored in planes"
+    QVB8_MMA_PLANES = 8,      /* the pack has rows stored in planes (bit 62 of their bit_off, see "rows stored in planes"
                                  above): with a row layout these are the rows of every whole 16-row tile that lies inside
                                  one run of a width 4..8; without one, whatever rows the records mark.  The call then asks
                                  for ids in operand order with non-temporal loads. */
+    QVB8_MMA_SILU_PAIRS = 16  /* gate and up of a gated MLP, the activation applied: positions 16 t .. 16 t + 7 are eight gate rows,
+                                 16 t + 8 .. 16 t + 15 the up rows of the same outputs (row Q / 2 + j when position 16 t + r is
+                                 row j; a pair that breaks this gives NaN), and Y is (M, Q / 2) = silu(gate) * up, both products,
+                                 SiLU and the result rounded to Y's type.  Needs QVB8_MMA_Y_F16 or _BF16, a row layout of whole
+                                 16-row tiles, no escapes, M <= 16.  The reference launches it as a kernel of its own between
+                                 the products (decode/fused_pointwise.py:60-67). */
 };
 
 /* Row records of the matrix-core path: qvb8_mma_rowinfo_bytes(Q) bytes (24 per row, 8-byte aligned), in tile order
@@ -218,7 +224,8 @@ int qvb8_launch_probe(int64_t blocks, int64_t threads, int64_t lds_bytes, void* 
  * escapes), row records from qvb8_mma_prepare for the same order.  gate+up is ONE pack of 2 * inter rows (rows
  * 0..inter-1 gate, the rest up) whose position order goes unit by unit: positions 32 u .. 32 u + 15 hold 16 gate rows,
  * 32 u + 16 .. 32 u + 31 the up rows of the same outputs (position 32 u + 16 + r is row inter + j when position 32 u + r is
- * row j; a pair that breaks this gives NaN for that output).  down: out_features rows of inter columns.
+ * row j; a pair that breaks this gives NaN for that output) -- or, unit by unit, each of its two tiles holds 8 gate rows and
+ * the 8 up rows of the same outputs, the order of QVB8_MMA_SILU_PAIRS.  down: out_features rows of inter columns.
  * hidden % 128 == 0, inter % 128 == 0, out_features % 16 == 0; anything else: QVB8_ERR_UNSUPPORTED (call the products
  * separately).  The weights' buffers must stay where they are while the plan is in use.
  * `workspace`: qvb8_mlp_workspace_bytes(inter) bytes of device memory, 16-byte aligned, the library's from qvb8_mlp_init

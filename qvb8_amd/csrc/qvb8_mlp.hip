@@ -309,11 +309,12 @@ __global__ void __launch_bounds__(kMlpThreads) mlp_kernel(const uint16_t* __rest
     auto publish = [&](int lu, int first_item, int stride) __attribute__((always_inline)) {
         const int valid1 = ranges1 < kMlpTileWaves ? ranges1 : kMlpTileWaves;
         const int items = kTileRows * M;
+        const bool halves = s_fin1[lu * 32 + 8].z >= (uint32_t)I;      // the unit's tiles hold 8 + 8 rows each, not 16 gate and 16 up
         for (int first = first_item; first < items; first += stride) {
             const int i = first + (lane >> 4), w = lane & 15;
             const bool item = i < items;
             const int rr = item ? i / M : 0, t = item ? i - rr * M : 0;
-            const int grow = lu * 32 + rr, urow = grow + 16;
+            const int grow = lu * 32 + (halves ? (rr & 7) + 2 * (rr & 8) : rr), urow = grow + (halves ? 8 : 16);
             const bool live = item && w < valid1;
             const int wr = live ? w : 0;
             const float pg = part1[((size_t)grow * kMlpTileWaves + wr) * M + t], pu = part1[((size_t)urow * kMlpTileWaves + wr) * M + t];

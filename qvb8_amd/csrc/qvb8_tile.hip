@@ -42,6 +42,15 @@ __device__ __forceinline__ void store_y(float* Y, int out_dt, int64_t i, float v
     else store_from_f32<2>(Y, i, v);
 }
 
+// silu(g) * u with every step rounded to the type `dt` (0 fp32, 1 fp16, 2 bf16)
+__device__ __forceinline__ float round_to(float v, int dt) {
+    return dt == 1 ? f16_bits_to_f32(f32_to_f16_bits(v)) : dt == 2 ? bf16_bits_to_f32(f32_to_bf16_bits(v)) : v;
+}
+__device__ __forceinline__ float silu_times(float yg, float yu, int dt) {
+    const float g = round_to(yg, dt), u = round_to(yu, dt);
+    return round_to(g / (1.0f + expf(-g)), dt) * u;             // (rounded when it is stored)
+}
+
 struct TileArgs {
     const uint16_t* X;            // (M, P) fp16 or bf16 bits
     const uint8_t* ids;
@@ -51,6 +60,7 @@ struct TileArgs {
     int64_t ids_bytes;
     int M, Q, P;
     int out_dt;                   // what Y holds: 0 fp32, 1 fp16, 2 bf16
+    int silu_pairs;               // a tile is 8 gate rows and the 8 up rows of the same outputs: Y (M, Q / 2) = silu(gate) * up
     int n_steps;                  // P / 128
     int W, G, panels;             // waves per tile, tile groups per workgroup, column panels
     int TW;                       // tiles per workgroup (multiple of G)
@@ -122,7 +132,8 @@ __global__ void __launch_bounds__((64 * tile_max_waves<NT, T, BF, PL>())) tile_k
     TileArgs a;
     a.X = X; a.ids = ids; a.loc = loc; a.fin = reinterpret_cast<const uint4*>(loc + rowinfo_loc_words(Q)); a.Y = Y;
     a.ids_bytes = ids_bytes; a.Q = Q; a.P = P; a.n_steps = P / kStepCols; a.TW = TW;
-    a.M = (int)(counts & 63u); a.out_dt = (int)((counts >> 6) & 3u); a.W = (int)((counts >> 8) & 15u); a.G = (int)((counts >> 12) & 15u); a.panels = (int)(counts >> 16);
+    a.M = (int)(counts & 63u); a.out_dt = (int)((counts >> 6) & 3u); a.W = (int)((counts >> 8) & 15u); a.G = (int)((counts >> 12) & 15u); a.panels = (int)((counts >> 16) & 0x7fffu);
+    a.silu_pairs = (int)(counts >> 31);
     a.first1 = first1; a.first2 = first2; a.n_classes = (int)((widths >> 24) & 0x7Fu); a.planes = PL ? 1 : 0;
     a.nb[0] = (int)(widths & 255u); a.nb[1] = (int)((widths >> 8) & 255u); a.nb[2] = (int)((widths >> 16) & 255u);
     using F = Fmt<BF>;
@@ -549,6 +560,53 @@ __global__ void __launch_bounds__((64 * tile_max_waves<NT, T, BF, PL>())) tile_k
     const int valid_ranges = all_ranges < ranges ? all_ranges : ranges;      // waves without any column never stored
     const int n_items = tiles_here * kTileRows * a.M;
     const int n_waves_here = (int)blockDim.x >> 6;
+    if (a.silu_pairs) {
+        // Gate and up of an output meet here: the activation is applied to the sums and Y holds the down product's input.  As
+        // launches of their own -- torch's SiLU and multiplication between the two products -- they cost a decode step of the 9B
+        // shapes 3.3 us a layer, a quarter of the down launch, for 50 KB of data (four layers 199.1 -> 186.0 us).  Both rows of an output lie in one
+        // tile (8 + 8 rows), so tiles are dealt to workgroups as for any other weight.
+        // y is rounded to Y's type where the separate chain rounds: both products, SiLU, the result.
+        const int half_q = a.Q >> 1, n_out = n_items >> 1;
+        auto put = [&](int rg, int t, double dg, double du, double xsum) __attribute__((always_inline)) {
+            const uint4 fg = s_fin[rg], fu = s_fin[rg + kTileRows / 2];
+            const float yg = (float)((double)__uint_as_float(fg.x) * dg + (double)__uint_as_float(fg.y) * xsum);
+            const float yu = (float)((double)__uint_as_float(fu.x) * du + (double)__uint_as_float(fu.y) * xsum);
+            float y = silu_times(yg, yu, a.out_dt);
+            if (fu.z != fg.z + (uint32_t)half_q) {                                // not the gate row's partner: whatever outputs lie here
+                y = __builtin_nanf("");
+                if (fu.z < (uint32_t)half_q) store_y(a.Y, a.out_dt, (int64_t)t * half_q + fu.z, y);
+            }
+            if (fg.z < (uint32_t)half_q) store_y(a.Y, a.out_dt, (int64_t)t * half_q + fg.z, y);
+        };
+        if (n_out <= 4 * n_waves_here) {
+            const int i = wave * 4 + (lane >> 4), w = lane & 15;                  // sixteen lanes an output, as below
+            const bool item = i < n_out;
+            const int o = item ? i / a.M : 0, t = item ? i - o * a.M : 0;
+            const int rg = (o >> 3) * kTileRows + (o & 7);
+            const bool live = item && w < valid_ranges;
+            const int wr = live ? w : 0;
+            const float pg = part[((size_t)rg * ranges + wr) * MS + t], pu = part[((size_t)(rg + kTileRows / 2) * ranges + wr) * MS + t], sv = sxs[wr * TM + t];
+            double dg = live ? (double)pg : 0.0, du = live ? (double)pu : 0.0, xsum = live ? (double)sv : 0.0;
+            dg += row16_from<8>(dg); du += row16_from<8>(du); xsum += row16_from<8>(xsum);
+            dg += row16_from<4>(dg); du += row16_from<4>(du); xsum += row16_from<4>(xsum);
+            dg += row16_from<2>(dg); du += row16_from<2>(du); xsum += row16_from<2>(xsum);
+            dg += row16_from<1>(dg); du += row16_from<1>(du); xsum += row16_from<1>(xsum);
+            if (item && w == 0) put(rg, t, dg, du, xsum);
+            return;
+        }
+        for (int i = tid; i < n_out; i += blockDim.x) {
+            const int o = i / a.M, t = i - o * a.M;
+            const int rg = (o >> 3) * kTileRows + (o & 7);
+            double dg = 0.0, du = 0.0, xsum = 0.0;
+            for (int w = 0; w < valid_ranges; ++w) {
+                dg += (double)part[((size_t)rg * ranges + w) * MS + t];
+                du += (double)part[((size_t)(rg + kTileRows / 2) * ranges + w) * MS + t];
+                xsum += (double)sxs[w * TM + t];
+            }
+            put(rg, t, dg, du, xsum);
+        }
+        return;
+    }
     if (n_items <= 4 * n_waves_here) {
         // Few results (one token, a few tiles): a thread per (result, range) instead of a thread per result that walks
         // the ranges one LDS trip after the other while every other wave idles.  Sixteen neighbouring lanes hold a result's
@@ -1310,8 +1368,9 @@ int launch_tile(TileArgs& a, hipStream_t s) {
             return host::fail(QVB8_ERR_LAUNCH, "qvb8_mma: cannot raise the kernel's LDS limit");
         attr[dev] = true;
     }
-    if (pl.panels > 0xffff) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_mma: rows too long");
-    const uint32_t counts = (uint32_t)a.M | ((uint32_t)a.out_dt << 6) | ((uint32_t)a.W << 8) | ((uint32_t)a.G << 12) | ((uint32_t)a.panels << 16);
+    if (pl.panels > 0x7fff) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_mma: rows too long");
+    const uint32_t counts = (uint32_t)a.M | ((uint32_t)a.out_dt << 6) | ((uint32_t)a.W << 8) | ((uint32_t)a.G << 12) | ((uint32_t)a.panels << 16)
+                            | ((uint32_t)a.silu_pairs << 31);
     hipLaunchKernelGGL((tile_kernel<NT, T, BF, XC, XP, PL>), dim3(pl.blocks), dim3(pl.threads), pl.lds, s,
                        a.X, a.ids, a.loc, a.Y, a.ids_bytes, a.Q, a.P, counts, a.TW, a.first1, a.first2,
                        (uint32_t)a.nb[0] | ((uint32_t)a.nb[1] << 8) | ((uint32_t)a.nb[2] << 16) | ((uint32_t)a.n_classes << 24));
@@ -1563,6 +1622,14 @@ extern "C" int qvb8_mma(const void* X, int x_dtype, int64_t M,
     const int out_dt = (flags & QVB8_MMA_Y_F16) ? 1 : (flags & QVB8_MMA_Y_BF16) ? 2 : 0;
     a.planes = (flags & QVB8_MMA_PLANES) ? 1 : 0;
     if (out_dt != 0 && n_esc > 0) return host::fail(QVB8_ERR_ARG, "qvb8_mma: fp16 / bf16 results need a weight without escapes (the correction adds to fp32 results)");
+    a.silu_pairs = (flags & QVB8_MMA_SILU_PAIRS) ? 1 : 0;
+    if (a.silu_pairs) {
+        if (!layout || out_dt == 0 || M > 16)
+            return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_mma: SiLU of row pairs needs a row layout, fp16 / bf16 results and at most 16 rows of X");
+        bool whole = Q % kTileRows == 0;
+        for (int c = 0; c < a.n_classes; ++c) whole = whole && layout->first_pos[c] % kTileRows == 0;
+        if (!whole) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_mma: SiLU of row pairs needs whole 16-row tiles of one width");
+    }
     a.Y = Y; a.out_dt = out_dt; a.ids_bytes = ids_bytes; a.M = (int)M; a.Q = (int)Q; a.P = (int)P; a.n_steps = (int)(P / kStepCols);
     // mode 0: fp16 X, fp16 operands; 1: bf16 X narrowed to saturated fp16 on the way in, fp16 operands; 2: bf16 operands
     const int mode = x_dtype == QVB8_F16 ? 0 : (flags & QVB8_MMA_SATURATE_X) ? 1 : 2;

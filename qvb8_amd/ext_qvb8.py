@@ -181,6 +181,7 @@ MMA_GEMM_MAX_M = 256          # with a row layout (rows stored in width order, w
 MMA_SATURATE_X = 1
 MMA_Y_F16, MMA_Y_BF16 = 2, 4                      # qvb8_mma_flags: results stored as fp16 / bf16
 MMA_PLANES = 8                                    # qvb8_mma_flags: the pack has rows stored in planes
+MMA_SILU_PAIRS, MMA_SILU_MAX_M = 16, 16           # qvb8_mma_flags: tiles of 8 gate and 8 up rows, the activation applied; its most rows of X
 
 
 def mma_prepare(row_nbits, row_bit_off, tau_s, min_s, P, ids_bytes, perm=None):
@@ -422,7 +423,7 @@ def sort_rows_by_width(ids, row_nbits, row_bit_off, P, perm, planes=False):
 
 
 def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, perm=None, saturate=True,
-              rowinfo=None, layout=None, out_dtype=None, planes=False):
+              rowinfo=None, layout=None, out_dtype=None, planes=False, silu_pairs=False):
     """Matrix-core path for P % 128 == 0: X (fp16 or bf16) times the fp32 band value, fp32 (M, Q).  1 <= M <= 48 always;
     49 <= M <= 256 (the workgroup-tiled decode + GEMM kernel) when `layout` is given and its widths are 4..8.
     `perm` (int32, position -> row) groups rows of equal width into tiles; `rowinfo` = mma_prepare(...) for the
@@ -431,7 +432,8 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
     is loaded and the product runs on fp16 operands, as every fp16 path of the reference does; without it bf16 X is
     multiplied as it is on bf16 operands.  `out_dtype` torch.float16 / torch.bfloat16: the kernels store the results
     rounded to that type (the same values as casting the fp32 result; only for a weight without escapes).  `planes`:
-    the pack has rows stored in planes (sort_rows_by_width(planes=True))."""
+    the pack has rows stored in planes (sort_rows_by_width(planes=True)).  `silu_pairs` (fp16 / bf16 results, at most 16
+    rows of X, rows stored by QVBandMLPV8): (M, Q / 2) silu(gate) * up, rounded at every step."""
     lib = _lib.load()
     Q = _check_pack(ids, min_s, row_nbits, row_bit_off, tau_s)
     n_esc = _check_escapes(esc_idx, esc_vals)
@@ -466,7 +468,7 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
             out_dtype, y_flag = torch.float32, 0
         else:
             raise RuntimeError("qvb8 mma-multi: results are fp32, fp16 or bf16")
-        Y = torch.empty((M, Q), dtype=out_dtype, device=Xc.device)
+        Y = torch.empty((M, Q // 2 if silu_pairs else Q), dtype=out_dtype, device=Xc.device)
         ei = esc_idx.contiguous() if n_esc else None
         ev = esc_vals.contiguous() if n_esc else None
         need = lib.qvb8_mma_workspace_bytes(M, Q, int(P))          # row records when none are passed; more for the tiled kernel
@@ -477,7 +479,8 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
                                  Q, int(P), _lib.ptr(ei), _lib.ptr(ev), n_esc, _lib.ptr(perm),
                                  None if rowinfo is None else rowinfo.contiguous().data_ptr(),
                                  None if layout is None else ctypes.addressof(layout),
-                                 (MMA_SATURATE_X if saturate else 0) | y_flag | (MMA_PLANES if planes else 0), _lib.ptr(Y),
+                                 (MMA_SATURATE_X if saturate else 0) | y_flag | (MMA_PLANES if planes else 0)
+                                 | (MMA_SILU_PAIRS if silu_pairs else 0), _lib.ptr(Y),
                                  None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel() * 8,
                                  _lib.stream_of(Xc)), lib)
     return Y

@@ -20,6 +20,7 @@ import os
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from qvb8_amd import ext_qvb8 as ext
 from .fuse import concat_linears
@@ -53,6 +54,13 @@ def unit_order(nbits: torch.Tensor, inter: int):
     return perm, new_nbits
 
 
+def tiles_of_pairs(perm: torch.Tensor) -> torch.Tensor:
+    """unit_order's positions with the rows of every unit dealt to its two tiles as 8 gate rows and the 8 up rows of the same
+    outputs (ext.MMA_SILU_PAIRS): each tile holds both sides of its outputs, so a launch may deal single tiles to its workgroups and
+    still apply the activation itself."""
+    return perm.view(-1, 2, 2, UNIT // 2).transpose(1, 2).reshape(-1).contiguous()
+
+
 def _whole_tiles(layout, rows: int) -> bool:
     return all(int(layout.first_pos[c]) % rows == 0 for c in range(int(layout.n_classes) + 1)) and \
         all(4 <= int(layout.nbits[c]) <= 8 for c in range(int(layout.n_classes)))
@@ -63,7 +71,8 @@ class QVBandMLPV8(nn.Module):
 
     max_rows = ext.MLP_MAX_ROWS
     # Whether 1..4 rows take the one-launch kernel.  Off by default: measured on the 9B shapes (hidden 4096, inter 12288) the
-    # one launch takes 29.6 us against 30.0 us for the two separate launches -- the hand-over inside the grid costs what the
+    # one launch takes 29.6 us against 30.0 us for the two separate launches (the activation counted on neither side; since
+    # the gate+up launch applies it itself it costs the separate launches nothing) -- the hand-over inside the grid costs what the
     # launch it saves costs (see the kernel's source) --, so the separate products, which every other row count uses anyway,
     # stay the default.  QVB8_MLP_FUSED=1 in the environment (or True here) switches it on.
     one_launch = False
@@ -76,12 +85,12 @@ class QVBandMLPV8(nn.Module):
         self.in_features = self.hidden
         self.gate_up = concat_linears([gate, up])[0]
         self.down = down
-        self.fused_ready = False
+        self.fused_ready = self._pairs_stored = False
         self._ws = self._plan = None
         self._prepare_fused()
 
     def _prepare_fused(self):
-        """Stores gate+up unit by unit and down in width order, both in planes; fused_ready says whether the one-launch
+        """Stores gate+up unit by unit (tiles_of_pairs) and down in width order, both in planes; fused_ready says whether the one-launch
         kernel can read them (no bias, no escapes, widths 4..8, at most three widths each, whole tiles)."""
         gu, dn = self.gate_up, self.down
         ok = (gu.ids.is_cuda and gu.bias is None and dn.bias is None and not gu.esc_idx.numel() and not dn.esc_idx.numel()
@@ -90,7 +99,8 @@ class QVBandMLPV8(nn.Module):
               and os.environ.get("QVB8_PLANES", "1") != "0")
         if ok:
             order = unit_order(gu.nbits, self.inter)
-            ok = order is not None and gu.store_in_order(*order)
+            ok = order is not None and gu.store_in_order(tiles_of_pairs(order[0]), order[1])
+            self._pairs_stored = self._pairs_stored or ok
         if ok:
             d = dn._mma_order()
             ok = d is not None and d[2] is not None and dn._planes and _whole_tiles(d[2], 16)
@@ -113,10 +123,32 @@ class QVBandMLPV8(nn.Module):
         return self._ws is not None and bool(self._ws[:8].view(torch.int32)[1].item())
 
     def separate(self, rows: torch.Tensor) -> torch.Tensor:
-        """The same chain with the two products launched separately (any row count and type)."""
+        """The same chain with the two products launched separately (any row count and type).  Up to 16 rows the gate+up launch
+        applies the activation to its sums and hands on what the down product reads: two launches, where SiLU and the product by
+        torch's kernels made four (a decode step of four 9B layers 199.1 -> 186.0 us)."""
+        h = self._activated(rows)
+        if h is not None:
+            return self.down(h)
         gu = self.gate_up(rows)
         g, u = gu[..., :self.inter], gu[..., self.inter:]
         return self.down(F.silu(g) * u)
+
+    def _activated(self, rows: torch.Tensor):
+        """silu(gate(rows)) * up(rows) as one launch, or None where that launch does not do what the separate calls do: other
+        types and layouts, and hooks that expect to see the gate+up product."""
+        gu = self.gate_up
+        if not (self._pairs_stored and rows.dtype in (torch.float16, torch.bfloat16) and rows.dim() == 2 and 1 <= rows.shape[0] <= ext.MMA_SILU_MAX_M
+                and rows.shape[1] == self.hidden and rows.is_contiguous() and rows.device == gu.min_s.device):
+            return None
+        if gu._forward_hooks or gu._forward_pre_hooks or _has_any_global_hook():
+            return None
+        order = gu._mma_order()
+        if order is None or order[2] is None:
+            return None
+        perm, rowinfo, layout = order
+        bf16_mode = bool(gu.bf16_certified) and rows.dtype == torch.bfloat16
+        return ext.mma_tiles(rows, gu.ids, gu.min_s, gu.nbits, gu.bit_off, self.hidden, gu.tau_s, None, None, perm=perm, saturate=not bf16_mode,
+                             rowinfo=rowinfo, layout=layout, out_dtype=rows.dtype, planes=gu._planes, silu_pairs=True)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         rows, out_dtype = activation_rows(x, self.gate_up.min_s.device)
