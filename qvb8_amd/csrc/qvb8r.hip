@@ -31,7 +31,8 @@ namespace qvb8 {
 
 constexpr int kRTiles = 8;             // tiles per workgroup (two per wave)
 constexpr int kRThreads = 32 * kRTiles;
-constexpr int kRing = 256;             // 32-bit words per tile ring: a pair takes <= 32, refilled every kRing / 2
+constexpr int kRing = 256;             // 32-bit words of a tile's window in LDS
+constexpr int kHalfRing = kRing / 2;
 
 struct RCore {
     const uint32_t* words; int64_t n_words;      // stream + at least 2048 zero words of pad (n_words counts the pad)
@@ -45,77 +46,138 @@ struct RCore {
     int n_tiles, n_blocks, K, Q, P;
 };
 
+// The walk of one tile.  Its words lie in a window of LDS that does not wrap: word `ptr` of the window is the next one to be
+// taken, and its address is its index and nothing else.  When half the window has been used, the other half moves to the front
+// and the next 128 words, asked for half a window ago, follow from registers.
+// A half without a tile or row walks along with the wave's other half on what it holds (never past `room`).
 struct Walker {
     uint32_t xl, xh;
-    int ptr, sb;
-    uint32_t pre[kRing / 64];
+    int ptr;                           // next word of the window, counted from the wave's first one
+    int sb;                            // the window's first word, counted from the tile's
+    uint32_t upper;                    // all ones in the upper half of the wave, zero in the lower
+    uint32_t pre[kHalfRing / 32];
     const uint32_t* wp;
 };
 
-// Returns the last word index (from the tile's first word) the walk may read ahead to: the end of the buffer, and -- when
-// the next tile's words follow this tile's, as every writer lays them out -- the tile's own last word.  The ring always
+// Per-workgroup set-up shared by the kernels: slot table into LDS, this half-wave's tile.
+//
+// `room` is the last word index (from the tile's first word) the walk may read ahead to: the end of the buffer, and -- when
+// the next tile's words follow this tile's, as every writer lays them out -- the tile's own last word.  The window always
 // asks for 128..384 words more than the walk has used; past the tile's end those lines belong to a tile that another
 // workgroup walks at another time, so they came from memory twice (measured at the 65B shapes, one row per tile of 1150
 // words: 325 MB fetched for 267 MB of stream).  Requests past the bound read the bound's word again.
-__device__ __forceinline__ int64_t walk_init(Walker& z, uint32_t* rg, const RCore& c, int tile, int l32) {
-    int64_t off = c.tile_off[tile];
-    const int64_t next = c.tile_off[tile + 1];
-    const int64_t last = c.n_words - (kRing + kRing / 2);                  // the furthest start that keeps every read inside
+//
+// A workgroup's start is a chain of trips to memory: its block, then the tile's place, then its first words; the slot table's 16
+// KB are asked for between the last two, all of them at once (a loop that waits for every 1 KB of them took longer than a fifth
+// of a short launch: 17408 x 5120, one row of X, 61.1 us a call with it, 55.0 without).
+struct TileCtx { bool has; int tile, r0, nr; int64_t room; };
+__device__ __forceinline__ TileCtx block_setup(Walker& z, const RCore& c, int block, uint32_t* st, uint32_t* own, int h8, int l32) {
+    int cls = c.blocks[3 * block], tb = c.blocks[3 * block + 1], ntb = c.blocks[3 * block + 2];
+    cls = cls < 0 ? 0 : (cls >= c.K ? c.K - 1 : cls);
+    TileCtx t;
+    t.tile = tb + h8;
+    t.has = h8 < ntb && t.tile >= 0 && t.tile < c.n_tiles;
+    if (!t.has) t.tile = 0;
+    int64_t off = c.tile_off[t.tile];
+    const int64_t next = c.tile_off[t.tile + 1];
+    const uint64_t s = c.states[(int64_t)t.tile * 32 + l32];
+    t.r0 = (int)c.tiles[3 * (int64_t)t.tile + 1];
+    t.nr = (int)c.tiles[3 * (int64_t)t.tile + 2];
+    constexpr int kPer = 4096 / kRThreads;
+    uint32_t E[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) E[k] = c.tab[(int64_t)cls * 4096 + k * kRThreads + (int)threadIdx.x];
+    __builtin_amdgcn_sched_barrier(0);
+
+    const int64_t last = c.n_words - (kRing + kHalfRing);                  // the furthest start that keeps every read inside
     off = off < 0 ? 0 : (off > last ? last : off);
     z.wp = c.words + off;
-    int64_t room = c.n_words - 1 - off;
-    if (next > off && next - off - 1 < room) room = next - off - 1;
-    const uint64_t s = c.states[(int64_t)tile * 32 + l32];
+    t.room = c.n_words - 1 - off;
+    if (next > off && next - off - 1 < t.room) t.room = next - off - 1;
     z.xl = (uint32_t)s; z.xh = (uint32_t)(s >> 32);
-    z.ptr = z.sb = 0;
+    z.sb = 0;
+    z.upper = (threadIdx.x & 32) ? 0xffffffffu : 0u; z.ptr = (int)(z.upper & kRing);
+    uint32_t first[kRing / 32];
 #pragma unroll
-    for (int q = 0; q < kRing / 32; ++q) {
-        const int64_t i = 32 * q + l32;
-        rg[32 * q + l32] = z.wp[i < room ? i : room];
-    }
+    for (int q = 0; q < kRing / 32; ++q) { const int64_t i = 32 * q + l32; first[q] = z.wp[i < t.room ? i : t.room]; }
 #pragma unroll
-    for (int q = 0; q < kRing / 64; ++q) {
-        const int64_t i = kRing + 32 * q + l32;
-        z.pre[q] = z.wp[i < room ? i : room];
-    }
-    return room;
+    for (int q = 0; q < kHalfRing / 32; ++q) { const int64_t i = kRing + 32 * q + l32; z.pre[q] = z.wp[i < t.room ? i : t.room]; }
+    __builtin_amdgcn_sched_barrier(0);
+    // the file's entry is (frequency - 1) << 22 | (slot - cumulative) << 11 | symbol with frequency <= 1024; the walk wants
+    // the frequency itself, one instruction per symbol less
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) st[k * kRThreads + threadIdx.x] = (((E[k] >> 22) + 1u) << 21) | (E[k] & 0x1FFFFFu);
+#pragma unroll
+    for (int q = 0; q < kRing / 32; ++q) own[32 * q + l32] = first[q];
+    if (!t.has) t.nr = 0;
+    if (t.r0 < 0 || t.r0 + t.nr > c.Q) { t.nr = 0; t.has = false; }
+    return t;
 }
 
-// one symbol: x' = f * (x >> 12) + d on the 64-bit state
+// one symbol: x' = f * (x >> 12) + d on the 64-bit state; the entry comes back with the symbol in its low 11 bits
 // `st` holds the slot table re-packed for the walk (block_setup): frequency << 21 | (slot - cumulative) << 11 | symbol.
 __device__ __forceinline__ uint32_t walk_dec(Walker& z, const uint32_t* st) {
     const uint32_t E = st[z.xl & 4095u];
     const uint32_t f = E >> 21, d = (E >> 11) & 1023u;
-    const uint64_t q = (((uint64_t)z.xh << 32) | z.xl) >> 12;
-    const uint64_t x = (uint64_t)f * q + d;
-    z.xl = (uint32_t)x; z.xh = (uint32_t)(x >> 32);
-    return E & 2047u;
+    const uint32_t q = __builtin_amdgcn_alignbit(z.xh, z.xl, 12);
+    const uint64_t lo = (uint64_t)f * q + d;
+    z.xl = (uint32_t)lo;
+    z.xh = f * (z.xh >> 12) + (uint32_t)(lo >> 32);                        // 11 bits x 20 bits: one 24-bit multiply-add
+    return E;
 }
 
-// Two symbols, then one renormalisation.  Called by whole half-waves (the lanes of a tile are all in or all out).
-// `room` = words the tile's stream may still be read ahead (clamps the read-ahead of a damaged stream inside the pad).
-__device__ __forceinline__ void walk_pair(Walker& z, const uint32_t* st, uint32_t* rg, int l32, int half, int64_t room,
-                                          uint32_t& s1, uint32_t& s2) {
-    s1 = walk_dec(z, st);
-    s2 = walk_dec(z, st);
-    const bool need = z.xh == 0u;
-    const uint64_t mk64 = __builtin_amdgcn_ballot_w64(need);
-    const uint32_t mk = half ? (uint32_t)(mk64 >> 32) : (uint32_t)mk64;
-    const uint32_t below = mk & ((1u << l32) - 1u);
-    if (need) { z.xh = z.xl; z.xl = rg[(z.ptr + __builtin_popcount(below)) & (kRing - 1)]; }
-    z.ptr += __builtin_popcount(mk);
-    if (z.ptr - z.sb >= kRing / 2) {                                       // uniform within the half
+// Four symbols, a renormalisation after every second one; `rg` is the wave's first window.  A pair takes at most 32 words of a
+// tile, so with the windows looked after every second pair at least 64 of their 256 words are always ahead.
+// Bound by vector instructions: 36 a pair and the multiply's extra slots, where a ring that wraps, looked after every pair, with a branch
+// around the words taken and the activations addressed per lane took 45.  17408 x 5120, one row: 66.2 -> 50.4 us a call with the
+// shorter start above; 16 rows 88.1 -> 71.2; 5120 x 17408, one row 95.2 -> 70.0.  (The pointers as wave scalars, one bit count
+// over the whole wave: fewer vector instructions, a longer chain: the same.  Waves of different priority, fewer resident
+// workgroups: nothing and worse.)
+__device__ __forceinline__ void walk_pairs2(Walker& z, const uint32_t* st, const uint32_t* rg, uint32_t (&e)[4]) {
 #pragma unroll
-        for (int q = 0; q < kRing / 64; ++q) rg[(z.sb + kRing + 32 * q + l32) & (kRing - 1)] = z.pre[q];
-        z.sb += kRing / 2;
+    for (int p = 0; p < 2; ++p) {
+        e[2 * p] = walk_dec(z, st);
+        e[2 * p + 1] = walk_dec(z, st);
+        asm("" : "+v"(z.xh));                                              // a 32-bit comparison, not one of the whole state
+        const bool need = z.xh == 0u;
+        const uint64_t mk = __builtin_amdgcn_ballot_w64(need);
+        const uint32_t mine = z.upper ? (uint32_t)(mk >> 32) : (uint32_t)mk;
+        int at = __builtin_popcount(mine & ((1u << (threadIdx.x & 31)) - 1u)) + z.ptr;
+        asm("" : "+v"(at));
+        const uint32_t w = rg[at];
+        z.xh = need ? z.xl : z.xh;
+        z.xl = need ? w : z.xl;
+        z.ptr += __builtin_popcount(mine);
+    }
+}
+// ... to be followed, before the next pairs, by a look at the windows (kept apart so that what the caller waits for in between is
+// not held up by words asked for here, which come from memory).
+// `room` = words the tile's stream may still be read ahead (clamps the read-ahead of a damaged stream inside the pad).
+__device__ __forceinline__ void walk_window(Walker& z, uint32_t* rg, int l32, int64_t room) {
+    if (z.ptr >= (int)(z.upper & kRing) + kHalfRing) {
+        z.ptr -= kHalfRing;
+        z.sb += kHalfRing;
+        uint32_t* mine = rg + (z.upper & (uint32_t)kRing) + l32;
+        uint32_t up[kHalfRing / 32];
+#pragma unroll
+        for (int q = 0; q < kHalfRing / 32; ++q) up[q] = mine[kHalfRing + 32 * q];
+#pragma unroll
+        for (int q = 0; q < kHalfRing / 32; ++q) { mine[32 * q] = up[q]; mine[kHalfRing + 32 * q] = z.pre[q]; }
         const int64_t at = (int64_t)z.sb + kRing;
 #pragma unroll
-        for (int q = 0; q < kRing / 64; ++q) {
+        for (int q = 0; q < kHalfRing / 32; ++q) {
             const int64_t i = at + 32 * q + l32;
             z.pre[q] = z.wp[i < room ? i : room];
         }
     }
 }
+// The words asked for last have arrived.  Said where a row starts: the compiler otherwise assumes at the head of a row's loop that
+// some may be pending from before it, and waits for every later request in each round of the loop.
+__device__ __forceinline__ void walk_settle(Walker& z) {
+#pragma unroll
+    for (int q = 0; q < kHalfRing / 32; ++q) asm volatile("" : "+v"(z.pre[q]));
+}
+constexpr uint32_t kSymMask = 2047u;
 
 __device__ __forceinline__ float half_sum(float v) {                       // sum over the 32 lanes of a half, to every lane
     v = dpp_add<0xB1>(v);     // quad_perm [1,0,3,2]
@@ -123,28 +185,6 @@ __device__ __forceinline__ float half_sum(float v) {                       // su
     v = dpp_add<0x141>(v);    // row_half_mirror
     v = dpp_add<0x140>(v);    // row_mirror: every lane of a 16-lane row holds the row sum
     return v + __shfl_xor(v, 16, 64);
-}
-
-// Per-workgroup set-up shared by the kernels: slot table into LDS, this half-wave's tile.
-struct TileCtx { bool has; int tile, r0, nr; int64_t room; };
-__device__ __forceinline__ TileCtx block_setup(const RCore& c, int block, uint32_t* st, int h8) {
-    int cls = c.blocks[3 * block], tb = c.blocks[3 * block + 1], ntb = c.blocks[3 * block + 2];
-    cls = cls < 0 ? 0 : (cls >= c.K ? c.K - 1 : cls);
-    // the file's entry is (frequency - 1) << 22 | (slot - cumulative) << 11 | symbol with frequency <= 1024; the walk wants
-    // the frequency itself, one instruction per symbol less
-    for (int i = threadIdx.x; i < 4096; i += blockDim.x) {
-        const uint32_t E = c.tab[(int64_t)cls * 4096 + i];
-        st[i] = (((E >> 22) + 1u) << 21) | (E & 0x1FFFFFu);
-    }
-    TileCtx t;
-    t.tile = tb + h8;
-    t.has = h8 < ntb && t.tile >= 0 && t.tile < c.n_tiles;
-    if (!t.has) t.tile = 0;
-    t.r0 = (int)c.tiles[3 * (int64_t)t.tile + 1];
-    t.nr = t.has ? (int)c.tiles[3 * (int64_t)t.tile + 2] : 0;
-    if (t.r0 < 0 || t.r0 + t.nr > c.Q) { t.nr = 0; t.has = false; }
-    t.room = 0;
-    return t;
 }
 
 // ---- dense rows -----------------------------------------------------------------------------------------------------
@@ -157,40 +197,41 @@ __global__ void __launch_bounds__(kRThreads) r_decode_kernel(RCore c, int b0, in
                                                              const int32_t* __restrict__ list) {
     __shared__ uint32_t st[4096];
     __shared__ uint32_t ring[kRTiles][kRing];
-    const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5, h8 = threadIdx.x >> 5;
+    const int lane = threadIdx.x & 63, l32 = lane & 31, h8 = threadIdx.x >> 5;
     int block_no = b0 + (int)blockIdx.x;
     if (list) {
         block_no = list[blockIdx.x];
         if (block_no < 0 || block_no >= c.n_blocks) return;                   // the whole workgroup: a bad entry writes nothing
     }
-    TileCtx t = block_setup(c, block_no, st, h8);
-    uint32_t* rg = ring[h8];
+    uint32_t* rg = ring[2 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];          // of the wave's two tiles
     Walker z;
-    t.room = walk_init(z, rg, c, t.tile, l32);
+    const TileCtx t = block_setup(z, c, block_no, st, ring[h8], h8, l32);
     __syncthreads();
     const int S = c.P >> 5;
     for (int r = 0; r < T; ++r) {
-        if (!(t.has && r < t.nr)) continue;                                // per half-wave
-        const int orow = c.perm[t.r0 + r];
+        const bool active = t.has && r < t.nr;                             // per half-wave
+        if (!__builtin_amdgcn_ballot_w64(active)) break;                   // neither tile has such a row
+        const int orow = active ? c.perm[t.r0 + r] : -1;
         const bool row_ok = orow >= 0 && orow < c.Q;
-        const float m = row_ok ? c.min_s[orow] : 0.f, ts = row_ok ? c.tau_s[orow] : 0.f;
-        const int dr = row_ok ? c.drow[orow] : 0;
+        const int row = row_ok ? orow : 0;
+        const float m = c.min_s[row], ts = c.tau_s[row];
+        const int dr = c.drow[row];
+        walk_settle(z);
         const int64_t at = list ? ((int64_t)blockIdx.x * kRTiles + h8) * T + r : row_base < 0 ? (int64_t)orow : (int64_t)(t.r0 + r) - row_base;
         const bool store = row_ok && at >= 0 && at < out_rows;
-        for (int s0 = 0; s0 < S; s0 += 2) {
-            uint32_t s1, s2;
-            walk_pair(z, st, rg, l32, half, t.room, s1, s2);
+        for (int s0 = 0; s0 < S; s0 += 4) {                                // (P is a multiple of 128)
+            uint32_t e[4];
+            walk_pairs2(z, st, rg, e);
             if (store) {
-                const int64_t i1 = at * c.P + (int64_t)s0 * 32 + l32, i2 = i1 + 32;
-                const int id1 = (int)s1 + dr, id2 = (int)s2 + dr;
-                if constexpr (DT == 3) {
-                    reinterpret_cast<int16_t*>(out)[i1] = (int16_t)id1;
-                    reinterpret_cast<int16_t*>(out)[i2] = (int16_t)id2;
-                } else {
-                    store_from_f32<DT>(out, i1, __builtin_fmaf((float)id1, ts, m));
-                    store_from_f32<DT>(out, i2, __builtin_fmaf((float)id2, ts, m));
+                const int64_t i0 = at * c.P + (int64_t)s0 * 32 + l32;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int id = (int)(e[k] & kSymMask) + dr;
+                    if constexpr (DT == 3) reinterpret_cast<int16_t*>(out)[i0 + 32 * k] = (int16_t)id;
+                    else store_from_f32<DT>(out, i0 + 32 * k, __builtin_fmaf((float)id, ts, m));
                 }
             }
+            walk_window(z, rg, l32, t.room);
         }
     }
 }
@@ -202,11 +243,10 @@ template <int DT, bool WALK_ONLY = false>
 __global__ void __launch_bounds__(kRThreads) r_gemv_kernel(RCore c, const void* __restrict__ X, float* __restrict__ Y, int T) {
     __shared__ uint32_t st[4096];
     __shared__ uint32_t ring[kRTiles][kRing];
-    const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5, h8 = threadIdx.x >> 5;
-    TileCtx t = block_setup(c, blockIdx.x, st, h8);
-    uint32_t* rg = ring[h8];
+    const int lane = threadIdx.x & 63, l32 = lane & 31, h8 = threadIdx.x >> 5;
+    uint32_t* rg = ring[2 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];          // of the wave's two tiles
     Walker z;
-    t.room = walk_init(z, rg, c, t.tile, l32);
+    const TileCtx t = block_setup(z, c, blockIdx.x, st, ring[h8], h8, l32);
     __syncthreads();
     const int S = c.P >> 5;
     float sx = 0.f;                  // sum of x over this lane's columns (the same for every row): taken while the first row is walked
@@ -216,38 +256,53 @@ __global__ void __launch_bounds__(kRThreads) r_gemv_kernel(RCore c, const void* 
         constexpr bool FIRST = decltype(first)::value;
         if constexpr (WALK_ONLY) {
             uint32_t keep = 0;
-            for (int s0 = 0; s0 < S; s0 += 2) {
-                uint32_t s1, s2;
-                walk_pair(z, st, rg, l32, half, t.room, s1, s2);
-                keep ^= s1 + s2;
+            for (int s0 = 0; s0 < S; s0 += 4) {
+                uint32_t e[4];
+                walk_pairs2(z, st, rg, e);
+                keep ^= (e[0] & kSymMask) + (e[1] & kSymMask);
+                keep ^= (e[2] & kSymMask) + (e[3] & kSymMask);
+                walk_window(z, rg, l32, t.room);
             }
             return (float)keep;
         } else {
             float acc = 0.f;
-            float x1 = load_as_f32<DT>(X, l32), x2 = load_as_f32<DT>(X, 32 + l32);
-            for (int s0 = 0; s0 < S; s0 += 2) {
-                const int sn = s0 + 2 < S ? s0 + 2 : s0;                   // the last pair reloads itself (unused)
-                const float n1 = load_as_f32<DT>(X, sn * 32 + l32), n2 = load_as_f32<DT>(X, (sn + 1) * 32 + l32);
-                uint32_t s1, s2;
-                walk_pair(z, st, rg, l32, half, t.room, s1, s2);
-                acc = __builtin_fmaf(x1, (float)s1, acc);
-                acc = __builtin_fmaf(x2, (float)s2, acc);
-                if constexpr (FIRST) sx += x1 + x2;
-                x1 = n1; x2 = n2;
+            for (int s0 = 0; s0 < S; s0 += 4) {
+                // columns 32 s0 + l32 ..: asked for ahead of the walk, there behind it
+                using Raw = std::conditional_t<DT == QVB8_F32, uint32_t, uint16_t>;
+                const Raw* base = reinterpret_cast<const Raw*>(X) + (size_t)s0 * 32;
+                Raw raw[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) raw[k] = base[(uint32_t)l32 + 32u * k];
+                __builtin_amdgcn_sched_barrier(0);
+                uint32_t e[4];
+                walk_pairs2(z, st, rg, e);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float x = DT == QVB8_F32 ? __builtin_bit_cast(float, (uint32_t)raw[k]) : DT == QVB8_F16 ? f16_bits_to_f32(raw[k]) : bf16_bits_to_f32(raw[k]);
+                    acc = __builtin_fmaf(x, (float)(e[k] & kSymMask), acc);
+                    if constexpr (FIRST) sx += x;
+                }
+                asm volatile("" : "+v"(acc));                              // the activations are used up before words are asked for
+                walk_window(z, rg, l32, t.room);
             }
             if constexpr (FIRST) sx = half_sum(sx);
             return acc;
         }
     };
     for (int r = 0; r < T; ++r) {
-        if (!(t.has && r < t.nr)) continue;                                // per half-wave
-        const int orow = c.perm[t.r0 + r];
+        const bool active = t.has && r < t.nr;                             // per half-wave
+        if (!__builtin_amdgcn_ballot_w64(active)) break;                   // neither tile has such a row
+        const int orow = active ? c.perm[t.r0 + r] : -1;
         const bool row_ok = orow >= 0 && orow < c.Q;
+        // the row's constants are asked for ahead of its walk, all at once
+        const int at = row_ok ? orow : 0;
+        const float m = c.min_s[at], ts = c.tau_s[at];
+        const int dr = c.drow[at];
+        walk_settle(z);
         const float acc = r == 0 ? walk_row(std::true_type{}) : walk_row(std::false_type{});
-        const double m = row_ok ? (double)c.min_s[orow] : 0.0, ts = row_ok ? (double)c.tau_s[orow] : 0.0;
-        const double dr = row_ok ? (double)c.drow[orow] : 0.0;
         const float a = half_sum(acc);
-        if (l32 == 0 && row_ok) Y[orow] = (float)(ts * ((double)a + dr * (double)sx) + m * (double)sx);
+        if (l32 == 0 && row_ok) Y[orow] = (float)((double)ts * ((double)a + (double)dr * (double)sx) + (double)m * (double)sx);
     }
 }
 
@@ -340,16 +395,15 @@ __global__ void __launch_bounds__(kRThreads) r_mma_kernel(RCore c, RPacked xp, i
     __shared__ int s_row[kRTiles];
     __shared__ float s_ts[kRTiles], s_min[kRTiles], s_dr[kRTiles];
     __shared__ double s_sx[16 * NT];
-    const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5, h8 = threadIdx.x >> 5, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, l32 = lane & 31, h8 = threadIdx.x >> 5, wave = threadIdx.x >> 6;
     if (threadIdx.x < 16 * NT) {
         double a = 0.0;
         for (int i = 0; i < xp.slabs; ++i) a += xp.sums[threadIdx.x * xp.slabs + i];
         s_sx[threadIdx.x] = a;
     }
-    TileCtx t = block_setup(c, blockIdx.x, st, h8);
-    uint32_t* rg = ring[h8];
+    uint32_t* rg = ring[2 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];          // of the wave's two tiles
     Walker z;
-    t.room = walk_init(z, rg, c, t.tile, l32);
+    const TileCtx t = block_setup(z, c, blockIdx.x, st, ring[h8], h8, l32);
     __syncthreads();
     const int S = c.P >> 5;
     const int n_batches = (c.P + kRBatchCols - 1) / kRBatchCols;
@@ -375,14 +429,18 @@ __global__ void __launch_bounds__(kRThreads) r_mma_kernel(RCore c, RPacked xp, i
             const int pairs = (S - b * 8) >> 1;                            // step pairs left in the row: a short last batch ends in zeros
             if (active) {
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    uint32_t out = 0;
-                    if (p < pairs) {                                       // uniform
-                        uint32_t s1, s2;
-                        walk_pair(z, st, rg, l32, half, t.room, s1, s2);
-                        out = __builtin_amdgcn_perm(u16_to_half_bits(s2), u16_to_half_bits(s1), 0x05040100u);
+                for (int p = 0; p < 4; p += 2) {
+                    uint32_t out[2] = {0u, 0u};
+                    if (p < pairs) {                                       // uniform (pairs come in twos: P is a multiple of 128)
+                        uint32_t e[4];
+                        walk_pairs2(z, st, rg, e);
+#pragma unroll
+                        for (int k = 0; k < 2; ++k)
+                            out[k] = __builtin_amdgcn_perm(u16_to_half_bits(e[2 * k + 1] & kSymMask), u16_to_half_bits(e[2 * k] & kSymMask), 0x05040100u);
+                        walk_window(z, rg, l32, t.room);
                     }
-                    sb[p * 32] = out;
+                    sb[p * 32] = out[0];
+                    sb[(p + 1) * 32] = out[1];
                 }
             } else {
 #pragma unroll

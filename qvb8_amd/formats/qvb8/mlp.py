@@ -76,6 +76,7 @@ class QVBandMLPV8(nn.Module):
     # launch it saves costs (see the kernel's source) --, so the separate products, which every other row count uses anyway,
     # stay the default.  QVB8_MLP_FUSED=1 in the environment (or True here) switches it on.
     one_launch = False
+    _pairs_stored = False          # gate+up lies in tiles_of_pairs order
 
     def __init__(self, gate: QVBandLinearV8, up: QVBandLinearV8, down: QVBandLinearV8):
         super().__init__()
@@ -85,7 +86,7 @@ class QVBandMLPV8(nn.Module):
         self.in_features = self.hidden
         self.gate_up = concat_linears([gate, up])[0]
         self.down = down
-        self.fused_ready = self._pairs_stored = False
+        self.fused_ready = False
         self._ws = self._plan = None
         self._prepare_fused()
 
@@ -140,7 +141,7 @@ class QVBandMLPV8(nn.Module):
         if not (self._pairs_stored and rows.dtype in (torch.float16, torch.bfloat16) and rows.dim() == 2 and 1 <= rows.shape[0] <= ext.MMA_SILU_MAX_M
                 and rows.shape[1] == self.hidden and rows.is_contiguous() and rows.device == gu.min_s.device):
             return None
-        if gu._forward_hooks or gu._forward_pre_hooks or _has_any_global_hook():
+        if gu._forward_hooks or gu._forward_pre_hooks or _has_any_global_hook() or gu.bias is not None or gu.esc_idx.numel() or gu.esc_idx_bf16.numel():
             return None
         order = gu._mma_order()
         if order is None or order[2] is None:

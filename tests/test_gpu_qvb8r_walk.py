@@ -1,0 +1,41 @@
+"""GPU tests of the QVB8R walk where its window of words moves most often and tiles of a wave differ: nearly uniform symbols (ten bits
+each, so a pair of steps takes some 20 of the 64 words kept ahead), rows of one step group and of many, tiles with fewer rows
+than their neighbour, blocks that are not full."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import qvb8_oracle as O
+from oracle import qvb8r_oracle as R
+from qvb8_amd import ext_qvb8r as ext
+from qvb8_amd.formats.qvb8 import pack as PK
+from qvb8_amd.formats.qvb8r import pack as RP
+from qvb8_amd.formats.qvb8r.module import QVBandLinearV8R
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("Q,P,kw", [(5, 128, dict(rows_per_tile=2)), (67, 384, dict(rows_per_tile=5, n_classes=3)), (130, 640, dict(rows_per_tile=1)),
+                                     (33, 2176, dict(rows_per_tile=4)), (19, 8192, dict())])
+def test_window_of_words(Q, P, kw):
+    g = torch.Generator().manual_seed(Q * P)
+    W = (0.1 * (2.0 * torch.rand(Q, P, generator=g) - 1.0)).to(torch.bfloat16).to(DEV)
+    enc = PK.encode_tensor(W, 1.3e-4, keep_ids=True)
+    d = RP.transcode(enc, **kw)
+    want = enc["ids_dense"].cpu().numpy().astype(np.int64)
+    assert np.array_equal(R.ids(d), want) and 32 * len(d["words"]) > 7 * Q * P
+    lin = QVBandLinearV8R(d, device=DEV)
+    assert np.array_equal(ext.ids(P, *lin._core(), T=lin.T).cpu().numpy().astype(np.int64), want)
+    Wr = R.reconstruct(d, enc["esc_idx"].cpu().numpy(), enc["esc_vals"].cpu().numpy())
+    assert np.array_equal(lin.dense(torch.float32).cpu().numpy().view(np.uint32), Wr.view(np.uint32))
+    for dtype in (torch.float32, torch.float16, torch.bfloat16):
+        for M in (1, 5, 33):
+            x = torch.randn(M, P, generator=torch.Generator().manual_seed(M)).to(dtype).to(DEV)
+            xs = x.float().cpu().numpy()
+            ref = O.linear_f64(xs, Wr)
+            eps = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+            tol = H.gemv_tolerance(ref, Wr, xs) + eps * np.abs(ref)
+            diff = np.abs(lin(x).float().cpu().numpy().astype(np.float64) - ref)
+            assert np.all(diff <= tol), (dtype, M, float((diff / tol).max()))
