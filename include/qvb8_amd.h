@@ -53,9 +53,9 @@ enum qvb8_status {
 /* Library identification: ABI version, bumped on any signature change or new entry point (3: row lookup, attention over
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
  * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*;
- * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS).  A binding compares the loaded library's answer
+ * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS; 12: qvb8r_gemv_as).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
-#define QVB8_ABI_VERSION 11
+#define QVB8_ABI_VERSION 12
 int qvb8_abi_version(void);
 /* Message of the calling thread's most recent failure ("" if none). Valid until that thread's next call. */
 const char* qvb8_last_error(void);
@@ -384,6 +384,10 @@ int64_t qvb8r_gemv_workspace_bytes(int64_t M, int64_t P);
  * (which multiplies fp16-rounded weights; this one keeps the fp32 band value). */
 int qvb8r_gemv(const void* X, int x_dtype, int64_t M, const qvb8r_core* core, int64_t max_tile_rows, float* Y,
                void* workspace, int64_t workspace_bytes, void* stream);
+/* The same with Y in y_dtype (QVB8_F32 / _F16 / _BF16): each result rounded to nearest even from the fp32 value qvb8r_gemv would
+ * store.  For weights without escapes: the correction adds to fp32 results. */
+int qvb8r_gemv_as(const void* X, int x_dtype, int64_t M, const qvb8r_core* core, int64_t max_tile_rows, void* Y, int y_dtype,
+                  void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Measurement aid: the launch of qvb8r_gemv for one row of X with the activations not read and the two multiply-adds per
  * symbol pair replaced by an exclusive-or of the symbols -- the rANS walk alone (slot lookups, 64-bit state updates, word

@@ -236,11 +236,18 @@ __global__ void __launch_bounds__(kRThreads) r_decode_kernel(RCore c, int b0, in
     }
 }
 
+// a result in the caller's type: a cast pass over the results cost a launch of its own (17408 x 5120, one row: 50.6 -> 48.6 us)
+__device__ __forceinline__ void store_y(void* Y, int y_dt, int64_t i, float v) {
+    if (y_dt == QVB8_F32) reinterpret_cast<float*>(Y)[i] = v;
+    else if (y_dt == QVB8_F16) store_from_f32<1>(Y, i, v);
+    else store_from_f32<2>(Y, i, v);
+}
+
 // ---- fused decode + product, one row of X ------------------------------------------------------------------------------
 // WALK_ONLY (a measurement aid, qvb8r_walk_probe): the same launch with the activations not read and the two multiply-adds
 // per pair replaced by an exclusive-or that keeps the symbols alive -- what the walk alone costs, the ceiling of this path.
 template <int DT, bool WALK_ONLY = false>
-__global__ void __launch_bounds__(kRThreads) r_gemv_kernel(RCore c, const void* __restrict__ X, float* __restrict__ Y, int T) {
+__global__ void __launch_bounds__(kRThreads) r_gemv_kernel(RCore c, const void* __restrict__ X, void* __restrict__ Y, int y_dt, int T) {
     __shared__ uint32_t st[4096];
     __shared__ uint32_t ring[kRTiles][kRing];
     const int lane = threadIdx.x & 63, l32 = lane & 31, h8 = threadIdx.x >> 5;
@@ -302,7 +309,7 @@ __global__ void __launch_bounds__(kRThreads) r_gemv_kernel(RCore c, const void* 
         walk_settle(z);
         const float acc = r == 0 ? walk_row(std::true_type{}) : walk_row(std::false_type{});
         const float a = half_sum(acc);
-        if (l32 == 0 && row_ok) Y[orow] = (float)((double)ts * ((double)a + (double)dr * (double)sx) + (double)m * (double)sx);
+        if (l32 == 0 && row_ok) store_y(Y, y_dt, orow, (float)((double)ts * ((double)a + (double)dr * (double)sx) + (double)m * (double)sx));
     }
 }
 
@@ -387,7 +394,7 @@ typedef _Float16 r_v8h_t __attribute__((ext_vector_type(8)));
 typedef float r_v4f_t __attribute__((ext_vector_type(4)));
 
 template <int NT, bool LO>
-__global__ void __launch_bounds__(kRThreads) r_mma_kernel(RCore c, RPacked xp, int M, float* __restrict__ Y, int T) {
+__global__ void __launch_bounds__(kRThreads) r_mma_kernel(RCore c, RPacked xp, int M, void* __restrict__ Y, int y_dt, int T) {
     __shared__ uint32_t st[4096];
     __shared__ uint32_t ring[kRTiles][kRing];
     __shared__ __align__(16) uint32_t sym[2][kRTiles][kRSymStride];
@@ -484,7 +491,7 @@ __global__ void __launch_bounds__(kRThreads) r_mma_kernel(RCore c, RPacked xp, i
             for (int w = 0; w < kRThreads / 64; ++w) a += (double)red[w][nt][at];
             const double sx = s_sx[m];
             const double v = (double)s_ts[n] * (a + (double)s_dr[n] * sx) + (double)s_min[n] * sx;
-            Y[(int64_t)m * c.Q + orow] = (float)__builtin_ldexp(v, -xp.kexp[m]);
+            store_y(Y, y_dt, (int64_t)m * c.Q + orow, (float)__builtin_ldexp(v, -xp.kexp[m]));
         }
         // red and s_row are written again only after the next row's batch barriers, which every thread reaches after this loop
     }
@@ -581,7 +588,7 @@ extern "C" int qvb8r_walk_probe(const qvb8r_core* core, int64_t max_tile_rows, f
     if (max_tile_rows < 1 || max_tile_rows > 0x7fffffff) return host::fail(QVB8_ERR_ARG, "qvb8r_walk_probe: bad rows-per-tile bound");
     if (c.Q == 0 || c.n_blocks == 0) return QVB8_OK;
     if (!Y) return host::fail(QVB8_ERR_ARG, "qvb8r_walk_probe: null pointer");
-    hipLaunchKernelGGL((r_gemv_kernel<0, true>), dim3((unsigned)c.n_blocks), dim3(kRThreads), 0, (hipStream_t)stream, c, (const void*)Y, Y, (int)max_tile_rows);
+    hipLaunchKernelGGL((r_gemv_kernel<0, true>), dim3((unsigned)c.n_blocks), dim3(kRThreads), 0, (hipStream_t)stream, c, (const void*)Y, (void*)Y, QVB8_F32, (int)max_tile_rows);
     return host::check_launch("qvb8r_walk_probe");
 }
 
@@ -593,10 +600,16 @@ extern "C" int64_t qvb8r_gemv_workspace_bytes(int64_t M, int64_t P) {
 
 extern "C" int qvb8r_gemv(const void* X, int x_dtype, int64_t M, const qvb8r_core* core, int64_t max_tile_rows, float* Y,
                           void* workspace, int64_t workspace_bytes, void* stream) {
+    return qvb8r_gemv_as(X, x_dtype, M, core, max_tile_rows, Y, QVB8_F32, workspace, workspace_bytes, stream);
+}
+
+extern "C" int qvb8r_gemv_as(const void* X, int x_dtype, int64_t M, const qvb8r_core* core, int64_t max_tile_rows, void* Y, int y_dtype,
+                             void* workspace, int64_t workspace_bytes, void* stream) {
     RCore c;
     if (int rc = check_core("qvb8r_gemv", core, c)) return rc;
     if (M < 1 || M > 48) return host::fail(QVB8_ERR_ARG, "qvb8r_gemv: M=%lld outside 1..48", (long long)M);
     if (x_dtype < QVB8_F32 || x_dtype > QVB8_BF16) return host::fail(QVB8_ERR_ARG, "qvb8r_gemv: bad activation dtype");
+    if (y_dtype < QVB8_F32 || y_dtype > QVB8_BF16) return host::fail(QVB8_ERR_ARG, "qvb8r_gemv: bad result dtype");
     if (max_tile_rows < 1 || max_tile_rows > 0x7fffffff) return host::fail(QVB8_ERR_ARG, "qvb8r_gemv: bad rows-per-tile bound");
     if (c.Q == 0 || c.n_blocks == 0) return QVB8_OK;
     if (!X || !Y) return host::fail(QVB8_ERR_ARG, "qvb8r_gemv: null pointer");
@@ -604,9 +617,9 @@ extern "C" int qvb8r_gemv(const void* X, int x_dtype, int64_t M, const qvb8r_cor
     dim3 grid((unsigned)c.n_blocks), block(kRThreads);
     const int T = (int)max_tile_rows;
     if (M == 1) {
-        if (x_dtype == QVB8_F32) hipLaunchKernelGGL(r_gemv_kernel<0>, grid, block, 0, s, c, X, Y, T);
-        else if (x_dtype == QVB8_F16) hipLaunchKernelGGL(r_gemv_kernel<1>, grid, block, 0, s, c, X, Y, T);
-        else hipLaunchKernelGGL(r_gemv_kernel<2>, grid, block, 0, s, c, X, Y, T);
+        if (x_dtype == QVB8_F32) hipLaunchKernelGGL(r_gemv_kernel<0>, grid, block, 0, s, c, X, Y, y_dtype, T);
+        else if (x_dtype == QVB8_F16) hipLaunchKernelGGL(r_gemv_kernel<1>, grid, block, 0, s, c, X, Y, y_dtype, T);
+        else hipLaunchKernelGGL(r_gemv_kernel<2>, grid, block, 0, s, c, X, Y, y_dtype, T);
         return host::check_launch("qvb8r_gemv");
     }
     const int64_t need = qvb8r_gemv_workspace_bytes(M, c.P);
@@ -626,8 +639,8 @@ extern "C" int qvb8r_gemv(const void* X, int x_dtype, int64_t M, const qvb8r_cor
     else if (x_dtype == QVB8_F16) hipLaunchKernelGGL((r_pack_x_kernel<1, false>), pgrid, dim3(256), 0, s, X, (int)M, c.P, NT, hi, lo, sums, kexp);
     else hipLaunchKernelGGL((r_pack_x_kernel<2, false>), pgrid, dim3(256), 0, s, X, (int)M, c.P, NT, hi, lo, sums, kexp);
     if (int rc = host::check_launch("qvb8r_gemv pack")) return rc;
-#define QVB8R_MMA(NT_) do { if (split) hipLaunchKernelGGL((r_mma_kernel<NT_, true>), grid, block, 0, s, c, xp, (int)M, Y, T); \
-                            else hipLaunchKernelGGL((r_mma_kernel<NT_, false>), grid, block, 0, s, c, xp, (int)M, Y, T); } while (0)
+#define QVB8R_MMA(NT_) do { if (split) hipLaunchKernelGGL((r_mma_kernel<NT_, true>), grid, block, 0, s, c, xp, (int)M, Y, y_dtype, T); \
+                            else hipLaunchKernelGGL((r_mma_kernel<NT_, false>), grid, block, 0, s, c, xp, (int)M, Y, y_dtype, T); } while (0)
     if (NT == 1) QVB8R_MMA(1); else if (NT == 2) QVB8R_MMA(2); else QVB8R_MMA(3);
 #undef QVB8R_MMA
     return host::check_launch("qvb8r_gemv");

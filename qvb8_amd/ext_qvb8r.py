@@ -46,7 +46,7 @@ def _rows_bound(tiles, T):
     return int(tiles.reshape(-1, 3)[:, 2].max()) if tiles.numel() else 1
 
 
-def _product(X, core, T):
+def _product(X, core, T, out_dtype=torch.float32):
     lib = _lib.load()
     _lib.require_cuda(X)
     if X.dim() == 1:
@@ -58,11 +58,11 @@ def _product(X, core, T):
         raise RuntimeError("qvb8r: X must be fp32, fp16 or bf16")
     c, Q, _ = _core(*core, P)
     Xc = X.contiguous()
-    with torch.cuda.device(Xc.device):
-        Y = torch.empty((M, Q), dtype=torch.float32, device=Xc.device)
+    with _lib.on_device_of(Xc):
+        Y = torch.empty((M, Q), dtype=out_dtype, device=Xc.device)
         ws = torch.empty(max(16, lib.qvb8r_gemv_workspace_bytes(M, P)), dtype=torch.uint8, device=Xc.device)
-        _lib._check(lib.qvb8r_gemv(Xc.data_ptr(), _lib.dtype_code(Xc.dtype), M, ctypes.byref(c), _rows_bound(core[3], T),
-                                   Y.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(Xc)), lib)
+        _lib._check(lib.qvb8r_gemv_as(Xc.data_ptr(), _lib.dtype_code(Xc.dtype), M, ctypes.byref(c), _rows_bound(core[3], T),
+                                      Y.data_ptr(), _lib.dtype_code(out_dtype), ws.data_ptr(), ws.numel(), _lib.stream_of(Xc)), lib)
     return Y
 
 
@@ -71,9 +71,10 @@ def gemv(X, words, off, states, tiles, blocks, tab, perm, mn, ts, drow, T=None):
     return _product(X.reshape(1, -1), (words, off, states, tiles, blocks, tab, perm, mn, ts, drow), T).reshape(-1)
 
 
-def multi(X, words, off, states, tiles, blocks, tab, perm, mn, ts, drow, T=None):
-    """M = 2..8 (here up to 48): X (M, P) fp32, fp16 or bf16 -> Y (M, Q) fp32 (qvb8r_cuda.cu:359-383)."""
-    return _product(X, (words, off, states, tiles, blocks, tab, perm, mn, ts, drow), T)
+def multi(X, words, off, states, tiles, blocks, tab, perm, mn, ts, drow, T=None, out_dtype=torch.float32):
+    """M = 2..8 (here up to 48): X (M, P) fp32, fp16 or bf16 -> Y (M, Q) fp32 (qvb8r_cuda.cu:359-383).  `out_dtype` fp16 / bf16:
+    the same values rounded to that type by the kernel."""
+    return _product(X, (words, off, states, tiles, blocks, tab, perm, mn, ts, drow), T, out_dtype)
 
 
 def tc(X, words, off, states, tiles, blocks, tab, perm, mn, ts, drow, T):

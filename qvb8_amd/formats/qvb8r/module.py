@@ -15,6 +15,7 @@ import torch
 import torch.nn as nn
 
 from qvb8_amd import ext_qvb8r as ext
+from qvb8_amd.ext_qvb8 import saturating_half
 from qvb8_amd.formats.qvb8.module import activation_rows, apply_keeping_fp32_metadata  # noqa: F401  (same metadata rule)
 from . import container as QF
 
@@ -154,18 +155,27 @@ class QVBandLinearV8R(nn.Module):
         return (self.words, self.off, self.states, self.tiles, self.blocks8, self.tab, self.perm, self.min_s, self.tau_s,
                 self.drow)
 
-    def _small(self, x2):
+    def _small(self, x2, out_dtype):
         xk = x2.contiguous()
+        if out_dtype in (torch.float16, torch.bfloat16) and self.bias is None and not self.esc_uq.numel():
+            return ext.multi(xk, *self._core(), T=self.T, out_dtype=out_dtype)       # nothing to add to fp32 results
         y = ext.multi(xk, *self._core(), T=self.T)
         return ext.fix_escapes(xk, self.esc_uq, self.esc_ptr, self.esc_c, self.esc_delta, y)
 
     def _chunked(self, x2, bf16: bool):
         dt = torch.bfloat16 if bf16 else torch.float16
-        xk = x2 if bf16 else x2.float().clamp(-65504, 65504).half()          # saturating fp16, as the small-M paths of QVB8
+        # saturating fp16, as the small-M paths of QVB8 (an infinity among fp16 rows, which saturating_half leaves alone, too)
+        xk = x2 if bf16 else x2.clamp(-65504, 65504) if x2.dtype == torch.float16 else saturating_half(x2)
         ef, ev = (self.esc_flat_bf16, self.esc_val_bf16) if bf16 else (self.esc_flat, self.esc_val)
         P = self.in_features
-        y = torch.empty(x2.shape[0], self.out_features, device=x2.device, dtype=torch.float32)
         code = 1 if bf16 else 0
+        if len(self.chunks) == 1:
+            # the whole weight at once: its rows in their own order, and the product is the result
+            W = ext.decode(*self._core(), P, code, 0, self.blocks8.shape[0], -1, 0, T=self.T)
+            if ef.numel():
+                W.view(-1)[ef] = ev.to(dt)
+            return torch.mm(xk, W.t(), out_dtype=torch.float32)              # 16-bit operands, fp32 accumulate and result
+        y = torch.empty(x2.shape[0], self.out_features, device=x2.device, dtype=torch.float32)
         for b0, nb, base, rows in self.chunks:
             W = ext.decode(*self._core(), P, code, b0, nb, base, rows, T=self.T)
             orows = self.perm[base:base + rows].long()
@@ -176,7 +186,7 @@ class QVBandLinearV8R(nn.Module):
                 pos = inv[ef // P]
                 keep = pos >= 0
                 W.view(-1)[pos[keep] * P + ef[keep] % P] = ev[keep].to(dt)
-            y[:, orows] = torch.mm(xk, W.t(), out_dtype=torch.float32)       # 16-bit operands, fp32 accumulate and result
+            y[:, orows] = torch.mm(xk, W.t(), out_dtype=torch.float32)
         return y
 
     def forward(self, x):
@@ -193,7 +203,7 @@ class QVBandLinearV8R(nn.Module):
             # one fused walk per call of at most ext.MAX_M rows; more rows are split evenly
             calls = -(-M // ext.MAX_M)
             per_call = -(-M // calls)
-            parts = [self._small(rows[at:at + per_call]) for at in range(0, M, per_call)]
+            parts = [self._small(rows[at:at + per_call], out_dtype) for at in range(0, M, per_call)]
             y = parts[0] if len(parts) == 1 else torch.cat(parts)
         else:
             y = self._chunked(rows, bf16=dense_bf16 and bool(self.bf16_certified))

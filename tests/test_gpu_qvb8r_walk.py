@@ -39,3 +39,39 @@ def test_window_of_words(Q, P, kw):
             tol = H.gemv_tolerance(ref, Wr, xs) + eps * np.abs(ref)
             diff = np.abs(lin(x).float().cpu().numpy().astype(np.float64) - ref)
             assert np.all(diff <= tol), (dtype, M, float((diff / tol).max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_results_in_the_callers_type(dtype):
+    """Rounded by the kernel where nothing is added afterwards: the values of casting the fp32 results, both sides bit for bit."""
+    enc = PK.encode_tensor(H.synth_weight(70, 512, seed=4).to(DEV), 2e-3, keep_ids=True)
+    assert enc["esc_idx"].numel() == 0
+    lin = QVBandLinearV8R(RP.transcode(enc, rows_per_tile=3), device=DEV)
+    for M in (1, 2, 17, 48):
+        x = torch.randn(M, 512, generator=torch.Generator().manual_seed(M)).to(dtype).to(DEV)
+        x[0, 7] = 3.0e4
+        y = lin(x)
+        assert y.dtype == dtype and torch.equal(y, ext.multi(x, *lin._core(), T=lin.T).to(dtype))
+    lin.bias = torch.nn.Parameter(torch.ones(70, device=DEV), requires_grad=False)
+    assert torch.equal(lin(x), (ext.multi(x, *lin._core(), T=lin.T) + 1.0).to(dtype))
+
+
+def test_whole_weight_in_one_chunk_and_in_several():
+    """More than 48 rows: the weight restored at once in its rows' own order, or chunk by chunk in the stream's."""
+    Q, P, M = 150, 512, 60
+    enc = PK.encode_tensor(H.synth_weight(Q, P, seed=9).to(DEV), 2e-3, force_escapes=torch.tensor([3, 700, P * Q - 1]), keep_ids=True)
+    d = RP.transcode(enc, rows_per_tile=3)
+    lin, several = QVBandLinearV8R(d, device=DEV), type("Several", (QVBandLinearV8R,), dict(CHUNK_BYTES=2 * P * 40))(d, device=DEV)
+    assert len(lin.chunks) == 1 and len(several.chunks) > 1
+    Wr = O.narrow_fp16(R.reconstruct(d, enc["esc_idx"].cpu().numpy(), enc["esc_vals"].cpu().numpy())).astype(np.float32)
+    for dtype in (torch.float32, torch.float16, torch.bfloat16):
+        x = torch.randn(M, P, generator=torch.Generator().manual_seed(1)).to(dtype).to(DEV)
+        x[2, 5] = 7.0e4 if dtype != torch.float16 else float("inf")                    # becomes 65504
+        xs = O.sat_half(x.float().cpu().numpy())
+        ref = O.linear_f64(xs, Wr)
+        eps = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+        tol = H.gemv_tolerance(ref, Wr, xs) + eps * np.abs(ref)
+        for m in (lin, several):
+            diff = np.abs(m(x).float().cpu().numpy().astype(np.float64) - ref)
+            finite = np.abs(ref) < (6.5e4 if dtype == torch.float16 else 1e30)
+            assert np.all(diff[finite] <= tol[finite]), (dtype, float((diff / tol)[finite].max()))
