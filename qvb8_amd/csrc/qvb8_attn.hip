@@ -31,6 +31,7 @@
 #include <stdint.h>
 
 #include "qvb8_amd.h"
+#include "qvb8_device.h"
 #include "qvb8_host.h"
 
 namespace qvb8 {
@@ -45,7 +46,8 @@ constexpr int kAttnThreads = 256;
 constexpr int kSStride = kKeys + 4;
 
 struct AttnArgs {
-    const uint16_t* q; int64_t sq_r, sq_h;
+    const void* q; int64_t sq_r, sq_h;                          // strides in elements
+    int q_dt; float q_scale;                                    // kQReady: fp16 as the products take it; else QVB8_F32 / _F16 / _BF16, to be prepared
     const void* ki; const void* vi; int64_t s_n, s_h;           // strides in ids
     const float* kmid; const float* kstep; const float* vmid; const float* vstep; const float* kc; const float* vc;
     const int32_t* ts; const int32_t* tl; const int32_t* tseg;
@@ -53,6 +55,29 @@ struct AttnArgs {
     int q_pos0, n_tiles, tps, n_rows, G, nhkv;
     float scale;
 };
+
+// Four neighbouring channels of one query, at element offset `at`.  What is not ready is multiplied by the softmax scale, then
+// clamped to fp16's finite range and rounded -- in this order, so that an outlier channel does not become an infinity.  Done by
+// the row-block kernel where it reads its queries, 16 or 32 rows a workgroup; the kernel of 128 rows takes them ready (every one of its
+// splits would prepare them again: 120 tokens over 16001 keys 118.3 us that way, 112.1 with a launch that does it once).
+constexpr int kQReady = -1;
+__device__ __forceinline__ h4_t load_query(const AttnArgs& a, int64_t at) {
+    if (a.q_dt == kQReady) return *reinterpret_cast<const h4_t*>(reinterpret_cast<const uint16_t*>(a.q) + at);
+    float v[4];
+    if (a.q_dt == QVB8_F32) {
+        const float4 f = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(a.q) + at);
+        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+    } else {
+        const uint2 w = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(a.q) + at);
+        const uint32_t u[4] = {w.x & 0xFFFFu, w.x >> 16, w.y & 0xFFFFu, w.y >> 16};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = a.q_dt == QVB8_F16 ? f16_bits_to_f32(u[k]) : bf16_bits_to_f32(u[k]);
+    }
+    uint32_t h[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) h[k] = sat_half_bits(v[k] * a.q_scale);
+    return __builtin_bit_cast(h4_t, uint2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)});
+}
 
 // Four neighbouring channels of one key, as they lie in memory.
 template <typename T> struct Quad;
@@ -135,10 +160,10 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
         const int row = row0 + rb * kRows + n16;
         const bool row_ok = row < a.n_rows;
         const int rr = row_ok ? row : 0;
-        const uint16_t* qp = a.q + (int64_t)(rr / a.G) * a.sq_r + (int64_t)(h * a.G + rr % a.G) * a.sq_h + dh * (D / 2) + 4 * kg;
+        const int64_t qp = (int64_t)(rr / a.G) * a.sq_r + (int64_t)(h * a.G + rr % a.G) * a.sq_h + dh * (D / 2) + 4 * kg;
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
-            const h4_t v = *reinterpret_cast<const h4_t*>(qp + 16 * ks);
+            const h4_t v = load_query(a, qp + 16 * ks);
             qa[rb][ks] = row_ok ? v : h4_t{0, 0, 0, 0};
         }
     }
@@ -436,7 +461,7 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
     h8_t qb[NKS];
     {
         const int rr = row_ok ? myrow : 0;
-        const uint16_t* qp = a.q + (int64_t)(rr / a.G) * a.sq_r + (int64_t)(h * a.G + rr % a.G) * a.sq_h + 8 * hf;
+        const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + (int64_t)(rr / a.G) * a.sq_r + (int64_t)(h * a.G + rr % a.G) * a.sq_h + 8 * hf;
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
             const h4_t lo = *reinterpret_cast<const h4_t*>(qp + 16 * ks), hi = *reinterpret_cast<const h4_t*>(qp + 16 * ks + 4);
@@ -613,53 +638,84 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
     }
 }
 
-// Splits -> the normalised result and the log-sum-exp.  One workgroup per (kv head, row, 16 channels): 64 groups of 4
-// threads share the splits (group g takes splits g, g + 64, ...), a thread holds four channels; the groups' maxima,
-// sums and partial results meet in LDS.  A thread has a few independent loads, so the launch costs a few trips to
-// memory, not one per split.
+// Splits -> the normalised result and the log-sum-exp.  A unit of W waves takes one (kv head, row, 16 channels): 16 W groups of 4
+// threads share the splits (group g takes splits g, g + 16 W, ...), a thread holds four channels.  A thread asks for everything of
+// its next splits at once and weighs them against their own largest maximum; the groups of a wave then join by lane exchanges and
+// the waves through LDS, each join weighing both sides against the larger maximum, all in a fixed order: one trip to memory, at most
+// one barrier.
+struct Joined { float top, total; f4_t acc; };
+__device__ __forceinline__ void join(Joined& a, float top, float total, const f4_t& acc) {
+    const float t = fmaxf(a.top, top), safe = t == -INFINITY ? 0.f : t;
+    const float wa = expf(a.top - safe), wb = expf(top - safe);
+    a.total = a.total * wa + total * wb;
+    a.acc = a.acc * wa + acc * wb;
+    a.top = t;
+}
+// K splits of the group, `step` apart, from s0 on (those past the end count nothing)
+template <int K>
+__device__ __forceinline__ void join_splits(Joined& j, const float* o, const float* m, const float* l, int s0, int step, int n_splits,
+                                            int64_t stride, int64_t hr, int D, int ch) {
+    float mv[K], lv[K];
+    f4_t ov[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int64_t at = min(s0 + step * k, n_splits - 1) * stride + hr;
+        mv[k] = m[at];
+        lv[k] = l ? l[at] : 1.f;
+        ov[k] = *reinterpret_cast<const f4_t*>(o + at * D + ch);
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < K; ++k) { if (s0 + step * k >= n_splits) mv[k] = -INFINITY; top = fmaxf(top, mv[k]); }
+    const float safe = top == -INFINITY ? 0.f : top;
+    float total = 0.f;
+    f4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const float w = expf(mv[k] - safe);
+        if (s0 + step * k < n_splits) { total += lv[k] * w; acc += ov[k] * w; }
+    }
+    join(j, top, total, acc);
+}
+__device__ __forceinline__ void store_joined(const Joined& j, int64_t hr, int n_rows, int nhkv, int G, int D, int ch, float* out, float* lse) {
+    const int h = (int)(hr / n_rows), r = (int)(hr - (int64_t)h * n_rows);
+    const int64_t dst = (int64_t)(r / G) * (nhkv * G) + h * G + r % G;
+    *reinterpret_cast<f4_t*>(out + dst * D + ch) = j.acc * (1.f / fmaxf(j.total, 1e-30f));
+    if (ch == 0) lse[dst] = j.total > 0.f ? j.top + logf(fmaxf(j.total, 1e-30f)) : -INFINITY;
+}
+template <int W>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restrict__ o, const float* __restrict__ m, const float* __restrict__ l,
                                                             int n_splits, int nhkv, int n_rows, int D, int G,
                                                             float* __restrict__ out, float* __restrict__ lse) {
-    __shared__ float s_top[64], s_total[64];
-    __shared__ __align__(16) float s_acc[64][16];
-    const int h = blockIdx.x / n_rows, r = blockIdx.x % n_rows;
-    const int grp = threadIdx.x >> 2, cl = threadIdx.x & 3, ch = blockIdx.y * 16 + cl * 4;
-    const int64_t hr = (int64_t)h * n_rows + r, stride = (int64_t)nhkv * n_rows;
-    float top = -INFINITY;
-    for (int s = grp; s < n_splits; s += 64) top = fmaxf(top, m[s * stride + hr]);
-    if (cl == 0) s_top[grp] = top;
-    __syncthreads();
+    constexpr int kGroups = 16 * W;
+    __shared__ float s_top[4], s_total[4];
+    __shared__ __align__(16) f4_t s_acc[4][4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int grp = (int)(threadIdx.x >> 2) % kGroups, cl = threadIdx.x & 3, ch = blockIdx.y * 16 + cl * 4, chc = min(ch, D - 4);
+    const int64_t stride = (int64_t)nhkv * n_rows, unit = (int64_t)blockIdx.x * (4 / W) + wave / W, hr = min(unit, stride - 1);
+    Joined j = {-INFINITY, 0.f, {0.f, 0.f, 0.f, 0.f}};
+    if (n_splits <= kGroups) join_splits<1>(j, o, m, l, grp, kGroups, n_splits, stride, hr, D, chc);
+    else for (int s0 = grp; s0 < n_splits; s0 += 4 * kGroups) join_splits<4>(j, o, m, l, s0, kGroups, n_splits, stride, hr, D, chc);
 #pragma unroll
-    for (int g = 0; g < 64; ++g) top = fmaxf(top, s_top[g]);
-    if (top == -INFINITY) top = 0.f;
-    float total = 0.f;
-    f4_t acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s = grp; s < n_splits; s += 64) {
-        const float w = expf(m[s * stride + hr] - top);
-        total += (l ? l[s * stride + hr] : 1.f) * w;
-        if (ch < D) acc += *reinterpret_cast<const f4_t*>(o + (s * stride + hr) * D + ch) * w;
+    for (int d = 4; d < 64; d <<= 1) {
+        f4_t acc;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] = __shfl_xor(j.acc[c], d);
+        const float top = __shfl_xor(j.top, d), total = __shfl_xor(j.total, d);
+        join(j, top, total, acc);
     }
-    if (cl == 0) s_total[grp] = total;
-    *reinterpret_cast<f4_t*>(&s_acc[grp][cl * 4]) = acc;
-    __syncthreads();
-    if (grp == 0) {
-        total = 0.f;
-        acc = f4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-        for (int g = 0; g < 64; ++g) {                    // fixed order: the result does not depend on timing
-            total += s_total[g];
-            acc += *reinterpret_cast<const f4_t*>(&s_acc[g][cl * 4]);
-        }
-        const int tok = r / G, qh = h * G + r % G;
-        const int64_t dst = (int64_t)tok * (nhkv * G) + qh;
-        if (ch < D) *reinterpret_cast<f4_t*>(out + dst * D + ch) = acc * (1.f / fmaxf(total, 1e-30f));
-        if (cl == 0 && blockIdx.y == 0) lse[dst] = total > 0.f ? top + logf(fmaxf(total, 1e-30f)) : -INFINITY;
+    if constexpr (W > 1) {
+        if (lane == 0) { s_top[wave] = j.top; s_total[wave] = j.total; }
+        if (lane < 4) s_acc[wave][cl] = j.acc;
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 1; w < 4; ++w) join(j, s_top[w], s_total[w], s_acc[w][cl]);
     }
+    if (lane < 4 && unit < stride && ch < D) store_joined(j, hr, n_rows, nhkv, G, D, ch, out, lse);
 }
 
-// The same for many rows: a thread holds four channels of one row and takes the splits in ascending order.  (The kernel above
-// spreads the splits over a workgroup, for launches of few rows; with thousands of rows and a few splits most of its
-// threads have nothing to do: 2880 rows of 256 channels from 21 splits 58.7 us there, 16.5 us here.)  Taken from 65536 threads on.
+// The same with no exchange: a thread holds four channels of one row and takes the splits in ascending order, eight at a time.
 __global__ __launch_bounds__(256) void attn_combine_rows_kernel(const float* __restrict__ o, const float* __restrict__ m, const float* __restrict__ l,
                                                                 int n_splits, int nhkv, int n_rows, int D, int G,
                                                                 float* __restrict__ out, float* __restrict__ lse) {
@@ -668,21 +724,9 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(const float* __r
     const int64_t hr = i / per_row;
     if (hr >= stride) return;
     const int ch = (int)(i - hr * per_row) * 4;
-    float top = -INFINITY;
-    for (int s = 0; s < n_splits; ++s) top = fmaxf(top, m[s * stride + hr]);
-    if (top == -INFINITY) top = 0.f;
-    float total = 0.f;
-    f4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int s = 0; s < n_splits; ++s) {
-        const float w = expf(m[s * stride + hr] - top);
-        total += (l ? l[s * stride + hr] : 1.f) * w;
-        acc += *reinterpret_cast<const f4_t*>(o + (s * stride + hr) * D + ch) * w;
-    }
-    const int h = (int)(hr / n_rows), r = (int)(hr - (int64_t)h * n_rows);
-    const int64_t dst = (int64_t)(r / G) * (nhkv * G) + h * G + r % G;
-    *reinterpret_cast<f4_t*>(out + dst * D + ch) = acc * (1.f / fmaxf(total, 1e-30f));
-    if (ch == 0) lse[dst] = total > 0.f ? top + logf(fmaxf(total, 1e-30f)) : -INFINITY;
+    Joined j = {-INFINITY, 0.f, {0.f, 0.f, 0.f, 0.f}};
+    for (int s = 0; s < n_splits; s += 8) join_splits<8>(j, o, m, l, s, 1, n_splits, stride, hr, D, ch);
+    store_joined(j, hr, n_rows, nhkv, G, D, ch, out, lse);
 }
 
 template <int D, typename T>
@@ -715,14 +759,15 @@ bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p
 }  // namespace
 }  // namespace qvb8
 
-extern "C" int qvb8_attn_fwd(const void* q, int64_t sq_r, int64_t sq_h, const void* ki, const void* vi, int id_bytes,
-                             int64_t s_n, int64_t s_h, const float* kmid, const float* kstep, const float* vmid,
-                             const float* vstep, const float* kc, const float* vc, const int32_t* ts, const int32_t* tl,
-                             const int32_t* tseg, int64_t n_tiles, float* o, float* m, float* l, int64_t n_splits,
-                             int64_t n_rows, int64_t n_kv_heads, int64_t head_dim, int64_t q_pos0, int64_t tps,
-                             double scale, int64_t G, void* stream) {
+namespace {
+// q_dt: qvb8::kQReady, or the type of queries that still have to be prepared with q_scale
+int attn_forward(const void* q, int q_dt, float q_scale, int64_t sq_r, int64_t sq_h, const void* ki, const void* vi, int id_bytes,
+                 int64_t s_n, int64_t s_h, const float* kmid, const float* kstep, const float* vmid,
+                 const float* vstep, const float* kc, const float* vc, const int32_t* ts, const int32_t* tl,
+                 const int32_t* tseg, int64_t n_tiles, float* o, float* m, float* l, int64_t n_splits,
+                 int64_t n_rows, int64_t n_kv_heads, int64_t head_dim, int64_t q_pos0, int64_t tps,
+                 double scale, int64_t G, const char* who, void* stream) {
     using namespace qvb8;
-    const char* who = "qvb8_attn_fwd";
     if (head_dim != 128 && head_dim != 256) return host::fail(-1, "%s: head_dim must be 128 or 256, got %lld", who, (long long)head_dim);
     if (id_bytes != 1 && id_bytes != 2) return host::fail(-1, "%s: ids are 1 or 2 bytes wide, got %d", who, id_bytes);
     if (n_rows < 0 || n_tiles < 0 || n_splits < 1 || tps < 1 || G < 1 || n_kv_heads < 1)
@@ -734,7 +779,8 @@ extern "C" int qvb8_attn_fwd(const void* q, int64_t sq_r, int64_t sq_h, const vo
     if (!q || !o || !m || !l) return host::fail(-1, "%s: null q / o / m / l", who);
     if (n_tiles > 0 && (!ki || !vi || !kmid || !kstep || !vmid || !vstep || !kc || !vc || !ts || !tl || !tseg))
         return host::fail(-1, "%s: null ids, constants or tile table", who);
-    if (!aligned(q, 8) || (sq_r & 3) || (sq_h & 3)) return host::fail(-1, "%s: q must be 8-byte aligned with strides that are multiples of 4", who);
+    if (!aligned(q, q_dt == QVB8_F32 ? 16 : 8) || (sq_r & 3) || (sq_h & 3))
+        return host::fail(-1, "%s: q must be aligned to four elements with strides that are multiples of 4", who);
     if (n_tiles > 0) {
         if (!aligned(ki, 4 * id_bytes) || !aligned(vi, 4 * id_bytes) || (s_n & 3) || (s_h & 3))
             return host::fail(-1, "%s: ids must be aligned to four ids with strides that are multiples of 4", who);
@@ -746,7 +792,7 @@ extern "C" int qvb8_attn_fwd(const void* q, int64_t sq_r, int64_t sq_h, const vo
     if (n_splits > 65535 || row_blocks > 65535 || n_tiles > INT32_MAX || n_rows > INT32_MAX || q_pos0 > INT32_MAX / 2 || q_pos0 < INT32_MIN / 2)
         return host::fail(-1, "%s: size beyond what one launch takes", who);
     AttnArgs a;
-    a.q = static_cast<const uint16_t*>(q); a.sq_r = sq_r; a.sq_h = sq_h;
+    a.q = q; a.q_dt = q_dt; a.q_scale = q_scale; a.sq_r = sq_r; a.sq_h = sq_h;
     a.ki = ki; a.vi = vi; a.s_n = s_n; a.s_h = s_h;
     a.kmid = kmid; a.kstep = kstep; a.vmid = vmid; a.vstep = vstep; a.kc = kc; a.vc = vc;
     a.ts = ts; a.tl = tl; a.tseg = tseg; a.o = o; a.m = m; a.l = l;
@@ -755,6 +801,50 @@ extern "C" int qvb8_attn_fwd(const void* q, int64_t sq_r, int64_t sq_h, const vo
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (head_dim == 256) return id_bytes == 1 ? launch_attn<256, uint8_t>(a, n_splits, s) : launch_attn<256, uint16_t>(a, n_splits, s);
     return id_bytes == 1 ? launch_attn<128, uint8_t>(a, n_splits, s) : launch_attn<128, uint16_t>(a, n_splits, s);
+}
+}  // namespace
+
+extern "C" int qvb8_attn_fwd(const void* q, int64_t sq_r, int64_t sq_h, const void* ki, const void* vi, int id_bytes,
+                             int64_t s_n, int64_t s_h, const float* kmid, const float* kstep, const float* vmid,
+                             const float* vstep, const float* kc, const float* vc, const int32_t* ts, const int32_t* tl,
+                             const int32_t* tseg, int64_t n_tiles, float* o, float* m, float* l, int64_t n_splits,
+                             int64_t n_rows, int64_t n_kv_heads, int64_t head_dim, int64_t q_pos0, int64_t tps,
+                             double scale, int64_t G, void* stream) {
+    return attn_forward(q, qvb8::kQReady, 1.f, sq_r, sq_h, ki, vi, id_bytes, s_n, s_h, kmid, kstep, vmid, vstep, kc, vc, ts, tl, tseg,
+                        n_tiles, o, m, l, n_splits, n_rows, n_kv_heads, head_dim, q_pos0, tps, scale, G, "qvb8_attn_fwd", stream);
+}
+
+extern "C" int64_t qvb8_attn_workspace_bytes(int64_t n_splits, int64_t n_kv_heads, int64_t n_rows, int64_t head_dim) {
+    if (n_splits <= 0 || n_kv_heads <= 0 || n_rows <= 0 || head_dim <= 0) return 0;
+    return 4 * n_splits * n_kv_heads * n_rows * (head_dim + 2) + (n_rows >= qvb8::kWideFrom ? 16 + 2 * n_kv_heads * n_rows * head_dim : 0);
+}
+
+extern "C" int qvb8_attend(const void* q, int q_dtype, double q_scale, int64_t sq_r, int64_t sq_h, const void* ki, const void* vi, int id_bytes,
+                           int64_t s_n, int64_t s_h, const float* kmid, const float* kstep, const float* vmid,
+                           const float* vstep, const float* kc, const float* vc, const int32_t* ts, const int32_t* tl,
+                           const int32_t* tseg, int64_t n_tiles, int64_t n_splits, int64_t n_rows, int64_t n_kv_heads,
+                           int64_t head_dim, int64_t q_pos0, int64_t tps, int64_t G, float* out, float* lse, void* workspace,
+                           int64_t workspace_bytes, void* stream) {
+    using namespace qvb8;
+    const char* who = "qvb8_attend";
+    if (q_dtype < QVB8_F32 || q_dtype > QVB8_BF16) return host::fail(QVB8_ERR_ARG, "%s: unknown query type %d", who, q_dtype);
+    const int64_t need = qvb8_attn_workspace_bytes(n_splits, n_kv_heads, n_rows, head_dim);
+    if (need > 0 && (!workspace || workspace_bytes < need || !aligned(workspace, 16)))
+        return host::fail(QVB8_ERR_WORKSPACE, "%s: needs %lld bytes of 16-byte aligned workspace", who, (long long)need);
+    float* const o = static_cast<float*>(workspace);
+    const int64_t rows = n_splits * n_kv_heads * n_rows;
+    float* const m = o + rows * head_dim;
+    if (n_rows >= kWideFrom && q) {
+        // prepared once for all splits of the kernel of 128 rows
+        if (sq_h != head_dim || sq_r != n_kv_heads * G * head_dim) return host::fail(QVB8_ERR_UNSUPPORTED, "%s: %d rows and more must be contiguous", who, kWideFrom);
+        void* const q16 = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(m + 2 * rows) + 15) & ~(uintptr_t)15);
+        if (int rc = qvb8_scale_sat_half(q, q_dtype, n_kv_heads * n_rows * head_dim, (float)q_scale, q16, stream)) return rc;
+        q = q16;
+        q_dtype = kQReady;
+    }
+    if (int rc = attn_forward(q, q_dtype, (float)q_scale, sq_r, sq_h, ki, vi, id_bytes, s_n, s_h, kmid, kstep, vmid, vstep, kc, vc, ts, tl, tseg,
+                              n_tiles, o, m, m + rows, n_splits, n_rows, n_kv_heads, head_dim, q_pos0, tps, 1.0, G, who, stream)) return rc;
+    return qvb8_attn_combine(o, m, m + rows, n_splits, n_kv_heads, n_rows, head_dim, G, out, lse, stream);
 }
 
 extern "C" int qvb8_attn_combine(const float* o, const float* m, const float* l, int64_t n_splits, int64_t n_kv_heads,
@@ -769,14 +859,21 @@ extern "C" int qvb8_attn_combine(const float* o, const float* m, const float* l,
     if (!o || !m || !out || !lse) return host::fail(-1, "%s: null pointer", who);
     if (!aligned(o, 16) || !aligned(out, 16)) return host::fail(-1, "%s: o and out must be 16-byte aligned", who);
     if (n_kv_heads * n_rows > INT32_MAX || n_splits > INT32_MAX) return host::fail(-1, "%s: size beyond what one launch takes", who);
-    const int64_t quads = n_kv_heads * n_rows * (head_dim / 4);
-    if (quads >= 65536 && n_splits <= 64) {
+    const int64_t units = n_kv_heads * n_rows, quads = units * (head_dim / 4);
+    const unsigned parts = (unsigned)((head_dim + 15) / 16);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+#define QVB8_COMBINE_ARGS o, m, l, (int)n_splits, (int)n_kv_heads, (int)n_rows, (int)head_dim, (int)G, out, lse
+    // Measured alone, partial results in the caches (us; a thread a quad / a wave / four waves a unit): 1536 quads from 8 splits
+    // 3.0 / 3.5 / 3.7, from 171 26.5 / 6.1 / 4.6; 6144 from 8 3.1 / 3.6 / 5.3, from 24 5.0 / 4.3 / 5.4; 15360 from 24 5.1 / 5.2 / 9.2, from 64
+    // 11.7 / 6.4 / 9.7; 30720 from 32 7.3 / 8.0 / 15.5, from 64 12.4 / 9.7 / 16.8; 46592 from 64 13.8 / 16.9 / 24.0.  Behind the attention
+    // kernel, whole calls: 2304 quads from 299 splits 69 / 30.4 / 27.8, 6144 from 125 49 / 33.4 / 34.5, 7680 from 77 34.8 / 30.7 / 28.0, 9216 from
+    // 94 40.1 / 35.4 / 31.6, 10240 from 79 34.6 / 27.0 / 29.2.  (Two passes over the splits and a walk over 64 groups' results, four waves a
+    // unit up to 65536 quads: 6.5 us at 1536 quads from 171 splits, 19.7 at 46592 from 16.)
+    if (quads >= 40960 || n_splits <= 8 + quads / 1024) {
         if (quads > (int64_t)INT32_MAX * 256) return host::fail(-1, "%s: size beyond what one launch takes", who);
-        hipLaunchKernelGGL(attn_combine_rows_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                           o, m, l, (int)n_splits, (int)n_kv_heads, (int)n_rows, (int)head_dim, (int)G, out, lse);
-        return host::check_launch(who);
-    }
-    hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)(n_kv_heads * n_rows), (unsigned)((head_dim + 15) / 16)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       o, m, l, (int)n_splits, (int)n_kv_heads, (int)n_rows, (int)head_dim, (int)G, out, lse);
+        hipLaunchKernelGGL(attn_combine_rows_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, QVB8_COMBINE_ARGS);
+    } else if (quads > 9216) hipLaunchKernelGGL(attn_combine_kernel<1>, dim3((unsigned)((units + 3) / 4), parts), dim3(256), 0, st, QVB8_COMBINE_ARGS);
+    else hipLaunchKernelGGL(attn_combine_kernel<4>, dim3((unsigned)units, parts), dim3(256), 0, st, QVB8_COMBINE_ARGS);
+#undef QVB8_COMBINE_ARGS
     return host::check_launch(who);
 }
