@@ -191,6 +191,16 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
     request_x(0);
 
     // ---- where the rows' ids are; the first step's requests ----
+    // In operand order a request touches sixteen rows, a lane each.  With up to 16 pairs the lanes ask for chunk lane % 4 of row
+    // lane / 4 instead, so that four neighbours read consecutive bytes, and the registers change lanes afterwards: 40 tokens of 128
+    // experts 141.6 -> 134.2 us, 20 of 64 91.8 -> 84.5; with more pairs LDS has operands enough to serve: 509 tokens 209.5 -> 218.5.
+    constexpr bool kByRow = NT == 1;
+    const int ask_row = kByRow ? lane >> 2 : r, ask_chunk = kByRow ? lane & 3 : kg, pull = 4 * (4 * r + kg);
+    auto to_operand = [&](const uint4& v) __attribute__((always_inline)) -> uint4 {
+        if constexpr (!kByRow) return v;
+        return uint4{(uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.x), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.y),
+                     (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.z), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.w)};
+    };
     uint4 lo[2], hi[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -198,11 +208,16 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
         q.ok = !off_is_plane(off[t]) && row_in_bounds(off[t], q.nb, a.P, a.ids_bytes);        // stacks hold rows back to back only
         const uint32_t nb = (uint32_t)q.nb;
         q.sliced = q.ok && nb >= 4 && nb <= 8 && (off[t] & 31) == 0;
-        if (q.sliced) {
-            q.at = (uint64_t)(off[t] >> 3) + (uint32_t)kg * 4u * nb;
-            q.tail = 4u * (nb - 4u);
-            q.stride = 16u * nb;
-        } else { q.at = 0; q.tail = 16; q.stride = 0; }
+        // the row this lane asks for: its own, or the one of the lane that owns it
+        uint64_t base = q.sliced ? (uint64_t)(off[t] >> 3) : 0;
+        uint32_t ask_nb = q.sliced ? nb : 0u;
+        if constexpr (kByRow) {
+            const uint32_t low = __shfl((uint32_t)base, ask_row, 64), high = __shfl((uint32_t)(base >> 32), ask_row, 64);
+            base = (uint64_t)high << 32 | low;
+            ask_nb = __shfl(ask_nb, ask_row, 64);
+        }
+        if (ask_nb) { q.at = base + (uint32_t)ask_chunk * 4u * ask_nb; q.tail = 4u * (ask_nb - 4u); q.stride = 16u * ask_nb; }
+        else { q.at = 0; q.tail = 16; q.stride = 0; }
         const float zero = rintf(-a.min_s[row_at + row0[t]] / a.tau_s[row_at + row0[t]]);
         const int c = q.sliced ? (int)fminf(fmaxf(zero, 0.f), (float)((1 << q.nb) - 1)) : 0;          // (NaN: 0)
         q.centre = c;
@@ -224,9 +239,13 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
     if constexpr (DOWN) {
         float top = 0.f;
         const float* hrow = reinterpret_cast<const float*>(xrow);
-        for (int c = sub * 4; c < a.P; c += L::TPR * 4) {
-            const float4 h = *reinterpret_cast<const float4*>(hrow + c);
-            top = fmaxf(fmaxf(fmaxf(top, fabsf(h.x)), fabsf(h.y)), fmaxf(fabsf(h.z), fabsf(h.w)));
+        // eight requests at a time: one by one, the 12 trips of a 768-column row were 8 of the launch's 95 us
+        for (int c0 = sub * 4; c0 < a.P; c0 += L::TPR * 4 * 8) {
+            float4 h[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) h[k] = *reinterpret_cast<const float4*>(hrow + min(c0 + k * L::TPR * 4, a.P - 4));
+#pragma unroll
+            for (int k = 0; k < 8; ++k) top = fmaxf(fmaxf(fmaxf(top, fabsf(h[k].x)), fabsf(h[k].y)), fmaxf(fabsf(h[k].z), fabsf(h[k].w)));
         }
 #pragma unroll
         for (int o = L::TPR / 2; o >= 1; o >>= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
@@ -253,7 +272,7 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const GroupRow& q = g[t];
-            const uint4 l = lo[t], h = hi[t];
+            const uint4 l = to_operand(lo[t]), h = to_operand(hi[t]);
             switch (q.mode) {
                 case 4: decode_centred<4>(l, h, q.negb, b[t]); break;
                 case 5: decode_centred<5>(l, h, q.negb, b[t]); break;
