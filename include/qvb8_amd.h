@@ -53,9 +53,9 @@ enum qvb8_status {
 /* Library identification: ABI version, bumped on any signature change or new entry point (3: row lookup, attention over
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
  * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*;
- * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS; 12: qvb8r_gemv_as; 13: qvb8_attend).  A binding compares the loaded library's answer
+ * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS; 12: qvb8r_gemv_as; 13: qvb8_attend; 14: qvb8_kv_measure, qvb8_kv_wait).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
-#define QVB8_ABI_VERSION 13
+#define QVB8_ABI_VERSION 14
 int qvb8_abi_version(void);
 /* Message of the calling thread's most recent failure ("" if none). Valid until that thread's next call. */
 const char* qvb8_last_error(void);
@@ -467,6 +467,16 @@ int qvb8_kv_check(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_
                   int orig_dtype, int bits, double tau, const uint8_t* widths, float* lo, float* span, float* report, void* stream);
 int qvb8_kv_pack(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, const float* lo, const float* span,
                  const uint8_t* widths, float* step, uint8_t* const* packed, void* stream);
+
+/* qvb8_kv_range and qvb8_kv_check (widths NULL) as two launches that leave their figures where the host can read them while it goes on:
+ * found[heads][3] (pinned host memory) = each head's largest span, the least width >= bits that puts half a step of it within tau, and the
+ * largest error that width leaves; minima and spans in `lo` / `span` as there.  `scratch`: qvb8_kv_measure_floats floats of device
+ * memory.  qvb8_kv_wait returns when the figures have arrived (or the stream has ended without them: an error); `found` stays the
+ * library's until then. */
+int64_t qvb8_kv_measure_floats(int64_t heads, int64_t seq, int64_t dim);
+int qvb8_kv_measure(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, int orig_dtype, int bits, double tau,
+                    float* scratch, float* lo, float* span, float* found, void* stream);
+int qvb8_kv_wait(const float* found, int64_t heads, void* stream);
 
 /* Packed heads into the id layout of qvb8_attn_fwd: per entry seq x dim ids to ids_out (u8 or u16 by id_bytes; keys row_stride ids
  * apart), mid_out[dim] = min + step * c, step_out[dim] = step, *centre_out = c = (2^bits - 1) / 2.  `list`: host array, any number

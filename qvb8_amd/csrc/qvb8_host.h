@@ -59,6 +59,10 @@ inline int raise_lds_limit(size_t bytes, const char* who) {
     return 0;
 }
 
+// A host that polls a word a kernel writes asks the runtime this rarely (every few hundred microseconds) whether the stream still
+// runs: the question puts a marker into the stream and takes longer than most of these waits (a banded segment 59 us instead of 45).
+constexpr int64_t kPollsPerQuery = 1 << 18;
+
 // Integer knob from the environment, read on every call (cheap; lets a test change it between calls).
 inline int env_int(const char* name, int dflt) {
     const char* e = getenv(name);

@@ -9,8 +9,9 @@
 //
 // All four are bound by memory: x is read once per kernel (8 MB per 4096-key segment of 4 heads x 256 channels stay in the
 // caches after the first), everything else is smaller.  Measured on such a segment, keys and values and their layout:
-// 2868 us as ~100 torch launches with 64-bit temporaries per bit, 182 us with these (65 of them kernels; the rest is the host,
-// which has to read the widths before it can allocate the streams).
+// 2868 us as ~100 torch launches with 64-bit temporaries per bit; 193 us with a launch for each of range, join, check and pack and the
+// check's thousand figures written to the host; 146 us with the join in the check, three figures a head, and the ids packed at the
+// width asked for while those are on their way.  What is left is launches: 250 keys of 2 x 64 channels take 95 (153 before).
 //
 // Arithmetic is the codec's own expression by expression: fp32 differences, one IEEE division, rounding to nearest even,
 // products and sums rounded separately (contraction is off in this file).
@@ -54,11 +55,12 @@ __device__ __forceinline__ void load_values(const void* x, int64_t at, float (&v
 }
 
 // grid (chunks, heads).  partial[head][chunk][2][dim]: minima, maxima of the chunk's rows.  A thread owns V neighbouring
-// channels and every `lanes`-th row; the row groups meet in LDS.
+// channels and every `lanes`-th row; the row groups meet in LDS.  `clear` (or null): two words per head, zeroed for the launch that follows.
 template <int DT, int V>
-__global__ void __launch_bounds__(kKvThreads) kv_range_kernel(const void* x, int seq, int dim, int rows_per_chunk, float* partial) {
+__global__ void __launch_bounds__(kKvThreads) kv_range_kernel(const void* x, int seq, int dim, int rows_per_chunk, float* partial, uint32_t* clear) {
     extern __shared__ float s_red[];                                   // [groups][dim] x 2
     const int head = blockIdx.y, chunk = blockIdx.x;
+    if (clear && chunk == 0 && threadIdx.x < 2) clear[2 * head + threadIdx.x] = 0u;
     const int nv = dim / V, across = min(nv, kKvThreads), groups = kKvThreads / across;
     const int cv0 = threadIdx.x % across, group = threadIdx.x / across;
     const int r0 = chunk * rows_per_chunk, r1 = min(seq, r0 + rows_per_chunk);
@@ -106,38 +108,58 @@ __device__ __forceinline__ float id_of(float x, float lo, float step, float top)
     return fminf(fmaxf(rintf((x - lo) / step), 0.f), top);
 }
 
-// Joins the partial minima and maxima: grid (ceil(dim / 64), heads); wave w takes every fourth chunk, the waves meet in LDS.
-__global__ void __launch_bounds__(kKvThreads) kv_join_kernel(int dim, int chunks, const float* partial, float* lo_out, float* span_out) {
-    __shared__ float s_lo[4][64], s_hi[4][64];
+// Joins the partial minima and maxima: grid (ceil(dim / 64), heads); wave w takes every sixteenth chunk, the waves meet in LDS.  A
+// chain of trips; the calls that wait for it (qvb8_kv_measure) join in the check instead.
+constexpr int kJoinWaves = 16;
+__global__ void __launch_bounds__(64 * kJoinWaves) kv_join_kernel(int dim, int chunks, const float* partial, float* lo_out, float* span_out) {
+    __shared__ float s_lo[kJoinWaves][64], s_hi[kJoinWaves][64];
     const int head = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
     const float* p = partial + (int64_t)head * chunks * 2 * dim + min(c, dim - 1);
     float lo = __builtin_inff(), hi = -__builtin_inff();
 #pragma unroll 8
-    for (int k = wave; k < chunks; k += 4) { lo = fminf(lo, p[(int64_t)k * 2 * dim]); hi = fmaxf(hi, p[(int64_t)k * 2 * dim + dim]); }
+    for (int k = wave; k < chunks; k += kJoinWaves) { lo = fminf(lo, p[(int64_t)k * 2 * dim]); hi = fmaxf(hi, p[(int64_t)k * 2 * dim + dim]); }
     s_lo[wave][lane] = lo;
     s_hi[wave][lane] = hi;
     __syncthreads();
     if (wave == 0 && c < dim) {
-        lo = fminf(fminf(s_lo[0][lane], s_lo[1][lane]), fminf(s_lo[2][lane], s_lo[3][lane]));
-        hi = fmaxf(fmaxf(s_hi[0][lane], s_hi[1][lane]), fmaxf(s_hi[2][lane], s_hi[3][lane]));
+#pragma unroll
+        for (int w = 1; w < kJoinWaves; ++w) { lo = fminf(lo, s_lo[w][lane]); hi = fmaxf(hi, s_hi[w][lane]); }
         lo_out[(int64_t)head * dim + c] = lo;
         span_out[(int64_t)head * dim + c] = hi - lo;
     }
 }
 
+// What qvb8_kv_measure adds: the partial ranges to join, two zeroed words per head (largest error, workgroups that are done), and
+// where the figures go -- found[head][3] in memory the host reads: largest span, width, largest error.
+struct KvShown { const float* partial; int partials; uint32_t* state; float* found; };
+
 // grid (chunks, heads).  Fixes the head's width -- `given`, or the least one >= bits with half a step within tau -- and measures
 // the chunk's largest |decoded - x|.  report[head][2 + chunks]: largest span, width, the chunks' errors.
 template <int DT, int V>
 __global__ void __launch_bounds__(kKvThreads) kv_check_kernel(const void* x, int seq, int dim, int rows_per_chunk, int orig_dt,
-                                                              int bits, double tau, int use_given, KvWidths given, const float* lo_in, const float* span_in,
-                                                              float* report) {
+                                                              int bits, double tau, int use_given, KvWidths given, float* lo_io, float* span_io,
+                                                              float* report, KvShown shown) {
     __shared__ float s_lo[kKvMaxDim], s_step[kKvMaxDim], s4[4];
     const int head = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
     float widest = 0.f;
     for (int c = threadIdx.x; c < dim; c += kKvThreads) {
-        s_lo[c] = lo_in[(int64_t)head * dim + c];
-        s_step[c] = span_in[(int64_t)head * dim + c];
-        widest = fmaxf(widest, s_step[c]);
+        float lo, span;
+        if (shown.found) {
+            // every workgroup joins the partial ranges itself (a few dozen per channel): a launch less in front of the host's wait
+            const float* p = shown.partial + (int64_t)head * shown.partials * 2 * dim + c;
+            float hi = -__builtin_inff();
+            lo = __builtin_inff();
+#pragma unroll 8
+            for (int k = 0; k < shown.partials; ++k) { lo = fminf(lo, p[(int64_t)k * 2 * dim]); hi = fmaxf(hi, p[(int64_t)k * 2 * dim + dim]); }
+            span = hi - lo;
+            if (chunk == 0) { lo_io[(int64_t)head * dim + c] = lo; span_io[(int64_t)head * dim + c] = span; }
+        } else {
+            lo = lo_io[(int64_t)head * dim + c];
+            span = span_io[(int64_t)head * dim + c];
+        }
+        s_lo[c] = lo;
+        s_step[c] = span;
+        widest = fmaxf(widest, span);
     }
     widest = block_max(widest, s4);
     int width = use_given ? (int)given.w[head] : bits;
@@ -173,6 +195,25 @@ __global__ void __launch_bounds__(kKvThreads) kv_check_kernel(const void* x, int
         }
     }
     worst = block_max(worst, s4);
+    if (shown.found) {
+        if (threadIdx.x == 0) {
+            // The head's largest error and the number of its workgroups that have added theirs, both as atomics at the device's
+            // point of coherence, the second issued when the first has returned: the last one finds every error in.
+            uint32_t* state = shown.state + 2 * head;
+            const uint32_t before = __hip_atomic_fetch_max(state, __builtin_bit_cast(uint32_t, worst), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("" :: "v"(before) : "memory");
+            __builtin_amdgcn_s_waitcnt(0x0F70);                        // vmcnt(0)
+            if (__hip_atomic_fetch_add(state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)chunks - 1u) {
+                const uint32_t all = __hip_atomic_fetch_max(state, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                // three words a head across the bus (a word per workgroup, written by each: 6 of 15.8 us)
+                uint32_t* to = reinterpret_cast<uint32_t*>(shown.found) + 3 * head;
+                __hip_atomic_store(to, __builtin_bit_cast(uint32_t, widest), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(to + 1, __builtin_bit_cast(uint32_t, (float)width), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(to + 2, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+        return;
+    }
     if (threadIdx.x == 0) {
         float* rep = report + (int64_t)head * (2 + chunks);
         rep[2 + chunk] = worst;
@@ -364,7 +405,8 @@ extern "C" int64_t qvb8_kv_chunks(int64_t heads, int64_t seq) {
     return std::max<int64_t>(1, std::min<int64_t>({want, (seq + 15) / 16, 256}));
 }
 
-extern "C" int qvb8_kv_range(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, float* partial, int64_t chunks, void* stream) {
+namespace {
+int kv_range(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, float* partial, int64_t chunks, uint32_t* clear, void* stream) {
     if (int rc = bad_shape("qvb8_kv_range", x, x_dtype, heads, seq, dim)) return rc;
     if (!partial || chunks < 1 || chunks > 65535) return host::fail(QVB8_ERR_ARG, "qvb8_kv_range: bad partial results");
     const bool vec = vectors_ok(x, dim);
@@ -373,10 +415,15 @@ extern "C" int qvb8_kv_range(const void* x, int x_dtype, int64_t heads, int64_t 
     const dim3 grid((unsigned)chunks, (unsigned)heads);
     by_dtype(x_dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        if (vec) hipLaunchKernelGGL((kv_range_kernel<DT, 8>), grid, dim3(kKvThreads), lds, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), partial);
-        else hipLaunchKernelGGL((kv_range_kernel<DT, 1>), grid, dim3(kKvThreads), lds, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), partial);
+        if (vec) hipLaunchKernelGGL((kv_range_kernel<DT, 8>), grid, dim3(kKvThreads), lds, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), partial, clear);
+        else hipLaunchKernelGGL((kv_range_kernel<DT, 1>), grid, dim3(kKvThreads), lds, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), partial, clear);
     });
     return host::check_launch("qvb8_kv_range");
+}
+}  // namespace
+
+extern "C" int qvb8_kv_range(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, float* partial, int64_t chunks, void* stream) {
+    return kv_range(x, x_dtype, heads, seq, dim, partial, chunks, nullptr, stream);
 }
 
 extern "C" int qvb8_kv_check(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, const float* partial, int64_t chunks, int orig_dtype,
@@ -385,7 +432,7 @@ extern "C" int qvb8_kv_check(const void* x, int x_dtype, int64_t heads, int64_t 
     if (!partial || !lo || !span || chunks < 1 || chunks > 65535 || orig_dtype < QVB8_F32 || orig_dtype > QVB8_BF16)
         return host::fail(QVB8_ERR_ARG, "qvb8_kv_check: bad argument");
     if (!widths)                                               // (asked again with other widths: minima and spans are there)
-        hipLaunchKernelGGL(kv_join_kernel, dim3((unsigned)((dim + 63) / 64), (unsigned)heads), dim3(kKvThreads), 0, (hipStream_t)stream, (int)dim, (int)chunks, partial, lo, span);
+        hipLaunchKernelGGL(kv_join_kernel, dim3((unsigned)((dim + 63) / 64), (unsigned)heads), dim3(64 * kJoinWaves), 0, (hipStream_t)stream, (int)dim, (int)chunks, partial, lo, span);
     if (!report) return host::check_launch("qvb8_kv_check");   // nothing to certify
     if (bits < 1 || bits > 16 || !(tau > 0)) return host::fail(QVB8_ERR_ARG, "qvb8_kv_check: widths are 1..16 bits, tau > 0");
     KvWidths given = {};
@@ -397,8 +444,8 @@ extern "C" int qvb8_kv_check(const void* x, int x_dtype, int64_t heads, int64_t 
     const dim3 grid((unsigned)chunks, (unsigned)heads);
     by_dtype(x_dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        if (vectors_ok(x, dim)) hipLaunchKernelGGL((kv_check_kernel<DT, 8>), grid, dim3(kKvThreads), 0, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), orig_dtype, bits, tau, widths ? 1 : 0, given, lo, span, report);
-        else hipLaunchKernelGGL((kv_check_kernel<DT, 1>), grid, dim3(kKvThreads), 0, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), orig_dtype, bits, tau, widths ? 1 : 0, given, lo, span, report);
+        if (vectors_ok(x, dim)) hipLaunchKernelGGL((kv_check_kernel<DT, 8>), grid, dim3(kKvThreads), 0, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), orig_dtype, bits, tau, widths ? 1 : 0, given, lo, span, report, KvShown{});
+        else hipLaunchKernelGGL((kv_check_kernel<DT, 1>), grid, dim3(kKvThreads), 0, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), orig_dtype, bits, tau, widths ? 1 : 0, given, lo, span, report, KvShown{});
     });
     return host::check_launch("qvb8_kv_check");
 }
@@ -418,6 +465,52 @@ extern "C" int qvb8_kv_pack(const void* x, int x_dtype, int64_t heads, int64_t s
     const dim3 grid((unsigned)((a.n + 32 * kKvThreads - 1) / (32 * kKvThreads)), (unsigned)heads);
     by_dtype(x_dtype, [&](auto dt) { hipLaunchKernelGGL((kv_pack_kernel<decltype(dt)::value>), grid, dim3(kKvThreads), 0, (hipStream_t)stream, a); });
     return host::check_launch("qvb8_kv_pack");
+}
+
+// Ranges, least widths and their errors as two launches, the figures on their way to the host when it has packed at the widths it
+// expects (qvb8_kv_pack) and comes to wait for them (qvb8_kv_wait).
+namespace {
+constexpr int64_t kMeasurePartials = 32;                       // per head: every workgroup of the check joins them
+int64_t measure_partials(int64_t seq) { return std::max<int64_t>(1, std::min<int64_t>(kMeasurePartials, (seq + 15) / 16)); }
+constexpr uint32_t kUnwritten = 0xBF800000u;                   // -1: none of the figures is negative
+}
+extern "C" int64_t qvb8_kv_measure_floats(int64_t heads, int64_t seq, int64_t dim) {
+    return heads < 1 || seq < 1 || dim < 1 ? 0 : heads * (measure_partials(seq) * 2 * dim + 2);
+}
+extern "C" int qvb8_kv_measure(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, int orig_dtype, int bits, double tau,
+                               float* scratch, float* lo, float* span, float* found, void* stream) {
+    if (int rc = bad_shape("qvb8_kv_measure", x, x_dtype, heads, seq, dim)) return rc;
+    if (!scratch || !lo || !span || !found || (reinterpret_cast<uintptr_t>(found) & 3u) || orig_dtype < QVB8_F32 || orig_dtype > QVB8_BF16 || bits < 1 || bits > 16 || !(tau > 0))
+        return host::fail(QVB8_ERR_ARG, "qvb8_kv_measure: bad argument");
+    const int64_t partials = measure_partials(seq), chunks = std::min<int64_t>(qvb8_kv_chunks(heads, seq), std::max<int64_t>(1, 2 * host::device_cus() / heads));
+    KvShown shown = {scratch, (int)partials, reinterpret_cast<uint32_t*>(scratch + heads * partials * 2 * dim), found};
+    uint32_t* words = reinterpret_cast<uint32_t*>(found);
+    for (int64_t i = 0; i < 3 * heads; ++i) __atomic_store_n(words + i, kUnwritten, __ATOMIC_RELEASE);
+    if (int rc = kv_range(x, x_dtype, heads, seq, dim, scratch, partials, shown.state, stream)) return rc;
+    const dim3 grid((unsigned)chunks, (unsigned)heads);
+    by_dtype(x_dtype, [&](auto dt) {
+        constexpr int DT = decltype(dt)::value;
+        if (vectors_ok(x, dim)) hipLaunchKernelGGL((kv_check_kernel<DT, 8>), grid, dim3(kKvThreads), 0, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), orig_dtype, bits, tau, 0, KvWidths{}, lo, span, nullptr, shown);
+        else hipLaunchKernelGGL((kv_check_kernel<DT, 1>), grid, dim3(kKvThreads), 0, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), orig_dtype, bits, tau, 0, KvWidths{}, lo, span, nullptr, shown);
+    });
+    return host::check_launch("qvb8_kv_measure");
+}
+
+extern "C" int qvb8_kv_wait(const float* found, int64_t heads, void* stream) {
+    if (!found || heads < 1 || heads > QVB8_KV_MAX_HEADS) return host::fail(QVB8_ERR_ARG, "qvb8_kv_wait: bad argument");
+    const uint32_t* words = reinterpret_cast<const uint32_t*>(found);
+    const int64_t n = 3 * heads;
+    int64_t at = 0;
+    for (int64_t spins = 1; at < n; ++spins) {                 // ends with the stream at the latest
+        while (at < n && __atomic_load_n(words + at, __ATOMIC_ACQUIRE) != kUnwritten) ++at;
+        if (at == n || spins % host::kPollsPerQuery) continue;
+        const hipError_t e = hipStreamQuery((hipStream_t)stream);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return host::fail(QVB8_ERR_LAUNCH, "qvb8_kv_wait: the check did not run: %s", hipGetErrorString(e));
+        for (; at < n; ++at)
+            if (__atomic_load_n(words + at, __ATOMIC_ACQUIRE) == kUnwritten) return host::fail(QVB8_ERR_LAUNCH, "qvb8_kv_wait: the check left no figures");
+    }
+    return 0;
 }
 
 extern "C" int qvb8_kv_unpack(const qvb8_kv_head* list, int64_t n_list, int64_t dim, int id_bytes, int64_t row_stride, void* stream) {

@@ -1239,7 +1239,7 @@ extern "C" int qvb8_moe_experts_checked(const void* X, int x_dtype, int64_t toke
     // The plan kernel writes the counter in the middle of its work; the products are queued behind it by now.  (An event between
     // the two, waited for instead, put 8 us of idle GPU there.)  The wait ends with the stream at the latest.
     for (int64_t spins = 1; __atomic_load_n(bad_pairs, __ATOMIC_ACQUIRE) < 0; ++spins) {
-        if (spins % 4096) continue;
+        if (spins % host::kPollsPerQuery) continue;
         const hipError_t e = hipStreamQuery((hipStream_t)stream);
         if (e == hipErrorNotReady) continue;
         if (e != hipSuccess || __atomic_load_n(bad_pairs, __ATOMIC_ACQUIRE) < 0)

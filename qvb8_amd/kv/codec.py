@@ -141,44 +141,62 @@ _STORED_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 
 def _band_on_gpu(t, orig_dtype, bits: int, tau: float, certify: bool) -> list:
-    """band_kv_heads on the HIP library: ranges, widths with the error they leave (one host read; a head that still misses tau
-    is checked again one bit wider), then the ids at their final widths straight into their packed streams."""
+    """band_kv_heads on the HIP library: ranges, and the least widths with the error they leave; while those figures are on their way to
+    the host, the ids are packed at the width asked for.  Heads that need more are packed again, checked again one bit wider while
+    they still miss tau."""
     heads, seq, dim = t.shape
     x = t.detach()
     x = (x if x.dtype in _STORED_DTYPES else x.to(torch.float32)).contiguous()
-    lib, dev, dt = _lib.load(), x.device, _lib.dtype_code(x.dtype)
+    lib, dev, dt, odt = _lib.load(), x.device, _lib.dtype_code(x.dtype), _lib.dtype_code(orig_dtype)
     certifying = bool(certify and tau > 0)
     with _lib.on_device_of(x):
-        stream = _lib.stream_of(x)
-        chunks = lib.qvb8_kv_chunks(heads, seq)
-        partial = torch.empty(heads * chunks * 2 * dim, dtype=torch.float32, device=dev)
-        lo, span, step = torch.empty((3, heads, dim), dtype=torch.float32, device=dev).unbind(0)
-        # the kernel writes its report where the host reads it: pinned memory, no copy behind it
-        report = torch.empty((heads, 2 + chunks), dtype=torch.float32, pin_memory=True) if certifying else None
-        _lib._check(lib.qvb8_kv_range(x.data_ptr(), dt, heads, seq, dim, partial.data_ptr(), chunks, stream), lib)
+        stream, x_at = _lib.stream_of(x), x.data_ptr()
+        grid = torch.empty((3, heads, dim), dtype=torch.float32, device=dev)                          # minima, steps, spans
+        lo_at, step_at, span_at = (grid.data_ptr() + 4 * heads * dim * i for i in range(3))
 
-        def check(widths):
-            given = None if widths is None else bytes(widths)
-            _lib._check(lib.qvb8_kv_check(x.data_ptr(), dt, heads, seq, dim, partial.data_ptr(), chunks, _lib.dtype_code(orig_dtype), bits,
-                                          float(tau), given, lo.data_ptr(), span.data_ptr(), report.data_ptr() if certifying else None, stream), lib)
-            if not certifying:
-                return None
-            torch.cuda.current_stream().synchronize()
-            return torch.cat([report[:, :2], report[:, 2:].amax(1, keepdim=True)], 1).tolist()        # span, width, largest error
+        def pack(widths):
+            packed = [torch.empty((seq * dim * w + 7) // 8, dtype=torch.uint8, device=dev) for w in widths]
+            where = (ctypes.c_void_p * heads)(*[p.data_ptr() for p in packed])
+            _lib._check(lib.qvb8_kv_pack(x_at, dt, heads, seq, dim, lo_at, span_at, bytes(widths), step_at, where, stream), lib)
+            return packed
 
-        found = check(None)
         widths = [bits] * heads
-        if certifying:
-            widths = [_first_width(r[0], bits, tau) for r in found]
-            if widths != [int(r[1]) for r in found]:         # a span on the edge of a power of two: the host's logarithm decides
-                found = check(widths)
-            while not all(r[2] <= tau for r in found):
-                widths = [w if r[2] <= tau else _next_width(i, w, r[2], tau, orig_dtype) for i, (w, r) in enumerate(zip(widths, found))]
-                found = check(widths)
-        packed = [torch.empty((seq * dim * w + 7) // 8, dtype=torch.uint8, device=dev) for w in widths]
-        where = (ctypes.c_void_p * heads)(*[p.data_ptr() for p in packed])
-        _lib._check(lib.qvb8_kv_pack(x.data_ptr(), dt, heads, seq, dim, lo.data_ptr(), span.data_ptr(), bytes(widths), step.data_ptr(), where, stream), lib)
-    return [BandedKV(packed[i], lo[i], step[i], widths[i], (seq, dim), orig_dtype, tau) for i in range(heads)]
+        if not certifying:
+            chunks = lib.qvb8_kv_chunks(heads, seq)
+            partial = torch.empty(heads * chunks * 2 * dim, dtype=torch.float32, device=dev)
+            _lib._check(lib.qvb8_kv_range(x_at, dt, heads, seq, dim, partial.data_ptr(), chunks, stream), lib)
+            _lib._check(lib.qvb8_kv_check(x_at, dt, heads, seq, dim, partial.data_ptr(), chunks, odt, bits, float(tau), None, lo_at, span_at, None, stream), lib)
+            packed = pack(widths)
+            los, steps = (g.unbind(0) for g in grid[:2].unbind(0))
+        else:
+            scratch = torch.empty(lib.qvb8_kv_measure_floats(heads, seq, dim), dtype=torch.float32, device=dev)
+            shown = torch.empty(3 * heads, dtype=torch.float32, pin_memory=True)
+            _lib._check(lib.qvb8_kv_measure(x_at, dt, heads, seq, dim, odt, bits, float(tau), scratch.data_ptr(), lo_at, span_at, shown.data_ptr(), stream), lib)
+            try:
+                packed = pack(widths)
+                los, steps = (g.unbind(0) for g in grid[:2].unbind(0))
+            finally:
+                _lib._check(lib.qvb8_kv_wait(shown.data_ptr(), heads, stream), lib)       # the figures are written whatever happened since
+            found = shown.tolist()
+            widths = [_first_width(found[3 * i], bits, tau) for i in range(heads)]
+            errors = found[2::3]
+
+            def check():
+                chunks = lib.qvb8_kv_chunks(heads, seq)
+                report = torch.empty((heads, 2 + chunks), dtype=torch.float32, pin_memory=True)
+                _lib._check(lib.qvb8_kv_check(x_at, dt, heads, seq, dim, scratch.data_ptr(), chunks, odt, bits, float(tau), bytes(widths), lo_at, span_at,
+                                              report.data_ptr(), stream), lib)
+                torch.cuda.current_stream().synchronize()
+                return report[:, 2:].amax(1).tolist()
+
+            if widths != [int(w) for w in found[1::3]]:          # a span on the edge of a power of two: the host's logarithm decides
+                errors = check()
+            while not all(e <= tau for e in errors):
+                widths = [w if e <= tau else _next_width(i, w, e, tau, orig_dtype) for i, (w, e) in enumerate(zip(widths, errors))]
+                errors = check()
+            if widths != [bits] * heads:
+                packed = pack(widths)
+    return [BandedKV(p, m, s, w, (seq, dim), orig_dtype, tau) for p, m, s, w in zip(packed, los, steps, widths)]
 
 
 def band_kv_heads(t: torch.Tensor, orig_dtype: torch.dtype, bits: int, tau: float = 0.0, certify: bool = True) -> list:

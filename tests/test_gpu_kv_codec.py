@@ -64,3 +64,26 @@ def test_tile_tables_of_many_segments(n_seg):
     want, got = (FA.QVLayout(ids.to(d), ids.to(d), *[p.to(d) for p in parts], lens, d) for d in ("cpu", DEV))
     for name in ("t_start", "t_len", "t_seg"):
         assert torch.equal(getattr(got, name).cpu(), getattr(want, name)), name
+
+
+@pytest.mark.parametrize("heads,seq,dim,dtype", [(1, 1, 3, torch.float32), (2, 16, 64, torch.bfloat16), (3, 17, 40, torch.float16), (32, 511, 8, torch.bfloat16),
+                                                 (2, 512, 256, torch.bfloat16), (1, 4096, 2048, torch.bfloat16)])
+@pytest.mark.parametrize("bits,tau", [(7, 0.25), (3, 0.01)])
+def test_figures_for_the_waiting_host_are_the_checks(heads, seq, dim, dtype, bits, tau):
+    """qvb8_kv_measure + qvb8_kv_wait (partial ranges joined by every workgroup, three words a head) against qvb8_kv_range + qvb8_kv_check."""
+    from qvb8_amd import _lib
+    lib, code = _lib.load(), {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype]
+    x = _values(heads, seq, dim, dtype, seed=seq).to(DEV)
+    s, chunks = _lib.stream_of(x), lib.qvb8_kv_chunks(heads, seq)
+    partial, both = torch.empty(heads * chunks * 2 * dim, device=DEV), torch.empty(2, 2, heads, dim, device=DEV)
+    report = torch.empty(heads, 2 + chunks, pin_memory=True)
+    _lib._check(lib.qvb8_kv_range(x.data_ptr(), code, heads, seq, dim, partial.data_ptr(), chunks, s), lib)
+    _lib._check(lib.qvb8_kv_check(x.data_ptr(), code, heads, seq, dim, partial.data_ptr(), chunks, code, bits, tau, None, both[0, 0].data_ptr(), both[0, 1].data_ptr(),
+                                  report.data_ptr(), s), lib)
+    scratch, found = torch.empty(lib.qvb8_kv_measure_floats(heads, seq, dim), device=DEV), torch.empty(heads, 3, pin_memory=True)
+    for _ in range(3):                                           # the words the workgroups meet in are cleared by every call
+        _lib._check(lib.qvb8_kv_measure(x.data_ptr(), code, heads, seq, dim, code, bits, tau, scratch.data_ptr(), both[1, 0].data_ptr(), both[1, 1].data_ptr(),
+                                        found.data_ptr(), s), lib)
+        _lib._check(lib.qvb8_kv_wait(found.data_ptr(), heads, s), lib)
+        assert torch.equal(both[0].view(torch.int32), both[1].view(torch.int32))
+        assert torch.equal(found, torch.cat([report[:, :2], report[:, 2:].amax(1, keepdim=True)], 1))
