@@ -50,7 +50,7 @@ def _decode_to(code, dtype, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_id
     n_esc = _check_escapes(esc_idx, esc_vals)
     ids, min_s, tau_s = ids.contiguous(), min_s.contiguous(), tau_s.contiguous()
     row_nbits, row_bit_off = row_nbits.contiguous(), row_bit_off.contiguous()
-    with torch.cuda.device(ids.device):
+    with _lib.on_device_of(ids):
         out = torch.empty((Q, int(P)), dtype=dtype, device=ids.device)
         st = _lib.stream_of(ids)
         if rowinfo is not None:
@@ -97,7 +97,7 @@ def lookup_rows(rows, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc
     ids, min_s, tau_s = ids.contiguous(), min_s.contiguous(), tau_s.contiguous()
     row_nbits, row_bit_off = row_nbits.contiguous(), row_bit_off.contiguous()
     code = _lib.dtype_code(out_dtype)
-    with torch.cuda.device(ids.device):
+    with _lib.on_device_of(ids):
         out = torch.empty((rows.numel(), int(P)), dtype=out_dtype, device=ids.device)
         ei = esc_idx.contiguous() if n_esc else None
         ev = esc_vals.contiguous() if n_esc else None
@@ -115,7 +115,7 @@ def certify(restored: torch.Tensor, original: torch.Tensor, tau: float):
     if restored.numel() != original.numel():
         raise RuntimeError("certify: tensors differ in size")
     a, b = restored.contiguous(), original.contiguous()
-    with torch.cuda.device(a.device):
+    with _lib.on_device_of(a):
         res = torch.empty(2, dtype=torch.int32, device=a.device)
         _lib._check(lib.qvb8_certify(_lib.ptr(a), _lib.dtype_code(a.dtype), _lib.ptr(b), _lib.dtype_code(b.dtype),
                                      a.numel(), float(tau), res.data_ptr(), _lib.stream_of(a)), lib)
@@ -132,7 +132,7 @@ def saturating_half(X: torch.Tensor) -> torch.Tensor:
     Xc = X.contiguous()
     if Xc.dtype not in (torch.float32, torch.bfloat16):
         Xc = Xc.float()
-    with torch.cuda.device(Xc.device):
+    with _lib.on_device_of(Xc):
         out = torch.empty(Xc.shape, dtype=torch.float16, device=Xc.device)
         _lib._check(lib.qvb8_sat_half(_lib.ptr(Xc), _lib.dtype_code(Xc.dtype), Xc.numel(), _lib.ptr(out),
                                       _lib.stream_of(Xc)), lib)
@@ -156,7 +156,7 @@ def gemv_multi(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_val
         Xc = Xc.float()
     ids, min_s, tau_s = ids.contiguous(), min_s.contiguous(), tau_s.contiguous()
     row_nbits, row_bit_off = row_nbits.contiguous(), row_bit_off.contiguous()
-    with torch.cuda.device(Xc.device):
+    with _lib.on_device_of(Xc):
         Y = torch.empty((M, Q), dtype=torch.float32, device=Xc.device)
         ei = esc_idx.contiguous() if n_esc else None
         ev = esc_vals.contiguous() if n_esc else None
@@ -197,7 +197,7 @@ def mma_prepare(row_nbits, row_bit_off, tau_s, min_s, P, ids_bytes, perm=None):
         perm = perm.contiguous()
     else:
         perm = None
-    with torch.cuda.device(row_nbits.device):
+    with _lib.on_device_of(row_nbits):
         out = torch.empty(lib.qvb8_mma_rowinfo_bytes(Q) // 8, dtype=torch.int64, device=row_nbits.device)
         _lib._check(lib.qvb8_mma_prepare(_lib.ptr(row_nbits), _lib.ptr(row_bit_off), _lib.ptr(tau_s), _lib.ptr(min_s),
                                          _lib.ptr(perm), Q, int(P),
@@ -438,14 +438,15 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
     Q = _check_pack(ids, min_s, row_nbits, row_bit_off, tau_s)
     n_esc = _check_escapes(esc_idx, esc_vals)
     _lib.require_cuda(X)
-    if X.dim() != 2 or X.shape[1] != int(P):
-        raise RuntimeError(f"X must be (M, {int(P)})")
+    P, x_dtype = int(P), X.dtype
+    if X.dim() != 2 or X.shape[1] != P:
+        raise RuntimeError(f"X must be (M, {P})")
     M = X.shape[0]
     if not 1 <= M <= (MMA_GEMM_MAX_M if layout is not None else MMA_MAX_M):
         raise RuntimeError(f"qvb8 mma-multi: M={M} outside 1..{MMA_GEMM_MAX_M if layout is not None else MMA_MAX_M}")
-    if int(P) % 128 != 0 or ids.data_ptr() % 4 != 0:
+    if P % 128 != 0 or ids.data_ptr() % 4 != 0:
         raise RuntimeError("qvb8 mma-multi: needs P%128==0 and 4-byte-aligned ids")
-    if X.dtype not in (torch.float16, torch.bfloat16):
+    if x_dtype is not torch.float16 and x_dtype is not torch.bfloat16:
         raise RuntimeError("qvb8 mma-multi: X must be fp16 or bf16")
     if perm is not None and perm.numel():
         if perm.dtype != torch.int32 or perm.numel() != Q or not perm.is_cuda:
@@ -453,36 +454,38 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
         perm = perm.contiguous()
     else:
         perm = None
-    if rowinfo is not None and (rowinfo.dtype != torch.int64 or rowinfo.numel() * 8 != lib.qvb8_mma_rowinfo_bytes(Q)
-                                or not rowinfo.is_cuda):
+    records = ((Q + 1) // 2 * 16 + Q * 16) if Q > 0 else 0             # qvb8_mma_rowinfo_bytes
+    if rowinfo is not None and (rowinfo.dtype != torch.int64 or rowinfo.numel() * 8 != records or not rowinfo.is_cuda):
         raise RuntimeError("qvb8 mma-multi: rowinfo must be the int64 GPU tensor mma_prepare returned")
+    if out_dtype is torch.float16 or out_dtype is torch.bfloat16:
+        if n_esc:
+            raise RuntimeError("qvb8 mma-multi: fp16 / bf16 results need a weight without escapes")
+        flags = MMA_Y_F16 if out_dtype is torch.float16 else MMA_Y_BF16
+    elif out_dtype in (None, torch.float32):
+        out_dtype, flags = torch.float32, 0
+    else:
+        raise RuntimeError("qvb8 mma-multi: results are fp32, fp16 or bf16")
+    flags |= (MMA_SATURATE_X if saturate else 0) | (MMA_PLANES if planes else 0) | (MMA_SILU_PAIRS if silu_pairs else 0)
     Xc = X.contiguous()
     ids, min_s, tau_s = ids.contiguous(), min_s.contiguous(), tau_s.contiguous()
     row_nbits, row_bit_off = row_nbits.contiguous(), row_bit_off.contiguous()
-    with torch.cuda.device(Xc.device):
-        if out_dtype in (torch.float16, torch.bfloat16):
-            if n_esc:
-                raise RuntimeError("qvb8 mma-multi: fp16 / bf16 results need a weight without escapes")
-            y_flag = MMA_Y_F16 if out_dtype == torch.float16 else MMA_Y_BF16
-        elif out_dtype in (None, torch.float32):
-            out_dtype, y_flag = torch.float32, 0
-        else:
-            raise RuntimeError("qvb8 mma-multi: results are fp32, fp16 or bf16")
+    ei, ev = (esc_idx.contiguous(), esc_vals.contiguous()) if n_esc else (None, None)
+    records_at = None if rowinfo is None else rowinfo.contiguous()
+    with _lib.on_device_of(Xc):
         Y = torch.empty((M, Q // 2 if silu_pairs else Q), dtype=out_dtype, device=Xc.device)
-        ei = esc_idx.contiguous() if n_esc else None
-        ev = esc_vals.contiguous() if n_esc else None
-        need = lib.qvb8_mma_workspace_bytes(M, Q, int(P))          # row records when none are passed; more for the tiled kernel
-        ws = None if (rowinfo is not None and need <= lib.qvb8_mma_rowinfo_bytes(Q)) else \
-            torch.empty((need + 7) // 8, dtype=torch.int64, device=Xc.device)
-        _lib._check(lib.qvb8_mma(_lib.ptr(Xc), _lib.dtype_code(Xc.dtype), M, _lib.ptr(ids), ids.numel(),
-                                 _lib.ptr(min_s), _lib.ptr(tau_s), _lib.ptr(row_nbits), _lib.ptr(row_bit_off),
-                                 Q, int(P), _lib.ptr(ei), _lib.ptr(ev), n_esc, _lib.ptr(perm),
-                                 None if rowinfo is None else rowinfo.contiguous().data_ptr(),
-                                 None if layout is None else ctypes.addressof(layout),
-                                 (MMA_SATURATE_X if saturate else 0) | y_flag | (MMA_PLANES if planes else 0)
-                                 | (MMA_SILU_PAIRS if silu_pairs else 0), _lib.ptr(Y),
-                                 None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel() * 8,
-                                 _lib.stream_of(Xc)), lib)
+        ws, ws_bytes = None, 0
+        if rowinfo is None or M > MMA_SILU_MAX_M:                      # up to 16 rows the records are all a call needs
+            need = lib.qvb8_mma_workspace_bytes(M, Q, P)
+            if rowinfo is None or need > records:
+                ws = torch.empty((need + 7) // 8, dtype=torch.int64, device=Xc.device)
+                ws_bytes = ws.numel() * 8
+        # (an empty tensor's address is 0: null)
+        rc = lib.qvb8_mma(Xc.data_ptr(), _lib.F16 if x_dtype is torch.float16 else _lib.BF16, M, ids.data_ptr(), ids.numel(), min_s.data_ptr(),
+                          tau_s.data_ptr(), row_nbits.data_ptr(), row_bit_off.data_ptr(), Q, P, None if ei is None else ei.data_ptr(),
+                          None if ev is None else ev.data_ptr(), n_esc, None if perm is None else perm.data_ptr(),
+                          None if records_at is None else records_at.data_ptr(), None if layout is None else ctypes.addressof(layout), flags,
+                          Y.data_ptr(), None if ws is None else ws.data_ptr(), ws_bytes, _lib.stream_of(Xc))
+        _lib._check(rc, lib)
     return Y
 
 
@@ -501,7 +504,7 @@ def mlp_init(gu_ids, gu_rowinfo, gu_layout, dn_ids, dn_rowinfo, dn_layout, hidde
     lib = _lib.load()
     _lib.require_cuda(gu_ids, gu_rowinfo, dn_ids, dn_rowinfo)
     plan = _lib.MlpPlan()
-    with torch.cuda.device(gu_ids.device):
+    with _lib.on_device_of(gu_ids):
         ws = torch.empty(int(lib.qvb8_mlp_workspace_bytes(int(inter))), dtype=torch.uint8, device=gu_ids.device)
         _lib._check(lib.qvb8_mlp_init(int(hidden), int(inter), int(out_features),
                                       gu_ids.data_ptr(), gu_ids.numel(), gu_rowinfo.data_ptr(), ctypes.addressof(gu_layout),
@@ -524,7 +527,7 @@ def mlp_fused(X, workspace, plan, mid_dtype=None, out_dtype=None, act=MLP_SILU_G
     mid_dtype = X.dtype if mid_dtype is None else mid_dtype
     out_dtype = X.dtype if out_dtype is None else out_dtype
     Xc = X.contiguous()
-    with torch.cuda.device(Xc.device):
+    with _lib.on_device_of(Xc):
         Y = torch.empty((M, int(plan.out_features)), dtype=out_dtype, device=Xc.device)
         _lib._check(lib.qvb8_mlp(ctypes.addressof(plan), _lib.ptr(Xc), _lib.dtype_code(Xc.dtype), M, int(act), _lib.dtype_code(mid_dtype),
                                  Y.data_ptr(), _lib.dtype_code(out_dtype), workspace.data_ptr(), _lib.stream_of(Xc)), lib)
@@ -588,7 +591,7 @@ def _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids
     if Xc.data_ptr() % 16:                      # a view into the middle of a buffer: the kernels load 16 bytes of a row at a time
         Xc = Xc.clone()
     tens = [t.contiguous() for t in (up_ids, up_min, up_tau, up_nb, up_off, dn_ids, dn_min, dn_tau, dn_nb, dn_off)]
-    with torch.cuda.device(Xc.device):
+    with _lib.on_device_of(Xc):
         out = torch.empty((T, int(Qdn)), dtype=Xc.dtype, device=Xc.device)
         if T == 0:
             return out
@@ -599,11 +602,11 @@ def _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids
         if checked:
             bad = torch.empty(1, dtype=torch.int32, pin_memory=True)
             entry, extra = lib.qvb8_moe_experts_checked, (bad.data_ptr(),)
+        at = [t.data_ptr() for t in tens]                       # (an empty tensor's address is 0: null)
         _lib._check(entry(
-            _lib.ptr(Xc), _lib.dtype_code(Xc.dtype), T, _lib.ptr(idxc), _lib.ptr(wc), k, E,
-            _lib.ptr(u[0]), u[0].numel(), _lib.ptr(u[1]), _lib.ptr(u[2]), _lib.ptr(u[3]), _lib.ptr(u[4]), int(Qup), int(Pup),
-            _lib.ptr(d[0]), d[0].numel(), _lib.ptr(d[1]), _lib.ptr(d[2]), _lib.ptr(d[3]), _lib.ptr(d[4]), int(Qdn), int(Pdn),
-            act, _lib.ptr(out), _lib.dtype_code(out.dtype), _lib.ptr(ws), ws.numel(), *extra, _lib.stream_of(Xc)), lib)
+            Xc.data_ptr(), _lib.dtype_code(Xc.dtype), T, idxc.data_ptr(), wc.data_ptr(), k, E,
+            at[0], u[0].numel(), *at[1:5], int(Qup), int(Pup), at[5], d[0].numel(), *at[6:], int(Qdn), int(Pdn),
+            act, out.data_ptr(), _lib.dtype_code(out.dtype), ws.data_ptr(), ws.numel(), *extra, _lib.stream_of(Xc)), lib)
         if checked and int(bad[0]):
             return None
     return out

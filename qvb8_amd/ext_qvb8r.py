@@ -91,7 +91,7 @@ def decode(words, off, states, tiles, blocks, tab, perm, mn, ts, drow, P, out_dt
     c, Q, _ = _core(words, off, states, tiles, blocks, tab, perm, mn, ts, drow, P)
     dt = _OUT[int(out_dtype)]
     rows = Q if row_base < 0 else int(nrows)
-    with torch.cuda.device(mn.device):
+    with _lib.on_device_of(mn):
         W = torch.empty((rows, int(P)), dtype=dt, device=mn.device)
         _lib._check(lib.qvb8r_decode(ctypes.byref(c), _rows_bound(tiles, T), _ABI_DT[dt], int(b0), int(nb), int(row_base),
                                      W.data_ptr(), rows, _lib.stream_of(mn)), lib)
@@ -110,7 +110,7 @@ def decode_blocks(block_list, words, off, states, tiles, blocks, tab, perm, mn, 
     Tb = _rows_bound(tiles, T)
     dt = torch.int16 if int(out_dtype) == 3 else _OUT[int(out_dtype)]
     n = block_list.numel()
-    with torch.cuda.device(mn.device):
+    with _lib.on_device_of(mn):
         W = torch.empty((n * 8 * Tb, int(P)), dtype=dt, device=mn.device)
         _lib._check(lib.qvb8r_decode_blocks(ctypes.byref(c), Tb, _ABI_DT[dt], block_list.data_ptr(), n, W.data_ptr(), W.shape[0],
                                             _lib.stream_of(mn)), lib)
@@ -121,7 +121,7 @@ def ids(P, words, off, states, tiles, blocks, tab, perm, mn, ts, drow, T=None):
     """The band ids (Q, P) int16 in original row order (qvb8r_cuda.cu:426-444)."""
     lib = _lib.load()
     c, Q, _ = _core(words, off, states, tiles, blocks, tab, perm, mn, ts, drow, P)
-    with torch.cuda.device(mn.device):
+    with _lib.on_device_of(mn):
         W = torch.empty((Q, int(P)), dtype=torch.int16, device=mn.device)
         _lib._check(lib.qvb8r_decode(ctypes.byref(c), _rows_bound(tiles, T), 3, 0, c.n_blocks, -1, W.data_ptr(), Q,
                                      _lib.stream_of(mn)), lib)
