@@ -53,9 +53,10 @@ enum qvb8_status {
 /* Library identification: ABI version, bumped on any signature change or new entry point (3: row lookup, attention over
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
  * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*;
- * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS; 12: qvb8r_gemv_as; 13: qvb8_attend; 14: qvb8_kv_measure, qvb8_kv_wait).  A binding compares the loaded library's answer
+ * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS; 12: qvb8r_gemv_as; 13: qvb8_attend; 14: qvb8_kv_measure, qvb8_kv_wait;
+ * 15: qvb8_mma_escapes_workspace_bytes).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
-#define QVB8_ABI_VERSION 14
+#define QVB8_ABI_VERSION 15
 int qvb8_abi_version(void);
 /* Message of the calling thread's most recent failure ("" if none). Valid until that thread's next call. */
 const char* qvb8_last_error(void);
@@ -176,6 +177,8 @@ typedef struct qvb8_mma_layout {
  * first); from 17 rows on, when P % 256 == 0, what the workgroup-tiled kernels need (narrowed activations, their sums per
  * column range, partial results of the column ranges). */
 int64_t qvb8_mma_workspace_bytes(int64_t M, int64_t Q, int64_t P);
+/* ... for fp16 / bf16 results of a weight with escapes. */
+int64_t qvb8_mma_escapes_workspace_bytes(int64_t M, int64_t Q, int64_t P);
 
 /* Y[m, q] = sum_c X[m, c] * value(q, c), fp32 accumulate on v_mfma 16x16x32, Y f32 (M, Q) row-major.
  * X is (M, P) fp16 or bf16 (x_dtype QVB8_F16 / QVB8_BF16), 16-byte aligned, P % 128 == 0, 1 <= M <= 48 (up to 256 under the

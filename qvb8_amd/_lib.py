@@ -14,13 +14,13 @@ import torch
 from .common.errors import NativeLibraryError
 
 _LIB = None
-EXPECTED_ABI = 14           # QVB8_ABI_VERSION of include/qvb8_amd.h that the argument lists below were written for
+EXPECTED_ABI = 15           # QVB8_ABI_VERSION of include/qvb8_amd.h that the argument lists below were written for
 F32, F16, BF16 = 0, 1, 2
 _DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
 # every symbol include/qvb8_amd.h declares
 SYMBOLS = ("qvb8_abi_version", "qvb8_last_error", "qvb8_decode", "qvb8_lookup_rows", "qvb8_scatter_escapes", "qvb8_certify",
-           "qvb8_sat_half", "qvb8_scale_sat_half", "qvb8_gemv_workspace_bytes", "qvb8_gemv", "qvb8_mma_rowinfo_bytes", "qvb8_mma_prepare", "qvb8_decode_tiles", "qvb8_mma_workspace_bytes", "qvb8_mma", "qvb8_launch_probe", "qvb8_mlp_workspace_bytes", "qvb8_mlp_init", "qvb8_mlp",
+           "qvb8_sat_half", "qvb8_scale_sat_half", "qvb8_gemv_workspace_bytes", "qvb8_gemv", "qvb8_mma_rowinfo_bytes", "qvb8_mma_prepare", "qvb8_decode_tiles", "qvb8_mma_workspace_bytes", "qvb8_mma_escapes_workspace_bytes", "qvb8_mma", "qvb8_launch_probe", "qvb8_mlp_workspace_bytes", "qvb8_mlp_init", "qvb8_mlp",
            "qvb8_moe_workspace_bytes", "qvb8_moe_experts", "qvb8_moe_experts_checked", "qvb8_moe_experts_static",
            "qvb8r_decode", "qvb8r_decode_blocks", "qvb8r_gemv_workspace_bytes", "qvb8r_gemv", "qvb8r_gemv_as", "qvb8r_walk_probe", "qvb8r_fix_escapes", "qvb8_attn_fwd", "qvb8_attn_combine", "qvb8_attn_workspace_bytes", "qvb8_attend",
            "qvb8_kv_chunks", "qvb8_kv_range", "qvb8_kv_check", "qvb8_kv_pack", "qvb8_kv_measure_floats", "qvb8_kv_measure", "qvb8_kv_wait", "qvb8_kv_unpack", "qvb8_kv_tiles")
@@ -81,6 +81,8 @@ def load(build_if_missing: bool = True):
     lib.qvb8_gemv.argtypes = [vp, i32, i64, vp, i64, vp, vp, vp, vp, i64, i64, vp, vp, i64, vp, vp, i64, vp]
     lib.qvb8_mma_workspace_bytes.argtypes = [i64, i64, i64]
     lib.qvb8_mma_workspace_bytes.restype = i64
+    lib.qvb8_mma_escapes_workspace_bytes.argtypes = [i64] * 3
+    lib.qvb8_mma_escapes_workspace_bytes.restype = i64
     lib.qvb8_mma_rowinfo_bytes.argtypes = [i64]
     lib.qvb8_mma_rowinfo_bytes.restype = i64
     lib.qvb8_mma_prepare.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, vp, vp]

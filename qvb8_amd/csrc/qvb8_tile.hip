@@ -668,6 +668,66 @@ __global__ void __launch_bounds__(256) tile_fix_escapes_kernel(const uint16_t* _
     Y[(size_t)t * Q + q] += acc;
 }
 
+// The same for results in the caller's 16-bit type: what the kernels left in fp32 (Y32) rounded into Y, rows with escapes corrected first.
+// Bound by its dependent trips to memory, so: a workgroup takes 64 rows by 16 tokens, finds its place in the ascending list 256 samples
+// at a time (one trip up to 65536 escapes, where a thread's own search is a trip per bisection) and marks each row's first escape;
+// a thread keeps one row and four tokens, so an escape's band value is read once for the four and what needs no escape is loaded before
+// the search.  A row's escapes are added in ascending order, no atomics: the values of tile_fix_escapes_kernel and a cast, which as two launches
+// took 34816 x 5120, 16 rows, 3000 escapes 39.3 us a call, 38.7 this way; 2000 x 2048, 7 rows, 500 escapes 28.4, 22.6.
+constexpr int kFinishRows = 64, kFinishTokens = 16;
+template <bool BF, bool XC>
+__global__ void __launch_bounds__(256) finish_escapes_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict__ ids, int64_t ids_bytes,
+        const float* __restrict__ min_s, const float* __restrict__ tau_s, const uint8_t* __restrict__ nbits, const int64_t* __restrict__ bit_off,
+        const int64_t* __restrict__ esc_idx, const float* __restrict__ esc_vals, int64_t n_esc, const float* __restrict__ Y32, void* __restrict__ Y, int out_dt, int Q, int P) {
+    __shared__ int64_t s_first[kFinishRows];
+    constexpr int kEach = kFinishTokens / 4;
+    const int tid = threadIdx.x, q0 = blockIdx.x * kFinishRows, rows = min(kFinishRows, Q - q0);
+    const int r = tid & (kFinishRows - 1), q = min(q0 + r, Q - 1), t0 = blockIdx.y * kFinishTokens + (tid >> 6) * kEach;
+    float v[kEach];
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) v[k] = Y32[(size_t)min(t0 + k, M - 1) * Q + q];
+    const int nb = nbits[q];
+    const int64_t bit0 = bit_off[q];
+    const float ts = tau_s[q], mn = min_s[q];
+    const int64_t from = (int64_t)q0 * P, to = from + (int64_t)rows * P;
+    if (tid < kFinishRows) s_first[tid] = -1;
+    int64_t lo = 0, left = n_esc;                              // the first escape at or behind `from` is in [lo, lo + left]
+    while (left > 256) {
+        const int64_t step = (left + 255) / 256, at = lo + (tid + 1) * step - 1;
+        const int64_t below = __syncthreads_count(at < lo + left && esc_idx[min(at, n_esc - 1)] < from);
+        lo += below * step;
+        left = min(step, left - below * step);
+    }
+    __syncthreads();
+    for (int64_t i0 = lo; i0 < n_esc; i0 += 256) {
+        const int64_t i = i0 + tid, at = i < n_esc ? esc_idx[i] : to, before = i > 0 && i <= n_esc ? esc_idx[i - 1] : -1;
+        if (at >= from && at < to) {
+            const int row = (int)((uint32_t)(at - from) / (uint32_t)P);
+            if (before < from + (int64_t)row * P) s_first[row] = i;
+        }
+        if (__syncthreads_or(at >= to)) break;                 // ascending: nothing behind it is of these rows
+    }
+    if (r >= rows) return;
+    const int64_t first = s_first[r], row0 = (int64_t)q * P;
+    if (first >= 0) {
+        const int64_t clamp_byte = (ids_bytes - 8) & ~(int64_t)3;
+        float acc[kEach] = {};
+        for (int64_t e = first; e < n_esc; ++e) {
+            const int64_t c = esc_idx[e] - row0;
+            if (c >= P) break;
+            const float off = esc_vals[e] - __builtin_fmaf((float)row_field(ids, bit0, nb, (int)c, clamp_byte), ts, mn);
+#pragma unroll
+            for (int k = 0; k < kEach; ++k)
+                acc[k] = __builtin_fmaf(XIn<BF, XC>::scalar(X[(size_t)min(t0 + k, M - 1) * P + c]), off, acc[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) v[k] += acc[k];
+    }
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (t0 + k < M) store_y(static_cast<float*>(Y), out_dt, (int64_t)(t0 + k) * Q + q, v[k]);
+}
+
 // ---- dense restore in tile order ------------------------------------------------------------------------------
 // The rows of a 16-row tile stored in planes lie together in memory but far apart in the weight: a wave that restores one
 // output row picks 16 bytes out of every 256 of its tile, and the lines it leaves are fetched again by whoever restores the
@@ -1576,6 +1636,12 @@ extern "C" int64_t qvb8_mma_workspace_bytes(int64_t M, int64_t Q, int64_t P) {
     return qvb8_mma_rowinfo_bytes(Q);
 }
 
+// fp32 results behind what the kernels need: those of a call whose own are 16-bit and corrected
+extern "C" int64_t qvb8_mma_escapes_workspace_bytes(int64_t M, int64_t Q, int64_t P) {
+    if (M < 1 || Q < 1 || P < 1) return 0;
+    return align256i(qvb8_mma_workspace_bytes(M, Q, P)) + M * Q * 4;
+}
+
 extern "C" int qvb8_mma(const void* X, int x_dtype, int64_t M,
                         const uint8_t* ids, int64_t ids_bytes, const float* min_s, const float* tau_s,
                         const uint8_t* nbits, const int64_t* bit_off, int64_t Q, int64_t P,
@@ -1619,9 +1685,19 @@ extern "C" int qvb8_mma(const void* X, int x_dtype, int64_t M,
         a.first2 = n > 2 ? layout->first_pos[2] : (int)Q;
         a.n_classes = n;
     }
-    const int out_dt = (flags & QVB8_MMA_Y_F16) ? 1 : (flags & QVB8_MMA_Y_BF16) ? 2 : 0;
+    int out_dt = (flags & QVB8_MMA_Y_F16) ? 1 : (flags & QVB8_MMA_Y_BF16) ? 2 : 0;
     a.planes = (flags & QVB8_MMA_PLANES) ? 1 : 0;
-    if (out_dt != 0 && n_esc > 0) return host::fail(QVB8_ERR_ARG, "qvb8_mma: fp16 / bf16 results need a weight without escapes (the correction adds to fp32 results)");
+    void* finished = nullptr;                                  // 16-bit results of a weight with escapes, and their type
+    int finished_dt = 0;
+    if (out_dt != 0 && n_esc > 0) {
+        const int64_t need = qvb8_mma_escapes_workspace_bytes(M, Q, P);
+        if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15u) || (flags & QVB8_MMA_SILU_PAIRS))
+            return host::fail(QVB8_ERR_ARG, "qvb8_mma: fp16 / bf16 results need a weight without escapes, or workspace for fp32 results (the correction adds to those)");
+        finished = Y;
+        finished_dt = out_dt;
+        Y = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(workspace) + align256i(qvb8_mma_workspace_bytes(M, Q, P)));
+        out_dt = 0;
+    }
     a.silu_pairs = (flags & QVB8_MMA_SILU_PAIRS) ? 1 : 0;
     if (a.silu_pairs) {
         if (!layout || out_dt == 0 || M > 16)
@@ -1711,6 +1787,15 @@ extern "C" int qvb8_mma(const void* X, int x_dtype, int64_t M,
 #undef QVB8_TILE_LAUNCH
 #undef QVB8_TILE_LAUNCH_P
         if (rc) return rc;
+    }
+    if (finished) {
+        const dim3 grid((unsigned)((Q + kFinishRows - 1) / kFinishRows), (unsigned)((M + kFinishTokens - 1) / kFinishTokens));
+#define QVB8_FINISH_ARGS grid, dim3(256), 0, s, (const uint16_t*)X, (int)M, ids, ids_bytes, min_s, tau_s, nbits, bit_off, esc_idx, esc_vals, n_esc, Y, finished, finished_dt, (int)Q, (int)P
+        if (mode == 0) hipLaunchKernelGGL((finish_escapes_kernel<false, false>), QVB8_FINISH_ARGS);
+        else if (mode == 1) hipLaunchKernelGGL((finish_escapes_kernel<false, true>), QVB8_FINISH_ARGS);
+        else hipLaunchKernelGGL((finish_escapes_kernel<true, false>), QVB8_FINISH_ARGS);
+#undef QVB8_FINISH_ARGS
+        return host::check_launch("qvb8_mma escapes");
     }
     if (n_esc > 0) {
         dim3 grid((unsigned)((n_esc + 255) / 256), (unsigned)M);

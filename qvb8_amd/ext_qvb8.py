@@ -423,7 +423,7 @@ def sort_rows_by_width(ids, row_nbits, row_bit_off, P, perm, planes=False):
 
 
 def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals, perm=None, saturate=True,
-              rowinfo=None, layout=None, out_dtype=None, planes=False, silu_pairs=False):
+              rowinfo=None, layout=None, out_dtype=None, planes=False, silu_pairs=False, escapes_first=False):
     """Matrix-core path for P % 128 == 0: X (fp16 or bf16) times the fp32 band value, fp32 (M, Q).  1 <= M <= 48 always;
     49 <= M <= 256 (the workgroup-tiled decode + GEMM kernel) when `layout` is given and its widths are 4..8.
     `perm` (int32, position -> row) groups rows of equal width into tiles; `rowinfo` = mma_prepare(...) for the
@@ -433,7 +433,8 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
     multiplied as it is on bf16 operands.  `out_dtype` torch.float16 / torch.bfloat16: the kernels store the results
     rounded to that type (the same values as casting the fp32 result; only for a weight without escapes).  `planes`:
     the pack has rows stored in planes (sort_rows_by_width(planes=True)).  `silu_pairs` (fp16 / bf16 results, at most 16
-    rows of X, rows stored by QVBandMLPV8): (M, Q / 2) silu(gate) * up, rounded at every step."""
+    rows of X, rows stored by QVBandMLPV8): (M, Q / 2) silu(gate) * up, rounded at every step.  `escapes_first`: `out_dtype` also
+    for a weight with escapes (ascending positions): corrected in fp32, then rounded."""
     lib = _lib.load()
     Q = _check_pack(ids, min_s, row_nbits, row_bit_off, tau_s)
     n_esc = _check_escapes(esc_idx, esc_vals)
@@ -458,7 +459,7 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
     if rowinfo is not None and (rowinfo.dtype != torch.int64 or rowinfo.numel() * 8 != records or not rowinfo.is_cuda):
         raise RuntimeError("qvb8 mma-multi: rowinfo must be the int64 GPU tensor mma_prepare returned")
     if out_dtype is torch.float16 or out_dtype is torch.bfloat16:
-        if n_esc:
+        if n_esc and not escapes_first:
             raise RuntimeError("qvb8 mma-multi: fp16 / bf16 results need a weight without escapes")
         flags = MMA_Y_F16 if out_dtype is torch.float16 else MMA_Y_BF16
     elif out_dtype in (None, torch.float32):
@@ -474,7 +475,10 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
     with _lib.on_device_of(Xc):
         Y = torch.empty((M, Q // 2 if silu_pairs else Q), dtype=out_dtype, device=Xc.device)
         ws, ws_bytes = None, 0
-        if rowinfo is None or M > MMA_SILU_MAX_M:                      # up to 16 rows the records are all a call needs
+        if n_esc and out_dtype is not torch.float32:
+            ws_bytes = lib.qvb8_mma_escapes_workspace_bytes(M, Q, P)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=Xc.device)
+        elif rowinfo is None or M > MMA_SILU_MAX_M:                    # up to 16 rows the records are all a call needs
             need = lib.qvb8_mma_workspace_bytes(M, Q, P)
             if rowinfo is None or need > records:
                 ws = torch.empty((need + 7) // 8, dtype=torch.int64, device=Xc.device)

@@ -340,13 +340,13 @@ class QVBandLinearV8(nn.Module):
         if order is not None:
             perm, rowinfo, layout = order
             xm = xk if xk.dtype in (torch.float16, torch.bfloat16) else ext.saturating_half(xk)
-            # without escapes and bias the kernels round the results to the caller's type themselves: no cast pass over Y
-            direct = out_dtype if (ei.numel() == 0 and self.bias is None and out_dtype in (torch.float16, torch.bfloat16)) else None
+            # without bias the library rounds the results to the caller's type itself: no cast pass over Y
+            direct = out_dtype if (self.bias is None and out_dtype in (torch.float16, torch.bfloat16)) else None
             # (the dict of the buffers: a module's attribute access costs as much as the launch's arguments)
             held = self._buffers
             y = ext.mma_tiles(xm, held["ids"], held["min_s"], held["nbits"], held["bit_off"], self.in_features, held["tau_s"],
                               ei, ev, perm=perm, saturate=not bf16_mode, rowinfo=rowinfo, layout=layout, out_dtype=direct,
-                              planes=self._planes)
+                              planes=self._planes, escapes_first=True)
             if direct is not None:
                 return y if len(orig) == 2 else y.reshape(*orig[:-1], self.out_features)
             return self._finish(y, orig, out_dtype)

@@ -1,0 +1,59 @@
+"""16-bit results of a weight with escapes: corrected in fp32, then rounded, in one launch behind the kernels (ext.mma_tiles with
+escapes_first)."""
+import pytest
+import torch
+
+from qvb8_amd import ext_qvb8 as ext
+from qvb8_amd.formats.qvb8 import pack as PK
+from qvb8_amd.formats.qvb8.module import QVBandLinearV8
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _sorted_pack(Q, P, seed):
+    d = H.mixed_width_pack(Q, P, [7, 6, 5], seed=seed)
+    d["tau_s"] = d["tau_s"] * (1.0 / 64)
+    ids, min_s, nbits, bit_off, P, tau_s, _, _ = H.to_device_args(d, DEV)
+    perm = torch.argsort(nbits.to(torch.int16), stable=True).to(torch.int32)
+    ids, bit_off, layout = ext.sort_rows_by_width(ids, nbits, bit_off, P, perm)
+    rowinfo = ext.mma_prepare(nbits, bit_off, tau_s, min_s, P, ids.numel(), perm)
+    return (ids, min_s, nbits, bit_off, P, tau_s), dict(perm=perm, rowinfo=rowinfo, layout=layout)
+
+
+def _escapes(positions, seed):
+    at = torch.tensor(sorted(set(positions)), dtype=torch.int64)
+    return at.to(DEV), torch.randn(at.numel(), generator=torch.Generator().manual_seed(seed)).to(DEV)
+
+
+@pytest.mark.parametrize("M", [1, 7, 16, 17, 64, 256])
+@pytest.mark.parametrize("x_dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16), (torch.bfloat16, torch.float16)])
+def test_same_values_as_rounding_the_corrected_fp32_results(M, x_dtype, out_dtype):
+    """Bit for bit, with escapes in the first and the last place of a row and of the 64 rows a workgroup takes, a row full of them,
+    none in whole workgroups, one in 29 columns, and Q that ends inside a workgroup."""
+    for Q, P in ((300, 768), (129, 2048)):
+        pack, order = _sorted_pack(Q, P, seed=M + Q)
+        x = torch.randn(M, P, generator=torch.Generator().manual_seed(M)).to(x_dtype).to(DEV)
+        edges = [0, P - 1, P, 63 * P, 64 * P - 1, 64 * P, 64 * P + P - 1, 128 * P + 5, Q * P - 1]
+        everywhere = list(range(0, Q * P, 29))
+        for positions in ([Q * P - 1], edges, edges + list(range(70 * P, 71 * P)), everywhere):
+            esc = _escapes(positions, seed=M)
+            for saturate in (True, False):
+                y32 = ext.mma_tiles(x, *pack, *esc, saturate=saturate, **order)
+                y16 = ext.mma_tiles(x, *pack, *esc, saturate=saturate, out_dtype=out_dtype, escapes_first=True, **order)
+                assert y16.dtype == out_dtype and torch.equal(y16, y32.to(out_dtype)), (Q, P, len(positions), saturate)
+
+
+@pytest.mark.parametrize("n_esc", [256, 257, 65536, 65537, 70000])
+def test_long_lists_through_the_module(n_esc):
+    """One search step more from 257 and from 65537 escapes on; the module against fp32 results rounded by torch."""
+    Q, P = 192, 1024
+    enc = PK.encode_tensor(H.synth_weight(Q, P, seed=3).to(DEV), 1e-3, restore="fp16")
+    enc["esc_idx"], enc["esc_vals"] = _escapes(torch.randperm(Q * P, generator=torch.Generator().manual_seed(n_esc))[:n_esc].tolist(), seed=4)
+    x = torch.randn(5, P, generator=torch.Generator().manual_seed(1)).to(torch.float16).to(DEV)
+    lin = QVBandLinearV8.from_encoded(enc)
+    y = lin(x)
+    perm, rowinfo, layout = lin._mma_order()
+    y32 = ext.mma_tiles(x, *H.pack_args(dict(enc, ids=lin.ids, nbits=lin.nbits, bit_off=lin.bit_off)), perm=perm, rowinfo=rowinfo, layout=layout, planes=lin._planes)
+    assert y.dtype == torch.float16 and torch.equal(y, y32.to(torch.float16))
