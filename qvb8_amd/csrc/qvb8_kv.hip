@@ -11,7 +11,8 @@
 // caches after the first), everything else is smaller.  Measured on such a segment, keys and values and their layout:
 // 2868 us as ~100 torch launches with 64-bit temporaries per bit; 193 us with a launch for each of range, join, check and pack and the
 // check's thousand figures written to the host; 146 us with the join in the check, three figures a head, and the ids packed at the
-// width asked for while those are on their way.  What is left is launches: 250 keys of 2 x 64 channels take 95 (153 before).
+// width asked for while those are on their way; 119 us with several rows' loads on their way at once and the heads' counters apart.
+// What is left is launches: the kernels take 57 of them, 250 keys of 2 x 64 channels take 95 (153 before).
 //
 // Arithmetic is the codec's own expression by expression: fp32 differences, one IEEE division, rounding to nearest even,
 // products and sums rounded separately (contraction is off in this file).
@@ -34,34 +35,53 @@ constexpr float kKvStepFloor = 1e-12f;
 
 __device__ __forceinline__ float finite_or_zero(float v) { return __builtin_fabsf(v) < __builtin_inff() ? v : 0.f; }   // NaN compares false
 
+// V neighbouring values of a row as they are stored, and as fp32 (NaN and infinities read as 0).  Loading and converting are apart, so
+// that the loads of several rows are on their way together.
+template <int DT, int V>
+struct Values {
+    static constexpr int kWords = V == 8 ? (DT == QVB8_F32 ? 8 : 4) : 1;
+    uint32_t w[kWords];
+    __device__ __forceinline__ void load(const void* x, int64_t at) {
+        if constexpr (V == 8) {
+            const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(x) + at * (DT == QVB8_F32 ? 4 : 2));
+#pragma unroll
+            for (int k = 0; k < kWords / 4; ++k) {
+                const uint4 q = p[k];
+                w[4 * k] = q.x; w[4 * k + 1] = q.y; w[4 * k + 2] = q.z; w[4 * k + 3] = q.w;
+            }
+        } else {
+            w[0] = DT == QVB8_F32 ? reinterpret_cast<const uint32_t*>(x)[at] : reinterpret_cast<const uint16_t*>(x)[at];
+        }
+    }
+    __device__ __forceinline__ float operator[](int k) const {
+        if constexpr (DT == QVB8_F32) return finite_or_zero(__builtin_bit_cast(float, w[k]));
+        const uint32_t h = (w[k / 2] >> (16 * (k % 2))) & 0xFFFFu;
+        return finite_or_zero(DT == QVB8_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h));
+    }
+};
 template <int DT, int V>
 __device__ __forceinline__ void load_values(const void* x, int64_t at, float (&v)[V]) {
-    if constexpr (V == 8 && DT == QVB8_F32) {
-        const float4 a = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(x) + at), b = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(x) + at + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else if constexpr (V == 8) {
-        const uint4 q = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(x) + at);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+    Values<DT, V> raw;
+    raw.load(x, at);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const uint32_t h = (w[k / 2] >> (16 * (k % 2))) & 0xFFFFu;
-            v[k] = DT == QVB8_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
-        }
-    } else {
-        v[0] = load_as_f32<DT>(x, at);
-    }
-#pragma unroll
-    for (int k = 0; k < V; ++k) v[k] = finite_or_zero(v[k]);
+    for (int k = 0; k < V; ++k) v[k] = raw[k];
 }
+// Rows in flight per thread (range: twice as many).  One row after the other, a trip to memory each, the range of 4 x 4096 x 256 bf16
+// values took 9.1 us; 5.4 this way.
+constexpr int kKvRows = 4;
 
 // grid (chunks, heads).  partial[head][chunk][2][dim]: minima, maxima of the chunk's rows.  A thread owns V neighbouring
-// channels and every `lanes`-th row; the row groups meet in LDS.  `clear` (or null): two words per head, zeroed for the launch that follows.
+// channels and every `groups`-th row; the row groups meet in LDS.  `clear` (or null): two words per head, zeroed for the launch that follows.
+// Words that many workgroups add to lie this far apart: atomics on one cache line wait for each other (128 workgroups of four heads on one
+// line: the check takes 20.2 us, 11.5 this way).
+constexpr int kStateApart = 64;
+constexpr int kRangeThreads = 512;            // there are few chunks: every workgroup that follows reads all their results
 template <int DT, int V>
-__global__ void __launch_bounds__(kKvThreads) kv_range_kernel(const void* x, int seq, int dim, int rows_per_chunk, float* partial, uint32_t* clear) {
+__global__ void __launch_bounds__(kRangeThreads) kv_range_kernel(const void* x, int seq, int dim, int rows_per_chunk, float* partial, uint32_t* clear) {
     extern __shared__ float s_red[];                                   // [groups][dim] x 2
     const int head = blockIdx.y, chunk = blockIdx.x;
-    if (clear && chunk == 0 && threadIdx.x < 2) clear[2 * head + threadIdx.x] = 0u;
-    const int nv = dim / V, across = min(nv, kKvThreads), groups = kKvThreads / across;
+    if (clear && chunk == 0 && threadIdx.x < 2) clear[(2 * head + threadIdx.x) * kStateApart] = 0u;
+    const int nv = dim / V, across = min(nv, kRangeThreads), groups = kRangeThreads / across;
     const int cv0 = threadIdx.x % across, group = threadIdx.x / across;
     const int r0 = chunk * rows_per_chunk, r1 = min(seq, r0 + rows_per_chunk);
     float* s_hi = s_red + groups * dim;
@@ -70,11 +90,14 @@ __global__ void __launch_bounds__(kKvThreads) kv_range_kernel(const void* x, int
             float lo[V], hi[V];
 #pragma unroll
             for (int k = 0; k < V; ++k) { lo[k] = __builtin_inff(); hi[k] = -__builtin_inff(); }
-            for (int r = r0 + group; r < r1; r += groups) {
-                float v[V];
-                load_values<DT, V>(x, ((int64_t)head * seq + r) * dim + cv * V, v);
+            for (int r = r0 + group; r < r1; r += groups * 2 * kKvRows) {
+                Values<DT, V> v[2 * kKvRows];                          // (a row past the end: the last one again)
 #pragma unroll
-                for (int k = 0; k < V; ++k) { lo[k] = fminf(lo[k], v[k]); hi[k] = fmaxf(hi[k], v[k]); }
+                for (int j = 0; j < 2 * kKvRows; ++j) v[j].load(x, ((int64_t)head * seq + min(r + j * groups, r1 - 1)) * dim + cv * V);
+#pragma unroll
+                for (int j = 0; j < 2 * kKvRows; ++j)
+#pragma unroll
+                    for (int k = 0; k < V; ++k) { lo[k] = fminf(lo[k], v[j][k]); hi[k] = fmaxf(hi[k], v[j][k]); }
             }
 #pragma unroll
             for (int k = 0; k < V; ++k) { s_red[group * dim + cv * V + k] = lo[k]; s_hi[group * dim + cv * V + k] = hi[k]; }
@@ -82,7 +105,7 @@ __global__ void __launch_bounds__(kKvThreads) kv_range_kernel(const void* x, int
     }
     __syncthreads();
     float* out = partial + ((int64_t)head * gridDim.x + chunk) * 2 * dim;
-    for (int c = threadIdx.x; c < dim; c += kKvThreads) {
+    for (int c = threadIdx.x; c < dim; c += kRangeThreads) {
         float lo = s_red[c], hi = s_hi[c];
         for (int g = 1; g < groups; ++g) { lo = fminf(lo, s_red[g * dim + c]); hi = fmaxf(hi, s_hi[g * dim + c]); }
         out[c] = lo;
@@ -131,6 +154,7 @@ __global__ void __launch_bounds__(64 * kJoinWaves) kv_join_kernel(int dim, int c
 
 // What qvb8_kv_measure adds: the partial ranges to join, two zeroed words per head (largest error, workgroups that are done), and
 // where the figures go -- found[head][3] in memory the host reads: largest span, width, largest error.
+constexpr int kJoinAtOnce = 16;                // (a partial result past the last: that one again)
 struct KvShown { const float* partial; int partials; uint32_t* state; float* found; };
 
 // grid (chunks, heads).  Fixes the head's width -- `given`, or the least one >= bits with half a step within tau -- and measures
@@ -141,6 +165,16 @@ __global__ void __launch_bounds__(kKvThreads) kv_check_kernel(const void* x, int
                                                               float* report, KvShown shown) {
     __shared__ float s_lo[kKvMaxDim], s_step[kKvMaxDim], s4[4];
     const int head = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
+    const int nv = dim / V, across = min(nv, kKvThreads), groups = kKvThreads / across;
+    const int cv0 = threadIdx.x % across, group = threadIdx.x / across;
+    const int r0 = chunk * rows_per_chunk, r1 = min(seq, r0 + rows_per_chunk);
+    Values<DT, V> v[kKvRows];
+    auto load_rows = [&](int r, int cv) __attribute__((always_inline)) {   // (a row past the end: the last one again)
+#pragma unroll
+        for (int j = 0; j < kKvRows; ++j) v[j].load(x, ((int64_t)head * seq + min(r + j * groups, r1 - 1)) * dim + cv * V);
+    };
+    const bool any = group < groups && r0 + group < r1;
+    if (any) load_rows(r0 + group, cv0);                       // on their way while the ranges are joined
     float widest = 0.f;
     for (int c = threadIdx.x; c < dim; c += kKvThreads) {
         float lo, span;
@@ -149,8 +183,17 @@ __global__ void __launch_bounds__(kKvThreads) kv_check_kernel(const void* x, int
             const float* p = shown.partial + (int64_t)head * shown.partials * 2 * dim + c;
             float hi = -__builtin_inff();
             lo = __builtin_inff();
-#pragma unroll 8
-            for (int k = 0; k < shown.partials; ++k) { lo = fminf(lo, p[(int64_t)k * 2 * dim]); hi = fmaxf(hi, p[(int64_t)k * 2 * dim + dim]); }
+            for (int k0 = 0; k0 < shown.partials; k0 += kJoinAtOnce) {
+                float l[kJoinAtOnce], h[kJoinAtOnce];
+#pragma unroll
+                for (int j = 0; j < kJoinAtOnce; ++j) {
+                    const float* at = p + (int64_t)min(k0 + j, shown.partials - 1) * 2 * dim;
+                    l[j] = at[0];
+                    h[j] = at[dim];
+                }
+#pragma unroll
+                for (int j = 0; j < kJoinAtOnce; ++j) { lo = fminf(lo, l[j]); hi = fmaxf(hi, h[j]); }
+            }
             span = hi - lo;
             if (chunk == 0) { lo_io[(int64_t)head * dim + c] = lo; span_io[(int64_t)head * dim + c] = span; }
         } else {
@@ -172,24 +215,25 @@ __global__ void __launch_bounds__(kKvThreads) kv_check_kernel(const void* x, int
     for (int c = threadIdx.x; c < dim; c += kKvThreads) s_step[c] = step_of(s_step[c], width);
     __syncthreads();
     const float top = (float)((1u << width) - 1u);
-    const int nv = dim / V, across = min(nv, kKvThreads), groups = kKvThreads / across;
-    const int cv0 = threadIdx.x % across, group = threadIdx.x / across;
-    const int r0 = chunk * rows_per_chunk, r1 = min(seq, r0 + rows_per_chunk);
     float worst = 0.f;
-    if (group < groups) {
+    if (any) {
         for (int cv = cv0; cv < nv; cv += across) {
             float lo[V], step[V];
 #pragma unroll
             for (int k = 0; k < V; ++k) { lo[k] = s_lo[cv * V + k]; step[k] = s_step[cv * V + k]; }
-            for (int r = r0 + group; r < r1; r += groups) {
-                float v[V];
-                load_values<DT, V>(x, ((int64_t)head * seq + r) * dim + cv * V, v);
+            for (int r = r0 + group; r < r1; r += groups * kKvRows) {
+                if (r != r0 + group || cv != cv0) load_rows(r, cv);
 #pragma unroll
-                for (int k = 0; k < V; ++k) {
-                    float shown = lo[k] + id_of(v[k], lo[k], step[k], top) * step[k];
-                    if (orig_dt == QVB8_F16) shown = f16_bits_to_f32(f32_to_f16_bits(shown));
-                    else if (orig_dt == QVB8_BF16) shown = bf16_bits_to_f32(f32_to_bf16_bits(shown));
-                    worst = fmaxf(worst, __builtin_fabsf(shown - v[k]));
+                for (int j = 0; j < kKvRows; ++j) {
+                    if (j > 0 && r + j * groups >= r1) break;
+#pragma unroll
+                    for (int k = 0; k < V; ++k) {
+                        const float given_value = v[j][k];
+                        float shown = lo[k] + id_of(given_value, lo[k], step[k], top) * step[k];
+                        if (orig_dt == QVB8_F16) shown = f16_bits_to_f32(f32_to_f16_bits(shown));
+                        else if (orig_dt == QVB8_BF16) shown = bf16_bits_to_f32(f32_to_bf16_bits(shown));
+                        worst = fmaxf(worst, __builtin_fabsf(shown - given_value));
+                    }
                 }
             }
         }
@@ -199,11 +243,11 @@ __global__ void __launch_bounds__(kKvThreads) kv_check_kernel(const void* x, int
         if (threadIdx.x == 0) {
             // The head's largest error and the number of its workgroups that have added theirs, both as atomics at the device's
             // point of coherence, the second issued when the first has returned: the last one finds every error in.
-            uint32_t* state = shown.state + 2 * head;
+            uint32_t *state = shown.state + 2 * head * kStateApart, *done = state + kStateApart;
             const uint32_t before = __hip_atomic_fetch_max(state, __builtin_bit_cast(uint32_t, worst), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             asm volatile("" :: "v"(before) : "memory");
             __builtin_amdgcn_s_waitcnt(0x0F70);                        // vmcnt(0)
-            if (__hip_atomic_fetch_add(state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)chunks - 1u) {
+            if (__hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)chunks - 1u) {
                 const uint32_t all = __hip_atomic_fetch_max(state, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 // three words a head across the bus (a word per workgroup, written by each: 6 of 15.8 us)
                 uint32_t* to = reinterpret_cast<uint32_t*>(shown.found) + 3 * head;
@@ -410,13 +454,13 @@ int kv_range(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim
     if (int rc = bad_shape("qvb8_kv_range", x, x_dtype, heads, seq, dim)) return rc;
     if (!partial || chunks < 1 || chunks > 65535) return host::fail(QVB8_ERR_ARG, "qvb8_kv_range: bad partial results");
     const bool vec = vectors_ok(x, dim);
-    const int nv = (int)(vec ? dim / 8 : dim), across = std::min(nv, kKvThreads), groups = kKvThreads / across;
+    const int nv = (int)(vec ? dim / 8 : dim), across = std::min(nv, kRangeThreads), groups = kRangeThreads / across;
     const size_t lds = (size_t)groups * dim * 8;
     const dim3 grid((unsigned)chunks, (unsigned)heads);
     by_dtype(x_dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        if (vec) hipLaunchKernelGGL((kv_range_kernel<DT, 8>), grid, dim3(kKvThreads), lds, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), partial, clear);
-        else hipLaunchKernelGGL((kv_range_kernel<DT, 1>), grid, dim3(kKvThreads), lds, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), partial, clear);
+        if (vec) hipLaunchKernelGGL((kv_range_kernel<DT, 8>), grid, dim3(kRangeThreads), lds, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), partial, clear);
+        else hipLaunchKernelGGL((kv_range_kernel<DT, 1>), grid, dim3(kRangeThreads), lds, (hipStream_t)stream, x, (int)seq, (int)dim, rows_per_chunk(seq, chunks), partial, clear);
     });
     return host::check_launch("qvb8_kv_range");
 }
@@ -475,7 +519,7 @@ int64_t measure_partials(int64_t seq) { return std::max<int64_t>(1, std::min<int
 constexpr uint32_t kUnwritten = 0xBF800000u;                   // -1: none of the figures is negative
 }
 extern "C" int64_t qvb8_kv_measure_floats(int64_t heads, int64_t seq, int64_t dim) {
-    return heads < 1 || seq < 1 || dim < 1 ? 0 : heads * (measure_partials(seq) * 2 * dim + 2);
+    return heads < 1 || seq < 1 || dim < 1 ? 0 : heads * (measure_partials(seq) * 2 * dim + 2 * kStateApart);
 }
 extern "C" int qvb8_kv_measure(const void* x, int x_dtype, int64_t heads, int64_t seq, int64_t dim, int orig_dtype, int bits, double tau,
                                float* scratch, float* lo, float* span, float* found, void* stream) {

@@ -43,6 +43,19 @@ def test_bands_are_those_of_the_cpu_codec(heads, seq, dim, dtype, bits, tau):
         assert torch.equal(getattr(got_lay, name).cpu(), getattr(want_lay, name)), name
 
 
+@pytest.mark.parametrize("heads,seq,dim,dtype", [(1, 4101, 8, torch.float32), (1, 201, 2048, torch.bfloat16), (2, 83, 2047, torch.float16), (2, 270, 1000, torch.float32),
+                                                 (32, 129, 16, torch.bfloat16), (4, 1500, 58, torch.float16), (3, 497, 72, torch.bfloat16)])
+def test_chunks_that_end_inside_a_batch_of_rows(heads, seq, dim, dtype):
+    """Several rows are loaded at once, the last one again where a chunk ends, and channels past the first pass follow behind."""
+    x = _values(heads, seq, dim, dtype, seed=seq).clamp(-12, 12)
+    want = C.band_kv_heads(x, dtype, 5, tau=0.06)
+    got = C.band_kv_heads(x.to(DEV), dtype, 5, tau=0.06)
+    for w, g in zip(want, got):
+        assert g.bits == w.bits
+        for name in ("min_s", "tau_s", "packed"):
+            assert torch.equal(getattr(g, name).cpu(), getattr(w, name)), name
+
+
 def test_a_bound_that_sixteen_bits_miss_is_refused():
     x = torch.tensor([[[0.0], [1.1], [3e4]]])
     for dev in ("cpu", DEV):
