@@ -58,7 +58,7 @@ struct AttnArgs {
 
 // Four neighbouring channels of one query, at element offset `at`.  What is not ready is multiplied by the softmax scale, then
 // clamped to fp16's finite range and rounded -- in this order, so that an outlier channel does not become an infinity.  Done by
-// the row-block kernel where it reads its queries, 16 or 32 rows a workgroup; the kernel of 128 rows takes them ready (every one of its
+// the row-block kernel where it reads its queries, 16 or 32 rows a workgroup; the kernel of many rows takes them ready (every one of its
 // splits would prepare them again: 120 tokens over 16001 keys 118.3 us that way, 112.1 with a launch that does it once).
 constexpr int kQReady = -1;
 __device__ __forceinline__ h4_t load_query(const AttnArgs& a, int64_t at) {
@@ -388,8 +388,8 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
     }
 }
 
-// ---- many query rows (a prompt chunk, a wide draft): 128 rows per workgroup -----------------------------------------------
-// With hundreds of rows the products bound the work, and what has to be shared is the restored tile: 4 waves x 32 query
+// ---- many query rows (a prompt chunk, a wide draft): 128 or 256 rows per workgroup -----------------------------------------
+// With hundreds of rows the products bound the work, and what has to be shared is the restored tile: 4 or 8 waves x 32 query
 // rows share one, in two LDS buffers (tile t is multiplied while tile t + 1 is restored; one barrier per tile).  The
 // products run transposed, S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_f16: a lane then holds the scores of ONE
 // query (column lane % 32), so
@@ -403,13 +403,15 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
 // 1, and the keys that matter most lie just below it, where fp16 is finest for their size.  (A reference that lags behind
 // the maximum by up to 2^8 saves the multiplications but puts them anywhere in their binade: 1 .. 2.5 % more error against
 // 64 bits over 33 .. 1024 rows.)
-// Two workgroups per CU (78 KB of LDS, at most 256 registers): one restores while the other one's products run.
+// Two workgroups of four waves per CU (78 KB of LDS, at most 256 registers): one restores while the other one's products run.  One of
+// eight waves restores half as much per wave; its waves run apart by what the barrier allows.
 // Bound by what a CU issues beside its products (restoring, exp2, conversions): 720 rows x 4 kv heads over 16001 keys of 256
-// channels 251.6 us in the row-block kernel (32 rows share a tile), 108.7 us here = 0.43 PFLOP/s, of which rescaling O takes 4.7.  Two
-// workgroups per CU against one, and the ids of tile t + 2 asked for between the two products against before the first one (the
-// sixteen registers they come back to are then spilled away from Q): 100.7 against 133 and 118 against 133 for the whole
-// call, measured with the lagging reference.
-constexpr int kWideRows = 128, kWaveRows = 32;
+// channels, whole calls: 107.2 us with four waves and the scale multiplied before the maximum is taken, 100.0 with eight, 98.5 with
+// the scale in the exponent's subtraction and the products first.  (Half of the eight waves at their products while the others restore,
+// by program order: 103.)  The ids of tile t + 2 are asked for between the two products where both sets of registers would not fit
+// (before the first one they are spilled away from Q); with 128 channels and eight waves before them: 960 rows 76.6 against
+// 78.5.
+constexpr int kWaveRows = 32;
 constexpr int kWideFrom = 33;                                 // fewest rows that take it: fused_attn.py has the measurements
 constexpr int kVRow = kKeys + 8;                              // halfs per row of V in LDS
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -427,10 +429,12 @@ __device__ __forceinline__ int lane_now() {
     return l;
 }
 
-template <int D, typename T>
-__global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2) void attn_wide_kernel(const AttnArgs a) {
+template <int D, typename T, int NW>
+__global__ __launch_bounds__(64 * NW, (D == 256 && sizeof(T) == 2) ? 1 : 2) void attn_wide_kernel(const AttnArgs a) {
     constexpr int CG = D / 4;                  // channel groups (four channels each) of a key
-    constexpr int KPT = kKeys * CG / kAttnThreads;            // consecutive keys a thread restores: 8 (D = 256) or 4
+    constexpr int kWideRows = NW * kWaveRows;
+    constexpr bool kAskEarly = D == 128 && NW == 8;           // the ids of tile t + 2 before the products of tile t, where registers allow it
+    constexpr int KPT = kKeys * CG / (64 * NW);               // consecutive keys a thread restores: 32 (D = 256) or 16 over the waves
     constexpr int KROW = krow_wide(D), NKS = D / 16, NF = D / 32, NFC = NF / 4;
     using QD = Quad<T>;
     using U = typename QD::type;
@@ -537,9 +541,11 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
             }
             _Float16* dst = Vt + ((buf * 4 + c) * CG + cg) * kVRow + key0;
             if constexpr (KPT == 8) *reinterpret_cast<uint4*>(dst) = uint4{w[0], w[1], w[2], w[3]};
-            else *reinterpret_cast<uint2*>(dst) = uint2{w[0], w[1]};
+            else if constexpr (KPT == 4) *reinterpret_cast<uint2*>(dst) = uint2{w[0], w[1]};
+            else *reinterpret_cast<uint32_t*>(dst) = w[0];
         }
     };
+    static_assert(KPT == 8 || KPT == 4 || KPT == 2);
 
     float m_run = -INFINITY, l_run = 0.f;                    // m: in powers of two; l: this half's keys
     f16_t acc[NF];
@@ -560,8 +566,12 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
             s = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t*>(ka + 16 * ks), qb[ks], s, 0, 0, 0);
+        float times = to_log2;                                // > 0: multiplied in the exponent's subtraction, below
+        if (!(times > 0.f)) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] *= to_log2;
+            for (int i = 0; i < 16; ++i) s[i] *= times;
+            times = 1.f;
+        }
         if (!(ref.nlen == kKeys && ref.start + kKeys - 1 <= wqmin)) {
             const int seen = row_ok ? min(ref.nlen, qpos - ref.start + 1) - half8 : 0;      // keys of the tile this row sees
 #pragma unroll
@@ -570,7 +580,7 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
         float mx = s[0];
 #pragma unroll
         for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = fmaxf(mx, __shfl_xor(mx, 32)) * times;
         const bool rises = mx > m_run;                        // also the first visible key: m_run is -inf
         if (__builtin_amdgcn_ballot_w64(rises)) {
             const float alpha = rises ? (m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - mx)) : 1.f;
@@ -584,7 +594,7 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
         const float m_safe = m_run == -INFINITY ? 0.f : m_run;
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
-            const h2_t pp = {(_Float16)__builtin_amdgcn_exp2f(s[i] - m_safe), (_Float16)__builtin_amdgcn_exp2f(s[i + 1] - m_safe)};
+            const h2_t pp = {(_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(s[i], times, -m_safe)), (_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], times, -m_safe))};
             l_run = __builtin_amdgcn_fdot2(pp, h2_t{(_Float16)1.f, (_Float16)1.f}, l_run, false);    // the rounded p, as the product sees it
             p[i >> 3][i & 7] = pp[0];
             p[i >> 3][(i & 7) + 1] = pp[1];
@@ -611,12 +621,15 @@ __global__ __launch_bounds__(kAttnThreads, (D == 256 && sizeof(T) == 2) ? 1 : 2)
             const TileRef now = cur;
             cur = next;
             if (cur.ok) restore(buf ^ 1, cur);
+            if (kAskEarly) { fetch(t + 2, next); __builtin_amdgcn_sched_barrier(0); }
             const bool mine = wave_ok && now.start <= wqmax;
             h8_t p[2] = {};
+            __builtin_amdgcn_s_setprio(1);                    // the wave at its products goes first, the one that restores fills in
             if (mine) scores(buf, now, p);
-            fetch(t + 2, next);
+            if (!kAskEarly) fetch(t + 2, next);
             __builtin_amdgcn_sched_barrier(0);
             if (mine) values(buf, p);
+            __builtin_amdgcn_s_setprio(0);
             __syncthreads();                                  // buffer buf ^ 1 is filled, buffer buf is free
             buf ^= 1;
         }
@@ -729,21 +742,33 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(const float* __r
     store_joined(j, hr, n_rows, nhkv, G, D, ch, out, lse);
 }
 
-template <int D, typename T>
+// Eight waves where at least 13/16 of their rows are used, and where workgroups of four waves would have to share CUs.  Whole calls in us,
+// four waves / eight, 4 kv heads: 256 channels, 720 rows (94 % used) over 16001 keys 107.2 / 98.5, 240 (94 %) over 65536 137.0 / 123.0, 1104
+// (86 %) 145.5 / 138.9; 600 (78 %) 98.0 / 95.8 but 808 (79 %) 119.5 / 122.4, 288 (56 %) 78.2 / 83.0; 128 channels, 960 rows (94 %) over
+// 16001 keys 86.9 / 76.6, 1024 (100 %) over 40000 171.4 / 149.7, 630 (82 %) over 30000 96.5 / 94.7.  Few workgroups: 2048 rows x 2
+// heads over 2048 keys (256 of four waves) 48.4 / 51.5, 256 rows over 5000 keys (184) 47.3 / 48.9.  16-bit ids stay with four waves.
+bool eight_waves(int64_t rows, int64_t heads_and_splits) {
+    return 16 * rows >= 13 * 256 * ((rows + 255) / 256) && heads_and_splits * ((rows + 127) / 128) > host::device_cus();
+}
+
+template <int D, typename T, int NW>
 int launch_attn_wide(const AttnArgs& a, int64_t n_splits, hipStream_t s) {
-    if (int rc = host::raise_lds_limit<attn_wide_kernel<D, T>>(wide_lds(D), "qvb8_attn_fwd")) return rc;
-    const dim3 grid((unsigned)a.nhkv, (unsigned)n_splits, (unsigned)((a.n_rows + kWideRows - 1) / kWideRows));
-    hipLaunchKernelGGL((attn_wide_kernel<D, T>), grid, dim3(kAttnThreads), wide_lds(D), s, a);
+    if (int rc = host::raise_lds_limit<attn_wide_kernel<D, T, NW>>(wide_lds(D), "qvb8_attn_fwd")) return rc;
+    const dim3 grid((unsigned)a.nhkv, (unsigned)n_splits, (unsigned)((a.n_rows + NW * kWaveRows - 1) / (NW * kWaveRows)));
+    hipLaunchKernelGGL((attn_wide_kernel<D, T, NW>), grid, dim3(64 * NW), wide_lds(D), s, a);
     return host::check_launch("qvb8_attn_fwd");
 }
 
 template <int D, typename T>
 int launch_attn(const AttnArgs& a, int64_t n_splits, hipStream_t s) {
-    // up to 16 rows: one block per workgroup; up to 32: two; beyond: the kernel of 128 rows.  QVB8_ATTN_ROW_BLOCKS forces this
+    // up to 16 rows: one block per workgroup; up to 32: two; beyond: the kernel of 128 or 256 rows.  QVB8_ATTN_ROW_BLOCKS forces this
     // kernel with 1, 2 or 4 blocks (256 channels: at most 2, four blocks' accumulators and Q do not fit the registers).
     int rb = a.n_rows <= kRows ? 1 : a.n_rows <= 2 * kRows ? 2 : 4;
     const int forced = host::env_int("QVB8_ATTN_ROW_BLOCKS", 0);
-    if (forced == 0 && a.n_rows >= kWideFrom) return launch_attn_wide<D, T>(a, n_splits, s);
+    if (forced == 0 && a.n_rows >= kWideFrom) {
+        if constexpr (sizeof(T) == 1) if (eight_waves(a.n_rows, n_splits * a.nhkv)) return launch_attn_wide<D, T, 8>(a, n_splits, s);
+        return launch_attn_wide<D, T, 4>(a, n_splits, s);
+    }
     if (forced == 1 || forced == 2 || forced == 4) rb = forced;
     if (D == 256 && rb > 2) rb = 2;
     const dim3 grid((unsigned)a.nhkv, (unsigned)n_splits, (unsigned)((a.n_rows + rb * kRows - 1) / (rb * kRows)));
@@ -835,7 +860,7 @@ extern "C" int qvb8_attend(const void* q, int q_dtype, double q_scale, int64_t s
     const int64_t rows = n_splits * n_kv_heads * n_rows;
     float* const m = o + rows * head_dim;
     if (n_rows >= kWideFrom && q) {
-        // prepared once for all splits of the kernel of 128 rows
+        // prepared once for all splits of the kernel of 128 or 256 rows
         if (sq_h != head_dim || sq_r != n_kv_heads * G * head_dim) return host::fail(QVB8_ERR_UNSUPPORTED, "%s: %d rows and more must be contiguous", who, kWideFrom);
         void* const q16 = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(m + 2 * rows) + 15) & ~(uintptr_t)15);
         if (int rc = qvb8_scale_sat_half(q, q_dtype, n_kv_heads * n_rows * head_dim, (float)q_scale, q16, stream)) return rc;

@@ -34,6 +34,27 @@ def test_wide_rows_match_the_oracle(D, Hkv, G, MQ, seg_len, q_pos0, bits, tps, a
     assert np.all(np.abs(lse[seen] - ref_lse[seen]) <= 1e-3 * np.abs(ref_lse[seen]) + 1e-3)
 
 
+@pytest.mark.parametrize("D,Hkv,G,MQ,seg_len,q_pos0,bits,tps,scale", [
+    (256, 1, 8, 26, [33, 1, 70], 78, 6, 2, 1.0), (128, 2, 5, 51, [300], 249, 7, 4, 1.0), (256, 2, 8, 32, [40, 64], -3, 6, 1, 1.0), (128, 1, 1, 257, [90], 20, 8, 3, 1.0),
+    (256, 1, 6, 72, [130, 31], 89, 8, 100, 0.4), (128, 1, 8, 64, [64, 64, 3], 67, 6, 2, 1.0), (256, 1, 4, 64, [97], 33, 7, 2, -0.5), (256, 1, 8, 27, [45], 18, 6, 1, 0.0)])
+def test_workgroups_of_256_rows_match_the_oracle(D, Hkv, G, MQ, seg_len, q_pos0, bits, tps, scale):
+    """208 (the fewest of them), 216, 255, 256 and 257 (too few for two) rows, blocks with empty waves, rows that see no key, one split of
+    every tile; a scale that is not positive is multiplied before the maximum is taken.  Splits without a tile make up the number of
+    workgroups from which that kernel takes over; once without them, for the other kernel."""
+    lay = make_layout(D + MQ + G, seg_len, Hkv, D, bits=bits)
+    rng = np.random.default_rng(MQ)
+    q = (rng.normal(0, 1, (MQ, Hkv * G, D)) * D ** -0.5).astype(np.float16)
+    want = A.fwd_split(q, lay["ki"], lay["vi"], lay["kmid"], lay["kstep"], lay["vmid"], lay["vstep"], lay["kc"], lay["vc"],
+                       lay["ts"], lay["tl"], lay["tseg"], q_pos0, tps, scale, G)
+    dl, q16 = to_device(lay, slack=MQ % 3), torch.from_numpy(q).to(DEV)
+    for empty in (512 // Hkv, 0):
+        o, m, l = (torch.full((w.shape[0] + empty,) + w.shape[1:], float("nan"), device=DEV) for w in want)
+        FA.fwd(q16, dl["ki"], dl["vi"], dl["kmid"], dl["kstep"], dl["vmid"], dl["vstep"], dl["kc"], dl["vc"], dl["ts"], dl["tl"], dl["tseg"], o, m, l, q_pos0, tps, scale, G)
+        S = want[0].shape[0]
+        check_split_outputs((o[:S].cpu().numpy(), m[:S].cpu().numpy(), l[:S].cpu().numpy()), want, lay)
+        assert torch.isneginf(m[S:]).all() and (l[S:] == 0).all() and (o[S:] == 0).all()
+
+
 def test_combining_many_rows_is_combining_few():
     """3 splits of 300 rows x 4 heads (a thread per four channels) against the CPU's combination, rows without a key among them."""
     g = torch.Generator().manual_seed(2)
