@@ -4,7 +4,7 @@
 // state up in the class's 4096-entry slot table (LDS, one class per workgroup), gets the symbol of column
 // 32 * step + j and advances  x' = f * (x >> 12) + d.  Steps go in pairs: after two symbols the lanes whose state
 // fell below 2^32 take the next 32-bit word of the tile's stream in lane order (ballot of the half + popcount).  Words
-// come from a per-tile LDS ring that is refilled from registers loaded half a ring ahead.  A wave64 therefore walks
+// come from a per-tile window in LDS whose rest moves to its front as the words requested a window ahead arrive.  A wave64 walks
 // TWO tiles at once, a workgroup of 256 threads eight: the block schedule of the format (runs of <= 8 tiles of one
 // class) maps one block to one workgroup.  id = symbol + drow[row]; value = fmaf(id, tau_s[row], min_s[row]).
 //

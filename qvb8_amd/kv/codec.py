@@ -3,8 +3,8 @@ segment of one kv head, one (min_s, tau_s) per channel,
 
     id = round((x - min_c) / step_c),  step_c = (max_c - min_c) / (2^B - 1),  recon = min_c + id * step_c,
 
-no escapes (minimum and maximum cover every value).  On the GPU the encoder is three launches of the HIP library (four when
-a head's width has to rise), on the CPU torch ops; both give the same bits.  The ids are kept bit-packed, LSB first,
+no escapes (minimum and maximum cover every value).  On the GPU the encoder is three launches of the HIP library (one more for
+each time a head's width has to rise), on the CPU torch ops; both give the same bits.  The ids are kept bit-packed, LSB first,
 row-major (codec.py:53-82), as the cache stores them between attention calls.
 """
 from __future__ import annotations
