@@ -76,7 +76,7 @@ class QVBandMLPV8(nn.Module):
     # launch it saves costs (see the kernel's source) --, so the separate products, which every other row count uses anyway,
     # stay the default.  QVB8_MLP_FUSED=1 in the environment (or True here) switches it on.
     one_launch = False
-    _pairs_stored = False          # gate+up lies in tiles_of_pairs order
+    _pairs_order = None            # the order (tiles_of_pairs) this module stored gate+up in
 
     def __init__(self, gate: QVBandLinearV8, up: QVBandLinearV8, down: QVBandLinearV8):
         super().__init__()
@@ -101,7 +101,8 @@ class QVBandMLPV8(nn.Module):
         if ok:
             order = unit_order(gu.nbits, self.inter)
             ok = order is not None and gu.store_in_order(tiles_of_pairs(order[0]), order[1])
-            self._pairs_stored = self._pairs_stored or ok
+            if ok:
+                self._pairs_order = gu._stored_perm
         if ok:
             d = dn._mma_order()
             ok = d is not None and d[2] is not None and dn._planes and _whole_tiles(d[2], 16)
@@ -136,9 +137,13 @@ class QVBandMLPV8(nn.Module):
 
     def _activated(self, rows: torch.Tensor):
         """silu(gate(rows)) * up(rows) as one launch, or None where that launch does not do what the separate calls do: other
-        types and layouts, and hooks that expect to see the gate+up product."""
+        types and layouts, a gate_up that was replaced or whose rows were stored in another order since, and hooks (or a forward of
+        its own) that expect to see the gate+up product."""
         gu = self.gate_up
-        if not (self._pairs_stored and rows.dtype in (torch.float16, torch.bfloat16) and rows.dim() == 2 and 1 <= rows.shape[0] <= ext.MMA_SILU_MAX_M
+        if self._pairs_order is None or gu.__dict__.get("_stored_perm") is not self._pairs_order \
+                or type(gu).forward is not QVBandLinearV8.forward or "forward" in gu.__dict__:
+            return None
+        if not (rows.dtype in (torch.float16, torch.bfloat16) and rows.dim() == 2 and 1 <= rows.shape[0] <= ext.MMA_SILU_MAX_M
                 and rows.shape[1] == self.hidden and rows.is_contiguous() and rows.device == gu.min_s.device):
             return None
         if gu._forward_hooks or gu._forward_pre_hooks or _has_any_global_hook() or gu.bias is not None or gu.esc_idx.numel() or gu.esc_idx_bf16.numel():

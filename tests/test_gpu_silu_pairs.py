@@ -1,5 +1,7 @@
 """GPU tests of the gate+up launch that applies the activation itself (ext.MMA_SILU_PAIRS through QVBandMLPV8): against the float64
 chain and the separate calls, at row counts and shapes where tiles, waves and the two ways of joining partial sums change."""
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -71,13 +73,48 @@ def test_what_takes_the_separate_calls():
         ext.mma_tiles(x, *args, **kw, out_dtype=torch.bfloat16, layout=layout)
 
 
-def test_rows_that_are_no_pairs_give_nan():
+def _other_order(gu):
     """The rows in unit_order's own order (16 gate rows, then their 16 up rows): no tile holds both rows of an output."""
+    assert gu.store_in_order(*unit_order(gu.nbits, gu.out_features // 2))
+
+
+def test_rows_that_are_no_pairs_give_nan():
     mlp, _ = _build(512, 256, 512, seed=4)
     gu = mlp.gate_up
-    assert gu.store_in_order(*unit_order(gu.nbits, 256))
+    _other_order(gu)
+    perm, rowinfo, layout = gu._mma_order()
     x = torch.randn(2, 512, device=DEV).to(torch.bfloat16)
-    assert bool(torch.isnan(mlp._activated(x).float()).all())
+    h = ext.mma_tiles(x, gu.ids, gu.min_s, gu.nbits, gu.bit_off, 512, gu.tau_s, None, None, perm=perm, rowinfo=rowinfo, layout=layout,
+                      out_dtype=torch.bfloat16, planes=gu._planes, silu_pairs=True)
+    assert bool(torch.isnan(h.float()).all())
+
+
+def test_gate_up_in_another_order_or_replaced_takes_the_separate_calls():
+    """The order the launch needs is a fact of gate_up's rows, and gate_up may be stored again, replaced, wrapped, copied and moved."""
+    for M in (1, 7, 16):
+        mlp, _ = _build(512, 256, 512, seed=4)
+        x = torch.randn(M, 512, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
+        gu = mlp.gate_up
+
+        def chain():
+            y = mlp.gate_up(x)
+            return mlp.down(F.silu(y[:, :256]) * y[:, 256:])
+
+        moved = copy.deepcopy(mlp).cpu().to(DEV)                       # the same bytes in the same order
+        for m in (mlp, moved):
+            assert m._activated(x) is not None
+        assert torch.equal(moved(x), mlp(x))
+        gu.forward = lambda rows: torch.zeros(rows.shape[0], 512, dtype=rows.dtype, device=rows.device)
+        assert mlp._activated(x) is None and not mlp(x).any()
+        del gu.forward
+        other, _ = _build(512, 256, 512, seed=5)
+        _other_order(other.gate_up)
+        mlp.gate_up = other.gate_up
+        assert mlp._activated(x) is None and torch.equal(mlp(x), chain()) and torch.isfinite(mlp(x)).all()
+        mlp.gate_up = gu
+        assert mlp._activated(x) is not None
+        _other_order(gu)
+        assert mlp._activated(x) is None and torch.equal(mlp(x), chain()) and torch.isfinite(mlp(x)).all()
 
 
 def test_tiles_of_pairs():
