@@ -702,7 +702,7 @@ __global__ void __launch_bounds__(256) finish_escapes_kernel(const uint16_t* __r
     for (int64_t i0 = lo; i0 < n_esc; i0 += 256) {
         const int64_t i = i0 + tid, at = i < n_esc ? esc_idx[i] : to, before = i > 0 && i <= n_esc ? esc_idx[i - 1] : -1;
         if (at >= from && at < to) {
-            const int row = (int)((uint32_t)(at - from) / (uint32_t)P);
+            const int row = (int)((at - from) / P);
             if (before < from + (int64_t)row * P) s_first[row] = i;
         }
         if (__syncthreads_or(at >= to)) break;                 // ascending: nothing behind it is of these rows
@@ -714,7 +714,7 @@ __global__ void __launch_bounds__(256) finish_escapes_kernel(const uint16_t* __r
         float acc[kEach] = {};
         for (int64_t e = first; e < n_esc; ++e) {
             const int64_t c = esc_idx[e] - row0;
-            if (c >= P) break;
+            if ((uint64_t)c >= (uint64_t)P) break;             // another row's, also where a list does not ascend
             const float off = esc_vals[e] - __builtin_fmaf((float)row_field(ids, bit0, nb, (int)c, clamp_byte), ts, mn);
 #pragma unroll
             for (int k = 0; k < kEach; ++k)

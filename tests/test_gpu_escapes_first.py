@@ -57,3 +57,24 @@ def test_long_lists_through_the_module(n_esc):
     perm, rowinfo, layout = lin._mma_order()
     y32 = ext.mma_tiles(x, *H.pack_args(dict(enc, ids=lin.ids, nbits=lin.nbits, bit_off=lin.bit_off)), perm=perm, rowinfo=rowinfo, layout=layout, planes=lin._planes)
     assert y.dtype == torch.float16 and torch.equal(y, y32.to(torch.float16))
+
+
+@pytest.mark.parametrize("M", [1, 20])
+def test_a_list_that_does_not_ascend_stays_inside_its_rows(M):
+    """Against its documented order the correction may miss a row, and never reads a column of another one: rows 5 and 7 are followed by
+    rows before them, row 0 comes last."""
+    Q, P = 100, 768
+    pack, order = _sorted_pack(Q, P, seed=2)
+    x = torch.randn(M, P, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
+    positions = [5 * P + 3, 5 * P + 700, 2 * P + 1, 7 * P, 6 * P + 5, 9 * P + 767, 0]
+    vals = torch.randn(len(positions), generator=torch.Generator().manual_seed(3)).to(DEV)
+    at = torch.tensor(positions, dtype=torch.int64)
+    by_row = torch.argsort(at)
+    whole = ext.mma_tiles(x, *pack, at[by_row].to(DEV), vals[by_row.to(DEV)], **order).to(torch.bfloat16)
+    none = ext.mma_tiles(x, *pack, None, None, **order).to(torch.bfloat16)
+    y = ext.mma_tiles(x, *pack, at.to(DEV), vals, out_dtype=torch.bfloat16, escapes_first=True, **order)
+    assert torch.equal(y[:, 5], whole[:, 5]) and torch.equal(y[:, 7], whole[:, 7]) and torch.equal(y[:, 9], whole[:, 9])
+    rest = [q for q in range(Q) if q not in (0, 2, 5, 6, 7, 9)]
+    assert torch.equal(y[:, rest], none[:, rest])
+    for q in (0, 2, 6):
+        assert torch.equal(y[:, q], whole[:, q]) or torch.equal(y[:, q], none[:, q])
