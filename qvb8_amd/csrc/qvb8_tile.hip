@@ -674,7 +674,11 @@ __global__ void __launch_bounds__(256) tile_fix_escapes_kernel(const uint16_t* _
 // a thread keeps one row and four tokens, so an escape's band value is read once for the four and what needs no escape is loaded before
 // the search.  A row's escapes are added in ascending order, no atomics: the values of tile_fix_escapes_kernel and a cast, which as two launches
 // took 34816 x 5120, 16 rows, 3000 escapes 39.3 us a call, 38.7 this way; 2000 x 2048, 7 rows, 500 escapes 28.4, 22.6.
-constexpr int kFinishRows = 64, kFinishTokens = 16;
+// A row with many more escapes than its neighbours is bound by the instructions of its one lane, some 170 an escape.  Once few rows of a
+// wave go on, all its lanes prepare their band values and activations, an escape each, and only the multiply-adds stay in order:
+// 4096 x 4096 with 4000 escapes in one row, 16 tokens, 259 us a call, 2000 without this, 1760 as the two launches.  While many go on, each
+// lane keeps its own row: 64 escapes in every row 52 us (50 without the looks in between), 420 as the two launches.
+constexpr int kFinishRows = 64, kFinishTokens = 16, kFinishAlone = 16, kFinishFew = 6;
 template <bool BF, bool XC>
 __global__ void __launch_bounds__(256) finish_escapes_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict__ ids, int64_t ids_bytes,
         const float* __restrict__ min_s, const float* __restrict__ tau_s, const uint8_t* __restrict__ nbits, const int64_t* __restrict__ bit_off,
@@ -702,27 +706,67 @@ __global__ void __launch_bounds__(256) finish_escapes_kernel(const uint16_t* __r
     for (int64_t i0 = lo; i0 < n_esc; i0 += 256) {
         const int64_t i = i0 + tid, at = i < n_esc ? esc_idx[i] : to, before = i > 0 && i <= n_esc ? esc_idx[i - 1] : -1;
         if (at >= from && at < to) {
-            const int row = (int)((at - from) / P);
+            const uint64_t in = (uint64_t)(at - from);
+            const int row = (in >> 32) ? (int)(in / (uint64_t)P) : (int)((uint32_t)in / (uint32_t)P);
             if (before < from + (int64_t)row * P) s_first[row] = i;
         }
         if (__syncthreads_or(at >= to)) break;                 // ascending: nothing behind it is of these rows
     }
-    if (r >= rows) return;
-    const int64_t first = s_first[r], row0 = (int64_t)q * P;
-    if (first >= 0) {
-        const int64_t clamp_byte = (ids_bytes - 8) & ~(int64_t)3;
+    const int64_t row0 = (int64_t)q * P, clamp_byte = (ids_bytes - 8) & ~(int64_t)3;
+    int64_t e = r < rows ? s_first[r] : -1;                    // (every lane stays: all of them prepare what follows)
+    bool open = e >= 0;
+    if (__builtin_amdgcn_ballot_w64(open)) {
         float acc[kEach] = {};
-        for (int64_t e = first; e < n_esc; ++e) {
-            const int64_t c = esc_idx[e] - row0;
-            if ((uint64_t)c >= (uint64_t)P) break;             // another row's, also where a list does not ascend
-            const float off = esc_vals[e] - __builtin_fmaf((float)row_field(ids, bit0, nb, (int)c, clamp_byte), ts, mn);
+        do {
+            if (open) {
+                const int64_t stop = min(e + kFinishAlone, n_esc);
+                for (; e < stop; ++e) {
+                    const int64_t c = esc_idx[e] - row0;
+                    if ((uint64_t)c >= (uint64_t)P) break;     // another row's, also where a list does not ascend
+                    const float off = esc_vals[e] - __builtin_fmaf((float)row_field(ids, bit0, nb, (int)c, clamp_byte), ts, mn);
 #pragma unroll
-            for (int k = 0; k < kEach; ++k)
-                acc[k] = __builtin_fmaf(XIn<BF, XC>::scalar(X[(size_t)min(t0 + k, M - 1) * P + c]), off, acc[k]);
+                    for (int k = 0; k < kEach; ++k)
+                        acc[k] = __builtin_fmaf(XIn<BF, XC>::scalar(X[(size_t)min(t0 + k, M - 1) * P + c]), off, acc[k]);
+                }
+                open = e == stop && e < n_esc;
+            }
+        } while (__builtin_popcountll(__builtin_amdgcn_ballot_w64(open)) > kFinishFew);
+        for (uint64_t rows_open = __builtin_amdgcn_ballot_w64(open); __builtin_expect(rows_open != 0, 0); rows_open &= rows_open - 1) {
+            const int src = __builtin_ctzll(rows_open);
+            auto of_src = [&](int w) __attribute__((always_inline)) { return __builtin_amdgcn_readlane(w, src); };
+            auto of_src64 = [&](int64_t w) __attribute__((always_inline)) { return (int64_t)((uint64_t)(uint32_t)of_src((int)(w >> 32)) << 32 | (uint32_t)of_src((int)w)); };
+            const int64_t row = of_src64(row0), off0 = of_src64(bit0);
+            const int width = of_src(nb);
+            const float step_s = __int_as_float(of_src(__float_as_int(ts))), low = __int_as_float(of_src(__float_as_int(mn)));
+            float sum[kEach];
+#pragma unroll
+            for (int k = 0; k < kEach; ++k) sum[k] = __int_as_float(of_src(__float_as_int(acc[k])));
+            for (int64_t e0 = of_src64(e);; e0 += 64) {
+                const int64_t i = e0 + r, at = i < n_esc ? esc_idx[i] - row : (int64_t)P;
+                const uint64_t others = ~__builtin_amdgcn_ballot_w64((uint64_t)at < (uint64_t)P);
+                const int n = others ? __builtin_ctzll(others) : 64;
+                int off = 0, x[kEach] = {};
+                if (r < n) {
+                    off = __float_as_int(esc_vals[i] - __builtin_fmaf((float)row_field(ids, off0, width, (int)at, clamp_byte), step_s, low));
+#pragma unroll
+                    for (int k = 0; k < kEach; ++k) x[k] = __float_as_int(XIn<BF, XC>::scalar(X[(size_t)min(t0 + k, M - 1) * P + at]));
+                }
+                for (int j = 0; j < n; ++j) {
+                    const float o = __int_as_float(__builtin_amdgcn_readlane(off, j));
+#pragma unroll
+                    for (int k = 0; k < kEach; ++k) sum[k] = __builtin_fmaf(__int_as_float(__builtin_amdgcn_readlane(x[k], j)), o, sum[k]);
+                }
+                if (n < 64) break;
+            }
+#pragma unroll
+            for (int k = 0; k < kEach; ++k) acc[k] = r == src ? sum[k] : acc[k];
         }
+        if (r < rows && s_first[r] >= 0) {
 #pragma unroll
-        for (int k = 0; k < kEach; ++k) v[k] += acc[k];
+            for (int k = 0; k < kEach; ++k) v[k] += acc[k];
+        }
     }
+    if (r >= rows) return;
 #pragma unroll
     for (int k = 0; k < kEach; ++k)
         if (t0 + k < M) store_y(static_cast<float*>(Y), out_dt, (int64_t)(t0 + k) * Q + q, v[k]);
