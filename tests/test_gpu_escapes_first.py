@@ -48,13 +48,13 @@ def test_same_values_as_rounding_the_corrected_fp32_results(M, x_dtype, out_dtyp
 @pytest.mark.parametrize("M", [1, 4, 5, 63, 64, 65, 130])
 def test_rows_of_many_escapes(M):
     """Rows that go on when their neighbours have ended: the last few of a wave are prepared by all its lanes, 64 escapes at a time.
-    Runs of 4 (a lane does them alone), 5, 64 + 4, 64 + 5, 128 + 4 and whole rows; two, six, seven and all rows of a wave; the list's end."""
+    Runs of 16 (a lane does them alone), 17, 64 + 16, 64 + 17, 128 + 16 and whole rows; two, six, seven and all rows of a wave; the list's end."""
     Q, P = 200, 768
     pack, order = _sorted_pack(Q, P, seed=M)
     x = torch.randn(M, P, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
     run = lambda row, n, at=0: list(range(row * P + at, row * P + at + n))                           # noqa: E731
-    lists = [run(3, 4) + run(4, 5) + run(40, 68) + run(63, P), run(Q - 1, 132, P - 132), sum((run(r, 69, 7 * r % 600) for r in range(6)), []) + [70 * P],
-             sum((run(r, 70 + r, 3) for r in range(64, 71)), []), sum((run(r, 12 + r % 9, r) for r in range(Q)), [])]
+    lists = [run(3, 16) + run(4, 17) + run(40, 80) + run(63, P), run(Q - 1, 144, P - 144), sum((run(r, 81, 7 * r % 600) for r in range(6)), []) + [70 * P],
+             sum((run(r, 82 + r, 3) for r in range(64, 71)), []), sum((run(r, 12 + r % 9, r) for r in range(Q)), [])]
     for positions in lists:
         esc = _escapes(positions, seed=M)
         for x_in, out_dtype, saturate in ((x, torch.bfloat16, True), (x.half(), torch.float16, True), (x, torch.bfloat16, False)):
