@@ -3,8 +3,9 @@ segment of one kv head, one (min_s, tau_s) per channel,
 
     id = round((x - min_c) / step_c),  step_c = (max_c - min_c) / (2^B - 1),  recon = min_c + id * step_c,
 
-no escapes (minimum and maximum cover every value).  On the GPU the encoder is three launches of the HIP library (one more for
-each time a head's width has to rise), on the CPU torch ops; both give the same bits.  The ids are kept bit-packed, LSB first,
+no escapes (minimum and maximum cover every value).  On the GPU the encoder is three launches of the HIP library (a fourth
+packs the heads that need more than the width asked for, one more checks each time a head still misses its bound), on the CPU torch
+ops; both give the same bits.  The ids are kept bit-packed, LSB first,
 row-major (codec.py:53-82), as the cache stores them between attention calls.
 """
 from __future__ import annotations
@@ -142,8 +143,9 @@ _STORED_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 def _band_on_gpu(t, orig_dtype, bits: int, tau: float, certify: bool) -> list:
     """band_kv_heads on the HIP library: ranges, and the least widths with the error they leave; while those figures are on their way to
-    the host, the ids are packed at the width asked for.  Heads that need more are packed again, checked again one bit wider while
-    they still miss tau."""
+    the host, the ids are packed at the width asked for.  Heads that need more are checked again, one bit wider while they still miss
+    tau, and packed again.  Keys of 4 heads x 4096 x 256: 38 us a call as asked, 44 when one head needs more, 48 when all do (65 in each
+    case with the widths awaited before the first id is packed); 32 heads x 4096 x 128: 113, 122, 166 (178)."""
     heads, seq, dim = t.shape
     x = t.detach()
     x = (x if x.dtype in _STORED_DTYPES else x.to(torch.float32)).contiguous()
@@ -154,26 +156,29 @@ def _band_on_gpu(t, orig_dtype, bits: int, tau: float, certify: bool) -> list:
         grid = torch.empty((3, heads, dim), dtype=torch.float32, device=dev)                          # minima, steps, spans
         lo_at, step_at, span_at = (grid.data_ptr() + 4 * heads * dim * i for i in range(3))
 
-        def pack(widths):
-            packed = [torch.empty((seq * dim * w + 7) // 8, dtype=torch.uint8, device=dev) for w in widths]
-            where = (ctypes.c_void_p * heads)(*[p.data_ptr() for p in packed])
-            _lib._check(lib.qvb8_kv_pack(x_at, dt, heads, seq, dim, lo_at, span_at, bytes(widths), step_at, where, stream), lib)
-            return packed
+        def pack(packed, widths, a=0):
+            """Heads a .. a + len(packed) - 1 into their streams."""
+            skip, n = 4 * dim * a, len(packed)
+            where = (ctypes.c_void_p * n)(*[p.data_ptr() for p in packed])
+            _lib._check(lib.qvb8_kv_pack(x_at + a * seq * dim * x.element_size() if a else x_at, dt, n, seq, dim, lo_at + skip, span_at + skip, bytes(widths),
+                                         step_at + skip, where, stream), lib)
 
-        widths = [bits] * heads
+        widths, stored = [bits] * heads, (seq * dim * bits + 7) // 8
         if not certifying:
             chunks = lib.qvb8_kv_chunks(heads, seq)
             partial = torch.empty(heads * chunks * 2 * dim, dtype=torch.float32, device=dev)
             _lib._check(lib.qvb8_kv_range(x_at, dt, heads, seq, dim, partial.data_ptr(), chunks, stream), lib)
             _lib._check(lib.qvb8_kv_check(x_at, dt, heads, seq, dim, partial.data_ptr(), chunks, odt, bits, float(tau), None, lo_at, span_at, None, stream), lib)
-            packed = pack(widths)
+            packed = [torch.empty(stored, dtype=torch.uint8, device=dev) for _ in widths]
+            pack(packed, widths)
             los, steps = (g.unbind(0) for g in grid[:2].unbind(0))
         else:
             scratch = torch.empty(lib.qvb8_kv_measure_floats(heads, seq, dim), dtype=torch.float32, device=dev)
             shown = torch.empty(3 * heads, dtype=torch.float32, pin_memory=True)
             _lib._check(lib.qvb8_kv_measure(x_at, dt, heads, seq, dim, odt, bits, float(tau), scratch.data_ptr(), lo_at, span_at, shown.data_ptr(), stream), lib)
             try:
-                packed = pack(widths)
+                packed = [torch.empty(stored, dtype=torch.uint8, device=dev) for _ in widths]
+                pack(packed, widths)
                 los, steps = (g.unbind(0) for g in grid[:2].unbind(0))
             finally:
                 _lib._check(lib.qvb8_kv_wait(shown.data_ptr(), heads, stream), lib)       # the figures are written whatever happened since
@@ -194,8 +199,12 @@ def _band_on_gpu(t, orig_dtype, bits: int, tau: float, certify: bool) -> list:
             while not all(e <= tau for e in errors):
                 widths = [w if e <= tau else _next_width(i, w, e, tau, orig_dtype) for i, (w, e) in enumerate(zip(widths, errors))]
                 errors = check()
-            if widths != [bits] * heads:
-                packed = pack(widths)
+            risen = [i for i, w in enumerate(widths) if w != bits]
+            if risen:                                            # one launch over them and what lies between (the same bytes again)
+                for i in risen:
+                    packed[i] = torch.empty((seq * dim * widths[i] + 7) // 8, dtype=torch.uint8, device=dev)
+                a, b = risen[0], risen[-1] + 1
+                pack(packed[a:b], widths[a:b], a)
     return [BandedKV(p, m, s, w, (seq, dim), orig_dtype, tau) for p, m, s, w in zip(packed, los, steps, widths)]
 
 

@@ -100,3 +100,30 @@ def test_figures_for_the_waiting_host_are_the_checks(heads, seq, dim, dtype, bit
         _lib._check(lib.qvb8_kv_wait(found.data_ptr(), heads, s), lib)
         assert torch.equal(both[0].view(torch.int32), both[1].view(torch.int32))
         assert torch.equal(found, torch.cat([report[:, :2], report[:, 2:].amax(1, keepdim=True)], 1))
+
+
+@pytest.mark.parametrize("risen", [[0], [2], [5], [1, 4], [0, 5], [0, 1, 2, 3, 4, 5]])
+@pytest.mark.parametrize("seq,dim", [(300, 64), (77, 30), (16, 7)])
+def test_heads_that_need_more_are_packed_again_and_no_others(risen, seq, dim, monkeypatch):
+    """Single heads, heads with others between them, all heads: the CPU codec's bits, and a second launch over those heads only."""
+    from qvb8_amd import _lib
+    x = _values(6, seq, dim, torch.bfloat16, seed=dim).clamp(-8, 8)
+    for n, i in enumerate(risen):
+        x[i, n, n] = 100.0 * (n + 1)
+    want = C.band_kv_heads(x, x.dtype, 7, tau=0.25)
+    assert [i for i, b in enumerate(want) if b.bits > 7] == risen
+    lib, packed = _lib.load(), []
+
+    class Watched:
+        def __getattr__(self, name):
+            if name == "qvb8_kv_pack":
+                return lambda *a: (packed.append((a[2], bytes(a[7]))), lib.qvb8_kv_pack(*a))[1]
+            return getattr(lib, name)
+
+    monkeypatch.setattr(_lib, "load", Watched)
+    got = C.band_kv_heads(x.to(DEV), x.dtype, 7, tau=0.25)
+    assert packed == [(6, bytes([7] * 6)), (risen[-1] + 1 - risen[0], bytes(b.bits for b in want[risen[0]:risen[-1] + 1]))]
+    for w, g in zip(want, got):
+        assert g.bits == w.bits
+        for name in ("min_s", "tau_s", "packed"):
+            assert torch.equal(getattr(g, name).cpu(), getattr(w, name)), name
