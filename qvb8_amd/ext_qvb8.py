@@ -13,6 +13,7 @@ saturating_half, lookup_rows (the embedding read, which the reference does in to
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -178,10 +179,16 @@ def gemv(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals):
 
 MMA_MAX_M = 48
 MMA_GEMM_MAX_M = 256          # with a row layout (rows stored in width order, widths 4..8): the workgroup-tiled kernel
+MMA_TILED_FROM = 17           # fewest rows of X whose kernels may want workspace beyond the row records
 MMA_SATURATE_X = 1
 MMA_Y_F16, MMA_Y_BF16 = 2, 4                      # qvb8_mma_flags: results stored as fp16 / bf16
 MMA_PLANES = 8                                    # qvb8_mma_flags: the pack has rows stored in planes
 MMA_SILU_PAIRS, MMA_SILU_MAX_M = 16, 16           # qvb8_mma_flags: tiles of 8 gate and 8 up rows, the activation applied; its most rows of X
+
+
+@functools.lru_cache(maxsize=1024)
+def _rowinfo_bytes(Q: int) -> int:
+    return _lib.load().qvb8_mma_rowinfo_bytes(Q)
 
 
 def mma_prepare(row_nbits, row_bit_off, tau_s, min_s, P, ids_bytes, perm=None):
@@ -455,7 +462,7 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
         perm = perm.contiguous()
     else:
         perm = None
-    records = ((Q + 1) // 2 * 16 + Q * 16) if Q > 0 else 0             # qvb8_mma_rowinfo_bytes
+    records = _rowinfo_bytes(Q)
     if rowinfo is not None and (rowinfo.dtype != torch.int64 or rowinfo.numel() * 8 != records or not rowinfo.is_cuda):
         raise RuntimeError("qvb8 mma-multi: rowinfo must be the int64 GPU tensor mma_prepare returned")
     if out_dtype is torch.float16 or out_dtype is torch.bfloat16:
@@ -478,7 +485,7 @@ def mma_tiles(X, ids, min_s, row_nbits, row_bit_off, P, tau_s, esc_idx, esc_vals
         if n_esc and out_dtype is not torch.float32:
             ws_bytes = lib.qvb8_mma_escapes_workspace_bytes(M, Q, P)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=Xc.device)
-        elif rowinfo is None or M > MMA_SILU_MAX_M:                    # up to 16 rows the records are all a call needs
+        elif rowinfo is None or M >= MMA_TILED_FROM:                   # below, the records are all a call needs
             need = lib.qvb8_mma_workspace_bytes(M, Q, P)
             if rowinfo is None or need > records:
                 ws = torch.empty((need + 7) // 8, dtype=torch.int64, device=Xc.device)

@@ -292,3 +292,21 @@ def test_unit_order_of_a_gate_up_pack():
     assert unit_order(nbits, inter - 1) is None and unit_order(nbits[:-1], inter) is None
     wide = nbits.clone(); wide[3] = 9
     assert unit_order(wide, inter) is None                                       # a row wider than 8 bits
+
+
+def test_workspace_of_few_rows_is_the_row_records(monkeypatch):
+    """What ext.mma_tiles relies on where it asks for no workspace: below MMA_TILED_FROM rows a call needs the row records only, whatever the
+    shape and the knob, and from there on kernels may want more."""
+    from qvb8_amd import _lib, ext_qvb8 as ext
+    lib = _lib.load()
+    for knob in (None, "1", "17", "30", "99"):
+        monkeypatch.delenv("QVB8_MMA_GEMM_FROM", raising=False)
+        if knob:
+            monkeypatch.setenv("QVB8_MMA_GEMM_FROM", knob)
+        for Q in (1, 2, 15, 16, 129, 4096, 34816):
+            for P in (128, 256, 640, 4096, 17408):
+                assert ext._rowinfo_bytes(Q) == lib.qvb8_mma_rowinfo_bytes(Q)
+                for M in range(1, ext.MMA_TILED_FROM):
+                    assert lib.qvb8_mma_workspace_bytes(M, Q, P) <= ext._rowinfo_bytes(Q), (M, Q, P)
+    monkeypatch.delenv("QVB8_MMA_GEMM_FROM", raising=False)
+    assert lib.qvb8_mma_workspace_bytes(ext.MMA_TILED_FROM, 4096, 4096) > ext._rowinfo_bytes(4096)
