@@ -310,3 +310,23 @@ def test_workspace_of_few_rows_is_the_row_records(monkeypatch):
                     assert lib.qvb8_mma_workspace_bytes(M, Q, P) <= ext._rowinfo_bytes(Q), (M, Q, P)
     monkeypatch.delenv("QVB8_MMA_GEMM_FROM", raising=False)
     assert lib.qvb8_mma_workspace_bytes(ext.MMA_TILED_FROM, 4096, 4096) > ext._rowinfo_bytes(4096)
+
+
+def test_longest_rows_of_the_tile_kernel():
+    """65535 panels of columns, whatever flags ride in the words beside their number: the host refuses more, and nothing less.  (Without a GPU:
+    an accepted call ends at the missing device, no address is followed.)"""
+    from qvb8_amd import _lib
+    if torch.cuda.is_available():
+        pytest.skip("the accepted calls would be launched")
+    lib = _lib.load()
+    here = ctypes.create_string_buffer(64)
+    at = (ctypes.addressof(here) + 15) & ~15
+
+    def message(P):
+        rc = lib.qvb8_mma(at, _lib.F16, 1, at, 1 << 40, at, at, at, at, 16, P, None, None, 0, None, at, None, 0, at, None, 0, None)
+        assert rc != 0
+        return lib.qvb8_last_error().decode()
+
+    panel = next(w * 4 * 128 for w in (8, 12) if "too long" in message(w * 4 * 128 * 65536))      # columns of a panel: 8 or 12 waves of four steps
+    assert "too long" not in message(panel * 65535) and "too long" not in message(panel * 32768) and "too long" not in message(4096)
+    assert "too long" in message(panel * 65535 + 128)
