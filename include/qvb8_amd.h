@@ -54,9 +54,9 @@ enum qvb8_status {
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
  * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*;
  * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS; 12: qvb8r_gemv_as; 13: qvb8_attend; 14: qvb8_kv_measure, qvb8_kv_wait;
- * 15: qvb8_mma_escapes_workspace_bytes).  A binding compares the loaded library's answer
+ * 15: qvb8_mma_escapes_workspace_bytes; 16: qvb8_attn_rows_per_workgroup).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
-#define QVB8_ABI_VERSION 15
+#define QVB8_ABI_VERSION 16
 int qvb8_abi_version(void);
 /* Message of the calling thread's most recent failure ("" if none). Valid until that thread's next call. */
 const char* qvb8_last_error(void);
@@ -442,6 +442,9 @@ int qvb8_attn_combine(const float* o, const float* m, const float* l, int64_t n_
  * strides in elements, multiples of 4, aligned to four elements, contiguous from 33 rows (tokens x G) on -- are multiplied by q_scale and
  * saturated to fp16, up to 32 rows by the kernel that reads them, beyond by a launch of its own.  `workspace`: qvb8_attn_workspace_bytes of device memory for the splits' partial results, 16-byte aligned.
  * Replaces: attend  kv/fused_attn.py:246-316. */
+/* Query rows a workgroup of the kernel of many rows (33 rows and more) will serve on a device of `cus` compute units: 128 or 256; 0 below 33
+ * rows.  For a caller that plans its splits. */
+int64_t qvb8_attn_rows_per_workgroup(int64_t n_rows, int64_t n_splits, int64_t n_kv_heads, int id_bytes, int64_t cus);
 int64_t qvb8_attn_workspace_bytes(int64_t n_splits, int64_t n_kv_heads, int64_t n_rows, int64_t head_dim);
 int qvb8_attend(const void* q, int q_dtype, double q_scale, int64_t sq_r, int64_t sq_h, const void* ki, const void* vi, int id_bytes,
                 int64_t s_n, int64_t s_h, const float* kmid, const float* kstep, const float* vmid, const float* vstep,

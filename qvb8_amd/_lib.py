@@ -14,7 +14,7 @@ import torch
 from .common.errors import NativeLibraryError
 
 _LIB = None
-EXPECTED_ABI = 15           # QVB8_ABI_VERSION of include/qvb8_amd.h that the argument lists below were written for
+EXPECTED_ABI = 16           # QVB8_ABI_VERSION of include/qvb8_amd.h that the argument lists below were written for
 F32, F16, BF16 = 0, 1, 2
 _DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
@@ -22,7 +22,7 @@ _DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 SYMBOLS = ("qvb8_abi_version", "qvb8_last_error", "qvb8_decode", "qvb8_lookup_rows", "qvb8_scatter_escapes", "qvb8_certify",
            "qvb8_sat_half", "qvb8_scale_sat_half", "qvb8_gemv_workspace_bytes", "qvb8_gemv", "qvb8_mma_rowinfo_bytes", "qvb8_mma_prepare", "qvb8_decode_tiles", "qvb8_mma_workspace_bytes", "qvb8_mma_escapes_workspace_bytes", "qvb8_mma", "qvb8_launch_probe", "qvb8_mlp_workspace_bytes", "qvb8_mlp_init", "qvb8_mlp",
            "qvb8_moe_workspace_bytes", "qvb8_moe_experts", "qvb8_moe_experts_checked", "qvb8_moe_experts_static",
-           "qvb8r_decode", "qvb8r_decode_blocks", "qvb8r_gemv_workspace_bytes", "qvb8r_gemv", "qvb8r_gemv_as", "qvb8r_walk_probe", "qvb8r_fix_escapes", "qvb8_attn_fwd", "qvb8_attn_combine", "qvb8_attn_workspace_bytes", "qvb8_attend",
+           "qvb8r_decode", "qvb8r_decode_blocks", "qvb8r_gemv_workspace_bytes", "qvb8r_gemv", "qvb8r_gemv_as", "qvb8r_walk_probe", "qvb8r_fix_escapes", "qvb8_attn_fwd", "qvb8_attn_combine", "qvb8_attn_rows_per_workgroup", "qvb8_attn_workspace_bytes", "qvb8_attend",
            "qvb8_kv_chunks", "qvb8_kv_range", "qvb8_kv_check", "qvb8_kv_pack", "qvb8_kv_measure_floats", "qvb8_kv_measure", "qvb8_kv_wait", "qvb8_kv_unpack", "qvb8_kv_tiles")
 
 
@@ -111,6 +111,8 @@ def load(build_if_missing: bool = True):
     lib.qvb8_attn_fwd.argtypes = ([vp, i64, i64, vp, vp, i32, i64, i64] + [vp] * 9 + [i64, vp, vp, vp] + [i64] * 6
                                   + [ctypes.c_double, i64, vp])
     lib.qvb8_attn_combine.argtypes = [vp, vp, vp, i64, i64, i64, i64, i64, vp, vp, vp]
+    lib.qvb8_attn_rows_per_workgroup.argtypes = [i64, i64, i64, i32, i64]
+    lib.qvb8_attn_rows_per_workgroup.restype = i64
     lib.qvb8_attn_workspace_bytes.argtypes = [i64] * 4
     lib.qvb8_attn_workspace_bytes.restype = i64
     lib.qvb8_attend.argtypes = ([vp, i32, ctypes.c_double, i64, i64, vp, vp, i32, i64, i64] + [vp] * 9 + [i64] * 8 + [vp, vp, vp, i64, vp])

@@ -747,8 +747,9 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(const float* __r
 // (86 %) 145.5 / 138.9; 600 (78 %) 98.0 / 95.8 but 808 (79 %) 119.5 / 122.4, 288 (56 %) 78.2 / 83.0; 128 channels, 960 rows (94 %) over
 // 16001 keys 86.9 / 76.6, 1024 (100 %) over 40000 171.4 / 149.7, 630 (82 %) over 30000 96.5 / 94.7.  Few workgroups: 2048 rows x 2
 // heads over 2048 keys (256 of four waves) 48.4 / 51.5, 256 rows over 5000 keys (184) 47.3 / 48.9.  16-bit ids stay with four waves.
-bool eight_waves(int64_t rows, int64_t heads_and_splits) {
-    return 16 * rows >= 13 * 256 * ((rows + 255) / 256) && heads_and_splits * ((rows + 127) / 128) > host::device_cus();
+// The only place of this rule: kv/fused_attn.py asks it (qvb8_attn_rows_per_workgroup) for the splits it plans.
+bool eight_waves(int64_t rows, int64_t heads_and_splits, int id_bytes, int64_t cus) {
+    return id_bytes == 1 && 16 * rows >= 13 * 256 * ((rows + 255) / 256) && heads_and_splits * ((rows + 127) / 128) > cus;
 }
 
 template <int D, typename T, int NW>
@@ -766,7 +767,7 @@ int launch_attn(const AttnArgs& a, int64_t n_splits, hipStream_t s) {
     int rb = a.n_rows <= kRows ? 1 : a.n_rows <= 2 * kRows ? 2 : 4;
     const int forced = host::env_int("QVB8_ATTN_ROW_BLOCKS", 0);
     if (forced == 0 && a.n_rows >= kWideFrom) {
-        if constexpr (sizeof(T) == 1) if (eight_waves(a.n_rows, n_splits * a.nhkv)) return launch_attn_wide<D, T, 8>(a, n_splits, s);
+        if constexpr (sizeof(T) == 1) if (eight_waves(a.n_rows, n_splits * a.nhkv, 1, host::device_cus())) return launch_attn_wide<D, T, 8>(a, n_splits, s);
         return launch_attn_wide<D, T, 4>(a, n_splits, s);
     }
     if (forced == 1 || forced == 2 || forced == 4) rb = forced;
@@ -837,6 +838,11 @@ extern "C" int qvb8_attn_fwd(const void* q, int64_t sq_r, int64_t sq_h, const vo
                              double scale, int64_t G, void* stream) {
     return attn_forward(q, qvb8::kQReady, 1.f, sq_r, sq_h, ki, vi, id_bytes, s_n, s_h, kmid, kstep, vmid, vstep, kc, vc, ts, tl, tseg,
                         n_tiles, o, m, l, n_splits, n_rows, n_kv_heads, head_dim, q_pos0, tps, scale, G, "qvb8_attn_fwd", stream);
+}
+
+extern "C" int64_t qvb8_attn_rows_per_workgroup(int64_t n_rows, int64_t n_splits, int64_t n_kv_heads, int id_bytes, int64_t cus) {
+    if (n_rows < qvb8::kWideFrom || n_splits < 1 || n_kv_heads < 1) return 0;
+    return qvb8::eight_waves(n_rows, n_splits * n_kv_heads, id_bytes, cus) ? 256 : 128;
 }
 
 extern "C" int64_t qvb8_attn_workspace_bytes(int64_t n_splits, int64_t n_kv_heads, int64_t n_rows, int64_t head_dim) {

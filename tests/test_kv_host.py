@@ -155,3 +155,34 @@ def test_split_plans(monkeypatch):
     assert plan(33) == (64, 64) and plan(96) == (128, 32)                        # 16 rows: 3 and 6 row blocks
     monkeypatch.setenv("QVB8_ATTN_ROW_BLOCKS", "4")
     assert plan(33, d=128) == (32, 128) and plan(33) == (64, 64)                 # 64 rows; 256 channels: 32 at most
+
+
+@pytest.mark.parametrize("cus", [256, 64, 304])
+def test_plans_are_for_the_workgroups_the_library_will_launch(cus, monkeypatch):
+    """plan_splits asks the library how many rows a workgroup will serve, then changes the splits, on which that answer depends: the final
+    splits have to get the answer that they were planned for."""
+    from types import SimpleNamespace
+    from qvb8_amd import _lib
+    lib = _lib.load()
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda device: SimpleNamespace(multi_processor_count=cus))
+    for name in ("QVB8_ATTN_ROW_BLOCKS", "QVB8_ATTN_WG_PER_CU"):
+        monkeypatch.delenv(name, raising=False)
+
+    def planned_for(answer, *args, **kw):
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "load", lambda: SimpleNamespace(qvb8_attn_rows_per_workgroup=lambda *a: answer))
+            return FA.plan_splits(*args, **kw)
+
+    seen = set()
+    for rows in (33, 128, 129, 207, 208, 256, 257, 400, 415, 416, 512, 630, 720, 768, 1100, 2048):
+        for hkv in (1, 2, 3, 4, 8, 16, 96):
+            for d in (128, 256):
+                for n_tiles in (*range(1, 140), 500, 511, 513, 2048, 4096):
+                    for wide in (False, True):
+                        args, kw = (n_tiles, hkv, rows, "cuda"), dict(d=d, wide=wide)
+                        tps, splits = FA.plan_splits(*args, **kw)
+                        block = lib.qvb8_attn_rows_per_workgroup(rows, splits, hkv, 2 if wide else 1, cus)
+                        assert (tps, splits) == planned_for(block, *args, **kw), (rows, hkv, d, n_tiles, wide, block)
+                        seen.add((block, wide))
+    assert seen == {(128, False), (256, False), (128, True)}
+    assert lib.qvb8_attn_rows_per_workgroup(32, 4, 4, 1, cus) == 0
