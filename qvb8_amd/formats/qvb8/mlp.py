@@ -16,6 +16,7 @@ input narrowed like every fp16-path activation -- what the separate modules and 
 from __future__ import annotations
 
 import os
+import weakref
 
 import torch
 import torch.nn as nn
@@ -76,6 +77,7 @@ class QVBandMLPV8(nn.Module):
     # launch it saves costs (see the kernel's source) --, so the separate products, which every other row count uses anyway,
     # stay the default.  QVB8_MLP_FUSED=1 in the environment (or True here) switches it on.
     one_launch = False
+    _reads = None                  # what the plan holds addresses of: both weights' ids (weakly), their row records
     _pairs_order = None            # the order (tiles_of_pairs) this module stored gate+up in
 
     def __init__(self, gate: QVBandLinearV8, up: QVBandLinearV8, down: QVBandLinearV8):
@@ -109,10 +111,20 @@ class QVBandMLPV8(nn.Module):
         if ok:
             ok = _whole_tiles(gu._mma_cache[2], 32)
         self.fused_ready = bool(ok)
-        self._ws = self._plan = None
+        self._ws = self._plan = self._reads = None
         if ok:
             self._ws, self._plan = ext.mlp_init(gu.ids, gu._mma_cache[1], gu._mma_cache[2], dn.ids, d[1], d[2],
                                                 self.hidden, self.inter, self.out_features)
+            self._reads = weakref.ref(gu.ids), weakref.ref(dn.ids), gu._mma_cache[1], d[1]
+
+    def _plan_stands(self) -> bool:
+        """Whether the plan still describes the weights: gate_up and down are public, may be stored in another order or replaced."""
+        return self._reads is not None and self._reads[0]() is self.gate_up.ids and self._reads[1]() is self.down.ids
+
+    def __getstate__(self):
+        state = self.__dict__.copy()
+        state["_reads"] = None         # a copy has weights of its own, at other addresses
+        return state
 
     def _apply(self, fn, recurse=True):
         out = super()._apply(fn, recurse)
@@ -160,7 +172,7 @@ class QVBandMLPV8(nn.Module):
         rows, out_dtype = activation_rows(x, self.gate_up.min_s.device)
         M = rows.shape[0]
         if (self.fused_ready and 1 <= M <= self.max_rows and rows.dtype in (torch.float16, torch.bfloat16)
-                and os.environ.get("QVB8_MLP_FUSED", "1" if self.one_launch else "0") != "0"):
+                and os.environ.get("QVB8_MLP_FUSED", "1" if self.one_launch else "0") != "0" and self._plan_stands()):
             y = ext.mlp_fused(rows, self._ws, self._plan, mid_dtype=rows.dtype, out_dtype=rows.dtype)
             return y.reshape(*x.shape[:-1], self.out_features).to(out_dtype)
         return self.separate(rows).reshape(*x.shape[:-1], self.out_features).to(out_dtype)

@@ -1,5 +1,7 @@
 """GPU tests of the one-launch MLP (qvb8_mlp through QVBandMLPV8): against the CPU oracle's chain, against the separate
 products on the same bytes, the state it carries from call to call, graph replay, and the bounded wait giving up."""
+import copy
+import io
 import os
 
 import numpy as np
@@ -194,6 +196,34 @@ def test_what_the_kernel_does_not_cover_goes_the_separate_way():
         ext.mlp_fused(torch.zeros(5, 512, dtype=torch.bfloat16, device=DEV), mlp._ws, mlp._plan)
     with pytest.raises(RuntimeError):                                  # a plan goes with the workspace it was made for
         ext.mlp_fused(torch.zeros(1, 512, dtype=torch.bfloat16, device=DEV), mlp._ws.clone(), mlp._plan)
+
+
+def test_a_plan_ends_with_the_bytes_it_was_made_for():
+    """The plan holds addresses: gate_up stored in another order, another down, a copy of the module and a cast that drops the row records all
+    get the product of the weights that are there now."""
+    mlp, Ws = _build(512, 768, 512, seed=3)
+    x = torch.randn(2, 512, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(DEV)
+    y = mlp(x)
+    mlp.half()                                                         # the records are made anew when next asked for
+    junk = [torch.full((n,), 0x7F, dtype=torch.uint8, device=DEV) for n in (1 << 15, 1 << 17, 1 << 20) for _ in range(8)]
+    assert mlp._plan_stands() and torch.equal(mlp(x), y)
+    saved = io.BytesIO()
+    torch.save(mlp, saved)
+    saved.seek(0)
+    for twin in (copy.deepcopy(mlp), torch.load(saved, weights_only=False)):
+        assert not twin._plan_stands() and torch.equal(twin(x), mlp.separate(x))
+    gu, down = mlp.gate_up, mlp.down
+    other, Wo = _build(512, 768, 512, seed=9)
+    mlp.down = other.down
+    assert not mlp._plan_stands() and torch.equal(mlp(x), mlp.separate(x))
+    _check(mlp(x), x, [Ws[0], Ws[1], Wo[2]], torch.bfloat16, 2)
+    mlp.down = down
+    assert mlp._plan_stands()
+    assert gu.store_in_order(*unit_order(gu.nbits, 768))
+    assert not mlp._plan_stands()
+    _check(mlp(x), x, Ws, torch.bfloat16, 2)
+    assert torch.equal(mlp(x), mlp.separate(x)) and not mlp.error_raised()
+    del junk
 
 
 def test_install_replaces_a_models_mlps():
