@@ -132,9 +132,11 @@ enum qvb8_mma_flags {
                                  multiply.  Without it bf16 X is used as it is, on bf16 operands (the reference's bf16
                                  mode).  No effect on fp16 X. */
     QVB8_MMA_Y_F16 = 2,       /* Y is (M, Q) fp16: each result rounded to nearest even from the fp32 value the call would */
-    QVB8_MMA_Y_BF16 = 4,      /* otherwise store; likewise bf16.  Only for a weight without escapes (n_esc == 0): the escape
-                                 correction adds to fp32 results.  Saves the caller's cast pass over Y (the reference's
-                                 operator casts the extension's fp32 result, formats/qvb8/module.py:430-441). */
+    QVB8_MMA_Y_BF16 = 4,      /* otherwise store; likewise bf16.  With escapes (n_esc > 0) the kernels leave fp32 results in the
+                                 workspace, which one launch corrects and rounds into Y: the call then needs
+                                 qvb8_mma_escapes_workspace_bytes, 16-byte aligned, esc_idx ascending, and no
+                                 QVB8_MMA_SILU_PAIRS; without that workspace it is refused.  Saves the caller's cast pass over
+                                 Y (the reference's operator casts the extension's fp32 result, formats/qvb8/module.py:430-441). */
     QVB8_MMA_PLANES = 8,      /* the pack has rows stored in planes (bit 62 of their bit_off, see "rows stored in planes"
                                  above): with a row layout these are the rows of every whole 16-row tile that lies inside
                                  one run of a width 4..8; without one, whatever rows the records mark.  The call then asks
@@ -177,10 +179,11 @@ typedef struct qvb8_mma_layout {
  * first); from 17 rows on, when P % 256 == 0, what the workgroup-tiled kernels need (narrowed activations, their sums per
  * column range, partial results of the column ranges). */
 int64_t qvb8_mma_workspace_bytes(int64_t M, int64_t Q, int64_t P);
-/* ... for fp16 / bf16 results of a weight with escapes. */
+/* ... for fp16 / bf16 results of a weight with escapes: the above and M x Q fp32 results behind it.  16-byte aligned. */
 int64_t qvb8_mma_escapes_workspace_bytes(int64_t M, int64_t Q, int64_t P);
 
-/* Y[m, q] = sum_c X[m, c] * value(q, c), fp32 accumulate on v_mfma 16x16x32, Y f32 (M, Q) row-major.
+/* Y[m, q] = sum_c X[m, c] * value(q, c), fp32 accumulate on v_mfma 16x16x32, Y f32 (M, Q) row-major -- or what the flags say it
+ * is: fp16 / bf16 (M, Q), or with QVB8_MMA_SILU_PAIRS (M, Q / 2); `Y` is then a pointer to that type.
  * X is (M, P) fp16 or bf16 (x_dtype QVB8_F16 / QVB8_BF16), 16-byte aligned, P % 128 == 0, 1 <= M <= 48 (up to 256 under the
  * conditions below).
  * The ids enter the matrix product exactly (as bias + id in X's own 16-bit format) and tau_s / min_s are applied

@@ -11,8 +11,8 @@
 // caches after the first), everything else is smaller.  Measured on such a segment, keys and values and their layout:
 // 2868 us as ~100 torch launches with 64-bit temporaries per bit; 193 us with a launch for each of range, join, check and pack and the
 // check's thousand figures written to the host; 146 us with the join in the check, three figures a head, and the ids packed at the
-// width asked for while those are on their way; 119 us with several rows' loads on their way at once and the heads' counters apart.
-// What is left is launches: the kernels take 57 of them, 250 keys of 2 x 64 channels take 95 (153 before).
+// width asked for while those are on their way; 126 us with several rows' loads on their way at once and the heads' counters apart.
+// What is left is launches: the kernels take 58 of them, 250 keys of 2 x 64 channels take 95 (153 before).
 //
 // Arithmetic is the codec's own expression by expression: fp32 differences, one IEEE division, rounding to nearest even,
 // products and sums rounded separately (contraction is off in this file).
@@ -514,7 +514,10 @@ extern "C" int qvb8_kv_pack(const void* x, int x_dtype, int64_t heads, int64_t s
 // Ranges, least widths and their errors as two launches, the figures on their way to the host when it has packed at the widths it
 // expects (qvb8_kv_pack) and comes to wait for them (qvb8_kv_wait).
 namespace {
-constexpr int64_t kMeasurePartials = 32;                       // per head: every workgroup of the check joins them
+// Partial ranges per head: every workgroup of the check joins them all.  Few heads and long segments leave CUs idle in the range pass (32
+// workgroups a head), and still gain by the launch saved; a tensor as asked, range + join + check with up to 256 partials a head / this,
+// us: 1 x 32768 x 128 55 / 42, 1 x 131072 x 256 166 / 152, 2 x 131072 x 128 127 / 107, 1 x 16384 x 2048 246 / 246, 4 x 4096 x 256 65 / 37.
+constexpr int64_t kMeasurePartials = 32;
 int64_t measure_partials(int64_t seq) { return std::max<int64_t>(1, std::min<int64_t>(kMeasurePartials, (seq + 15) / 16)); }
 constexpr uint32_t kUnwritten = 0xBF800000u;                   // -1: none of the figures is negative
 }

@@ -19,7 +19,7 @@
 // Error of a call's fp32 results against 64 bits (17 .. 64 tokens, activations that fp16 holds): 2.3e-7 .. 3.3e-7 of their norm; the
 // general path's fp32 products 5.4e-7 .. 6.9e-7; with c in the middle of the width instead, 1.0e-6 .. 1.4e-6.
 //
-// Measured (hidden 2048, 128 experts of 2 x 768 / 768 columns, top-8, bf16): a layer of 509 tokens 207 us, where one pass per
+// Measured (hidden 2048, 128 experts of 2 x 768 / 768 columns, top-8, bf16): a layer of 509 tokens 212 us, where one pass per
 // expert over its own modules took 12.2 ms, nearly all of it launches; kernels alone, under the profiler, up 109, down 89, plan 13,
 // combine 8.  40 tokens 132 us against 410 on the general path.  The up launch moves 300 MB at 2.7 TB/s: its vector units are 46 %
 // busy with the decode, its L1 59 % with requests that touch sixteen rows each, the matrix pipes 14 %.

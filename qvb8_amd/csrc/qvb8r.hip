@@ -128,8 +128,8 @@ __device__ __forceinline__ uint32_t walk_dec(Walker& z, const uint32_t* st) {
 
 // Four symbols, a renormalisation after every second one; `rg` is the wave's first window.  A pair takes at most 32 words of a
 // tile, so with the windows looked after every second pair at least 64 of their 256 words are always ahead.
-// Bound by vector instructions: 36 a pair and the multiply's extra slots, where a ring that wraps, looked after every pair, with a branch
-// around the words taken and the activations addressed per lane took 45.  17408 x 5120, one row: 66.2 -> 50.4 us a call with the
+// Bound by vector instructions: 42 a pair by the counters, besides 2.9 scalar and 3.6 of LDS, where a ring that wraps, looked after every
+// pair, with a branch around the words taken and the activations addressed per lane took 45, 12 and 3.5.  17408 x 5120, one row: 66.2 -> 50.4 us a call with the
 // shorter start above; 16 rows 88.1 -> 71.2; 5120 x 17408, one row 95.2 -> 70.0.  (The pointers as wave scalars, one bit count
 // over the whole wave: fewer vector instructions, a longer chain: the same.  Waves of different priority, fewer resident
 // workgroups: nothing and worse.)

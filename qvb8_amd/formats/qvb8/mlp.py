@@ -71,11 +71,10 @@ class QVBandMLPV8(nn.Module):
     """gate_proj / up_proj / down_proj (QVBandLinearV8, no bias, no escapes) with gated SiLU between them."""
 
     max_rows = ext.MLP_MAX_ROWS
-    # Whether 1..4 rows take the one-launch kernel.  Off by default: measured on the 9B shapes (hidden 4096, inter 12288) the
-    # one launch takes 29.6 us against 30.0 us for the two separate launches (the activation counted on neither side; since
-    # the gate+up launch applies it itself it costs the separate launches nothing) -- the hand-over inside the grid costs what the
-    # launch it saves costs (see the kernel's source) --, so the separate products, which every other row count uses anyway,
-    # stay the default.  QVB8_MLP_FUSED=1 in the environment (or True here) switches it on.
+    # Whether 1..4 rows take the one-launch kernel.  Off by default: measured on the 9B shapes (hidden 4096, inter 12288; 16 layers'
+    # MLPs in a graph, us a layer) one launch / gate+up with the activation and down as two: 1 row 28.9 / 30.4, 2 rows 32.2 / 30.6, 4
+    # rows 36.8 / 32.0 -- the hand-over inside the grid costs about what the launch it saves costs (see the kernel's source) --, so
+    # the separate launches, which every other row count uses anyway, stay the default.  QVB8_MLP_FUSED=1 in the environment (or True here) switches it on.
     one_launch = False
     _reads = None                  # what the plan holds addresses of: both weights' ids (weakly), their row records
     _pairs_order = None            # the order (tiles_of_pairs) this module stored gate+up in

@@ -115,6 +115,20 @@ def test_one_launch_against_the_oracle_and_the_separate_products(shape, dtype):
     assert not mlp.error_raised()
 
 
+def test_units_stored_as_a_gate_tile_and_an_up_tile():
+    """The other order the kernel reads (16 gate rows, then their 16 up rows), which the module itself does not store."""
+    for hidden, inter, out, spread in (SHAPES[0], SHAPES[1]):
+        mlp, Ws = _build(hidden, inter, out, seed=hidden, spread=spread)
+        gu, dn = mlp.gate_up, mlp.down
+        assert gu.store_in_order(*unit_order(gu.nbits, inter))
+        records, d = gu._mma_order(), dn._mma_order()
+        ws, plan = ext.mlp_init(gu.ids, records[1], records[2], dn.ids, d[1], d[2], hidden, inter, out)
+        for M in (1, 3, 4):
+            x = torch.randn(M, hidden, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
+            _check(ext.mlp_fused(x, ws, plan), x, Ws, torch.bfloat16, M)
+        assert int(ws[4:8].view(torch.int32)[0]) == 0
+
+
 def test_fewer_workgroups_than_cus_and_step_variants(monkeypatch):
     """A grid of 24 workgroups walks several units and tiles each; three and four steps per wave in the down phase."""
     mlp, Ws = _build(1024, 2048, 1024, seed=5, spread=True)
