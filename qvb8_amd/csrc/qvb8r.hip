@@ -284,12 +284,14 @@ __global__ void __launch_bounds__(kRThreads) r_gemv_kernel(RCore c, const void* 
                 uint32_t e[4];
                 walk_pairs2(z, st, rg, e);
                 __builtin_amdgcn_sched_barrier(0);
+                float x[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    const float x = DT == QVB8_F32 ? __builtin_bit_cast(float, (uint32_t)raw[k]) : DT == QVB8_F16 ? f16_bits_to_f32(raw[k]) : bf16_bits_to_f32(raw[k]);
-                    acc = __builtin_fmaf(x, (float)(e[k] & kSymMask), acc);
-                    if constexpr (FIRST) sx += x;
+                    x[k] = DT == QVB8_F32 ? __builtin_bit_cast(float, (uint32_t)raw[k]) : DT == QVB8_F16 ? f16_bits_to_f32(raw[k]) : bf16_bits_to_f32(raw[k]);
+                    acc = __builtin_fmaf(x[k], (float)(e[k] & kSymMask), acc);
                 }
+                // (in pairs: added one by one, results of fp32 rows are 1 .. 11 % further from 64 bits)
+                if constexpr (FIRST) { sx += x[0] + x[1]; sx += x[2] + x[3]; }
                 asm volatile("" : "+v"(acc));                              // the activations are used up before words are asked for
                 walk_window(z, rg, l32, t.room);
             }

@@ -75,3 +75,36 @@ def test_whole_weight_in_one_chunk_and_in_several():
             diff = np.abs(m(x).float().cpu().numpy().astype(np.float64) - ref)
             finite = np.abs(ref) < (6.5e4 if dtype == torch.float16 else 1e30)
             assert np.all(diff[finite] <= tol[finite]), (dtype, float((diff / tol)[finite].max()))
+
+
+@pytest.mark.parametrize("P", [128, 640, 2176, 5120])
+def test_sums_of_one_fp32_row_are_taken_in_pairs(P):
+    """A weight of one symbol, a power of two, has exact products: each lane adds its columns one by one to the product's sum, and in pairs
+    to the sum of x; the lanes meet in a tree.  Bit for bit, so that the error against 64 bits stays what it was."""
+    Q = 24
+    W = torch.linspace(-0.05, 0.05, Q).to(torch.bfloat16).view(Q, 1).expand(Q, P).contiguous().to(DEV)
+    lin = QVBandLinearV8R(RP.transcode(PK.encode_tensor(W, 2e-3, keep_ids=True)), device=DEV)
+    ts, dr, mn = (t.cpu().numpy().astype(np.float64) for t in (lin.tau_s, lin.drow, lin.min_s))
+    symbols = ext.ids(P, *lin._core(), T=lin.T).cpu().numpy() - dr.reshape(Q, 1)
+    c = np.float32(symbols[0, 0])
+    assert (symbols == c).all() and (c == 0 or np.log2(c) % 1 == 0)
+
+    def tree(v):
+        while v.size > 1:
+            v = v[0::2] + v[1::2]
+        return np.float64(v[0])
+
+    for seed in range(4):
+        x = torch.randn(1, P, generator=torch.Generator().manual_seed(seed)) * 3.0
+        sx, acc = np.zeros(32, np.float32), np.zeros(32, np.float32)
+        for first, second in x.numpy().reshape(P // 64, 2, 32):          # (pair of steps, step, lane)
+            acc = (acc + c * first) + c * second
+            sx = sx + (first + second)
+        assert sx.dtype == acc.dtype == np.float32
+        a, b = tree(acc), tree(sx)
+        want = (ts * (a + dr * b) + mn * b).astype(np.float32)
+        got = ext.multi(x.to(DEV), *lin._core(), T=lin.T).cpu().numpy()[0]
+        # (the double expression may be contracted: its last bit, relative to its largest term)
+        room = 2.0 ** -50 * (np.abs(ts) * (abs(a) + np.abs(dr * b)) + np.abs(mn * b))
+        lo, hi = ((ts * (a + dr * b) + mn * b + s * room).astype(np.float32) for s in (-1, 1))
+        assert np.all((got >= np.minimum(lo, want)) & (got <= np.maximum(hi, want))), (P, seed)
