@@ -707,7 +707,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
     const int grp = (int)(threadIdx.x >> 2) % kGroups, cl = threadIdx.x & 3, ch = blockIdx.y * 16 + cl * 4, chc = min(ch, D - 4);
     const int64_t stride = (int64_t)nhkv * n_rows, unit = (int64_t)blockIdx.x * (4 / W) + wave / W, hr = min(unit, stride - 1);
     Joined j = {-INFINITY, 0.f, {0.f, 0.f, 0.f, 0.f}};
-    if (n_splits <= kGroups) join_splits<1>(j, o, m, l, grp, kGroups, n_splits, stride, hr, D, chc);
+    if (W > 1 && n_splits <= kGroups) join_splits<1>(j, o, m, l, grp, kGroups, n_splits, stride, hr, D, chc);
     else for (int s0 = grp; s0 < n_splits; s0 += 4 * kGroups) join_splits<4>(j, o, m, l, s0, kGroups, n_splits, stride, hr, D, chc);
 #pragma unroll
     for (int d = 4; d < 64; d <<= 1) {

@@ -1,6 +1,6 @@
-"""Attention of many query rows over the banded KV cache (the kernel of 128 rows per workgroup) against the oracle, at the sizes
+"""Attention of many query rows over the banded KV cache (the kernel of 128 or 256 rows per workgroup) against the oracle, at the sizes
 where its tiles change: the fewest rows it takes, one row more than a wave and a workgroup hold, tokens cut across both, key
-tiles of one key and of none a row sees, segment changes, 16-bit ids, scores that keep rising (the lazy rescale) or jump."""
+tiles of one key and of none a row sees, segment changes, 16-bit ids, scores that keep rising (a rescale at every tile) or jump."""
 import numpy as np
 import pytest
 import torch
@@ -8,6 +8,7 @@ import torch
 from oracle import kv_attn_oracle as A
 from tests.test_gpu_kv_attn import DEV, check_split_outputs, run_fwd, to_device, vmax
 from tests.test_oracle_kv_attn import make_layout
+from qvb8_amd import _lib
 from qvb8_amd.kv import fused_attn as FA
 
 pytestmark = pytest.mark.gpu
@@ -47,7 +48,10 @@ def test_workgroups_of_256_rows_match_the_oracle(D, Hkv, G, MQ, seg_len, q_pos0,
     want = A.fwd_split(q, lay["ki"], lay["vi"], lay["kmid"], lay["kstep"], lay["vmid"], lay["vstep"], lay["kc"], lay["vc"],
                        lay["ts"], lay["tl"], lay["tseg"], q_pos0, tps, scale, G)
     dl, q16 = to_device(lay, slack=MQ % 3), torch.from_numpy(q).to(DEV)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
     for empty in (512 // Hkv, 0):
+        block = _lib.load().qvb8_attn_rows_per_workgroup(MQ * G, want[0].shape[0] + empty, Hkv, 1, cus)
+        assert block == (256 if empty and MQ * G != 257 else 128)
         o, m, l = (torch.full((w.shape[0] + empty,) + w.shape[1:], float("nan"), device=DEV) for w in want)
         FA.fwd(q16, dl["ki"], dl["vi"], dl["kmid"], dl["kstep"], dl["vmid"], dl["vstep"], dl["kc"], dl["vc"], dl["ts"], dl["tl"], dl["tseg"], o, m, l, q_pos0, tps, scale, G)
         S = want[0].shape[0]

@@ -63,6 +63,24 @@ def test_rows_of_many_escapes(M):
             assert torch.equal(y16, y32.to(out_dtype)), (len(positions), saturate)
 
 
+@pytest.mark.parametrize("M", [1, 16, 64])
+def test_corrected_results_in_a_graph(M):
+    """The fp32 results between the two launches live in the graph's own memory; every replay against the eager call, with eager calls between."""
+    enc = PK.encode_tensor(H.synth_weight(300, 1024, seed=5).to(DEV), 1e-3, restore="fp16", force_escapes=torch.arange(0, 300 * 1024, 997))
+    lin = QVBandLinearV8.from_encoded(enc).prepare()
+    x = torch.zeros(M, 1024, dtype=torch.bfloat16, device=DEV)
+    lin(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = lin(x)
+    for i in range(4):
+        x.copy_(torch.randn(M, 1024, generator=torch.Generator().manual_seed(i)).to(torch.bfloat16))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert y.dtype == torch.bfloat16 and torch.equal(y, lin(x.clone()))
+
+
 @pytest.mark.parametrize("n_esc", [256, 257, 65536, 65537, 70000])
 def test_long_lists_through_the_module(n_esc):
     """One search step more from 257 and from 65537 escapes on; the module against fp32 results rounded by torch."""
