@@ -165,7 +165,14 @@ class QVBandLinearV8R(nn.Module):
     def _chunked(self, x2, bf16: bool):
         dt = torch.bfloat16 if bf16 else torch.float16
         # saturating fp16, as the small-M paths of QVB8 (an infinity among fp16 rows, which saturating_half leaves alone, too)
-        xk = x2 if bf16 else x2.clamp(-65504, 65504) if x2.dtype == torch.float16 else saturating_half(x2)
+        if bf16:
+            xk = x2
+        elif x2.dtype == torch.float16:
+            xk = x2.clamp(-65504, 65504)
+        elif torch.is_grad_enabled() and x2.requires_grad:
+            xk = x2.float().clamp(-65504, 65504).half()          # the library's pass leaves autograd's graph: a backward would be answered without x's part
+        else:
+            xk = saturating_half(x2)
         ef, ev = (self.esc_flat_bf16, self.esc_val_bf16) if bf16 else (self.esc_flat, self.esc_val)
         P = self.in_features
         code = 1 if bf16 else 0

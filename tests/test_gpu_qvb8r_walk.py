@@ -77,6 +77,22 @@ def test_whole_weight_in_one_chunk_and_in_several():
             assert np.all(diff[finite] <= tol[finite]), (dtype, float((diff / tol)[finite].max()))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_rows_that_want_a_gradient_stay_in_the_graph(dtype):
+    """The dense product has no derivative.  A backward through it is refused, as for a call that is part of a larger graph: the rest of
+    the graph must not be answered without this product's part.  The values are those of a call without a gradient."""
+    lin = QVBandLinearV8R(RP.transcode(PK.encode_tensor(H.synth_weight(64, 256, seed=3).to(DEV), 2e-3, keep_ids=True)), device=DEV)
+    x = torch.randn(70, 256, generator=torch.Generator().manual_seed(2)).to(dtype).to(DEV)
+    x[1, 2] = 7.0e4
+    with torch.no_grad():
+        want = lin(x)
+    x.requires_grad_()
+    y = lin(x)
+    assert torch.equal(y.detach(), want) and y.requires_grad
+    with pytest.raises(RuntimeError, match="not implemented"):
+        (y.float().sum() + x.float().sum()).backward()
+
+
 @pytest.mark.parametrize("P", [128, 640, 2176, 5120])
 def test_sums_of_one_fp32_row_are_taken_in_pairs(P):
     """A weight of one symbol, a power of two, has exact products: each lane adds its columns one by one to the product's sum, and in pairs
