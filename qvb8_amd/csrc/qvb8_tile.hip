@@ -117,6 +117,8 @@ __device__ __forceinline__ void decode_slice8_top(const uint4& lo, const uint4& 
 // slots.  After one barrier the whole workgroup combines the column ranges of each row in a fixed order.
 // The kernel's arguments are 56 bytes of scalars (measured: every further 64 bytes of kernel arguments cost about a
 // microsecond per launch): fin follows loc, n_steps follows P, the small counts share one word.
+// The first sixteen words arrive in registers, `widths` is fetched: what every launch asks early goes before it.  (The flag of SiLU pairs in
+// TW's top bit or in widths': a decode step of four layers of 4096 / 8960, 4 rows, 183.7 / 185.8 us; of 4096 / 12288, one row, 185.3 / 186.2.)
 // Waves a workgroup of this variant may have: twelve (three per SIMD) where the registers allow it -- long rows then take
 // fewer panels (12288 columns: two instead of three) --, else eight.
 constexpr uint32_t kTileTransitRow = 272;                     // bytes between rows of a wave's transit region (256 + 16: see XT)
@@ -131,9 +133,9 @@ __global__ void __launch_bounds__((64 * tile_max_waves<NT, T, BF, PL>())) tile_k
     constexpr bool XL = XP > 0;                              // X goes through LDS, XP 16-byte pieces per thread
     TileArgs a;
     a.X = X; a.ids = ids; a.loc = loc; a.fin = reinterpret_cast<const uint4*>(loc + rowinfo_loc_words(Q)); a.Y = Y;
-    a.ids_bytes = ids_bytes; a.Q = Q; a.P = P; a.n_steps = P / kStepCols; a.TW = TW;
+    a.ids_bytes = ids_bytes; a.Q = Q; a.P = P; a.n_steps = P / kStepCols; a.TW = TW & 0x7fffffff;
     a.M = (int)(counts & 63u); a.out_dt = (int)((counts >> 6) & 3u); a.W = (int)((counts >> 8) & 15u); a.G = (int)((counts >> 12) & 15u); a.panels = (int)(counts >> 16);
-    a.silu_pairs = (int)(widths >> 31);
+    a.silu_pairs = (int)((uint32_t)TW >> 31);
     a.first1 = first1; a.first2 = first2; a.n_classes = (int)((widths >> 24) & 0x7Fu); a.planes = PL ? 1 : 0;
     a.nb[0] = (int)(widths & 255u); a.nb[1] = (int)((widths >> 8) & 255u); a.nb[2] = (int)((widths >> 16) & 255u);
     using F = Fmt<BF>;
@@ -1475,8 +1477,8 @@ int launch_tile(TileArgs& a, hipStream_t s) {
     }
     const uint32_t counts = (uint32_t)a.M | ((uint32_t)a.out_dt << 6) | ((uint32_t)a.W << 8) | ((uint32_t)a.G << 12) | ((uint32_t)a.panels << 16);
     hipLaunchKernelGGL((tile_kernel<NT, T, BF, XC, XP, PL>), dim3(pl.blocks), dim3(pl.threads), pl.lds, s,
-                       a.X, a.ids, a.loc, a.Y, a.ids_bytes, a.Q, a.P, counts, a.TW, a.first1, a.first2,
-                       (uint32_t)a.nb[0] | ((uint32_t)a.nb[1] << 8) | ((uint32_t)a.nb[2] << 16) | ((uint32_t)a.n_classes << 24) | ((uint32_t)a.silu_pairs << 31));
+                       a.X, a.ids, a.loc, a.Y, a.ids_bytes, a.Q, a.P, counts, (int)((uint32_t)a.TW | ((uint32_t)a.silu_pairs << 31)), a.first1, a.first2,
+                       (uint32_t)a.nb[0] | ((uint32_t)a.nb[1] << 8) | ((uint32_t)a.nb[2] << 16) | ((uint32_t)a.n_classes << 24));
     return host::check_launch("qvb8_mma");
 }
 // One to sixteen rows of X on the NT = 1 kernel: X goes through LDS when all of it fits (the limits below, and the
