@@ -441,13 +441,14 @@ int qvb8_attn_fwd(const void* q, int64_t sq_r, int64_t sq_h, const void* ki, con
 int qvb8_attn_combine(const float* o, const float* m, const float* l, int64_t n_splits, int64_t n_kv_heads,
                       int64_t n_rows, int64_t head_dim, int64_t G, float* out, float* lse, void* stream);
 
+/* Query rows a workgroup of the kernel of many rows (33 rows and more) will serve on a device of `cus` compute units: 128 or 256; 0 below 33
+ * rows.  For a caller that plans its splits. */
+int64_t qvb8_attn_rows_per_workgroup(int64_t n_rows, int64_t n_splits, int64_t n_kv_heads, int id_bytes, int64_t cus);
+
 /* qvb8_scale_sat_half, qvb8_attn_fwd (scale 1) and qvb8_attn_combine as one call: the queries -- q_dtype QVB8_F32 / _F16 / _BF16,
  * strides in elements, multiples of 4, aligned to four elements, contiguous from 33 rows (tokens x G) on -- are multiplied by q_scale and
  * saturated to fp16, up to 32 rows by the kernel that reads them, beyond by a launch of its own.  `workspace`: qvb8_attn_workspace_bytes of device memory for the splits' partial results, 16-byte aligned.
  * Replaces: attend  kv/fused_attn.py:246-316. */
-/* Query rows a workgroup of the kernel of many rows (33 rows and more) will serve on a device of `cus` compute units: 128 or 256; 0 below 33
- * rows.  For a caller that plans its splits. */
-int64_t qvb8_attn_rows_per_workgroup(int64_t n_rows, int64_t n_splits, int64_t n_kv_heads, int id_bytes, int64_t cus);
 int64_t qvb8_attn_workspace_bytes(int64_t n_splits, int64_t n_kv_heads, int64_t n_rows, int64_t head_dim);
 int qvb8_attend(const void* q, int q_dtype, double q_scale, int64_t sq_r, int64_t sq_h, const void* ki, const void* vi, int id_bytes,
                 int64_t s_n, int64_t s_h, const float* kmid, const float* kstep, const float* vmid, const float* vstep,
