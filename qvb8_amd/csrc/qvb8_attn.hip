@@ -859,6 +859,10 @@ extern "C" int qvb8_attend(const void* q, int q_dtype, double q_scale, int64_t s
     using namespace qvb8;
     const char* who = "qvb8_attend";
     if (q_dtype < QVB8_F32 || q_dtype > QVB8_BF16) return host::fail(QVB8_ERR_ARG, "%s: unknown query type %d", who, q_dtype);
+    // ahead of the first launch: the workspace is laid out by these, and as many queries are read as they say
+    if (n_rows < 0 || n_splits < 1 || G < 1 || n_kv_heads < 1 || head_dim < 1 || n_rows % G != 0)
+        return host::fail(QVB8_ERR_ARG, "%s: bad size (rows %lld, splits %lld, G %lld, kv heads %lld, head_dim %lld)", who, (long long)n_rows, (long long)n_splits,
+                          (long long)G, (long long)n_kv_heads, (long long)head_dim);
     const int64_t need = qvb8_attn_workspace_bytes(n_splits, n_kv_heads, n_rows, head_dim);
     if (need > 0 && (!workspace || workspace_bytes < need || !aligned(workspace, 16)))
         return host::fail(QVB8_ERR_WORKSPACE, "%s: needs %lld bytes of 16-byte aligned workspace", who, (long long)need);

@@ -186,3 +186,20 @@ def test_plans_are_for_the_workgroups_the_library_will_launch(cus, monkeypatch):
                         seen.add((block, wide))
     assert seen == {(128, False), (256, False), (128, True)}
     assert lib.qvb8_attn_rows_per_workgroup(32, 4, 4, 1, cus) == 0
+
+
+@pytest.mark.parametrize("wrong", [dict(n_splits=0), dict(n_splits=-3), dict(G=0), dict(n_rows=65), dict(n_kv_heads=0), dict(n_rows=-2), dict(head_dim=0)])
+def test_attend_refuses_bad_sizes_before_its_first_launch(wrong):
+    """The preparation of many queries is a launch ahead of the attention kernel's own checks: with no splits it would be asked for no
+    workspace and write in front of it, with rows that are no whole tokens read queries that are not there."""
+    import ctypes
+    from qvb8_amd import _lib
+    lib = _lib.load()
+    size = dict(n_rows=64, n_splits=2, n_kv_heads=4, head_dim=128, G=2)
+    size.update(wrong)
+    here = ctypes.create_string_buffer(64)
+    at = (ctypes.addressof(here) + 15) & ~15
+    d, g, heads = size["head_dim"], size["G"], size["n_kv_heads"]
+    rc = lib.qvb8_attend(at, _lib.F16, 1.0, heads * g * d, d, at, at, 1, heads * d, d, *[at] * 9, 4, size["n_splits"], size["n_rows"], heads, d, 0, 2, g,
+                         at, at, at, 1 << 40, None)
+    assert rc == -1 and "bad size" in lib.qvb8_last_error().decode()
