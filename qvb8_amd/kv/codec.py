@@ -156,12 +156,11 @@ def _band_on_gpu(t, orig_dtype, bits: int, tau: float, certify: bool) -> list:
         grid = torch.empty((3, heads, dim), dtype=torch.float32, device=dev)                          # minima, steps, spans
         lo_at, step_at, span_at = (grid.data_ptr() + 4 * heads * dim * i for i in range(3))
 
-        def pack(packed, widths, a=0):
-            """Heads a .. a + len(packed) - 1 into their streams."""
-            skip, n = 4 * dim * a, len(packed)
+        def pack(packed, widths, x_at=x_at, skip=0):
+            """Some neighbouring heads into their streams, the first one's values at x_at, its constants `skip` bytes into theirs."""
+            n = len(packed)
             where = (ctypes.c_void_p * n)(*[p.data_ptr() for p in packed])
-            _lib._check(lib.qvb8_kv_pack(x_at + a * seq * dim * x.element_size() if a else x_at, dt, n, seq, dim, lo_at + skip, span_at + skip, bytes(widths),
-                                         step_at + skip, where, stream), lib)
+            _lib._check(lib.qvb8_kv_pack(x_at, dt, n, seq, dim, lo_at + skip, span_at + skip, bytes(widths), step_at + skip, where, stream), lib)
 
         widths, stored = [bits] * heads, (seq * dim * bits + 7) // 8
         if not certifying:
@@ -199,12 +198,12 @@ def _band_on_gpu(t, orig_dtype, bits: int, tau: float, certify: bool) -> list:
             while not all(e <= tau for e in errors):
                 widths = [w if e <= tau else _next_width(i, w, e, tau, orig_dtype) for i, (w, e) in enumerate(zip(widths, errors))]
                 errors = check()
-            risen = [i for i, w in enumerate(widths) if w != bits]
-            if risen:                                            # one launch over them and what lies between (the same bytes again)
+            if widths != [bits] * heads:                         # one launch over the heads that rose and what lies between (the same bytes again)
+                risen = [i for i, w in enumerate(widths) if w != bits]
                 for i in risen:
                     packed[i] = torch.empty((seq * dim * widths[i] + 7) // 8, dtype=torch.uint8, device=dev)
                 a, b = risen[0], risen[-1] + 1
-                pack(packed[a:b], widths[a:b], a)
+                pack(packed[a:b], widths[a:b], x_at + a * seq * dim * x.element_size(), 4 * dim * a)
     return [BandedKV(p, m, s, w, (seq, dim), orig_dtype, tau) for p, m, s, w in zip(packed, los, steps, widths)]
 
 
