@@ -14,6 +14,13 @@ typedef float v4f_t __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u_t __attribute__((ext_vector_type(4)));
 typedef float v16f_t __attribute__((ext_vector_type(16)));
 
+// a result into Y in the caller's format (wave-uniform choice)
+__device__ __forceinline__ void store_y(float* Y, int out_dt, int64_t i, float v) {
+    if (out_dt == 0) Y[i] = v;
+    else if (out_dt == 1) store_from_f32<1>(Y, i, v);
+    else store_from_f32<2>(Y, i, v);
+}
+
 constexpr int kTileRows = 16;
 constexpr int kStepCols = 128;          // columns one wave step covers (4 lane groups x 32 ids)
 

@@ -18,6 +18,7 @@
 #include <stdint.h>
 
 #include "../../include/qvb8_amd.h"
+#include "qvb8_columns.h"
 #include "qvb8_device.h"
 #include "qvb8_host.h"
 #include "qvb8_mma_device.h"
@@ -34,13 +35,6 @@ namespace qvb8 {
 // loc has Q rounded up to even entries, so that fin is 16-byte aligned.
 constexpr uint64_t kRowOffMask = (1ull << 48) - 1;
 __host__ __device__ inline size_t rowinfo_loc_words(int64_t Q) { return (size_t)((Q + 1) & ~(int64_t)1); }
-
-// a result into Y in the caller's format (wave-uniform choice)
-__device__ __forceinline__ void store_y(float* Y, int out_dt, int64_t i, float v) {
-    if (out_dt == 0) Y[i] = v;
-    else if (out_dt == 1) store_from_f32<1>(Y, i, v);
-    else store_from_f32<2>(Y, i, v);
-}
 
 // silu(g) * u with every step rounded to the type `dt` (0 fp32, 1 fp16, 2 bf16)
 __device__ __forceinline__ float round_to(float v, int dt) {
@@ -1584,6 +1578,8 @@ GemmPlan plan_gemm_for(int64_t M, int64_t Q, int64_t P) { return M >= gemm2_from
 // projections, 8 layers: M = 17 0.641 ms against 0.721 for the tile kernel with two token tiles, M = 32 0.70 / 0.87)
 int gemm_from() { const int v = host::env_int("QVB8_MMA_GEMM_FROM", 17); return v < 17 ? 17 : (v > 49 ? 49 : v); }
 
+bool columns_take(int64_t M) { return M >= gemm_from() && M <= kColumnsMaxM && host::env_int("QVB8_COLUMNS", 1) != 0; }
+
 template <int MT, bool BF, bool XC, int RT>
 int launch_gemm_as(const GemmArgs& a, const GemmPlan& g, int row_blocks, hipStream_t s) {
     static bool attr[64] = {false};
@@ -1677,8 +1673,11 @@ extern "C" int qvb8_decode_tiles(const uint8_t* ids, int64_t ids_bytes, const fl
 }
 
 extern "C" int64_t qvb8_mma_workspace_bytes(int64_t M, int64_t Q, int64_t P) {
-    if (M >= gemm_from() && M <= 256 && Q > 0 && P > 0 && (P % (2 * kGemmStageCols)) == 0) return plan_gemm_for(M, Q, P).bytes;
-    return qvb8_mma_rowinfo_bytes(Q);
+    int64_t need = qvb8_mma_rowinfo_bytes(Q);
+    if (M < gemm_from() || M > 256 || Q < 1 || P < 1) return need;
+    if (P % (2 * kGemmStageCols) == 0) need = std::max(need, plan_gemm_for(M, Q, P).bytes);
+    if (columns_take(M) && P % kStepCols == 0) need = std::max(need, plan_columns(M, Q, P).bytes);
+    return need;
 }
 
 // fp32 results behind what the kernels need: those of a call whose own are 16-bit and corrected
@@ -1755,6 +1754,14 @@ extern "C" int qvb8_mma(const void* X, int x_dtype, int64_t M,
     // mode 0: fp16 X, fp16 operands; 1: bf16 X narrowed to saturated fp16 on the way in, fp16 operands; 2: bf16 operands
     const int mode = x_dtype == QVB8_F16 ? 0 : (flags & QVB8_MMA_SATURATE_X) ? 1 : 2;
     int rc;
+    bool columns = columns_take(M) && layout && mode != 2 && (M <= 48 || P % (2 * kGemmStageCols) == 0) && workspace
+                   && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
+    ColumnsPlan cp = {};
+    if (columns) {
+        for (int c = 0; c < a.n_classes; ++c) columns = columns && a.nb[c] >= 4 && a.nb[c] <= 8;
+        cp = plan_columns(M, Q, P);
+        columns = columns && cp.taken && workspace_bytes >= cp.bytes;
+    }
     // Many rows of X: the workgroup-tiled kernel.  It addresses rows arithmetically and decodes whole slices only; from 17
     // rows on it is also the faster one (the tile kernel then keeps too few bytes in flight), so it is taken whenever it
     // can read the weight and the caller brought its workspace.
@@ -1764,7 +1771,22 @@ extern "C" int qvb8_mma(const void* X, int x_dtype, int64_t M,
         tiled = true;
         for (int c = 0; c < a.n_classes; ++c) tiled = tiled && a.nb[c] >= 4 && a.nb[c] <= (mode == 2 ? 7 : 8);
     }
-    if (tiled) {
+    if (columns) {
+        unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
+        ColumnsArgs ca = {};
+        ca.ids = ids; ca.fin = a.fin; ca.M = (int)M; ca.Q = (int)Q; ca.P = (int)P;
+        ca.out = cp.splits > 1 ? reinterpret_cast<float*>(ws + cp.part_at) : Y;
+        ca.out_dt = cp.splits > 1 ? 0 : out_dt;
+        ca.planes = a.planes;
+        ca.first1 = a.first1; ca.first2 = a.first2;
+        ca.widths = (uint32_t)a.nb[0] | ((uint32_t)a.nb[1] << 8) | ((uint32_t)a.nb[2] << 16);
+        if ((rc = launch_columns(cp, ca, a.X, mode, reinterpret_cast<uint16_t*>(ws + cp.x16_at), reinterpret_cast<float*>(ws + cp.sx_at), s))) return rc;
+        if (cp.splits > 1) {
+            const int64_t n = M * Q;
+            hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ca.out, Y, n, cp.splits, out_dt);
+            if (int rc2 = host::check_launch("qvb8_mma reduce")) return rc2;
+        }
+    } else if (tiled) {
         if (!layout) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_mma: M > 48 needs rows stored in width order (a row layout)");
         if ((P % (2 * kGemmStageCols)) != 0) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_mma: M > 48 needs P %% 256 == 0");
         for (int c = 0; c < a.n_classes; ++c)

@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import itertools
 
 import torch
 
@@ -309,9 +310,9 @@ def repack_rows(ids, row_nbits, row_bit_off, P, new_nbits, chunk_rows=256):
 
 def widen_rows_to_whole_tiles(ids, row_nbits, row_bit_off, P, tile_rows=16, top=8):
     """Stores a few rows with more bits than they need so that, sorted by width, every run of one width is a whole number
-    of 16-row tiles: of each width (ascending) the last `count % 16` rows move up to the next width present (up to
+    of 16-row tiles (of `tile_rows` rows: a multiple of 16): of each width (ascending) the last `count % tile_rows` rows move up to the next width present (up to
     `top`).  A row's ids, tau_s and min_s stay what they are -- only the field its ids are stored in gets wider, so
-    every value of the weight is unchanged -- and at most 15 rows per width grow by a bit or two each.  Returns
+    every value of the weight is unchanged -- and at most tile_rows - 1 rows per width grow by a bit or two each.  Returns
     (ids, row_nbits, row_bit_off) with the widened rows appended to a copy of `ids`, or None when nothing moves."""
     P = int(P)
     ids, row_bit_off = rows_back_to_back(ids, row_nbits, row_bit_off, P)
@@ -344,22 +345,26 @@ def widen_rows_to_whole_tiles(ids, row_nbits, row_bit_off, P, tile_rows=16, top=
             final[q] = (final[q][0] if q in final else w0, up)
     if not final:
         return None
-    new_nb, new_off = row_nbits.clone(), row_bit_off.clone()
+    dev = ids.device
     base = (ids.numel() - 8 + 15) // 16 * 16                               # the pad bytes of the old end are reused
-    parts, at = [], base
-    cols = torch.arange(P, device=ids.device, dtype=torch.int64)
-    for q, (w0, up) in sorted(final.items()):
-        pos = row_bit_off[q] + cols * w0
-        byte, sh = pos >> 3, pos & 7
-        word = ids[byte].to(torch.int64) | (ids[byte + 1].to(torch.int64) << 8) | (ids[byte + 2].to(torch.int64) << 16)
-        val = (word >> sh) & ((1 << w0) - 1)
-        bits = ((val[:, None] >> torch.arange(up, device=ids.device)) & 1).reshape(-1, 8)
-        parts.append((bits << torch.arange(8, device=ids.device)).sum(1).to(torch.uint8))
-        new_nb[q], new_off[q] = up, at * 8
-        at += P * up // 8
-    out_ids = torch.zeros(at + 8, dtype=torch.uint8, device=ids.device)
+    rows = sorted(final)
+    starts = [base, *itertools.accumulate((P * final[q][1] // 8 for q in rows), initial=base)][1:]
+    out_ids = torch.zeros(starts[-1] + 8, dtype=torch.uint8, device=dev)
     out_ids[: ids.numel() - 8] = ids[: ids.numel() - 8]
-    out_ids[base:at] = torch.cat(parts)
+    new_nb, new_off = row_nbits.clone(), row_bit_off.clone()
+    cols = torch.arange(P, device=dev, dtype=torch.int64)
+    for w0, up in sorted(set(final.values())):
+        kind = [i for i, q in enumerate(rows) if final[q] == (w0, up)]
+        for k in range(0, len(kind), 32):                                  # bounded index tensors
+            q, to = (torch.tensor([v[i] for i in kind[k:k + 32]], device=dev, dtype=torch.int64) for v in (rows, starts))
+            pos = row_bit_off[q][:, None] + cols * w0
+            byte, sh = pos >> 3, pos & 7
+            word = ids[byte].to(torch.int64) | (ids[byte + 1].to(torch.int64) << 8) | (ids[byte + 2].to(torch.int64) << 16)
+            val = ((word >> sh) & ((1 << w0) - 1)).to(torch.int32)
+            bits = ((val[:, :, None] >> torch.arange(up, device=dev, dtype=torch.int32)) & 1).reshape(q.numel(), -1, 8)
+            packed = (bits << torch.arange(8, device=dev, dtype=torch.int32)).sum(2).to(torch.uint8)
+            out_ids[to[:, None] + torch.arange(P * up // 8, device=dev)] = packed
+            new_nb[q], new_off[q] = up, to * 8
     return out_ids, new_nb, new_off
 
 
