@@ -259,7 +259,8 @@ def bench_moe(args, dev):
                                       g_["nbits"].data_ptr(), g_["bit_off"].data_ptr(), g_["Q"], g_["P"],
                                       d_["ids"].data_ptr(), d_["ids"].numel(), d_["min_s"].data_ptr(), d_["tau_s"].data_ptr(),
                                       d_["nbits"].data_ptr(), d_["bit_off"].data_ptr(), d_["Q"], d_["P"],
-                                      (0x100 if g_["regular"] else 0) | (0x200 if d_["regular"] else 0),   # what the operator passes
+                                      (0x100 if g_["regular"] else 0) | (0x200 if d_["regular"] else 0)    # what the operator passes
+                                      | (0x800 if g_["planes"] else 0) | (0x1000 if d_["planes"] else 0),
                                       out.data_ptr(), 2, ws.data_ptr(), ws.numel(), s)
             if rc != 0:
                 raise RuntimeError(lib.qvb8_last_error().decode())

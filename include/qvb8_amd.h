@@ -277,7 +277,11 @@ enum qvb8_moe_act {
     QVB8_MOE_DOWN_REGULAR = 0x200,
     /* More than 16 tokens: an infinity among fp16 activations stays one.  Without the flag it becomes +-65504, as every value beyond
      * fp16's range does in the other activation types (up to 16 tokens fp16 activations are always taken as they are). */
-    QVB8_MOE_KEEP_INF = 0x400
+    QVB8_MOE_KEEP_INF = 0x400,
+    /* With QVB8_MOE_*_REGULAR, P a multiple of 128 and whole 16-row tiles (of each half, where gate and up are halves): every tile is
+     * stored in planes, as QVB8_MMA_PLANES describes; bit_off keeps the places of rows back to back. */
+    QVB8_MOE_UP_PLANES = 0x800,
+    QVB8_MOE_DOWN_PLANES = 0x1000
 };
 
 /* Bytes of workspace qvb8_moe_experts needs (routing plan + fp32 H (pairs, P_dn) + fp32 Yd (pairs, Q_dn)). */

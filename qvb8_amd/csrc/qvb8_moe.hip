@@ -169,6 +169,7 @@ struct MoeGemvArgs {
     int units_per_block;
     int keep_inf;                  // QVB8_MOE_KEEP_INF
     int x_rows;                    // activation rows a workgroup stages at a time: min(kMoeMB, tokens)
+    int planes;                    // every 16-row tile is stored in planes (QVB8_MOE_*_PLANES)
 };
 
 template <int NB, int J>
@@ -230,7 +231,21 @@ __device__ __forceinline__ void moe_chunk_any(int nb, const uint4& lo, const uin
 }
 
 // Row record a workgroup keeps in LDS for each of its rows: flags = width | ok << 8 | fast << 9
-struct MoeRow { int64_t bit0; float ts, mn; int flags; int pad; };
+struct MoeRow { int64_t bit0; float ts, mn; int flags; int slot; };       // slot: the row's number in its tile
+// first and last four dwords of slice `cg` (32 columns) of a row: back to back, or of a tile in planes (bit0 = the tile's first bit)
+__device__ __forceinline__ void moe_slice(const uint8_t* ids, int64_t bit0, int nb, int slot, int cg, bool planes, uint4& lo, uint4& hi) {
+    const uint8_t* p = ids + (bit0 >> 3);
+    if (planes) {
+        const uint32_t at = (uint32_t)slot + 16u * (uint32_t)(cg & 3);
+        p += (size_t)(cg >> 2) * (256u * (uint32_t)nb);
+        lo = *reinterpret_cast<const uint4*>(p + at * 16u);
+        hi = *reinterpret_cast<const uint4*>(p + 1008u + (at + 1u) * (4u * (uint32_t)(nb - 4)));
+    } else {
+        p += (size_t)cg * (4u * (uint32_t)nb);
+        lo = *reinterpret_cast<const uint4*>(p);
+        hi = *reinterpret_cast<const uint4*>(p + 4 * (nb - 4));
+    }
+}
 
 // STAGE 0: up projection + activation -> H.  STAGE 1: down projection -> Yd.
 // grid = (unit blocks, expert slots); a workgroup serves `units_per_block` output units of one selected expert for
@@ -257,12 +272,14 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
     // the odd ones the matching up rows (Q/2 + u)
     for (int lr = tid; lr < n_rows_blk; lr += blockDim.x) {
         const int u = u_begin + lr / rpu;
-        const size_t mi = (size_t)e * a.Q + ((rpu == 2 && (lr & 1)) ? gate_rows + u : u);
+        const int row = (rpu == 2 && (lr & 1)) ? gate_rows + u : u;
+        const size_t mi = (size_t)e * a.Q + row;
         const int nb = a.nbits[mi];
-        const int64_t bit0 = a.bit_off[mi];
-        const bool ok = nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + (int64_t)nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
+        const int64_t bit0 = a.planes ? a.bit_off[mi - (row & 15)] : a.bit_off[mi];
+        bool ok = nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + (int64_t)nb * a.P * (a.planes ? 16 : 1) + 7) >> 3) + 8 <= a.ids_bytes;
         const bool fast = ok && nb >= 4 && nb <= 8 && (bit0 & 31) == 0;
-        s_row[lr] = MoeRow{ok ? bit0 : 0, a.tau_s[mi], a.min_s[mi], nb | (ok ? 256 : 0) | (fast ? 512 : 0), 0};
+        if (a.planes) ok = fast;
+        s_row[lr] = MoeRow{ok ? bit0 : 0, a.tau_s[mi], a.min_s[mi], nb | (ok ? 256 : 0) | (fast ? 512 : 0), row & 15};
     }
     const int64_t clamp_byte = (a.ids_bytes - 8) & ~(int64_t)3;
     const int n_items = ((u_end - u_begin - wave + n_waves - 1) / n_waves) * rpu;   // rows this wave walks through
@@ -271,9 +288,7 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
     auto request = [&](const MoeRow& r, uint4& lo, uint4& hi) {
         const int nb = r.flags & 255;
         const bool use = (r.flags & 512) && lane * 32 < a.P;
-        const uint8_t* p = a.ids + (use ? (r.bit0 >> 3) + (int64_t)lane * 4 * nb : 0);
-        lo = *reinterpret_cast<const uint4*>(p);
-        hi = *reinterpret_cast<const uint4*>(p + (use ? 4 * (nb - 4) : 16));
+        moe_slice(a.ids, use ? r.bit0 : 0, use ? nb : 8, r.slot, use ? lane : 0, use && a.planes, lo, hi);
     };
 
     for (int pc = p_begin; pc < p_end; pc += a.x_rows) {
@@ -324,8 +339,9 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
             if (cur.flags & 512) {
                 if (lane * 32 < a.P) moe_chunk_any(nb, lo, hi, xs, a.P, lane * 32, n, acc);
                 for (int c0 = (kWave + lane) * 32; c0 < a.P; c0 += kWave * 32) {          // rows longer than 2048 columns
-                    const uint8_t* p = a.ids + (cur.bit0 >> 3) + (int64_t)(c0 >> 5) * 4 * nb;
-                    moe_chunk_any(nb, *reinterpret_cast<const uint4*>(p), *reinterpret_cast<const uint4*>(p + 4 * (nb - 4)), xs, a.P, c0, n, acc);
+                    uint4 l, h;
+                    moe_slice(a.ids, cur.bit0, nb, cur.slot, c0 >> 5, a.planes != 0, l, h);
+                    moe_chunk_any(nb, l, h, xs, a.P, c0, n, acc);
                 }
             } else if (cur.flags & 256) {
                 for (int c = lane; c < a.P; c += kWave) {
@@ -396,6 +412,7 @@ struct MoeOneArgs {
     int E, Q, P, topk;
     int units, gated;              // up: outputs per expert; whether the rows come as (gate, up) halves
     int tiles_per_wg;              // up: unit tiles per workgroup
+    int planes;                    // every 16-row tile is stored in planes (REG only)
 };
 
 // REG: the caller states that every row of the stack has one width and that the rows lie at regular places (row q of
@@ -490,27 +507,32 @@ __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
     // + chunk (four neighbouring lanes read 16 nb consecutive bytes of one row: far fewer L1 accesses per request than a row
     // per lane) and to_operand moves the registers into operand order (lane = row + 16 * chunk) across the wave.
     const int pull = 4 * (4 * r + kg);
+    const bool planes = REG && a.planes != 0;                 // already in operand order: lane l asks for entry l
     auto to_operand = [&](const uint4& v) -> uint4 {
         if constexpr (!REG) return v;
+        if (planes) return v;
         return uint4{(uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.x), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.y),
                      (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.z), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.w)};
     };
     auto request_ids = [&](Round& q, uint4 (&lo)[T], uint4 (&hi)[T]) {
-        q.ok = q.e_ok && q.nb >= 1 && q.nb <= 14 && q.bit0 >= 0 && ((q.bit0 + (int64_t)q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
+        const int64_t end_row = planes ? (int64_t)(16 - r) : 1;  // (in planes a row ends with its tile)
+        q.ok = q.e_ok && q.nb >= 1 && q.nb <= 14 && q.bit0 >= 0 && ((q.bit0 + end_row * q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
         q.sliced = q.ok && q.nb >= 4 && q.nb <= 8 && (q.bit0 & 31) == 0;
         // the row and chunk this lane asks for: its own (row r, chunk kg), or in REG mode row lane / 4, chunk lane % 4 of the
         // same tile (rows of a tile follow each other at P * nb bits; all 16 are usable or none is)
-        const int64_t ask_bit0 = REG ? q.bit0 + (int64_t)((lane >> 2) - r) * a.P * q.nb : q.bit0;
+        const int64_t ask_bit0 = REG ? q.bit0 + (int64_t)((planes ? 0 : lane >> 2) - r) * a.P * q.nb : q.bit0;
         const int ask_chunk = REG ? (lane & 3) : kg;
         const bool ask_sliced = !REG ? q.sliced : (q.e_ok && q.nb >= 4 && q.nb <= 8 && ask_bit0 >= 0 && (ask_bit0 & 31) == 0
-                                                   && ((ask_bit0 + (int64_t)q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes);
-        const uint64_t row_off = (uint64_t)(ask_bit0 >> 3) + (uint64_t)(step0 * 4 + ask_chunk) * (4u * (uint32_t)q.nb);
+                                                   && ((ask_bit0 + (planes ? 16 : 1) * (int64_t)q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes);
+        const uint32_t nbu = (uint32_t)q.nb, per_step = planes ? 256u * nbu : 16u * nbu;
+        const uint64_t row_off = (uint64_t)(ask_bit0 >> 3) + (planes ? (uint64_t)step0 * per_step + 16u * (uint32_t)lane : (uint64_t)(step0 * 4 + ask_chunk) * (4u * nbu));
+        const uint32_t to_hi = planes ? 1008u + (uint32_t)(lane + 1) * (4u * (nbu - 4u)) - 16u * (uint32_t)lane : 4u * (nbu - 4u);
 #pragma unroll
         for (int it = 0; it < T; ++it) {
             const bool use = ask_sliced && (step0 + it) < n_steps;     // a wave without a tile reads tile 0's again: no address shared by the whole chip
-            const uint64_t off = use ? row_off + (uint64_t)it * (16u * (uint32_t)q.nb) : 0;
+            const uint64_t off = use ? row_off + (uint64_t)it * per_step : 0;
             lo[it] = *reinterpret_cast<const uint4*>(a.ids + off);
-            hi[it] = *reinterpret_cast<const uint4*>(a.ids + off + (use ? 4u * (uint32_t)(q.nb - 4) : 16u));
+            hi[it] = *reinterpret_cast<const uint4*>(a.ids + off + (use ? to_hi : 16u));
         }
     };
     auto multiply = [&](const Round& q, const uint4 (&lo_)[T], const uint4 (&hi_)[T], const uint16_t* xrow) {
@@ -660,6 +682,7 @@ struct MoeWalkArgs {
     int units, gated;              // up: outputs per expert; whether the rows come as (gate, up) halves
     int tiles_per_seg;             // unit tiles (up) / row tiles (down) per segment
     int max_tokens;                // most pairs an expert can have in this call (the LDS is laid out for it)
+    int planes;                    // every 16-row tile is stored in planes (REG only)
 };
 constexpr int kWalkWaves = 4;          // waves per workgroup: two workgroups share a CU
 constexpr int kWalkMaxRowTiles = 16;   // row tiles per segment: one row record per thread
@@ -697,6 +720,7 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
     const int reg_nb = REG ? (int)a.nbits[0] : 0;
     const int64_t reg_base = REG ? a.bit_off[0] : 0;
     const int64_t reg_stride = REG ? a.bit_off[a.E > 1 ? a.Q : 0] - reg_base : 0;
+    const bool planes = REG && a.planes != 0;                 // already in operand order: lane l asks for entry l of its tile
     const int n_active = a.plan.n_bad[1];
     const int per_expert = max(1, (int)gridDim.x / max(1, n_active));
     const int sl = (int)blockIdx.x / per_expert;
@@ -745,7 +769,8 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
         }
         bool row_usable = false;
         if (tid < n_rows) {
-            const bool ok = e_ok && nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + (int64_t)nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
+            const int64_t end_row = planes ? (int64_t)(16 - (row_in_expert & 15)) : 1;      // (in planes a row ends with its tile)
+            const bool ok = e_ok && nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + end_row * nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
             const bool sliced = ok && nb >= 4 && nb <= 8 && (bit0 & 31) == 0;
             row_usable = ok;
             // REG: the record is complete without anything read from memory; tau_s and min_s go to LDS further down,
@@ -786,23 +811,26 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
             const WalkRow rec = s_row[i * 16 + r];
             // REG: the lane asks for chunk lane % 4 of row lane / 4 of the tile (neighbouring lanes, neighbouring bytes: far
             // fewer L1 accesses per request than a row per lane); to_operand brings the registers into operand order
-            const WalkRow ask = REG ? s_row[i * 16 + (lane >> 2)] : rec;
+            const WalkRow ask = REG ? s_row[i * 16 + (planes ? 0 : lane >> 2)] : rec;
             const int ask_chunk = REG ? (lane & 3) : kg;
             const uint32_t nbr = (uint32_t)ask.flags & 255u;
             const bool sliced = (ask.flags & 512) != 0;
-            const uint64_t row_off = (uint64_t)(ask.bit0 >> 3) + (uint64_t)(step0 * 4 + ask_chunk) * (4u * nbr);
+            const uint32_t per_step = planes ? 256u * nbr : 16u * nbr;
+            const uint64_t row_off = (uint64_t)(ask.bit0 >> 3) + (planes ? (uint64_t)step0 * per_step + 16u * (uint32_t)lane : (uint64_t)(step0 * 4 + ask_chunk) * (4u * nbr));
+            const uint32_t to_hi = planes ? 1008u + (uint32_t)(lane + 1) * (4u * (nbr - 4u)) - 16u * (uint32_t)lane : 4u * (nbr - 4u);
 #pragma unroll
             for (int it = 0; it < T; ++it) {
                 const bool use = sliced && (step0 + it) < n_steps;
-                const uint64_t off = use ? row_off + (uint64_t)it * (16u * nbr) : 0;
+                const uint64_t off = use ? row_off + (uint64_t)it * per_step : 0;
                 lo[it] = *reinterpret_cast<const uint4*>(a.ids + off);
-                hi[it] = *reinterpret_cast<const uint4*>(a.ids + off + (use ? 4u * (nbr - 4u) : 16u));
+                hi[it] = *reinterpret_cast<const uint4*>(a.ids + off + (use ? to_hi : 16u));
             }
             return rec;
         };
         const int pull = 4 * (4 * r + kg);
         auto to_operand = [&](const uint4& v) __attribute__((always_inline)) -> uint4 {
             if constexpr (!REG) return v;
+            if (planes) return v;
             return uint4{(uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.x), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.y),
                          (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.z), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.w)};
         };
@@ -1108,10 +1136,14 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
                 const uint8_t* dn_nb, const int64_t* dn_off, int64_t Q_dn, int64_t P_dn,
                 int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes, int32_t* bad_out, void* stream) {
     if (tokens < 0 || topk < 1 || n_experts < 1 || n_experts > 8192) return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: bad token / top-k / expert count");
-    constexpr int kActFlags = QVB8_MOE_UP_REGULAR | QVB8_MOE_DOWN_REGULAR | QVB8_MOE_KEEP_INF;
+    constexpr int kActFlags = QVB8_MOE_UP_REGULAR | QVB8_MOE_DOWN_REGULAR | QVB8_MOE_KEEP_INF | QVB8_MOE_UP_PLANES | QVB8_MOE_DOWN_PLANES;
     if ((act & ~kActFlags) != 0 && (act & ~kActFlags) != 1)
         return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: act must be 0 (gated SiLU) or 1 (ReLU squared), with the QVB8_MOE_* flags at most");
     const bool up_regular = (act & QVB8_MOE_UP_REGULAR) != 0, dn_regular = (act & QVB8_MOE_DOWN_REGULAR) != 0, keep_inf = (act & QVB8_MOE_KEEP_INF) != 0;
+    const bool up_planes = (act & QVB8_MOE_UP_PLANES) != 0, dn_planes = (act & QVB8_MOE_DOWN_PLANES) != 0;
+    if ((up_planes && (!up_regular || P_up % kStepCols || Q_up % 16)) || (dn_planes && (!dn_regular || P_dn % kStepCols || Q_dn % 16))
+        || (up_planes && (act & 0xFF) == 0 && P_dn % 16))
+        return host::fail(QVB8_ERR_ARG, "moe: tiles in planes need a regular stack, whole 128-column steps and whole 16-row tiles");
     act &= 0xFF;
     if (Q_up <= 0 || P_up <= 0 || Q_dn <= 0 || P_dn <= 0 || Q_up > 0x7fffffff || P_up > 0x7fffffff || Q_dn > 0x7fffffff || P_dn > 0x7fffffff)
         return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: bad shape");
@@ -1151,13 +1183,13 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
         const int64_t cap = kOneMaxTiles / RT;
         if (per_wg > cap) per_wg = cap;
         if (per_wg < 1) per_wg = 1;
-        o.tiles_per_wg = (int)per_wg;
+        o.tiles_per_wg = (int)per_wg; o.planes = up_planes ? 1 : 0;
         const unsigned up_blocks = (unsigned)((total_ut + per_wg - 1) / per_wg);
         const unsigned tk = (unsigned)tokens;
         if (int rc = x_dtype == QVB8_BF16 ? launch_moe_one<false, true, 0>(o, up_regular, up_blocks, tk, s) : launch_moe_one<false, false, 0>(o, up_regular, up_blocks, tk, s)) return rc;
         o.X = reinterpret_cast<const uint16_t*>(H); o.ids = dn_ids; o.ids_bytes = dn_ids_bytes;
         o.min_s = dn_min; o.tau_s = dn_tau; o.nbits = dn_nb; o.bit_off = dn_off; o.out = out;
-        o.Q = (int)Q_dn; o.P = (int)P_dn; o.units = (int)Q_dn; o.gated = 0; o.tiles_per_wg = 0;
+        o.Q = (int)Q_dn; o.P = (int)P_dn; o.units = (int)Q_dn; o.gated = 0; o.tiles_per_wg = 0; o.planes = dn_planes ? 1 : 0;
         const unsigned dn_blocks = (unsigned)(Q_dn / 16);
         if (out_dtype == QVB8_F32) return launch_moe_one<true, false, 0>(o, dn_regular, dn_blocks, tk, s);
         if (out_dtype == QVB8_F16) return launch_moe_one<true, false, 1>(o, dn_regular, dn_blocks, tk, s);
@@ -1176,24 +1208,25 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
         wa.X = reinterpret_cast<const uint16_t*>(X); wa.plan = pl; wa.ids = up_ids; wa.ids_bytes = up_ids_bytes;
         wa.min_s = up_min; wa.tau_s = up_tau; wa.nbits = up_nb; wa.bit_off = up_off; wa.out = H;                // H as fp16 (pairs, P_dn)
         wa.E = (int)n_experts; wa.Q = (int)Q_up; wa.P = (int)P_up; wa.topk = (int)topk; wa.units = (int)P_dn; wa.gated = act == 0 ? 1 : 0;
-        wa.tiles_per_seg = 1; wa.max_tokens = 1;
+        wa.tiles_per_seg = 1; wa.max_tokens = 1; wa.planes = up_planes ? 1 : 0;
         if (int rc = x_dtype == QVB8_BF16 ? launch_moe_walk<false, true>(wa, up_regular, slots, tokens, s) : launch_moe_walk<false, false>(wa, up_regular, slots, tokens, s)) return rc;
         wa.X = reinterpret_cast<const uint16_t*>(H); wa.ids = dn_ids; wa.ids_bytes = dn_ids_bytes;
         wa.min_s = dn_min; wa.tau_s = dn_tau; wa.nbits = dn_nb; wa.bit_off = dn_off; wa.out = Yd;
-        wa.Q = (int)Q_dn; wa.P = (int)P_dn; wa.units = (int)Q_dn; wa.gated = 0;
+        wa.Q = (int)Q_dn; wa.P = (int)P_dn; wa.units = (int)Q_dn; wa.gated = 0; wa.planes = dn_planes ? 1 : 0;
         if (int rc = launch_moe_walk<true, false>(wa, dn_regular, slots, tokens, s)) return rc;
         return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
     }
-    if (tokens > 16 && (reinterpret_cast<uintptr_t>(X) & 15u) == 0 && moe_group_shapes_ok(P_up, Q_dn, P_dn)) {
+    // (the general kernel reads a row at a time, which leaves most of a tile's lines in planes to be fetched again)
+    if ((tokens > 16 || up_planes || dn_planes) && (reinterpret_cast<uintptr_t>(X) & 15u) == 0 && moe_group_shapes_ok(P_up, Q_dn, P_dn)) {
         MoeGroupArgs ga;
         ga.X = X; ga.plan = pl; ga.ids = up_ids; ga.ids_bytes = up_ids_bytes;
         ga.min_s = up_min; ga.tau_s = up_tau; ga.nbits = up_nb; ga.bit_off = up_off; ga.out = H;
         ga.E = (int)n_experts; ga.Q = (int)Q_up; ga.P = (int)P_up; ga.topk = (int)topk; ga.units = (int)P_dn; ga.gated = act == 0 ? 1 : 0;
-        ga.row_blocks = ga.items = 0; ga.keep_inf = keep_inf ? 1 : 0;
+        ga.row_blocks = ga.items = 0; ga.keep_inf = keep_inf ? 1 : 0; ga.planes = up_planes ? 1 : 0;
         if (int rc = launch_moe_group(false, x_dtype, ga, np, s)) return rc;
         ga.X = H; ga.ids = dn_ids; ga.ids_bytes = dn_ids_bytes;
         ga.min_s = dn_min; ga.tau_s = dn_tau; ga.nbits = dn_nb; ga.bit_off = dn_off; ga.out = Yd;
-        ga.Q = (int)Q_dn; ga.P = (int)P_dn; ga.units = (int)Q_dn; ga.gated = 0;
+        ga.Q = (int)Q_dn; ga.P = (int)P_dn; ga.units = (int)Q_dn; ga.gated = 0; ga.planes = dn_planes ? 1 : 0;
         if (int rc = launch_moe_group(true, QVB8_F32, ga, np, s)) return rc;
         return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
     }
@@ -1201,10 +1234,10 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
     MoeGemvArgs a;
     a.X = X; a.ids = up_ids; a.ids_bytes = up_ids_bytes; a.min_s = up_min; a.tau_s = up_tau; a.nbits = up_nb; a.bit_off = up_off;
     a.out = H; a.plan = pl; a.Q = (int)Q_up; a.P = (int)P_up; a.topk = (int)topk; a.x_dtype = x_dtype; a.act = act;
-    a.units = (int)P_dn; a.keep_inf = keep_inf ? 1 : 0; a.units_per_block = 0; a.x_rows = (int)(tokens < kMoeMB ? tokens : kMoeMB);
+    a.units = (int)P_dn; a.planes = up_planes ? 1 : 0; a.keep_inf = keep_inf ? 1 : 0; a.units_per_block = 0; a.x_rows = (int)(tokens < kMoeMB ? tokens : kMoeMB);
     if (int rc = launch_moe_gemv(0, a, slots, s)) return rc;
     a.X = H; a.ids = dn_ids; a.ids_bytes = dn_ids_bytes; a.min_s = dn_min; a.tau_s = dn_tau; a.nbits = dn_nb; a.bit_off = dn_off;
-    a.out = Yd; a.Q = (int)Q_dn; a.P = (int)P_dn; a.x_dtype = QVB8_F32; a.units = (int)Q_dn;
+    a.out = Yd; a.Q = (int)Q_dn; a.P = (int)P_dn; a.x_dtype = QVB8_F32; a.units = (int)Q_dn; a.planes = dn_planes ? 1 : 0;
     if (int rc = launch_moe_gemv(1, a, slots, s)) return rc;
 
     return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);

@@ -19,10 +19,12 @@
 // Error of a call's fp32 results against 64 bits (17 .. 64 tokens, activations that fp16 holds): 2.3e-7 .. 3.3e-7 of their norm; the
 // general path's fp32 products 5.4e-7 .. 6.9e-7; with c in the middle of the width instead, 1.0e-6 .. 1.4e-6.
 //
-// Measured (hidden 2048, 128 experts of 2 x 768 / 768 columns, top-8, bf16): a layer of 509 tokens 212 us, where one pass per
-// expert over its own modules took 12.2 ms, nearly all of it launches; kernels alone, under the profiler, up 109, down 89, plan 13,
-// combine 8.  40 tokens 132 us against 410 on the general path.  The up launch moves 300 MB at 2.7 TB/s: its vector units are 46 %
-// busy with the decode, its L1 59 % with requests that touch sixteen rows each, the matrix pipes 14 %.
+// Measured (hidden 2048, 128 experts of 2 x 768 / 768 columns, top-8, bf16): a layer of 509 tokens 184 us, where one pass per
+// expert over its own modules took 12.2 ms, nearly all of it launches; kernels alone, under the profiler, up 87, down 77, plan 13,
+// combine 8.  With the rows back to back 210 us, up 109, down 89: a request then touches sixteen rows, and L1 was busy 59 % of the time
+// with that.  In planes (PL) a request is one run and the tiles' places are scalar registers.  The up launch moves 300 MB at 3.4 TB/s; its
+// first 512 workgroups, two a CU, run at 4.9 and the other 256 alone on their CUs.  A second step of ids on its way, operands of X
+// a quarter of a step ahead, three workgroups a CU (80 registers) and non-temporal ids changed nothing or lost (88, 94, 121, 89 us).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <algorithm>
@@ -111,6 +113,7 @@ __device__ __forceinline__ void decode_centred(const uint4& lo, const uint4& hi,
 
 // a row tile of the wave: what a lane needs for its row (r = lane % 16)
 struct GroupRow {
+    const uint8_t* base;           // in planes: the next step of the tile
     uint64_t at;                   // byte of the first four dwords of the lane's slice of the next step
     uint32_t tail, stride;         // from there to its last four dwords; to the next step
     uint32_t negb;
@@ -118,7 +121,7 @@ struct GroupRow {
     bool sliced, ok;
 };
 
-template <int NT, bool DOWN, int XDT>
+template <int NT, bool DOWN, int XDT, bool PL>
 __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned char* smem, int e, int first, int n, int rb) {
     using L = GroupTile<NT, DOWN, XDT>;
     using F = Fmt<false>;
@@ -145,7 +148,13 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
     GroupRow g[2];
     int64_t off[2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) { g[t].nb = a.nbits[row_at + row0[t]]; off[t] = a.bit_off[row_at + row0[t]]; }
+    for (int t = 0; t < 2; ++t) {
+        // in planes: one width, and the tile's first row says where it is
+        const size_t at = PL ? (size_t)e * a.Q + row0[t] : row_at + row0[t];
+        g[t].nb = a.nbits[at];
+        off[t] = a.bit_off[at];
+        if constexpr (PL) g[t].nb = __builtin_amdgcn_readfirstlane(g[t].nb);
+    }
     // ---- the row this thread stages, its pair ----
     const int rho = tid / L::TPR, sub = tid % L::TPR;
     const bool stages = rho < 16 * NT;                         // (48 rows: a quarter of the threads has none)
@@ -194,7 +203,8 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
     // In operand order a request touches sixteen rows, a lane each.  With up to 16 pairs the lanes ask for chunk lane % 4 of row
     // lane / 4 instead, so that four neighbours read consecutive bytes, and the registers change lanes afterwards: 40 tokens of 128
     // experts 141.6 -> 134.2 us, 20 of 64 91.8 -> 84.5; with more pairs LDS has operands enough to serve: 509 tokens 209.5 -> 218.5.
-    constexpr bool kByRow = NT == 1;
+    // Tiles in planes: lane l asks for entry l, which is operand order and one contiguous run.
+    constexpr bool kByRow = NT == 1 && !PL;
     const int ask_row = kByRow ? lane >> 2 : r, ask_chunk = kByRow ? lane & 3 : kg, pull = 4 * (4 * r + kg);
     auto to_operand = [&](const uint4& v) __attribute__((always_inline)) -> uint4 {
         if constexpr (!kByRow) return v;
@@ -205,9 +215,10 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         GroupRow& q = g[t];
-        q.ok = !off_is_plane(off[t]) && row_in_bounds(off[t], q.nb, a.P, a.ids_bytes);        // stacks hold rows back to back only
+        q.ok = !off_is_plane(off[t]) && row_in_bounds(off[t], q.nb, PL ? (int64_t)16 * a.P : a.P, a.ids_bytes);
         const uint32_t nb = (uint32_t)q.nb;
         q.sliced = q.ok && nb >= 4 && nb <= 8 && (off[t] & 31) == 0;
+        if (PL) q.ok = q.sliced;
         // the row this lane asks for: its own, or the one of the lane that owns it
         uint64_t base = q.sliced ? (uint64_t)(off[t] >> 3) : 0;
         uint32_t ask_nb = q.sliced ? nb : 0u;
@@ -216,18 +227,29 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
             base = (uint64_t)high << 32 | low;
             ask_nb = __shfl(ask_nb, ask_row, 64);
         }
-        if (ask_nb) { q.at = base + (uint32_t)ask_chunk * 4u * ask_nb; q.tail = 4u * (ask_nb - 4u); q.stride = 16u * ask_nb; }
+        if constexpr (PL) {                                    // the same for all lanes: kept in scalar registers
+            q.base = a.ids + (((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base));
+        }
+        else if (ask_nb) { q.at = base + (uint32_t)ask_chunk * 4u * ask_nb; q.tail = 4u * (ask_nb - 4u); q.stride = 16u * ask_nb; }
         else { q.at = 0; q.tail = 16; q.stride = 0; }
         const float zero = rintf(-a.min_s[row_at + row0[t]] / a.tau_s[row_at + row0[t]]);
         const int c = q.sliced ? (int)fminf(fmaxf(zero, 0.f), (float)((1 << q.nb) - 1)) : 0;          // (NaN: 0)
         q.centre = c;
         q.negb = pack_half2((_Float16)(float)(-1024 - c), (_Float16)(float)(-1024 - c));
         const int mine = q.sliced ? q.nb : 0, lead = __builtin_amdgcn_readfirstlane(mine);
-        q.mode = __builtin_amdgcn_ballot_w64(mine != lead) == 0 ? lead : 0;
+        q.mode = PL || __builtin_amdgcn_ballot_w64(mine != lead) == 0 ? lead : 0;
     }
     auto issue = [&](bool last) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
+            if constexpr (PL) {
+                // (a tile outside the buffer reads the buffer's first bytes)
+                const uint32_t nb = g[t].ok ? (uint32_t)g[t].nb : 4u;
+                lo[t] = *reinterpret_cast<const uint4*>(g[t].base + (g[t].ok ? (uint32_t)lane * 16u : 0u));
+                hi[t] = *reinterpret_cast<const uint4*>(g[t].base + (g[t].ok ? 1008u + (uint32_t)(lane + 1) * (4u * (nb - 4u)) : 0u));
+                g[t].base += last || !g[t].ok ? 0u : 256u * nb;
+                continue;
+            }
             lo[t] = *reinterpret_cast<const uint4*>(a.ids + g[t].at);
             hi[t] = *reinterpret_cast<const uint4*>(a.ids + g[t].at + g[t].tail);
             g[t].at += last ? 0u : g[t].stride;                // past the end: the last step's lines again, nothing under a branch
@@ -282,6 +304,7 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
                 default:
 #pragma unroll
                     for (int j = 0; j < 4; ++j) b[t][j] = v4u_t{0u, 0u, 0u, 0u};
+                    if constexpr (PL) break;
                     if (q.sliced && q.nb == 4) decode_centred<4>(l, h, q.negb, b[t]);
                     if (q.sliced && q.nb == 5) decode_centred<5>(l, h, q.negb, b[t]);
                     if (q.sliced && q.nb == 6) decode_centred<6>(l, h, q.negb, b[t]);
@@ -319,6 +342,7 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
 
     // ---- rows the slicing cannot read (width outside 4..8, not dword aligned): id by id, in place of what stands there ----
     const int64_t clamp_byte = (a.ids_bytes - 8) & ~(int64_t)3;
+    if constexpr (!PL)
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         uint64_t odd = __builtin_amdgcn_ballot_w64(kg == 0 && !g[t].sliced && g[t].ok);
@@ -383,7 +407,7 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
         }
 }
 
-template <bool DOWN, int XDT>
+template <bool DOWN, int XDT, bool PL>
 __global__ void __launch_bounds__(kGroupThreads, 4) moe_group_kernel(MoeGroupArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     // workgroup b runs on XCD b % 8: an item's row blocks follow each other on ONE XCD, whose L2 then serves its
@@ -404,18 +428,22 @@ __global__ void __launch_bounds__(kGroupThreads, 4) moe_group_kernel(MoeGroupArg
     const int n = __builtin_amdgcn_readfirstlane(min(kGroupTokens, slot.z - first));
     const int e = __builtin_amdgcn_readfirstlane(slot.x);
     switch ((n + 15) / 16) {
-        case 1: moe_group_body<1, DOWN, XDT>(a, smem, e, first, n, rb); break;
-        case 2: moe_group_body<2, DOWN, XDT>(a, smem, e, first, n, rb); break;
-        case 3: moe_group_body<3, DOWN, XDT>(a, smem, e, first, n, rb); break;
-        default: moe_group_body<4, DOWN, XDT>(a, smem, e, first, n, rb); break;
+        case 1: moe_group_body<1, DOWN, XDT, PL>(a, smem, e, first, n, rb); break;
+        case 2: moe_group_body<2, DOWN, XDT, PL>(a, smem, e, first, n, rb); break;
+        case 3: moe_group_body<3, DOWN, XDT, PL>(a, smem, e, first, n, rb); break;
+        default: moe_group_body<4, DOWN, XDT, PL>(a, smem, e, first, n, rb); break;
     }
 }
 
+template <bool DOWN, int XDT, bool PL>
+int launch_stored(const MoeGroupArgs& a, unsigned blocks, hipStream_t s) {
+    if (int rc = host::raise_lds_limit<moe_group_kernel<DOWN, XDT, PL>>(kGroupLds, "qvb8_moe_experts")) return rc;
+    hipLaunchKernelGGL((moe_group_kernel<DOWN, XDT, PL>), dim3(blocks), dim3(kGroupThreads), kGroupLds, s, a);
+    return host::check_launch("qvb8_moe_experts");
+}
 template <bool DOWN, int XDT>
 int launch_as(const MoeGroupArgs& a, unsigned blocks, hipStream_t s) {
-    if (int rc = host::raise_lds_limit<moe_group_kernel<DOWN, XDT>>(kGroupLds, "qvb8_moe_experts")) return rc;
-    hipLaunchKernelGGL((moe_group_kernel<DOWN, XDT>), dim3(blocks), dim3(kGroupThreads), kGroupLds, s, a);
-    return host::check_launch("qvb8_moe_experts");
+    return a.planes ? launch_stored<DOWN, XDT, true>(a, blocks, s) : launch_stored<DOWN, XDT, false>(a, blocks, s);
 }
 
 }  // namespace

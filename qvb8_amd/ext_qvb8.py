@@ -629,6 +629,7 @@ def _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids
 
 
 MOE_UP_REGULAR, MOE_DOWN_REGULAR = 0x100, 0x200      # qvb8_moe_act flags: one width per stack, rows at regular places
+MOE_UP_PLANES, MOE_DOWN_PLANES = 0x800, 0x1000       # ... and every 16-row tile stored in planes
 MOE_KEEP_INF = 0x400                                 # ... an infinity among fp16 activations stays one (more than 16 tokens)
 
 
@@ -643,14 +644,29 @@ def stack_is_regular(nbits, bit_off, P) -> bool:
     return bool((nbits == nbits.reshape(-1)[0]).all() & (bit_off == want).all())
 
 
+def stack_in_planes(ids, bit_off, P, w) -> None:
+    """Stores every 16-row tile of a regular stack of width w (4..8, P a multiple of 128) in planes, in place: `bit_off`, (experts, Q), stays
+    what it is for rows back to back."""
+    Q, dwords = bit_off.shape[1], int(P) * int(w) // 2                     # of a tile
+    to_planes, to_native = _plane_index(int(P), int(w), ids.device)
+    source = torch.empty_like(to_planes)
+    source[to_planes] = to_native
+    for first in (bit_off[:, 0] // 8).tolist():
+        tiles = ids[first:first + Q // 16 * dwords * 4].view(torch.int32).view(-1, dwords)
+        for k in range(0, tiles.shape[0], 256):                            # bounded temporaries
+            tiles[k:k + 256] = tiles[k:k + 256][:, source]
+
+
 def moe_experts(X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn,
-                regular=(False, False), keep_inf=False, checked=False):
+                regular=(False, False), keep_inf=False, checked=False, planes=(False, False)):
     """Routed gated-SiLU expert stack on the stacked layout (reference: qvb8_cuda.cu:937-992); returns (tokens, Qdn)
-    in X's dtype.  `regular` = (up, down): the caller states that the stack is regular (stack_is_regular).  `keep_inf`: fp16
+    in X's dtype.  `regular` = (up, down): the caller states that the stack is regular (stack_is_regular); `planes`: and that its tiles are
+    stored in planes (stack_in_planes).  `keep_inf`: fp16
     activations beyond 16 tokens are taken as they are, infinities too (else they become +-65504).  `checked` (17 tokens
     or more): the host waits for the routing plan, not for the products, and gets None where an entry lies outside the
     stack (else such an entry makes the whole result NaN)."""
-    act = 0 | (MOE_UP_REGULAR if regular[0] else 0) | (MOE_DOWN_REGULAR if regular[1] else 0) | (MOE_KEEP_INF if keep_inf else 0)
+    act = 0 | (MOE_UP_REGULAR if regular[0] else 0) | (MOE_DOWN_REGULAR if regular[1] else 0) | (MOE_KEEP_INF if keep_inf else 0) \
+        | (MOE_UP_PLANES if planes[0] else 0) | (MOE_DOWN_PLANES if planes[1] else 0)
     return _moe(act, X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn, checked)
 
 
