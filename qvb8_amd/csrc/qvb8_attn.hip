@@ -23,7 +23,10 @@
 //   * the softmax is computed once per workgroup (wave w rows 4 w .. 4 w + 3, sixteen lanes a row, two keys a lane, row
 //     maxima and sums by data-parallel rotations inside the row); the probabilities, rounded to fp16, and the rows'
 //     rescale factors reach the four waves through LDS in the A-operand layout of the second product;
-//   * O += P V: wave w owns a quarter of the output channels.
+//   * O += P V: wave w owns a quarter of the output channels, its operands asked for ahead of the softmax.
+// A workgroup has few tiles (6 of 1024 for one token over 32768 keys), so its start counts: the tile table, then ids, queries and the
+// first segment's constants in one trip.  With the queries loaded before, each waited for, and the operands of either product two at a
+// time: 27.4 us a call, 26.7 now.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <algorithm>
@@ -56,27 +59,41 @@ struct AttnArgs {
     float scale;
 };
 
-// Four neighbouring channels of one query, at element offset `at`.  What is not ready is multiplied by the softmax scale, then
+// N x four channels of one query, 16 apart, from element offset `at`.  What is not ready is multiplied by the softmax scale, then
 // clamped to fp16's finite range and rounded -- in this order, so that an outlier channel does not become an infinity.  Done by
 // the row-block kernel where it reads its queries, 16 or 32 rows a workgroup; the kernel of many rows takes them ready (every one of its
 // splits would prepare them again: 120 tokens over 16001 keys 118.3 us that way, 112.1 with a launch that does it once).
+// All N requests stand together under one choice of type: with a choice per request every one was waited for before the next.
 constexpr int kQReady = -1;
-__device__ __forceinline__ h4_t load_query(const AttnArgs& a, int64_t at) {
-    if (a.q_dt == kQReady) return *reinterpret_cast<const h4_t*>(reinterpret_cast<const uint16_t*>(a.q) + at);
-    float v[4];
+template <int N>
+__device__ __forceinline__ void load_query(const AttnArgs& a, int64_t at, h4_t (&q)[N]) {
+    auto narrow = [&](const float (&v)[4]) __attribute__((always_inline)) {
+        uint32_t h[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) h[k] = sat_half_bits(v[k] * a.q_scale);
+        return __builtin_bit_cast(h4_t, uint2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)});
+    };
     if (a.q_dt == QVB8_F32) {
-        const float4 f = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(a.q) + at);
-        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
-    } else {
-        const uint2 w = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(a.q) + at);
-        const uint32_t u[4] = {w.x & 0xFFFFu, w.x >> 16, w.y & 0xFFFFu, w.y >> 16};
+        float4 f[N];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = a.q_dt == QVB8_F16 ? f16_bits_to_f32(u[k]) : bf16_bits_to_f32(u[k]);
+        for (int i = 0; i < N; ++i) f[i] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(a.q) + at + 16 * i);
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = narrow({f[i].x, f[i].y, f[i].z, f[i].w});
+        return;
     }
-    uint32_t h[4];
+    uint2 w[N];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) h[k] = sat_half_bits(v[k] * a.q_scale);
-    return __builtin_bit_cast(h4_t, uint2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)});
+    for (int i = 0; i < N; ++i) w[i] = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(a.q) + at + 16 * i);
+    if (a.q_dt == kQReady) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = __builtin_bit_cast(h4_t, w[i]);
+    } else if (a.q_dt == QVB8_F16) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = narrow({f16_bits_to_f32(w[i].x & 0xFFFFu), f16_bits_to_f32(w[i].x >> 16), f16_bits_to_f32(w[i].y & 0xFFFFu), f16_bits_to_f32(w[i].y >> 16)});
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = narrow({bf16_bits_to_f32(w[i].x & 0xFFFFu), bf16_bits_to_f32(w[i].x >> 16), bf16_bits_to_f32(w[i].y & 0xFFFFu), bf16_bits_to_f32(w[i].y >> 16)});
+    }
 }
 
 // Four neighbouring channels of one key, as they lie in memory.
@@ -155,18 +172,17 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
 
     // the lane's query rows (one per block) as the A operand of S = Q K^T: Q[row][16 ks + 4 kg .. + 3], ks in the wave's half
     h4_t qa[RB][NKS];
+    auto queries = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-        const int row = row0 + rb * kRows + n16;
-        const bool row_ok = row < a.n_rows;
-        const int rr = row_ok ? row : 0;
-        const int64_t qp = (int64_t)(rr / a.G) * a.sq_r + (int64_t)(h * a.G + rr % a.G) * a.sq_h + dh * (D / 2) + 4 * kg;
+        for (int rb = 0; rb < RB; ++rb) {
+            const int row = row0 + rb * kRows + n16;
+            const bool row_ok = row < a.n_rows;
+            const int rr = row_ok ? row : 0;
+            load_query<NKS>(a, (int64_t)(rr / a.G) * a.sq_r + (int64_t)(h * a.G + rr % a.G) * a.sq_h + dh * (D / 2) + 4 * kg, qa[rb]);
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const h4_t v = load_query(a, qp + 16 * ks);
-            qa[rb][ks] = row_ok ? v : h4_t{0, 0, 0, 0};
+            for (int ks = 0; ks < NKS; ++ks) qa[rb][ks] = row_ok ? qa[rb][ks] : h4_t{0, 0, 0, 0};
         }
-    }
+    };
     const int qmin = a.q_pos0 + row0 / a.G;                                   // first position of the block's rows
     // the softmax's own split of the block: this lane's row and pair of keys
     const int srow = 4 * wave + (lane >> 4), kpair = lane & 15;             // row within a block
@@ -215,23 +231,27 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
 
     int cur_seg = -1;
     float km[4] = {0.f, 0.f, 0.f, 0.f}, ks_[4] = {0.f, 0.f, 0.f, 0.f}, vm[4] = {0.f, 0.f, 0.f, 0.f}, vs_[4] = {0.f, 0.f, 0.f, 0.f}, kc = 0.f, vc = 0.f;
+    // a segment's constants for this thread's four channels
+    auto constants = [&](int seg) __attribute__((always_inline)) {
+        const int64_t pb = ((int64_t)seg * a.nhkv + h) * D + 4 * cg;
+        const float4 kmid = *reinterpret_cast<const float4*>(a.kmid + pb), kstep = *reinterpret_cast<const float4*>(a.kstep + pb);
+        const float4 vmid = *reinterpret_cast<const float4*>(a.vmid + pb), vstep = *reinterpret_cast<const float4*>(a.vstep + pb);
+        kc = a.kc[seg * a.nhkv + h]; vc = a.vc[seg * a.nhkv + h];
+        km[0] = kmid.x; km[1] = kmid.y; km[2] = kmid.z; km[3] = kmid.w;
+        ks_[0] = kstep.x; ks_[1] = kstep.y; ks_[2] = kstep.z; ks_[3] = kstep.w;
+        vm[0] = vmid.x; vm[1] = vmid.y; vm[2] = vmid.z; vm[3] = vmid.w;
+        vs_[0] = vstep.x; vs_[1] = vstep.y; vs_[2] = vstep.z; vs_[3] = vstep.w;
+        cur_seg = seg;
+    };
     // One tile: restore the ids of register set (rk, rv) into LDS, refill the set with tile t + 2, S, softmax, O.
     auto tile = [&](int t, U (&rk)[UNITS][4], U (&rv)[UNITS][4], TileRef& ref) {
         const int start = ref.start, nlen = ref.ok ? ref.nlen : 0, seg = ref.seg;      // a tile that is not wanted: no key counts
         if (seg != cur_seg) {
-            // A new segment (every few thousand keys): its constants for this thread's four channels.  The wait stands
-            // INSIDE the branch: the requests of the next tiles' ids are older than these, and a wait placed where the
-            // constants are first used would hold every tile until its successors' ids had arrived.
-            const int64_t pb = ((int64_t)seg * a.nhkv + h) * D + 4 * cg;
-            const float4 kmid = *reinterpret_cast<const float4*>(a.kmid + pb), kstep = *reinterpret_cast<const float4*>(a.kstep + pb);
-            const float4 vmid = *reinterpret_cast<const float4*>(a.vmid + pb), vstep = *reinterpret_cast<const float4*>(a.vstep + pb);
-            kc = a.kc[seg * a.nhkv + h]; vc = a.vc[seg * a.nhkv + h];
-            km[0] = kmid.x; km[1] = kmid.y; km[2] = kmid.z; km[3] = kmid.w;
-            ks_[0] = kstep.x; ks_[1] = kstep.y; ks_[2] = kstep.z; ks_[3] = kstep.w;
-            vm[0] = vmid.x; vm[1] = vmid.y; vm[2] = vmid.z; vm[3] = vmid.w;
-            vs_[0] = vstep.x; vs_[1] = vstep.y; vs_[2] = vstep.z; vs_[3] = vstep.w;
+            // A new segment (every few thousand keys).  The wait stands INSIDE the branch: the requests of the next tiles' ids are
+            // older than these, and a wait placed where the constants are first used would hold every tile until its successors'
+            // ids had arrived.
+            constants(seg);
             __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0)
-            cur_seg = seg;
         }
         // Keys past the tile's length hold a copy of its last key: their scores are replaced by -inf before any use, so K
         // needs no blanking; their V must be zero (0 * inf would poison the sums), done on the packed halves.
@@ -276,12 +296,14 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) sc[rb] = f4_t{0.f, 0.f, 0.f, 0.f};
             const _Float16* kp = Ks + (16 * kf + n16) * KROW + dh * (D / 2) + 4 * kg;
+            h4_t kb[NKS];                                         // all asked for before the first product
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-                const h4_t kb = *reinterpret_cast<const h4_t*>(kp + 16 * ks);
+            for (int ks = 0; ks < NKS; ++ks) kb[ks] = *reinterpret_cast<const h4_t*>(kp + 16 * ks);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int rb = 0; rb < RB; ++rb) sc[rb] = __builtin_amdgcn_mfma_f32_16x16x16f16(qa[rb][ks], kb, sc[rb], 0, 0, 0);
-            }
+            for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) sc[rb] = __builtin_amdgcn_mfma_f32_16x16x16f16(qa[rb][ks], kb[ks], sc[rb], 0, 0, 0);
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -291,6 +313,7 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
 
         // ---- softmax, once per workgroup: wave w takes rows 4 w .. 4 w + 3 of every block, sixteen lanes a row, two keys
         //      a lane; the probabilities (fp16) and the rows' rescale factors go to LDS for all four waves ----
+        h4_t vb[2][NF];                                   // the second product's operands: here when the softmax is done
         {
             // every key of the tile counts for every row of the workgroup (rows past n_rows compute on zeros, never stored)
             const bool all_seen = nlen == kKeys && start + kKeys - 1 <= qmin;
@@ -301,6 +324,17 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
                 const int sqpos = a.q_pos0 + (srow_ok ? (row0 + prow) / a.G : 0);
                 const float2 sa = *reinterpret_cast<const float2*>(Ss + ((2 * rb) * kRows + srow) * kSStride + 2 * kpair);
                 const float2 sb = *reinterpret_cast<const float2*>(Ss + ((2 * rb + 1) * kRows + srow) * kSStride + 2 * kpair);
+                if (rb == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                        for (int f = 0; f < NF; ++f) {
+                            const int ch = wave * (D / 4) + 16 * f + n16;
+                            vb[kk][f] = *reinterpret_cast<const h4_t*>(Vt + ch * kKeys + 4 * ((4 * kk + kg) ^ ((ch >> 2) & 7)));
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 const bool ok0 = all_seen || (srow_ok && 2 * kpair < nlen && start + 2 * kpair <= sqpos);
                 const bool ok1 = all_seen || (srow_ok && 2 * kpair + 1 < nlen && start + 2 * kpair + 1 <= sqpos);
                 const float sv0 = ok0 ? (sa.x + sb.x) * a.scale : -INFINITY, sv1 = ok1 ? (sa.y + sb.y) * a.scale : -INFINITY;
@@ -337,12 +371,9 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-            for (int f = 0; f < NF; ++f) {
-                const int ch = wave * (D / 4) + 16 * f + n16;
-                const h4_t b = *reinterpret_cast<const h4_t*>(Vt + ch * kKeys + 4 * ((4 * kk + kg) ^ ((ch >> 2) & 7)));
+            for (int f = 0; f < NF; ++f)
 #pragma unroll
-                for (int rb = 0; rb < RB; ++rb) acc[rb][f] = __builtin_amdgcn_mfma_f32_16x16x16f16(pa[rb][kk], b, acc[rb][f], 0, 0, 0);
-            }
+                for (int rb = 0; rb < RB; ++rb) acc[rb][f] = __builtin_amdgcn_mfma_f32_16x16x16f16(pa[rb][kk], vb[kk][f], acc[rb][f], 0, 0, 0);
         __syncthreads();                                  // the tile in LDS is free again
     };
 
@@ -353,6 +384,9 @@ __global__ __launch_bounds__(kAttnThreads, ((D == 256 && sizeof(T) == 2) || RB >
         __builtin_amdgcn_sched_barrier(0);                 // set 0 is the older one, as in every later round of the loop
         fetch(t0 + 1, rk1, rv1, ref1);
         __builtin_amdgcn_sched_barrier(0);
+        // queries and the first segment's constants travel with the first ids: one trip to memory where there were ten
+        constants(ref0.seg);
+        queries();
         // The loop has one way out, at its head, and takes tiles in pairs; when the last pair has no second tile, that
         // one is run as an empty tile (no key counts: nothing changes).  A way out of the middle would be turned into a
         // path through the loop's end back to its head, on which set 0 is the younger one, and the compiler would make
@@ -434,6 +468,9 @@ __global__ __launch_bounds__(64 * NW, (D == 256 && sizeof(T) == 2) ? 1 : 2) void
     constexpr int CG = D / 4;                  // channel groups (four channels each) of a key
     constexpr int kWideRows = NW * kWaveRows;
     constexpr bool kAskEarly = D == 128 && NW == 8;           // the ids of tile t + 2 before the products of tile t, where registers allow it
+    // operands of a product on their way from LDS, as many as registers hold without a spill (one at a time: 720 rows x 4 heads over
+    // 16001 keys 98.9 .. 99.9 us a call, 95.3 .. 97.6 this way)
+    constexpr int kAhead = NW == 8 ? 6 : 4;
     constexpr int KPT = kKeys * CG / (64 * NW);               // consecutive keys a thread restores: 32 (D = 256) or 16 over the waves
     constexpr int KROW = krow_wide(D), NKS = D / 16, NF = D / 32, NFC = NF / 4;
     using QD = Quad<T>;
@@ -563,9 +600,16 @@ __global__ __launch_bounds__(64 * NW, (D == 256 && sizeof(T) == 2) ? 1 : 2) void
         const int ln = lane_now(), half8 = 8 * (ln >> 5);
         const int key = (ln & 19) | ((ln & 4) << 1) | ((ln & 8) >> 1);                   // A row ln % 32 of S^T is this key of the tile
         const _Float16* const ka = Ks + (buf * kKeys + key) * KROW + half8;
+        h8_t k[kAhead];
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks)
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t*>(ka + 16 * ks), qb[ks], s, 0, 0, 0);
+        for (int i = 0; i < kAhead; ++i) k[i] = *reinterpret_cast<const h8_t*>(ka + 16 * i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k[ks % kAhead], qb[ks], s, 0, 0, 0);
+            if (ks + kAhead < NKS) k[ks % kAhead] = *reinterpret_cast<const h8_t*>(ka + 16 * (ks + kAhead));
+            __builtin_amdgcn_sched_barrier(0);
+        }
         float times = to_log2;                                // > 0: multiplied in the exponent's subtraction, below
         if (!(times > 0.f)) {
 #pragma unroll
@@ -603,11 +647,17 @@ __global__ __launch_bounds__(64 * NW, (D == 256 && sizeof(T) == 2) ? 1 : 2) void
     auto values = [&](int buf, const h8_t (&p)[2]) __attribute__((always_inline)) {
         const int ln = lane_now();
         const _Float16* const va = Vt + (buf * D + (ln & 31)) * kVRow + 8 * (ln >> 5);
+        auto operand = [&](int i) __attribute__((always_inline)) { return *reinterpret_cast<const h8_t*>(va + 32 * (i % NF) * kVRow + 16 * (i / NF)); };
+        h8_t v[kAhead];
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
+        for (int i = 0; i < kAhead; ++i) v[i] = operand(i);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int f = 0; f < NF; ++f)
-                acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t*>(va + 32 * f * kVRow + 16 * k), p[k], acc[f], 0, 0, 0);
+        for (int i = 0; i < 2 * NF; ++i) {
+            acc[i % NF] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[i % kAhead], p[i / NF], acc[i % NF], 0, 0, 0);
+            if (i + kAhead < 2 * NF) v[i % kAhead] = operand(i + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
 
     if (t0 < t1) {
