@@ -33,6 +33,8 @@ constexpr int kRTiles = 8;             // tiles per workgroup (two per wave)
 constexpr int kRThreads = 32 * kRTiles;
 constexpr int kRing = 256;             // 32-bit words of a tile's window in LDS
 constexpr int kHalfRing = kRing / 2;
+constexpr uint32_t kSymMask = 2047u;   // a symbol's bits in an entry of the slot table
+constexpr int kFurthestWord = 0x7fffff00;
 
 struct RCore {
     const uint32_t* words; int64_t n_words;      // stream + at least 2048 zero words of pad (n_words counts the pad)
@@ -49,7 +51,7 @@ struct RCore {
 // The walk of one tile.  Its words lie in a window of LDS that does not wrap: word `ptr` of the window is the next one to be
 // taken, and its address is its index and nothing else.  When half the window has been used, the other half moves to the front
 // and the next 128 words, asked for half a window ago, follow from registers.
-// A half without a tile or row walks along with the wave's other half on what it holds (never past `room`).
+// A half without a tile or row walks along with the wave's other half on what it holds (never past `last_at`).
 struct Walker {
     uint32_t xl, xh;
     int ptr;                           // next word of the window, counted from the wave's first one
@@ -61,17 +63,19 @@ struct Walker {
 
 // Per-workgroup set-up shared by the kernels: slot table into LDS, this half-wave's tile.
 //
-// `room` is the last word index (from the tile's first word) the walk may read ahead to: the end of the buffer, and -- when
-// the next tile's words follow this tile's, as every writer lays them out -- the tile's own last word.  The window always
-// asks for 128..384 words more than the walk has used; past the tile's end those lines belong to a tile that another
-// workgroup walks at another time, so they came from memory twice (measured at the 65B shapes, one row per tile of 1150
-// words: 325 MB fetched for 267 MB of stream).  Requests past the bound read the bound's word again.
+// A tile's words are asked for 128 at a time, the last time where its last word is (`last_at`, from the tile's first word; a tile whose
+// end is not known -- the next tile's words do not follow, as every writer lays them out -- ends with the buffer); later requests ask
+// for the same again.  Without that end a walk reads 128..384 words more than it uses, lines of a tile that another workgroup walks at another
+// time (65B shapes, one row per tile of 1150 words: 325 MB fetched for 267 MB of stream).  One clamp a request: clamped word by
+// word, in 64 bits, the windows took 25 vector instructions each time instead of 5, a twelfth of the walk's.
 //
 // A workgroup's start is a chain of trips to memory: its block, then the tile's place, then its first words; the slot table's 16
 // KB are asked for between the last two, all of them at once (a loop that waits for every 1 KB of them took longer than a fifth
 // of a short launch: 17408 x 5120, one row of X, 61.1 us a call with it, 55.0 without).
-struct TileCtx { bool has; int tile, r0, nr; int64_t room; };
-__device__ __forceinline__ TileCtx block_setup(Walker& z, const RCore& c, int block, uint32_t* st, uint32_t* own, int h8, int l32) {
+struct TileCtx { bool has; int tile, r0, nr; int last_at; };
+constexpr int kTabPerThread = 4096 / kRThreads;
+struct BlockWords { uint32_t entry[kTabPerThread], first[kRing / 32]; };
+__device__ __forceinline__ TileCtx block_request(Walker& z, BlockWords& b, const RCore& c, int block, int h8, int l32) {
     int cls = c.blocks[3 * block], tb = c.blocks[3 * block + 1], ntb = c.blocks[3 * block + 2];
     cls = cls < 0 ? 0 : (cls >= c.K ? c.K - 1 : cls);
     TileCtx t;
@@ -83,39 +87,45 @@ __device__ __forceinline__ TileCtx block_setup(Walker& z, const RCore& c, int bl
     const uint64_t s = c.states[(int64_t)t.tile * 32 + l32];
     t.r0 = (int)c.tiles[3 * (int64_t)t.tile + 1];
     t.nr = (int)c.tiles[3 * (int64_t)t.tile + 2];
-    constexpr int kPer = 4096 / kRThreads;
-    uint32_t E[kPer];
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) E[k] = c.tab[(int64_t)cls * 4096 + k * kRThreads + (int)threadIdx.x];
+    for (int k = 0; k < kTabPerThread; ++k) b.entry[k] = c.tab[(int64_t)cls * 4096 + k * kRThreads + (int)threadIdx.x];
     __builtin_amdgcn_sched_barrier(0);
 
     const int64_t last = c.n_words - (kRing + kHalfRing);                  // the furthest start that keeps every read inside
     off = off < 0 ? 0 : (off > last ? last : off);
     z.wp = c.words + off;
-    t.room = c.n_words - 1 - off;
-    if (next > off && next - off - 1 < t.room) t.room = next - off - 1;
+    int64_t room = c.n_words - 1 - off;
+    if (next > off && next - off - 1 < room) room = next - off - 1;
+    // (never further than a request of 128 words stays inside the buffer; 64 bits of index are for the buffer, not for one tile)
+    int64_t last_at = room & ~(int64_t)(kHalfRing - 1);
+    if (last_at > c.n_words - off - kHalfRing) last_at = c.n_words - off - kHalfRing;
+    t.last_at = (int)(last_at < kFurthestWord ? last_at : kFurthestWord);
     z.xl = (uint32_t)s; z.xh = (uint32_t)(s >> 32);
     z.sb = 0;
     z.upper = (threadIdx.x & 32) ? 0xffffffffu : 0u; z.ptr = (int)(z.upper & kRing);
-    uint32_t first[kRing / 32];
 #pragma unroll
-    for (int q = 0; q < kRing / 32; ++q) { const int64_t i = 32 * q + l32; first[q] = z.wp[i < t.room ? i : t.room]; }
+    for (int k = 0; k < 3; ++k) {
+        const uint32_t* const from = z.wp + (uint64_t)(uint32_t)(min(k * kHalfRing, t.last_at) + l32);
 #pragma unroll
-    for (int q = 0; q < kHalfRing / 32; ++q) { const int64_t i = kRing + 32 * q + l32; z.pre[q] = z.wp[i < t.room ? i : t.room]; }
+        for (int q = 0; q < kHalfRing / 32; ++q) (k < 2 ? b.first[4 * k + q] : z.pre[q]) = from[32 * q];
+    }
     __builtin_amdgcn_sched_barrier(0);
-    // the file's entry is (frequency - 1) << 22 | (slot - cumulative) << 11 | symbol with frequency <= 1024; the walk wants
-    // the frequency itself, one instruction per symbol less
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) st[k * kRThreads + threadIdx.x] = (((E[k] >> 22) + 1u) << 21) | (E[k] & 0x1FFFFFu);
-#pragma unroll
-    for (int q = 0; q < kRing / 32; ++q) own[32 * q + l32] = first[q];
     if (!t.has) t.nr = 0;
     if (t.r0 < 0 || t.r0 + t.nr > c.Q) { t.nr = 0; t.has = false; }
     return t;
 }
+// What was requested goes to LDS.  The file's entry is (frequency - 1) << 22 | (slot - cumulative) << 11 | symbol with frequency <=
+// 1024; the walk wants the frequency itself, one instruction per symbol less.  `least` (no symbol is smaller) is taken off the symbols.
+__device__ __forceinline__ void block_fill(const BlockWords& b, uint32_t* st, uint32_t* own, int l32, uint32_t least = 0u) {
+#pragma unroll
+    for (int k = 0; k < kTabPerThread; ++k) st[k * kRThreads + threadIdx.x] = ((((b.entry[k] >> 22) + 1u) << 21) | (b.entry[k] & 0x1FFFFFu)) - least;
+#pragma unroll
+    for (int q = 0; q < kRing / 32; ++q) own[32 * q + l32] = b.first[q];
+    __syncthreads();
+}
 
 // one symbol: x' = f * (x >> 12) + d on the 64-bit state; the entry comes back with the symbol in its low 11 bits
-// `st` holds the slot table re-packed for the walk (block_setup): frequency << 21 | (slot - cumulative) << 11 | symbol.
+// `st` holds the slot table re-packed for the walk (block_fill): frequency << 21 | (slot - cumulative) << 11 | symbol.
 __device__ __forceinline__ uint32_t walk_dec(Walker& z, const uint32_t* st) {
     const uint32_t E = st[z.xl & 4095u];
     const uint32_t f = E >> 21, d = (E >> 11) & 1023u;
@@ -128,11 +138,13 @@ __device__ __forceinline__ uint32_t walk_dec(Walker& z, const uint32_t* st) {
 
 // Four symbols, a renormalisation after every second one; `rg` is the wave's first window.  A pair takes at most 32 words of a
 // tile, so with the windows looked after every second pair at least 64 of their 256 words are always ahead.
-// Bound by vector instructions: 42 a pair by the counters, besides 2.9 scalar and 3.6 of LDS, where a ring that wraps, looked after every
-// pair, with a branch around the words taken and the activations addressed per lane took 45, 12 and 3.5.  17408 x 5120, one row: 66.2 -> 50.4 us a call with the
-// shorter start above; 16 rows 88.1 -> 71.2; 5120 x 17408, one row 95.2 -> 70.0.  (The pointers as wave scalars, one bit count
-// over the whole wave: fewer vector instructions, a longer chain: the same.  Waves of different priority, fewer resident
-// workgroups: nothing and worse.)
+// Bound by vector instructions -- 34 a pair in the loop of one bf16 row (two of them, the 64-bit multiply-adds, count several times) --
+// and by the three dependent LDS lookups of a pair.  With a ring that wraps, looked after every pair, a branch around the words taken and the
+// activations addressed per lane: 66.2 us a call of 17408 x 5120, one row, 50.4 without and with the shorter start above; 16 rows 88.1 -> 71.2.  Then
+// 48.5 -> 45.9 by symbols that fit a byte, the half's bits picked by one instruction and one clamp per request of words; 5120 x
+// 17408, one row, 66.5 -> 62.1.  Nothing or slower: the pointers as wave scalars, one bit count over the whole wave; waves of different
+// priority; fewer resident workgroups; two tiles a half-wave, of two blocks that share the table (53.3); a 64-bit shift for both halves
+// of the state (the compiler splits it again).
 __device__ __forceinline__ void walk_pairs2(Walker& z, const uint32_t* st, const uint32_t* rg, uint32_t (&e)[4]) {
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
@@ -141,7 +153,9 @@ __device__ __forceinline__ void walk_pairs2(Walker& z, const uint32_t* st, const
         asm("" : "+v"(z.xh));                                              // a 32-bit comparison, not one of the whole state
         const bool need = z.xh == 0u;
         const uint64_t mk = __builtin_amdgcn_ballot_w64(need);
-        const uint32_t mine = z.upper ? (uint32_t)(mk >> 32) : (uint32_t)mk;
+        uint32_t mk_hi = (uint32_t)(mk >> 32);
+        asm("" : "+v"(mk_hi));
+        const uint32_t mine = __builtin_amdgcn_bitop3_b32(z.upper, mk_hi, (uint32_t)mk, 0xCA);         // upper ? high half : low half
         int at = __builtin_popcount(mine & ((1u << (threadIdx.x & 31)) - 1u)) + z.ptr;
         asm("" : "+v"(at));
         const uint32_t w = rg[at];
@@ -152,8 +166,9 @@ __device__ __forceinline__ void walk_pairs2(Walker& z, const uint32_t* st, const
 }
 // ... to be followed, before the next pairs, by a look at the windows (kept apart so that what the caller waits for in between is
 // not held up by words asked for here, which come from memory).
-// `room` = words the tile's stream may still be read ahead (clamps the read-ahead of a damaged stream inside the pad).
-__device__ __forceinline__ void walk_window(Walker& z, uint32_t* rg, int l32, int64_t room) {
+// `last_at` = where the last request of 128 words starts, counted from the tile's first (later ones ask for it again; this also keeps
+// the read-ahead of a damaged stream inside the pad).
+__device__ __forceinline__ void walk_window(Walker& z, uint32_t* rg, int l32, int last_at) {
     if (z.ptr >= (int)(z.upper & kRing) + kHalfRing) {
         z.ptr -= kHalfRing;
         z.sb += kHalfRing;
@@ -163,12 +178,10 @@ __device__ __forceinline__ void walk_window(Walker& z, uint32_t* rg, int l32, in
         for (int q = 0; q < kHalfRing / 32; ++q) up[q] = mine[kHalfRing + 32 * q];
 #pragma unroll
         for (int q = 0; q < kHalfRing / 32; ++q) { mine[32 * q] = up[q]; mine[kHalfRing + 32 * q] = z.pre[q]; }
-        const int64_t at = (int64_t)z.sb + kRing;
+        const uint32_t at = min((uint32_t)z.sb + kRing, (uint32_t)last_at) + (uint32_t)l32;
+        const uint32_t* const from = z.wp + (uint64_t)at;
 #pragma unroll
-        for (int q = 0; q < kHalfRing / 32; ++q) {
-            const int64_t i = at + 32 * q + l32;
-            z.pre[q] = z.wp[i < room ? i : room];
-        }
+        for (int q = 0; q < kHalfRing / 32; ++q) z.pre[q] = from[32 * q];
     }
 }
 // The words asked for last have arrived.  Said where a row starts: the compiler otherwise assumes at the head of a row's loop that
@@ -177,8 +190,6 @@ __device__ __forceinline__ void walk_settle(Walker& z) {
 #pragma unroll
     for (int q = 0; q < kHalfRing / 32; ++q) asm volatile("" : "+v"(z.pre[q]));
 }
-constexpr uint32_t kSymMask = 2047u;
-
 __device__ __forceinline__ float half_sum(float v) {                       // sum over the 32 lanes of a half, to every lane
     v = dpp_add<0xB1>(v);     // quad_perm [1,0,3,2]
     v = dpp_add<0x4E>(v);     // quad_perm [2,3,0,1]
@@ -205,8 +216,9 @@ __global__ void __launch_bounds__(kRThreads) r_decode_kernel(RCore c, int b0, in
     }
     uint32_t* rg = ring[2 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];          // of the wave's two tiles
     Walker z;
-    const TileCtx t = block_setup(z, c, block_no, st, ring[h8], h8, l32);
-    __syncthreads();
+    BlockWords words;
+    const TileCtx t = block_request(z, words, c, block_no, h8, l32);
+    block_fill(words, st, ring[h8], l32);
     const int S = c.P >> 5;
     for (int r = 0; r < T; ++r) {
         const bool active = t.has && r < t.nr;                             // per half-wave
@@ -231,7 +243,7 @@ __global__ void __launch_bounds__(kRThreads) r_decode_kernel(RCore c, int b0, in
                     else store_from_f32<DT>(out, i0 + 32 * k, __builtin_fmaf((float)id, ts, m));
                 }
             }
-            walk_window(z, rg, l32, t.room);
+            walk_window(z, rg, l32, t.last_at);
         }
     }
 }
@@ -246,58 +258,80 @@ __device__ __forceinline__ void store_y(void* Y, int y_dt, int64_t i, float v) {
 // ---- fused decode + product, one row of X ------------------------------------------------------------------------------
 // WALK_ONLY (a measurement aid, qvb8r_walk_probe): the same launch with the activations not read and the two multiply-adds
 // per pair replaced by an exclusive-or that keeps the symbols alive -- what the walk alone costs, the ceiling of this path.
-template <int DT, bool WALK_ONLY = false>
+// From as many weights per CU (rows of 1024 columns and more) the kernel looks for symbols that fit a byte: below, a launch is bound by the walk's
+// chain of lookups, not by its instructions, and the two barriers that takes show (us without / with: 1000 x 5120 16.6 / 16.8, 4096 x
+// 4096 16.0 / 16.1, 8192 x 2048 16.4 / 16.6, 17000 x 512 18.2 / 18.7; 8192 x 5120 27.2 / 26.4, 12288 x 4096 30.5 / 29.6, 5120 x 17408 66.5 / 62.1).
+constexpr int64_t kByteFrom = 1 << 17;
+template <int DT, bool BYTES, bool WALK_ONLY = false>
 __global__ void __launch_bounds__(kRThreads) r_gemv_kernel(RCore c, const void* __restrict__ X, void* __restrict__ Y, int y_dt, int T) {
     __shared__ uint32_t st[4096];
     __shared__ uint32_t ring[kRTiles][kRing];
-    const int lane = threadIdx.x & 63, l32 = lane & 31, h8 = threadIdx.x >> 5;
-    uint32_t* rg = ring[2 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];          // of the wave's two tiles
+    const int lane = threadIdx.x & 63, l32 = lane & 31, h8 = threadIdx.x >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t* rg = ring[2 * wave];                                         // of the wave's two tiles
     Walker z;
-    const TileCtx t = block_setup(z, c, blockIdx.x, st, ring[h8], h8, l32);
-    __syncthreads();
+    BlockWords words;
+    const TileCtx t = block_request(z, words, c, blockIdx.x, h8, l32);
+    // BYTES (16-bit activations): the class's least symbol is taken off all of them (it goes to the row's constant with the sum of x);
+    // where they fit a byte then, they are converted to fp32 where they lie, without a mask first: two instructions less per pair.
+    // fp32 rows keep products of whole symbols.
+    uint32_t least = 0u;
+    bool byte_symbols = false;
+    if constexpr (BYTES) {
+        uint32_t lo = kSymMask, hi = 0u;
+#pragma unroll
+        for (int k = 0; k < kTabPerThread; ++k) { lo = min(lo, words.entry[k] & kSymMask); hi = max(hi, words.entry[k] & kSymMask); }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) { lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64)); hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64)); }
+        if (lane == 0) { st[wave] = lo; st[4 + wave] = hi; }               // (where the table will be)
+        __syncthreads();
+        least = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(min(st[0], st[1]), min(st[2], st[3])));
+        byte_symbols = (uint32_t)__builtin_amdgcn_readfirstlane((int)max(max(st[4], st[5]), max(st[6], st[7]))) - least < 256u;
+        __syncthreads();
+    }
+    block_fill(words, st, ring[h8], l32, least);
     const int S = c.P >> 5;
-    float sx = 0.f;                  // sum of x over this lane's columns (the same for every row): taken while the first row is walked
-    // one row: the walk with two multiply-adds per pair; FIRST also adds the activations up (a second copy of the loop
-    // instead of a test per pair: the loop is bound by its instruction count)
-    auto walk_row = [&](auto first) __attribute__((always_inline)) {
+    float sx = 0.f;                  // sum of x over this lane's columns (the same for every row): taken while the first row is walked.  (By the
+                                     // workgroup before the walk: 49.3 us for 47.4; a quarter by each wave: nothing, and short rows lose.)
+    // one row: the walk with two multiply-adds per pair; FIRST also adds the activations up (copies of the loop instead of
+    // tests per pair: the loop is bound by its instruction count)
+    float acc = 0.f;
+    auto walk_row = [&](auto bytes, auto first) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first)::value;
-        if constexpr (WALK_ONLY) {
-            uint32_t keep = 0;
-            for (int s0 = 0; s0 < S; s0 += 4) {
-                uint32_t e[4];
+        constexpr uint32_t mask = decltype(bytes)::value ? 255u : kSymMask;
+        using Raw = std::conditional_t<DT == QVB8_F32, uint32_t, uint16_t>;
+        for (int s0 = 0; s0 < S; s0 += 4) {
+            uint32_t e[4];
+            if constexpr (WALK_ONLY) {
                 walk_pairs2(z, st, rg, e);
-                keep ^= (e[0] & kSymMask) + (e[1] & kSymMask);
-                keep ^= (e[2] & kSymMask) + (e[3] & kSymMask);
-                walk_window(z, rg, l32, t.room);
-            }
-            return (float)keep;
-        } else {
-            float acc = 0.f;
-            for (int s0 = 0; s0 < S; s0 += 4) {
+                uint32_t keep = __builtin_bit_cast(uint32_t, acc);
+                keep ^= (e[0] & mask) + (e[1] & mask);
+                keep ^= (e[2] & mask) + (e[3] & mask);
+                acc = __builtin_bit_cast(float, keep);
+            } else {
                 // columns 32 s0 + l32 ..: asked for ahead of the walk, there behind it
-                using Raw = std::conditional_t<DT == QVB8_F32, uint32_t, uint16_t>;
                 const Raw* base = reinterpret_cast<const Raw*>(X) + (size_t)s0 * 32;
                 Raw raw[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) raw[k] = base[(uint32_t)l32 + 32u * k];
                 __builtin_amdgcn_sched_barrier(0);
-                uint32_t e[4];
                 walk_pairs2(z, st, rg, e);
                 __builtin_amdgcn_sched_barrier(0);
                 float x[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     x[k] = DT == QVB8_F32 ? __builtin_bit_cast(float, (uint32_t)raw[k]) : DT == QVB8_F16 ? f16_bits_to_f32(raw[k]) : bf16_bits_to_f32(raw[k]);
-                    acc = __builtin_fmaf(x[k], (float)(e[k] & kSymMask), acc);
+                    acc = __builtin_fmaf(x[k], (float)(e[k] & mask), acc);
                 }
                 // (in pairs: added one by one, results of fp32 rows are 1 .. 11 % further from 64 bits)
                 if constexpr (FIRST) { sx += x[0] + x[1]; sx += x[2] + x[3]; }
                 asm volatile("" : "+v"(acc));                              // the activations are used up before words are asked for
-                walk_window(z, rg, l32, t.room);
             }
-            if constexpr (FIRST) sx = half_sum(sx);
-            return acc;
+            walk_window(z, rg, l32, t.last_at);
         }
+    };
+    auto walk = [&](auto first) __attribute__((always_inline)) {
+        if constexpr (BYTES) { if (byte_symbols) return walk_row(std::true_type{}, first); }
+        walk_row(std::false_type{}, first);
     };
     for (int r = 0; r < T; ++r) {
         const bool active = t.has && r < t.nr;                             // per half-wave
@@ -309,9 +343,16 @@ __global__ void __launch_bounds__(kRThreads) r_gemv_kernel(RCore c, const void* 
         const float m = c.min_s[at], ts = c.tau_s[at];
         const int dr = c.drow[at];
         walk_settle(z);
-        const float acc = r == 0 ? walk_row(std::true_type{}) : walk_row(std::false_type{});
+        acc = 0.f;
+        if (r == 0 && !WALK_ONLY) {
+            walk(std::true_type{});
+            sx = half_sum(sx);
+        } else {
+            walk(std::false_type{});
+        }
+        if constexpr (WALK_ONLY) acc = (float)__builtin_bit_cast(uint32_t, acc);
         const float a = half_sum(acc);
-        if (l32 == 0 && row_ok) store_y(Y, y_dt, orow, (float)((double)ts * ((double)a + (double)dr * (double)sx) + (double)m * (double)sx));
+        if (l32 == 0 && row_ok) store_y(Y, y_dt, orow, (float)((double)ts * ((double)a + (double)(dr + (int)least) * (double)sx) + (double)m * (double)sx));
     }
 }
 
@@ -412,8 +453,9 @@ __global__ void __launch_bounds__(kRThreads) r_mma_kernel(RCore c, RPacked xp, i
     }
     uint32_t* rg = ring[2 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];          // of the wave's two tiles
     Walker z;
-    const TileCtx t = block_setup(z, c, blockIdx.x, st, ring[h8], h8, l32);
-    __syncthreads();
+    BlockWords words;
+    const TileCtx t = block_request(z, words, c, blockIdx.x, h8, l32);
+    block_fill(words, st, ring[h8], l32);
     const int S = c.P >> 5;
     const int n_batches = (c.P + kRBatchCols - 1) / kRBatchCols;
     const int n16 = lane & 15, kg = lane >> 4;
@@ -446,7 +488,7 @@ __global__ void __launch_bounds__(kRThreads) r_mma_kernel(RCore c, RPacked xp, i
 #pragma unroll
                         for (int k = 0; k < 2; ++k)
                             out[k] = __builtin_amdgcn_perm(u16_to_half_bits(e[2 * k + 1] & kSymMask), u16_to_half_bits(e[2 * k] & kSymMask), 0x05040100u);
-                        walk_window(z, rg, l32, t.room);
+                        walk_window(z, rg, l32, t.last_at);
                     }
                     sb[p * 32] = out[0];
                     sb[(p + 1) * 32] = out[1];
@@ -590,7 +632,7 @@ extern "C" int qvb8r_walk_probe(const qvb8r_core* core, int64_t max_tile_rows, f
     if (max_tile_rows < 1 || max_tile_rows > 0x7fffffff) return host::fail(QVB8_ERR_ARG, "qvb8r_walk_probe: bad rows-per-tile bound");
     if (c.Q == 0 || c.n_blocks == 0) return QVB8_OK;
     if (!Y) return host::fail(QVB8_ERR_ARG, "qvb8r_walk_probe: null pointer");
-    hipLaunchKernelGGL((r_gemv_kernel<0, true>), dim3((unsigned)c.n_blocks), dim3(kRThreads), 0, (hipStream_t)stream, c, (const void*)Y, (void*)Y, QVB8_F32, (int)max_tile_rows);
+    hipLaunchKernelGGL((r_gemv_kernel<0, false, true>), dim3((unsigned)c.n_blocks), dim3(kRThreads), 0, (hipStream_t)stream, c, (const void*)Y, (void*)Y, QVB8_F32, (int)max_tile_rows);
     return host::check_launch("qvb8r_walk_probe");
 }
 
@@ -619,9 +661,12 @@ extern "C" int qvb8r_gemv_as(const void* X, int x_dtype, int64_t M, const qvb8r_
     dim3 grid((unsigned)c.n_blocks), block(kRThreads);
     const int T = (int)max_tile_rows;
     if (M == 1) {
-        if (x_dtype == QVB8_F32) hipLaunchKernelGGL(r_gemv_kernel<0>, grid, block, 0, s, c, X, Y, y_dtype, T);
-        else if (x_dtype == QVB8_F16) hipLaunchKernelGGL(r_gemv_kernel<1>, grid, block, 0, s, c, X, Y, y_dtype, T);
-        else hipLaunchKernelGGL(r_gemv_kernel<2>, grid, block, 0, s, c, X, Y, y_dtype, T);
+        const bool bytes = c.P >= 1024 && (int64_t)c.n_blocks * kRTiles * c.P >= kByteFrom * host::device_cus() / T;
+        if (x_dtype == QVB8_F32) hipLaunchKernelGGL((r_gemv_kernel<0, false>), grid, block, 0, s, c, X, Y, y_dtype, T);
+        else if (x_dtype == QVB8_F16 && bytes) hipLaunchKernelGGL((r_gemv_kernel<1, true>), grid, block, 0, s, c, X, Y, y_dtype, T);
+        else if (x_dtype == QVB8_F16) hipLaunchKernelGGL((r_gemv_kernel<1, false>), grid, block, 0, s, c, X, Y, y_dtype, T);
+        else if (bytes) hipLaunchKernelGGL((r_gemv_kernel<2, true>), grid, block, 0, s, c, X, Y, y_dtype, T);
+        else hipLaunchKernelGGL((r_gemv_kernel<2, false>), grid, block, 0, s, c, X, Y, y_dtype, T);
         return host::check_launch("qvb8r_gemv");
     }
     const int64_t need = qvb8r_gemv_workspace_bytes(M, c.P);

@@ -124,3 +124,27 @@ def test_sums_of_one_fp32_row_are_taken_in_pairs(P):
         room = 2.0 ** -50 * (np.abs(ts) * (abs(a) + np.abs(dr * b)) + np.abs(mn * b))
         lo, hi = ((ts * (a + dr * b) + mn * b + s * room).astype(np.float32) for s in (-1, 1))
         assert np.all((got >= np.minimum(lo, want)) & (got <= np.maximum(hi, want))), (P, seed)
+
+
+@pytest.mark.parametrize("levels", [6, 256, 257, 700])
+@pytest.mark.parametrize("Q,P,T", [(19, 640, 2), (3, 1024, 1), (70, 1152, 3), (9, 4224, 1)])
+def test_one_row_of_16_bits_and_symbols_around_a_byte(Q, P, T, levels):
+    """A large enough launch on rows of 1024 columns and more takes a class's least symbol off all of them and treats those that fit a byte
+    then apart.  Large by a schedule that lists its blocks over and over.  Bound: fp32 sums of P / 32 terms a lane, a tree over the lanes."""
+    g = torch.Generator().manual_seed(levels)
+    level = torch.randint(0, levels, (Q, P), generator=g)
+    level[:, 0], level[:, 1] = 0, levels - 1
+    W = (level.float() / levels).to(DEV)
+    lin = QVBandLinearV8R(RP.transcode(PK.encode_tensor(W, 0.5 / levels, keep_ids=True), rows_per_tile=T, n_classes=1), device=DEV)
+    core = list(lin._core())
+    ids = ext.ids(P, *core, T=lin.T).cpu().numpy().astype(np.float64)
+    ts, mn = (t.cpu().numpy().astype(np.float64) for t in (lin.tau_s, lin.min_s))
+    dense = mn[:, None] + ts[:, None] * ids
+    blocks, enough = core[4], 2 ** 17 * torch.cuda.get_device_properties(0).multi_processor_count // (8 * T * P) + 1
+    for dtype in (torch.float16, torch.bfloat16):
+        x = (torch.randn(1, P, generator=g) + 0.5).to(dtype).to(DEV)
+        xs = x.double().cpu().numpy()[0]
+        for core[4] in (blocks, blocks.repeat(-(-enough // blocks.shape[0]), 1)):
+            got = ext.multi(x, *core, T=lin.T).double().cpu().numpy()[0]
+            size = np.abs(xs).sum() * (ts * 2048.0 + np.abs(mn))
+            assert np.all(np.abs(got - dense @ xs) <= (P / 32 + 8) * 2.0 ** -24 * size + 2.0 ** -24 * np.abs(got)), (dtype, core[4].shape)
