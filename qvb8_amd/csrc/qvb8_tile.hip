@@ -1578,7 +1578,8 @@ GemmPlan plan_gemm_for(int64_t M, int64_t Q, int64_t P) { return M >= gemm2_from
 // projections, 8 layers: M = 17 0.641 ms against 0.721 for the tile kernel with two token tiles, M = 32 0.70 / 0.87)
 int gemm_from() { const int v = host::env_int("QVB8_MMA_GEMM_FROM", 17); return v < 17 ? 17 : (v > 49 ? 49 : v); }
 
-bool columns_take(int64_t M) { return M >= gemm_from() && M <= kColumnsMaxM && host::env_int("QVB8_COLUMNS", 1) != 0; }
+// (the sizes first: a call of a few rows, bound by the host, does not look at the environment for it)
+bool columns_take(int64_t M) { return M >= 17 && M <= kColumnsMaxM && M >= gemm_from() && host::env_int("QVB8_COLUMNS", 1) != 0; }
 
 template <int MT, bool BF, bool XC, int RT>
 int launch_gemm_as(const GemmArgs& a, const GemmPlan& g, int row_blocks, hipStream_t s) {
