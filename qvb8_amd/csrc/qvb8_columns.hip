@@ -327,6 +327,11 @@ static ColumnsPlan make_plan(int64_t M, int64_t Q, int64_t P) {
     // The kernels that stage X in LDS (gemm_kernel) keep: up to 32 rows, weights of more than a round of units (34816 x 5120, 20 rows, 40.8 us
     // against 45.7) or of more than 8192 columns (20000 x 9984, 20 rows, 35.9 / 42.0); few rows of W and long ones, whose columns they split over the chip (5120 x 17408, 24 rows 23.8 / 36.5, 64 rows 33.3 / 37).
     p.taken = splits > 1 ? M > 32 && tiles >= 1024 : (M > 32 || (units_best <= cus && n_steps <= 8 * kColumnsWaves)) && (10 * units_best >= 7 * cus || n_steps <= 4 * kColumnsWaves);
+    // ... and, where they can read the weight (P a multiple of 256), long rows with any number of rows of X (us them / here: 26675 x 8960, 33
+    // rows 64.6 / 70.1, 64 rows 67.7 / 79.3; up to 32 rows from 48 steps on: 12290 x 7936, 17 rows 27.5 / 29.4, 40 rows 36.6 / 33.5) and large weights whose waves would have a single step each (32603 x 1024, 17 rows 14.9 / 18.5,
+    // 64 rows 24.2 / 24.6; of ten steps, 15339 x 1280, 19.4 / 16.6 and 30.3 / 22.6).  The tile kernel, which takes the others, is behind (29291 x 8320,
+    // 40 rows, 136 / 80).
+    if (P % 256 == 0 && (n_steps > (M <= 32 ? 6 : 8) * kColumnsWaves || (n_steps <= kColumnsWaves && tiles >= 1024))) p.taken = false;
     p.steps_per_split = (int)((n_steps + splits - 1) / splits);
     p.splits = (int)((n_steps + p.steps_per_split - 1) / p.steps_per_split);
     p.x16_at = align256(qvb8_mma_rowinfo_bytes(Q));
