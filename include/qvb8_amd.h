@@ -27,8 +27,9 @@
  *   plane B, 64 x 4 (nb - 4) bytes:  entry l holds dwords 4..nb-1 of that slice (empty for nb = 4).
  * Row r of such a tile is marked in its bit_off word: bit 62 set, bits 0..47 = bit offset of the TILE's first byte (a
  * multiple of 32), bits 48..51 = r.  Every entry point that takes a pack reads such rows (qvb8_gemv and the escape
- * corrections id by id); qvb8_mma is told of them with QVB8_MMA_PLANES.  The expert stacks of qvb8_moe_experts do not
- * take them (a marked row there comes out as NaN, like any row whose metadata points outside its buffer).
+ * corrections id by id); qvb8_mma is told of them with QVB8_MMA_PLANES, the expert stacks of qvb8_moe_experts with
+ * QVB8_MOE_UP_PLANES / QVB8_MOE_DOWN_PLANES (without them a marked row there comes out as NaN, like any row whose metadata
+ * points outside its buffer).
  */
 #ifndef QVB8_AMD_H
 #define QVB8_AMD_H
@@ -54,9 +55,9 @@ enum qvb8_status {
  * the banded KV cache, query preparation; 4: qvb8_moe_experts_static; 5: result-type flags of qvb8_mma; 6: rows stored
  * in planes, QVB8_MMA_PLANES; 7: qvb8_mlp, qvb8r_walk_probe; 8: qvb8_kv_*;
  * 9: qvb8_decode_tiles; 10: its constants, qvb8_moe_experts_checked; 11: QVB8_MMA_SILU_PAIRS; 12: qvb8r_gemv_as; 13: qvb8_attend; 14: qvb8_kv_measure, qvb8_kv_wait;
- * 15: qvb8_mma_escapes_workspace_bytes; 16: qvb8_attn_rows_per_workgroup).  A binding compares the loaded library's answer
+ * 15: qvb8_mma_escapes_workspace_bytes; 16: qvb8_attn_rows_per_workgroup; 17: QVB8_MOE_*_PLANES).  A binding compares the loaded library's answer
  * with the QVB8_ABI_VERSION it was written for before it makes any other call. */
-#define QVB8_ABI_VERSION 16
+#define QVB8_ABI_VERSION 17
 int qvb8_abi_version(void);
 /* Message of the calling thread's most recent failure ("" if none). Valid until that thread's next call. */
 const char* qvb8_last_error(void);
@@ -278,8 +279,10 @@ enum qvb8_moe_act {
     /* More than 16 tokens: an infinity among fp16 activations stays one.  Without the flag it becomes +-65504, as every value beyond
      * fp16's range does in the other activation types (up to 16 tokens fp16 activations are always taken as they are). */
     QVB8_MOE_KEEP_INF = 0x400,
-    /* With QVB8_MOE_*_REGULAR, P a multiple of 128 and whole 16-row tiles (of each half, where gate and up are halves): every tile is
-     * stored in planes, as QVB8_MMA_PLANES describes; bit_off keeps the places of rows back to back. */
+    /* With QVB8_MOE_*_REGULAR, one width of 4..8, P a multiple of 128 and whole 16-row tiles (of each half, where gate and up are
+     * halves): every tile is stored in planes and every row's bit_off word is marked (rows stored in planes, above); "starts at bit"
+     * is then said of the tiles: that of rows 16 t .. 16 t + 15 of expert e lies where row 16 t would.  An unmarked stack with the
+     * flag, a marked one without it and tiles off a dword give NaN. */
     QVB8_MOE_UP_PLANES = 0x800,
     QVB8_MOE_DOWN_PLANES = 0x1000
 };

@@ -275,11 +275,10 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
         const int row = (rpu == 2 && (lr & 1)) ? gate_rows + u : u;
         const size_t mi = (size_t)e * a.Q + row;
         const int nb = a.nbits[mi];
-        const int64_t bit0 = a.planes ? a.bit_off[mi - (row & 15)] : a.bit_off[mi];
-        bool ok = nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + (int64_t)nb * a.P * (a.planes ? 16 : 1) + 7) >> 3) + 8 <= a.ids_bytes;
+        const int64_t off = a.bit_off[mi], bit0 = off & kOffBitsMask;
+        const bool ok = off_is_plane(off) == (a.planes != 0) && row_in_bounds(off, nb, a.P, a.ids_bytes);     // stored as the call says
         const bool fast = ok && nb >= 4 && nb <= 8 && (bit0 & 31) == 0;
-        if (a.planes) ok = fast;
-        s_row[lr] = MoeRow{ok ? bit0 : 0, a.tau_s[mi], a.min_s[mi], nb | (ok ? 256 : 0) | (fast ? 512 : 0), row & 15};
+        s_row[lr] = MoeRow{ok ? bit0 : 0, a.tau_s[mi], a.min_s[mi], nb | (ok ? 256 : 0) | (fast ? 512 : 0), off_plane_row(off)};
     }
     const int64_t clamp_byte = (a.ids_bytes - 8) & ~(int64_t)3;
     const int n_items = ((u_end - u_begin - wave + n_waves - 1) / n_waves) * rpu;   // rows this wave walks through
@@ -370,7 +369,7 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
                         if (lane == mb) {
                             if constexpr (STAGE == 0) {
                                 if (a.act == 0) v = (y_gate[mb] / (1.0f + __expf(-y_gate[mb]))) * y[mb];
-                                else { const float r = fmaxf(y[mb], 0.f); v = r * r; }
+                                else { const float r = fmaxf(y[mb], 0.f); v = y[mb] != y[mb] ? y[mb] : r * r; }
                             } else {
                                 v = y[mb];
                             }
@@ -401,6 +400,14 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
 // outside the stack gives NaN.
 constexpr int kOneMaxTiles = 16;       // row tiles per workgroup
 constexpr int kOneWaves = 8;
+
+// The first bit and the bits from one expert to the next of a regular stack, from the offsets of row 0 of its first two experts.  Marks of
+// rows in planes and what the call says have to agree: else no row is found inside the buffer, and results are NaN.
+__device__ __forceinline__ void regular_places(bool planes, int64_t& base, int64_t& stride) {
+    const bool agree = base >= 0 && stride >= 0 && off_is_plane(base) == planes && off_is_plane(stride) == planes;
+    base = agree ? base & kOffBitsMask : -kPlaneFlag;
+    stride = agree ? (stride & kOffBitsMask) - base : 0;
+}
 
 struct MoeOneArgs {
     const uint16_t* X;             // up: the token's activations (P), fp16 or bf16 bits; down: H (topk, P) fp16 bits
@@ -450,8 +457,8 @@ __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
     const v4u_t ones = {F::one_bits, F::one_bits, F::one_bits, F::one_bits};
     // REG: the stack's width, first bit and bits from one expert to the next (three reads that depend on nothing)
     const int reg_nb = REG ? (int)a.nbits[0] : 0;
-    const int64_t reg_base = REG ? a.bit_off[0] : 0;
-    const int64_t reg_stride = REG ? a.bit_off[a.E > 1 ? a.Q : 0] - reg_base : 0;
+    int64_t reg_base = REG ? a.bit_off[0] : 0, reg_stride = REG ? a.bit_off[a.E > 1 ? a.Q : 0] : 0;
+    if (REG) regular_places(a.planes != 0, reg_base, reg_stride);
 
     // A round = the row tiles the workgroup's waves work on at the same time.  (Two rounds of the up kernel in flight
     // together were measured: no faster -- a CU's share of the bytes, not the chain of trips, sets the time -- and the
@@ -518,6 +525,7 @@ __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
         const int64_t end_row = planes ? (int64_t)(16 - r) : 1;  // (in planes a row ends with its tile)
         q.ok = q.e_ok && q.nb >= 1 && q.nb <= 14 && q.bit0 >= 0 && ((q.bit0 + end_row * q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
         q.sliced = q.ok && q.nb >= 4 && q.nb <= 8 && (q.bit0 & 31) == 0;
+        if (planes) q.ok = q.sliced;                          // (no such row in planes is read id by id)
         // the row and chunk this lane asks for: its own (row r, chunk kg), or in REG mode row lane / 4, chunk lane % 4 of the
         // same tile (rows of a tile follow each other at P * nb bits; all 16 are usable or none is)
         const int64_t ask_bit0 = REG ? q.bit0 + (int64_t)((planes ? 0 : lane >> 2) - r) * a.P * q.nb : q.bit0;
@@ -718,8 +726,8 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
 
     // REG (one width, rows at regular places, see moe_one_kernel): the stack's width, first bit, bits between experts
     const int reg_nb = REG ? (int)a.nbits[0] : 0;
-    const int64_t reg_base = REG ? a.bit_off[0] : 0;
-    const int64_t reg_stride = REG ? a.bit_off[a.E > 1 ? a.Q : 0] - reg_base : 0;
+    int64_t reg_base = REG ? a.bit_off[0] : 0, reg_stride = REG ? a.bit_off[a.E > 1 ? a.Q : 0] : 0;
+    if (REG) regular_places(a.planes != 0, reg_base, reg_stride);
     const bool planes = REG && a.planes != 0;                 // already in operand order: lane l asks for entry l of its tile
     const int n_active = a.plan.n_bad[1];
     const int per_expert = max(1, (int)gridDim.x / max(1, n_active));
@@ -770,8 +778,9 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
         bool row_usable = false;
         if (tid < n_rows) {
             const int64_t end_row = planes ? (int64_t)(16 - (row_in_expert & 15)) : 1;      // (in planes a row ends with its tile)
-            const bool ok = e_ok && nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + end_row * nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
+            bool ok = e_ok && nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + end_row * nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
             const bool sliced = ok && nb >= 4 && nb <= 8 && (bit0 & 31) == 0;
+            if (planes) ok = sliced;
             row_usable = ok;
             // REG: the record is complete without anything read from memory; tau_s and min_s go to LDS further down,
             // behind the first requests for ids

@@ -215,7 +215,8 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& a, unsigned c
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         GroupRow& q = g[t];
-        q.ok = !off_is_plane(off[t]) && row_in_bounds(off[t], q.nb, PL ? (int64_t)16 * a.P : a.P, a.ids_bytes);
+        q.ok = off_is_plane(off[t]) == PL && row_in_bounds(off[t], q.nb, a.P, a.ids_bytes);           // stored as the call says
+        off[t] &= kOffBitsMask;
         const uint32_t nb = (uint32_t)q.nb;
         q.sliced = q.ok && nb >= 4 && nb <= 8 && (off[t] & 31) == 0;
         if (PL) q.ok = q.sliced;

@@ -36,7 +36,7 @@ struct MoeGroupArgs {
     int E, Q, P, topk;
     int units, gated;              // up: outputs per expert; whether the rows come as (gate, up) halves
     int keep_inf;                  // up: an infinity among fp16 activations stays one
-    int planes;                    // every 16-row tile is stored in planes (a regular stack; bit_off as with rows back to back)
+    int planes;                    // every 16-row tile is stored in planes (a regular stack; bit_off marked)
     int row_blocks, items;         // set by the launcher
 };
 bool moe_group_shapes_ok(int64_t P_up, int64_t Q_dn, int64_t P_dn);

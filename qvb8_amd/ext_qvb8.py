@@ -644,9 +644,9 @@ def stack_is_regular(nbits, bit_off, P) -> bool:
     return bool((nbits == nbits.reshape(-1)[0]).all() & (bit_off == want).all())
 
 
-def stack_in_planes(ids, bit_off, P, w) -> None:
-    """Stores every 16-row tile of a regular stack of width w (4..8, P a multiple of 128) in planes, in place: `bit_off`, (experts, Q), stays
-    what it is for rows back to back."""
+def stack_in_planes(ids, bit_off, P, w):
+    """Stores every 16-row tile of a regular stack of width w (4..8, P a multiple of 128, Q of 16) in planes, in place.  Returns the
+    (experts, Q) table of offsets that goes with them: marked, so that nothing takes the rows for rows back to back."""
     Q, dwords = bit_off.shape[1], int(P) * int(w) // 2                     # of a tile
     to_planes, to_native = _plane_index(int(P), int(w), ids.device)
     source = torch.empty_like(to_planes)
@@ -655,13 +655,15 @@ def stack_in_planes(ids, bit_off, P, w) -> None:
         tiles = ids[first:first + Q // 16 * dwords * 4].view(torch.int32).view(-1, dwords)
         for k in range(0, tiles.shape[0], 256):                            # bounded temporaries
             tiles[k:k + 256] = tiles[k:k + 256][:, source]
+    row = torch.arange(Q, device=ids.device)
+    return bit_off[:, row - row % 16] | (row % 16) << 48 | PLANE_FLAG
 
 
 def moe_experts(X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn,
                 regular=(False, False), keep_inf=False, checked=False, planes=(False, False)):
     """Routed gated-SiLU expert stack on the stacked layout (reference: qvb8_cuda.cu:937-992); returns (tokens, Qdn)
     in X's dtype.  `regular` = (up, down): the caller states that the stack is regular (stack_is_regular); `planes`: and that its tiles are
-    stored in planes (stack_in_planes).  `keep_inf`: fp16
+    stored in planes (stack_in_planes; without it such a stack comes out as NaN).  `keep_inf`: fp16
     activations beyond 16 tokens are taken as they are, infinities too (else they become +-65504).  `checked` (17 tokens
     or more): the host waits for the routing plan, not for the products, and gets None where an entry lies outside the
     stack (else such an entry makes the whole result NaN)."""
@@ -671,6 +673,8 @@ def moe_experts(X, idx, w, gu_ids, gu_min, gu_tau, gu_nb, gu_off, Qgu, Pgu, dn_i
 
 
 def moe_experts_relu2(X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn,
-                      regular=(False, False)):
-    """Non-gated expert stack with H = relu(up(x))^2 (reference: qvb8_cuda.cu:1002-1055)."""
-    return _moe(1 | (MOE_UP_REGULAR if regular[0] else 0) | (MOE_DOWN_REGULAR if regular[1] else 0), X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn)
+                      regular=(False, False), planes=(False, False)):
+    """Non-gated expert stack with H = relu(up(x))^2 (reference: qvb8_cuda.cu:1002-1055); `regular` and `planes` as in moe_experts."""
+    act = 1 | (MOE_UP_REGULAR if regular[0] else 0) | (MOE_DOWN_REGULAR if regular[1] else 0) \
+        | (MOE_UP_PLANES if planes[0] else 0) | (MOE_DOWN_PLANES if planes[1] else 0)
+    return _moe(act, X, idx, w, up_ids, up_min, up_tau, up_nb, up_off, Qup, Pup, dn_ids, dn_min, dn_tau, dn_nb, dn_off, Qdn, Pdn)

@@ -28,16 +28,17 @@ _INDEX_DTYPES = (torch.int64, torch.int32, torch.int16, torch.int8, torch.uint8)
 PLANES_FROM_BYTES = 16 << 20
 
 
-def stack_projection(mods, halves: int = 1) -> dict:
+def stack_projection(mods, halves: int = 1, planes: bool = False) -> dict:
     """One projection of every expert as ONE launch operand: the experts' packed ids back to back in a single buffer
     (each part starting on a 16-byte boundary, 64 spare bytes at the end), the row vectors as (experts, Q) tables, bit
-    offsets counted from the start of the shared buffer.  `halves`: 2 where a projection's rows are gate rows and up rows.  Every module is re-pointed at the shared buffer (its own
-    bit_off moved accordingly), so the separate copies can be freed and the modules keep working.
+    offsets counted from the start of the shared buffer.  `halves`: 2 where a projection's rows are gate rows and up rows.  `planes`: the
+    tiles of a large regular stack may be stored in planes; the result's "planes" says whether they are, and a call has to be told so
+    (ext.moe_experts).  Every module is re-pointed at the shared buffer (its own bit_off moved accordingly), so the separate copies can be
+    freed and the modules keep working.
     Layout of the reference's stacked call (src/qv_band/formats/qvb8/backends_experts.py:145-195).
     Unlike the reference's build_stack, which only re-points the experts' ids, this one may store the rows again: wider
     fields for some rows (every row of a 16-row tile in the tile's widest width, or every row of the stack in one width when
-    that costs at most QVB8_MOE_ONE_WIDTH_GROWTH = 4 % more bytes), the tiles of a large regular stack in planes (`planes`; the table's
-    bit_off stays that of rows back to back), all others' rows back to back.  The
+    that costs at most QVB8_MOE_ONE_WIDTH_GROWTH = 4 % more bytes), tiles in planes, all others' rows back to back.  The
     experts' nbits / ids / bit_off change with it (their values do not), so a footprint taken before the stack is built
     differs from one taken after by up to that growth."""
     uniform = os.environ.get("QVB8_MOE_UNIFORM_TILES", "1") != "0"
@@ -86,13 +87,12 @@ def stack_projection(mods, halves: int = 1) -> dict:
     regular = uniform and ext.stack_is_regular(table["nbits"], table["bit_off"], mods[0].in_features)
     sliced = bool(((table["nbits"] >= 4) & (table["nbits"] <= 8) & (table["bit_off"] % 32 == 0)).all())       # no row is read id by id
     P, Q = int(mods[0].in_features), int(mods[0].out_features)
-    planes = (regular and sliced and total >= PLANES_FROM_BYTES and P % 128 == 0 and Q % (16 * halves) == 0
+    planes = (planes and regular and sliced and total >= PLANES_FROM_BYTES and P % 128 == 0 and Q % (16 * halves) == 0
               and bool((table["bit_off"][:, 0] % 128 == 0).all()) and os.environ.get("QVB8_PLANES", "1") != "0")
     if planes:
-        ext.stack_in_planes(shared, table["bit_off"], P, int(table["nbits"][0, 0]))
-        row = torch.arange(Q, device=shared.device)
+        table["bit_off"] = ext.stack_in_planes(shared, table["bit_off"], P, int(table["nbits"][0, 0]))
         for m, off in zip(mods, table["bit_off"]):           # the modules' own offsets say where their rows are now
-            m.bit_off = off[row - row % 16] | (row % 16) << 48 | ext.PLANE_FLAG
+            m.bit_off = off.clone()
             m._planes = True
     return dict(ids=shared, Q=Q, P=P, regular=regular, sliced=sliced, planes=planes, **table)
 
@@ -167,7 +167,7 @@ class QVBandExpertsV8(nn.Module):
             gu, dn = list(self.gate_up_experts), list(self.down_experts)
             ok = (self._act_code() is not None and _stackable(gu) and _stackable(dn)
                   and gu[0].out_features == 2 * dn[0].in_features and gu[0].in_features == dn[0].out_features)
-            self._stk = (stack_projection(gu, 2), stack_projection(dn)) if ok else False
+            self._stk = (stack_projection(gu, 2, planes=True), stack_projection(dn, planes=True)) if ok else False
         return self._stk is not False
 
     def _whole_steps(self) -> bool:

@@ -44,11 +44,65 @@ def test_planes_change_no_result(T, k, dtype, tau, growth, monkeypatch):
         assert torch.equal(a, b)
 
 
+def _ops(s):
+    return s["ids"], s["min_s"], s["tau_s"], s["nbits"], s["bit_off"], s["Q"], s["P"]
+
+
+def _two_stacks(monkeypatch, E, hidden, inter, gated):
+    """The same experts as stacks back to back and in planes, (up, down) each."""
+    monkeypatch.setattr(BE, "PLANES_FROM_BYTES", 0)
+    out = []
+    for planes in (False, True):
+        gu, dn = _experts(E, hidden, inter, 2e-3)
+        up = gu if gated else [m.row_subset(torch.arange(inter, device=DEV)) for m in gu]
+        out.append((BE.stack_projection(up, 2 if gated else 1, planes=planes), BE.stack_projection(dn, planes=planes)))
+        assert [s["planes"] for s in out[-1]] == [planes] * 2 and all(s["regular"] for s in out[-1])
+    return out
+
+
+CALLS = [(1, torch.bfloat16), (5, torch.float16), (8, torch.bfloat16), (16, torch.float16), (3, torch.float32), (40, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_every_entry_point_reads_a_stack_in_planes_or_says_nan(gated, monkeypatch):
+    E, hidden, inter = 3, 256, 384
+    plain, planes = _two_stacks(monkeypatch, E, hidden, inter, gated)
+    for a, b in zip(plain, planes):                     # restored and looked up through the stack's own table
+        assert ext.rows_in_planes(b["bit_off"]) and not ext.rows_in_planes(a["bit_off"])
+        rows = [(s["ids"], s["min_s"].reshape(-1), s["nbits"].reshape(-1), s["bit_off"].reshape(-1), s["P"], s["tau_s"].reshape(-1), None, None) for s in (a, b)]
+        assert torch.equal(*(ext.decode_f32(*r) for r in rows))
+        some = torch.tensor([0, 17, a["Q"], E * a["Q"] - 1], device=DEV)
+        assert torch.equal(*(ext.lookup_rows(some, *r) for r in rows))
+    fn = ext.moe_experts if gated else ext.moe_experts_relu2
+    off_a_dword = [dict(s, bit_off=s["bit_off"] + 8) for s in planes]
+    unmarked = [dict(p, bit_off=s["bit_off"]) for s, p in zip(plain, planes)]
+    for T, dtype in CALLS:
+        g = torch.Generator(device=DEV).manual_seed(T)
+        x = torch.randn(T, hidden, device=DEV, generator=g).to(dtype)
+        w, idx = torch.softmax(torch.randn(T, E, device=DEV, generator=g), -1).topk(2, -1)
+        yes = dict(regular=(True, True))
+        want, got = fn(x, idx, w, *_ops(plain[0]), *_ops(plain[1]), **yes), fn(x, idx, w, *_ops(planes[0]), *_ops(planes[1]), **yes, planes=(True, True))
+        assert bool(want.isfinite().all())
+        assert torch.equal(got, want) if dtype != torch.float32 else float((got - want).norm() / want.norm()) < 2e-6
+        # one projection at a time: marked and not said so, regular or not; said to be in planes and not marked; off a dword
+        for stack, regular, said in ((planes, True, False), (planes, False, False), (unmarked, True, True), (off_a_dword, True, True)):
+            for bad in (0, 1):
+                ops = [*_ops((stack if bad == 0 else planes)[0]), *_ops((stack if bad == 1 else planes)[1])]
+                flags = dict(regular=(bad == 1 or regular, bad == 0 or regular), planes=(bad == 1 or said, bad == 0 or said))
+                assert bool(fn(x, idx, w, *ops, **flags).isnan().all()), (T, dtype, bad, regular, said)
+
+
+def test_a_stack_is_back_to_back_unless_planes_are_asked_for(monkeypatch):
+    monkeypatch.setattr(BE, "PLANES_FROM_BYTES", 0)
+    gu, dn = _experts(2, 256, 128, 2e-3)
+    for s in (BE.stack_projection(gu), BE.stack_projection(dn)):
+        assert not s["planes"] and not ext.rows_in_planes(s["bit_off"])
+
+
 def test_planes_without_what_they_need_are_refused():
     E, hidden, inter = 2, 256, 128
     gu, dn = _experts(E, hidden, inter, 2e-3)
     g, d = BE.stack_projection(gu, 2), BE.stack_projection(dn)
     x, idx, w = torch.randn(3, hidden, device=DEV), torch.zeros(3, 1, dtype=torch.int64, device=DEV), torch.ones(3, 1, device=DEV)
-    ops = lambda s: (s["ids"], s["min_s"], s["tau_s"], s["nbits"], s["bit_off"], s["Q"], s["P"])       # noqa: E731
     with pytest.raises(RuntimeError, match="regular"):
-        ext.moe_experts(x, idx, w, *ops(g), *ops(d), planes=(True, False))
+        ext.moe_experts(x, idx, w, *_ops(g), *_ops(d), planes=(True, False))

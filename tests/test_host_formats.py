@@ -270,6 +270,25 @@ def test_tile_uniform_widths_and_repack_rows_on_the_host():
     assert not ext.stack_is_regular(nb, off2, 64) and not ext.stack_is_regular(nb2, off, 64)
 
 
+def test_a_stack_in_planes_is_marked():
+    """stack_in_planes on CPU tensors: the table it returns marks every row, is not taken for a regular stack back to back, and rows_back_to_back
+    undoes it byte by byte (whatever reads the permuted bytes through a table sees where they are)."""
+    import torch
+    from qvb8_amd import ext_qvb8 as ext
+    E, Q, P = 3, 48, 256
+    for w in (4, 5, 6, 7, 8):
+        step = Q * P * w + 256
+        nb = torch.full((E, Q), w, dtype=torch.uint8)
+        off = torch.arange(E).view(E, 1) * step + torch.arange(Q).view(1, Q) * (P * w)
+        ids = torch.randint(0, 256, (E * step // 8 + 64,), dtype=torch.uint8)
+        stored = ids.clone()
+        marked = ext.stack_in_planes(stored, off, P, w)
+        assert ext.rows_in_planes(marked[1, 5:6]) and not torch.equal(stored, ids)
+        assert ext.stack_is_regular(nb, off, P) and not ext.stack_is_regular(nb, marked, P)
+        back, plain = ext.rows_back_to_back(stored, nb.reshape(-1), marked.reshape(-1), P)
+        assert torch.equal(back, ids) and torch.equal(plain, off.reshape(-1))
+
+
 def test_unit_order_of_a_gate_up_pack():
     """Units of 16 outputs, gate rows then up rows, every row of a unit at the unit's widest width, widths ascending."""
     import torch
