@@ -29,6 +29,7 @@ namespace qvb8 {
 
 constexpr int kMoeMB = 8;              // pairs that share one pass over an expert's rows
 constexpr int kMoeThreads = 256;
+constexpr int kPlaneRows = 4;          // rows of a tile in planes that a wave of the general kernel takes at a time
 
 constexpr int kPlanMaxThreads = 1024;
 constexpr int kPlanTableExperts = 512;
@@ -169,7 +170,6 @@ struct MoeGemvArgs {
     int units_per_block;
     int keep_inf;                  // QVB8_MOE_KEEP_INF
     int x_rows;                    // activation rows a workgroup stages at a time: min(kMoeMB, tokens)
-    int planes;                    // every 16-row tile is stored in planes (QVB8_MOE_*_PLANES)
 };
 
 template <int NB, int J>
@@ -231,28 +231,41 @@ __device__ __forceinline__ void moe_chunk_any(int nb, const uint4& lo, const uin
 }
 
 // Row record a workgroup keeps in LDS for each of its rows: flags = width | ok << 8 | fast << 9
-struct MoeRow { int64_t bit0; float ts, mn; int flags; int slot; };       // slot: the row's number in its tile
-// first and last four dwords of slice `cg` (32 columns) of a row: back to back, or of a tile in planes (bit0 = the tile's first bit)
-__device__ __forceinline__ void moe_slice(const uint8_t* ids, int64_t bit0, int nb, int slot, int cg, bool planes, uint4& lo, uint4& hi) {
-    const uint8_t* p = ids + (bit0 >> 3);
-    if (planes) {
-        const uint32_t at = (uint32_t)slot + 16u * (uint32_t)(cg & 3);
-        p += (size_t)(cg >> 2) * (256u * (uint32_t)nb);
-        lo = *reinterpret_cast<const uint4*>(p + at * 16u);
-        hi = *reinterpret_cast<const uint4*>(p + 1008u + (at + 1u) * (4u * (uint32_t)(nb - 4)));
-    } else {
-        p += (size_t)cg * (4u * (uint32_t)nb);
-        lo = *reinterpret_cast<const uint4*>(p);
-        hi = *reinterpret_cast<const uint4*>(p + 4 * (nb - 4));
+// (in planes bit0 is the tile's first bit and slot the row's number there)
+struct MoeRow { int64_t bit0; float ts, mn; int flags; int slot; };
+
+// v + the value of lane ^ X
+template <int X>
+__device__ __forceinline__ float add_lane_xor(float v) {
+    if constexpr (X == 4) {
+        const int low = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104, 0xF, 0x5, false);          // row_shl:4 for lanes without the bit
+        return v + __int_as_float(__builtin_amdgcn_update_dpp(low, __float_as_int(v), 0x114, 0xF, 0xA, false));
+    } else if constexpr (X == 8) return dpp_add<0x128>(v);                                                   // row_ror:8
+    else {
+        const uint32_t u = __builtin_bit_cast(uint32_t, v);
+        const auto pair = X == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        const uint32_t own = pair[0], other = pair[1];
+        return __builtin_bit_cast(float, own) + __builtin_bit_cast(float, other);
     }
 }
+// Sums over the lanes that agree in lane % 4, added up in wave_sum's order of their numbers / 4
+__device__ __forceinline__ float rows_sum(float v) { return add_lane_xor<32>(add_lane_xor<16>(add_lane_xor<8>(add_lane_xor<4>(v)))); }
 
 // STAGE 0: up projection + activation -> H.  STAGE 1: down projection -> Yd.
 // grid = (unit blocks, expert slots); a workgroup serves `units_per_block` output units of one selected expert for
 // all pairs routed to it, kMoeMB pairs at a time, with those pairs' activation rows staged in LDS as fp32.  A wave
 // walks through its rows with the next row's ids already requested while it multiplies the current one.
-template <int STAGE>
+//
+// R = 1: rows back to back, a row at a time, lane l slice l (32 columns), then l + 64, ...  R = 4: tiles in planes, where 16 bytes of a row
+// lie beside those of its neighbours: four rows at a time, lane l = 4 q + j slices q, q + 16, ... of row j.  Products and sums are those of
+// R = 1 bit for bit: the slices whose numbers agree modulo 64 first, then pairs of these.
+// R rows at a time because a request's lines go down with R (fp32, us a call, rows back to back / in planes R = 4 / R = 2 / a row at a time, both
+// layouts in one kernel, which cost either 13 registers: 128 experts of 2048/768, top-8, 1 token 31.8 / 33.7 / 35.8 / 40.6, 8 tokens 125 / 100 / 109 /
+// 146; 8 of 4096/8192, top-2, 1 token 82 / 70 / 99 / 115).  A second request on its way: 239 registers, 45.3 and 168 us.
+template <int STAGE, int R>
 __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
+    static_assert(R == 1 || R == 4);
+    constexpr bool PL = R > 1;
     extern __shared__ __align__(16) unsigned char smem[];
     const int rpu = (STAGE == 0 && a.act == 0) ? 2 : 1;             // rows per output unit (gate and up)
     // stage 0 multiplies activations that were narrowed to fp16: they are kept as fp16 (half the LDS and LDS traffic)
@@ -276,18 +289,30 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
         const size_t mi = (size_t)e * a.Q + row;
         const int nb = a.nbits[mi];
         const int64_t off = a.bit_off[mi], bit0 = off & kOffBitsMask;
-        const bool ok = off_is_plane(off) == (a.planes != 0) && row_in_bounds(off, nb, a.P, a.ids_bytes);     // stored as the call says
+        bool ok = off_is_plane(off) == PL && row_in_bounds(off, nb, a.P, a.ids_bytes);           // stored as the call says
         const bool fast = ok && nb >= 4 && nb <= 8 && (bit0 & 31) == 0;
+        if (PL) ok = fast;                                         // (no row in planes is read id by id)
         s_row[lr] = MoeRow{ok ? bit0 : 0, a.tau_s[mi], a.min_s[mi], nb | (ok ? 256 : 0) | (fast ? 512 : 0), off_plane_row(off)};
     }
     const int64_t clamp_byte = (a.ids_bytes - 8) & ~(int64_t)3;
-    const int n_items = ((u_end - u_begin - wave + n_waves - 1) / n_waves) * rpu;   // rows this wave walks through
-    auto local_row = [&](int i) { return ((wave + (i / rpu) * n_waves) * rpu) + (i % rpu); };
-    // the lane's slice of the first 2048 columns of a row (fast rows; other lanes / rows read the buffer's first bytes)
-    auto request = [&](const MoeRow& r, uint4& lo, uint4& hi) {
+    const int n_items = (((u_end - u_begin) / R - wave + n_waves - 1) / n_waves) * rpu;       // rows (R at a time) this wave walks through
+    const int in_group = lane % R, first_slice = lane / R;
+    auto local_row = [&](int i) { return (((wave + (i / rpu) * n_waves) * R + in_group) * rpu) + (i % rpu); };
+    // the lane's slice of the first 2048 columns of a row, or slice cg (fast rows; other lanes / rows read the buffer's first bytes)
+    auto request = [&](const MoeRow& r, int cg, uint4& lo, uint4& hi) {
         const int nb = r.flags & 255;
-        const bool use = (r.flags & 512) && lane * 32 < a.P;
-        moe_slice(a.ids, use ? r.bit0 : 0, use ? nb : 8, r.slot, use ? lane : 0, use && a.planes, lo, hi);
+        const bool use = (r.flags & 512) && cg * 32 < a.P;
+        const uint8_t* p = a.ids;
+        if constexpr (PL) {
+            const uint32_t at = use ? (uint32_t)r.slot + 16u * (uint32_t)(cg & 3) : 0u;
+            p += use ? (r.bit0 >> 3) + (int64_t)(cg >> 2) * (256 * nb) : 0;
+            lo = *reinterpret_cast<const uint4*>(p + at * 16u);
+            hi = *reinterpret_cast<const uint4*>(p + (use ? 1008u + (at + 1u) * (4u * (uint32_t)(nb - 4)) : 16u));
+        } else {
+            p += use ? (r.bit0 >> 3) + (int64_t)cg * 4 * nb : 0;
+            lo = *reinterpret_cast<const uint4*>(p);
+            hi = *reinterpret_cast<const uint4*>(p + (use ? 4 * (nb - 4) : 16));
+        }
     };
 
     for (int pc = p_begin; pc < p_end; pc += a.x_rows) {
@@ -295,7 +320,7 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
         __syncthreads();                                            // the previous chunk's rows are no longer read; s_row is written
         uint4 lo, hi;
         MoeRow cur;
-        if (n_items > 0) { cur = s_row[local_row(0)]; request(cur, lo, hi); }
+        if (n_items > 0) { cur = s_row[local_row(0)]; request(cur, first_slice, lo, hi); }
         // ---- stage the chunk's activation rows and their sums ----
         for (int mb = 0; mb < n; ++mb) {
             const int p = a.plan.order[pc + mb];
@@ -328,45 +353,75 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
 #pragma unroll
         for (int mb = 0; mb < kMoeMB; ++mb) y_gate[mb] = 0.f;
         for (int i = 0; i < n_items; ++i) {
-            uint4 lo_n = lo, hi_n = hi;
+            [[maybe_unused]] uint4 lo_n = lo, hi_n = hi;
             MoeRow nxt = cur;
-            if (i + 1 < n_items) { nxt = s_row[local_row(i + 1)]; request(nxt, lo_n, hi_n); }
-            const int nb = cur.flags & 255;
-            float acc[kMoeMB];
-#pragma unroll
-            for (int mb = 0; mb < kMoeMB; ++mb) acc[mb] = 0.f;
-            if (cur.flags & 512) {
-                if (lane * 32 < a.P) moe_chunk_any(nb, lo, hi, xs, a.P, lane * 32, n, acc);
-                for (int c0 = (kWave + lane) * 32; c0 < a.P; c0 += kWave * 32) {          // rows longer than 2048 columns
-                    uint4 l, h;
-                    moe_slice(a.ids, cur.bit0, nb, cur.slot, c0 >> 5, a.planes != 0, l, h);
-                    moe_chunk_any(nb, l, h, xs, a.P, c0, n, acc);
-                }
-            } else if (cur.flags & 256) {
-                for (int c = lane; c < a.P; c += kWave) {
-                    const float idf = (float)load_field(a.ids, cur.bit0 + (int64_t)c * nb, nb, clamp_byte);
-#pragma unroll
-                    for (int mb = 0; mb < kMoeMB; ++mb)
-                        if (mb < n) acc[mb] = __builtin_fmaf((float)xs[(size_t)mb * a.P + c], idf, acc[mb]);
-                }
-            }
+            if (i + 1 < n_items) { nxt = s_row[local_row(i + 1)]; if constexpr (!PL) request(nxt, lane, lo_n, hi_n); }
             float y[kMoeMB];
+            if constexpr (PL) {
+                const int nb = __builtin_amdgcn_readfirstlane(cur.flags & 255);          // one width
+                const int n_slices = a.P / 32, passes = (n_slices + kWave - 1) / kWave;
+                float pair[kMoeMB];
+#pragma unroll 1
+                for (int part = 0; part < R; ++part) {
+                    float acc[kMoeMB];
 #pragma unroll
-            for (int mb = 0; mb < kMoeMB; ++mb) {
-                y[mb] = 0.f;
-                if (mb < n) {                                                            // wave-uniform
-                    const float sum = wave_sum(acc[mb]);
-                    y[mb] = (cur.flags & 256) ? (float)((double)cur.ts * (double)sum + (double)cur.mn * (double)sxs[mb]) : __builtin_nanf("");
+                    for (int mb = 0; mb < kMoeMB; ++mb) acc[mb] = 0.f;
+#pragma unroll 1
+                    for (int pass = 0; pass < passes; ++pass) {
+                        const int cg = pass * kWave + part * (kWave / R) + first_slice;
+                        const bool last = pass + 1 == passes, done = last && part + 1 == R;
+                        uint4 lo_n, hi_n;
+                        request(done ? nxt : cur, done ? first_slice : last ? cg - pass * kWave + kWave / R : cg + kWave, lo_n, hi_n);
+                        if (cg < n_slices) moe_chunk_any(nb, lo, hi, xs, a.P, cg * 32, n, acc);
+                        lo = lo_n; hi = hi_n;
+                    }
+#pragma unroll
+                    for (int mb = 0; mb < kMoeMB; ++mb) {
+                        if (mb >= n) break;
+                        const float sum = rows_sum(acc[mb]);
+                        pair[mb] = part & 1 ? pair[mb] + sum : sum;
+                        if (part & 1) y[mb] = part == 3 ? y[mb] + pair[mb] : pair[mb];
+                    }
+                }
+#pragma unroll
+                for (int mb = 0; mb < kMoeMB; ++mb)
+                    y[mb] = mb < n ? ((cur.flags & 256) ? (float)((double)cur.ts * (double)y[mb] + (double)cur.mn * (double)sxs[mb]) : __builtin_nanf("")) : 0.f;
+            } else {
+                const int nb = cur.flags & 255;
+                float acc[kMoeMB];
+#pragma unroll
+                for (int mb = 0; mb < kMoeMB; ++mb) acc[mb] = 0.f;
+                if (cur.flags & 512) {
+                    if (lane * 32 < a.P) moe_chunk_any(nb, lo, hi, xs, a.P, lane * 32, n, acc);
+                    for (int c0 = (kWave + lane) * 32; c0 < a.P; c0 += kWave * 32) {          // rows longer than 2048 columns
+                        const uint8_t* p = a.ids + (cur.bit0 >> 3) + (int64_t)(c0 >> 5) * 4 * nb;
+                        moe_chunk_any(nb, *reinterpret_cast<const uint4*>(p), *reinterpret_cast<const uint4*>(p + 4 * (nb - 4)), xs, a.P, c0, n, acc);
+                    }
+                } else if (cur.flags & 256) {
+                    for (int c = lane; c < a.P; c += kWave) {
+                        const float idf = (float)load_field(a.ids, cur.bit0 + (int64_t)c * nb, nb, clamp_byte);
+#pragma unroll
+                        for (int mb = 0; mb < kMoeMB; ++mb)
+                            if (mb < n) acc[mb] = __builtin_fmaf((float)xs[(size_t)mb * a.P + c], idf, acc[mb]);
+                    }
+                }
+#pragma unroll
+                for (int mb = 0; mb < kMoeMB; ++mb) {
+                    y[mb] = 0.f;
+                    if (mb < n) {                                                            // wave-uniform
+                        const float sum = wave_sum(acc[mb]);
+                        y[mb] = (cur.flags & 256) ? (float)((double)cur.ts * (double)sum + (double)cur.mn * (double)sxs[mb]) : __builtin_nanf("");
+                    }
                 }
             }
             const bool unit_done = (i % rpu) == rpu - 1;
             if (unit_done) {
-                const int u = u_begin + wave + (i / rpu) * n_waves;
-                if (lane < n) {
+                const int u = u_begin + (wave + (i / rpu) * n_waves) * R + in_group;
+                if (first_slice < n) {
                     float v = 0.f;
 #pragma unroll
-                    for (int mb = 0; mb < kMoeMB; ++mb) {           // lane mb takes result mb (no dynamic register index)
-                        if (lane == mb) {
+                    for (int mb = 0; mb < kMoeMB; ++mb) {           // lane mb (of its row's) takes result mb (no dynamic register index)
+                        if (first_slice == mb) {
                             if constexpr (STAGE == 0) {
                                 if (a.act == 0) v = (y_gate[mb] / (1.0f + __expf(-y_gate[mb]))) * y[mb];
                                 else { const float r = fmaxf(y[mb], 0.f); v = y[mb] != y[mb] ? y[mb] : r * r; }
@@ -375,13 +430,14 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
                             }
                         }
                     }
-                    a.out[(size_t)a.plan.order[pc + lane] * a.units + u] = v;
+                    a.out[(size_t)a.plan.order[pc + first_slice] * a.units + u] = v;
                 }
             } else {
 #pragma unroll
                 for (int mb = 0; mb < kMoeMB; ++mb) y_gate[mb] = y[mb];
             }
-            cur = nxt; lo = lo_n; hi = hi_n;
+            cur = nxt;
+            if constexpr (!PL) { lo = lo_n; hi = hi_n; }
         }
     }
 }
@@ -1017,29 +1073,24 @@ constexpr size_t kMoeLdsLimit = 144 * 1024;
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-int launch_moe_gemv(int stage, MoeGemvArgs a, int64_t slots, hipStream_t s) {
-    // enough workgroups to fill the chip four times over the selected experts, at least one unit per wave
+template <int STAGE, int R>
+int launch_moe_gemv(MoeGemvArgs a, int64_t slots, hipStream_t s) {
+    // enough workgroups to fill the chip four times over the selected experts, at least R units per wave
     const int waves = kMoeThreads / 64;
     // measured on the 35B-A3B shapes: four workgroups per CU are best for a handful of selected experts, eight for dozens
     const int64_t target_blocks = ((int64_t)host::env_int("QVB8_MOE_WGS_PER_CU", slots > 16 ? 8 : 4) * host::device_cus() + slots - 1) / slots;
     int64_t upb = (a.units + target_blocks - 1) / target_blocks;
-    upb = (upb + waves - 1) / waves * waves;
+    upb = (upb + waves * R - 1) / (waves * R) * (waves * R);
+    auto lds_of = [&](int64_t units) {
+        return (((size_t)a.x_rows * a.P * (STAGE == 0 ? 2 : 4) + 15) & ~(size_t)15) + (kMoeMB + kMoeMB * (kMoeThreads / 64)) * 4 + (size_t)units * 2 * sizeof(MoeRow);
+    };
+    while (R > 1 && upb > waves * R && lds_of(upb) > kMoeLdsLimit) upb -= waves * R;         // (what is rounded up above is no reason to refuse)
     a.units_per_block = (int)upb;
-    const size_t lds = (((size_t)a.x_rows * a.P * (stage == 0 ? 2 : 4) + 15) & ~(size_t)15) + (kMoeMB + kMoeMB * (kMoeThreads / 64)) * 4
-                       + (size_t)upb * 2 * sizeof(MoeRow);
+    const size_t lds = lds_of(upb);
     if (lds > kMoeLdsLimit) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_moe_experts: P=%d does not fit the workgroup's LDS", a.P);
-    static bool attr[2][64] = {{false}};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return host::fail(QVB8_ERR_LAUNCH, "qvb8_moe_experts: no current device");
-    if (!attr[stage][dev]) {
-        const void* f = stage == 0 ? (const void*)moe_gemv_kernel<0> : (const void*)moe_gemv_kernel<1>;
-        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMoeLdsLimit) != hipSuccess)
-            return host::fail(QVB8_ERR_LAUNCH, "qvb8_moe_experts: cannot raise the kernel's LDS limit");
-        attr[stage][dev] = true;
-    }
+    if (int rc = host::raise_lds_limit<moe_gemv_kernel<STAGE, R>>(kMoeLdsLimit, "qvb8_moe_experts")) return rc;
     dim3 grid((unsigned)((a.units + upb - 1) / upb), (unsigned)slots);
-    if (stage == 0) hipLaunchKernelGGL(moe_gemv_kernel<0>, grid, dim3(kMoeThreads), lds, s, a);
-    else hipLaunchKernelGGL(moe_gemv_kernel<1>, grid, dim3(kMoeThreads), lds, s, a);
+    hipLaunchKernelGGL((moe_gemv_kernel<STAGE, R>), grid, dim3(kMoeThreads), lds, s, a);
     return host::check_launch("qvb8_moe_experts");
 }
 int launch_moe_combine(const float* Yd, const float* w, void* out, int out_dtype, int64_t topk, int64_t D, int64_t tokens, const MoePlan& pl, hipStream_t s) {
@@ -1225,8 +1276,7 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
         if (int rc = launch_moe_walk<true, false>(wa, dn_regular, slots, tokens, s)) return rc;
         return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
     }
-    // (the general kernel reads a row at a time, which leaves most of a tile's lines in planes to be fetched again)
-    if ((tokens > 16 || up_planes || dn_planes) && (reinterpret_cast<uintptr_t>(X) & 15u) == 0 && moe_group_shapes_ok(P_up, Q_dn, P_dn)) {
+    if (tokens > 16 && (reinterpret_cast<uintptr_t>(X) & 15u) == 0 && moe_group_shapes_ok(P_up, Q_dn, P_dn)) {
         MoeGroupArgs ga;
         ga.X = X; ga.plan = pl; ga.ids = up_ids; ga.ids_bytes = up_ids_bytes;
         ga.min_s = up_min; ga.tau_s = up_tau; ga.nbits = up_nb; ga.bit_off = up_off; ga.out = H;
@@ -1243,11 +1293,11 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
     MoeGemvArgs a;
     a.X = X; a.ids = up_ids; a.ids_bytes = up_ids_bytes; a.min_s = up_min; a.tau_s = up_tau; a.nbits = up_nb; a.bit_off = up_off;
     a.out = H; a.plan = pl; a.Q = (int)Q_up; a.P = (int)P_up; a.topk = (int)topk; a.x_dtype = x_dtype; a.act = act;
-    a.units = (int)P_dn; a.planes = up_planes ? 1 : 0; a.keep_inf = keep_inf ? 1 : 0; a.units_per_block = 0; a.x_rows = (int)(tokens < kMoeMB ? tokens : kMoeMB);
-    if (int rc = launch_moe_gemv(0, a, slots, s)) return rc;
+    a.units = (int)P_dn; a.keep_inf = keep_inf ? 1 : 0; a.units_per_block = 0; a.x_rows = (int)(tokens < kMoeMB ? tokens : kMoeMB);
+    if (int rc = up_planes ? launch_moe_gemv<0, kPlaneRows>(a, slots, s) : launch_moe_gemv<0, 1>(a, slots, s)) return rc;
     a.X = H; a.ids = dn_ids; a.ids_bytes = dn_ids_bytes; a.min_s = dn_min; a.tau_s = dn_tau; a.nbits = dn_nb; a.bit_off = dn_off;
-    a.out = Yd; a.Q = (int)Q_dn; a.P = (int)P_dn; a.x_dtype = QVB8_F32; a.units = (int)Q_dn; a.planes = dn_planes ? 1 : 0;
-    if (int rc = launch_moe_gemv(1, a, slots, s)) return rc;
+    a.out = Yd; a.Q = (int)Q_dn; a.P = (int)P_dn; a.x_dtype = QVB8_F32; a.units = (int)Q_dn;
+    if (int rc = dn_planes ? launch_moe_gemv<1, kPlaneRows>(a, slots, s) : launch_moe_gemv<1, 1>(a, slots, s)) return rc;
 
     return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
 }
