@@ -457,12 +457,24 @@ __global__ void __launch_bounds__(kMoeThreads) moe_gemv_kernel(MoeGemvArgs a) {
 constexpr int kOneMaxTiles = 16;       // row tiles per workgroup
 constexpr int kOneWaves = 8;
 
+// How a stack is stored, as the call says: anyhow; regular (QVB8_MOE_*_REGULAR); regular with every 16-row tile in planes.  Chosen when a
+// kernel is compiled: told apart at run time, the 16-row kernels kept lane changes, addresses and spilled scalars of both (us a call, bf16,
+// rows back to back without planes / both in one kernel / now: 128 experts of 2048/768, top-8, in planes, 1 token 15.1 / 15.4 / 14.4, 8 tokens 53.8 /
+// 53.1 / 50.6, 16 tokens 86.7 / 82.7 / 77.7; 8 of 4096/4096, top-2, 8 tokens 108 / 107 / 90; 16 of 2048/256, back to back, 1 token 12.4 / 14.0 / 12.5).
+enum MoeStored { kAnyhow, kRegular, kInPlanes };
+MoeStored moe_stored(bool regular, bool planes) { return planes ? kInPlanes : regular ? kRegular : kAnyhow; }
+
 // The first bit and the bits from one expert to the next of a regular stack, from the offsets of row 0 of its first two experts.  Marks of
 // rows in planes and what the call says have to agree: else no row is found inside the buffer, and results are NaN.
-__device__ __forceinline__ void regular_places(bool planes, int64_t& base, int64_t& stride) {
-    const bool agree = base >= 0 && stride >= 0 && off_is_plane(base) == planes && off_is_plane(stride) == planes;
-    base = agree ? base & kOffBitsMask : -kPlaneFlag;
-    stride = agree ? (stride & kOffBitsMask) - base : 0;
+template <bool PL>
+__device__ __forceinline__ void regular_places(int64_t& base, int64_t& stride) {
+    if constexpr (PL) {
+        const bool agree = base >= 0 && stride >= 0 && off_is_plane(base) && off_is_plane(stride);
+        base = agree ? base & kOffBitsMask : -kPlaneFlag;
+        stride = agree ? (stride & kOffBitsMask) - base : 0;
+    } else {
+        stride -= base;                                            // (a marked row lies far outside)
+    }
 }
 
 struct MoeOneArgs {
@@ -475,14 +487,15 @@ struct MoeOneArgs {
     int E, Q, P, topk;
     int units, gated;              // up: outputs per expert; whether the rows come as (gate, up) halves
     int tiles_per_wg;              // up: unit tiles per workgroup
-    int planes;                    // every 16-row tile is stored in planes (REG only)
 };
 
 // REG: the caller states that every row of the stack has one width and that the rows lie at regular places (row q of
 // expert e at bit_off[0] + e * (bit_off[Q] - bit_off[0]) + q * P * width): the kernel then works a row's place out
-// instead of reading it, which takes one dependent memory trip out of every round.
-template <int T, bool DOWN, bool XC, int DT, bool REG>
+// instead of reading it, which takes one dependent memory trip out of every round.  PL: its tiles lie in planes, a request is one run
+// in operand order, and all of a tile's rows can be read or none.
+template <int T, bool DOWN, bool XC, int DT, MoeStored ST>
 __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
+    constexpr bool REG = ST != kAnyhow, PL = ST == kInPlanes;
     using F = Fmt<false>;
     using XI = XIn<false, XC>;
     __shared__ float s_part[kOneMaxTiles][kOneWaves][16];    // [row tile][column range][row]
@@ -514,7 +527,7 @@ __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
     // REG: the stack's width, first bit and bits from one expert to the next (three reads that depend on nothing)
     const int reg_nb = REG ? (int)a.nbits[0] : 0;
     int64_t reg_base = REG ? a.bit_off[0] : 0, reg_stride = REG ? a.bit_off[a.E > 1 ? a.Q : 0] : 0;
-    if (REG) regular_places(a.planes != 0, reg_base, reg_stride);
+    if constexpr (REG) regular_places<PL>(reg_base, reg_stride);
 
     // A round = the row tiles the workgroup's waves work on at the same time.  (Two rounds of the up kernel in flight
     // together were measured: no faster -- a CU's share of the bytes, not the chain of trips, sets the time -- and the
@@ -559,7 +572,7 @@ __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
         const size_t mi = (size_t)(q.e_ok ? e : 0) * a.Q + row0_of(q.i) + r;
         if constexpr (REG) {
             q.nb = reg_nb;
-            q.bit0 = reg_base + (int64_t)(q.e_ok ? e : 0) * reg_stride + (int64_t)(row0_of(q.i) + r) * a.P * reg_nb;
+            q.bit0 = reg_base + (int64_t)(q.e_ok ? e : 0) * reg_stride + (int64_t)(row0_of(q.i) + (PL ? 0 : r)) * a.P * reg_nb;      // PL: the tile's
         } else {
             q.nb = a.nbits[mi];
             q.bit0 = a.bit_off[mi];
@@ -570,33 +583,40 @@ __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
     // + chunk (four neighbouring lanes read 16 nb consecutive bytes of one row: far fewer L1 accesses per request than a row
     // per lane) and to_operand moves the registers into operand order (lane = row + 16 * chunk) across the wave.
     const int pull = 4 * (4 * r + kg);
-    const bool planes = REG && a.planes != 0;                 // already in operand order: lane l asks for entry l
     auto to_operand = [&](const uint4& v) -> uint4 {
-        if constexpr (!REG) return v;
-        if (planes) return v;
+        if constexpr (!REG || PL) return v;
         return uint4{(uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.x), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.y),
                      (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.z), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.w)};
     };
     auto request_ids = [&](Round& q, uint4 (&lo)[T], uint4 (&hi)[T]) {
-        const int64_t end_row = planes ? (int64_t)(16 - r) : 1;  // (in planes a row ends with its tile)
-        q.ok = q.e_ok && q.nb >= 1 && q.nb <= 14 && q.bit0 >= 0 && ((q.bit0 + end_row * q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
+        if constexpr (PL) {
+            q.ok = q.sliced = q.e_ok && q.nb >= 4 && q.nb <= 8 && q.bit0 >= 0 && (q.bit0 & 31) == 0 && (q.bit0 >> 3) + (int64_t)a.P * q.nb * 2 + 8 <= a.ids_bytes;
+            const uint8_t* at = a.ids + (q.ok ? (uint64_t)(q.bit0 >> 3) + (uint64_t)(uint32_t)step0 * (256u * (uint32_t)q.nb) : 0u);
+            const uint32_t to_lo = (uint32_t)lane * 16u, to_hi = 1008u + (uint32_t)(lane + 1) * (4u * (uint32_t)(q.nb - 4));
+#pragma unroll
+            for (int it = 0; it < T; ++it) {
+                const bool use = q.ok && (step0 + it) < n_steps;       // (else the buffer's first bytes)
+                const uint8_t* step = use ? at + (uint32_t)it * (256u * (uint32_t)q.nb) : a.ids;
+                lo[it] = *reinterpret_cast<const uint4*>(step + (use ? to_lo : 0u));
+                hi[it] = *reinterpret_cast<const uint4*>(step + (use ? to_hi : 16u));
+            }
+            return;
+        }
+        q.ok = q.e_ok && q.nb >= 1 && q.nb <= 14 && q.bit0 >= 0 && ((q.bit0 + (int64_t)q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
         q.sliced = q.ok && q.nb >= 4 && q.nb <= 8 && (q.bit0 & 31) == 0;
-        if (planes) q.ok = q.sliced;                          // (no such row in planes is read id by id)
         // the row and chunk this lane asks for: its own (row r, chunk kg), or in REG mode row lane / 4, chunk lane % 4 of the
         // same tile (rows of a tile follow each other at P * nb bits; all 16 are usable or none is)
-        const int64_t ask_bit0 = REG ? q.bit0 + (int64_t)((planes ? 0 : lane >> 2) - r) * a.P * q.nb : q.bit0;
+        const int64_t ask_bit0 = REG ? q.bit0 + (int64_t)((lane >> 2) - r) * a.P * q.nb : q.bit0;
         const int ask_chunk = REG ? (lane & 3) : kg;
         const bool ask_sliced = !REG ? q.sliced : (q.e_ok && q.nb >= 4 && q.nb <= 8 && ask_bit0 >= 0 && (ask_bit0 & 31) == 0
-                                                   && ((ask_bit0 + (planes ? 16 : 1) * (int64_t)q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes);
-        const uint32_t nbu = (uint32_t)q.nb, per_step = planes ? 256u * nbu : 16u * nbu;
-        const uint64_t row_off = (uint64_t)(ask_bit0 >> 3) + (planes ? (uint64_t)step0 * per_step + 16u * (uint32_t)lane : (uint64_t)(step0 * 4 + ask_chunk) * (4u * nbu));
-        const uint32_t to_hi = planes ? 1008u + (uint32_t)(lane + 1) * (4u * (nbu - 4u)) - 16u * (uint32_t)lane : 4u * (nbu - 4u);
+                                                   && ((ask_bit0 + (int64_t)q.nb * a.P + 7) >> 3) + 8 <= a.ids_bytes);
+        const uint64_t row_off = (uint64_t)(ask_bit0 >> 3) + (uint64_t)(step0 * 4 + ask_chunk) * (4u * (uint32_t)q.nb);
 #pragma unroll
         for (int it = 0; it < T; ++it) {
             const bool use = ask_sliced && (step0 + it) < n_steps;     // a wave without a tile reads tile 0's again: no address shared by the whole chip
-            const uint64_t off = use ? row_off + (uint64_t)it * per_step : 0;
+            const uint64_t off = use ? row_off + (uint64_t)it * (16u * (uint32_t)q.nb) : 0;
             lo[it] = *reinterpret_cast<const uint4*>(a.ids + off);
-            hi[it] = *reinterpret_cast<const uint4*>(a.ids + off + (use ? to_hi : 16u));
+            hi[it] = *reinterpret_cast<const uint4*>(a.ids + off + (use ? 4u * (uint32_t)(q.nb - 4) : 16u));
         }
     };
     auto multiply = [&](const Round& q, const uint4 (&lo_)[T], const uint4 (&hi_)[T], const uint16_t* xrow) {
@@ -609,7 +629,7 @@ __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
         const uint32_t info0 = REG ? ((uint32_t)reg_nb | ((reg_nb >= 4 && reg_nb <= 8) ? 256u : 0u)) : (uint32_t)__builtin_amdgcn_readfirstlane((int)info);
         // (a regular stack whose rows do not start on dword boundaries has no sliced row: its lanes then multiply id 0 here and
         // the rows are redone element by element below, as without the statement)
-        const bool uniform = REG ? ((info0 >> 8) == 1u && __builtin_amdgcn_ballot_w64(q.e_ok && !sliced) == 0)
+        const bool uniform = REG ? ((info0 >> 8) == 1u && (PL || __builtin_amdgcn_ballot_w64(q.e_ok && !sliced) == 0))
                                  : (__builtin_amdgcn_ballot_w64(info != info0) == 0 && (info0 >> 8) == 1u);
 #pragma unroll
         for (int it = 0; it < T; ++it) {
@@ -648,7 +668,8 @@ __global__ void __launch_bounds__(64 * kOneWaves) moe_one_kernel(MoeOneArgs a) {
         if (kg == 0) s_part[i][wc][r] = __builtin_fmaf(-F::bias, sx[0], acc[0]);
         if (lane == 0) s_sx[i][wc] = sx[0];
         if (kg == 0 && wc == 0) s_fin[i][r] = float2{q.ts, q.mn};
-        if (lane == 0 && wc == 0) s_ok[i] = q.e_ok ? 1 : 0;
+        if (lane == 0 && wc == 0) s_ok[i] = (PL ? q.ok : q.e_ok) ? 1 : 0;
+        if constexpr (PL) return;
         // rows the slicing cannot read: element by element over this wave's columns
         uint64_t odd = __builtin_amdgcn_ballot_w64(kg == 0 && !sliced);
         while (odd) {
@@ -746,15 +767,15 @@ struct MoeWalkArgs {
     int units, gated;              // up: outputs per expert; whether the rows come as (gate, up) halves
     int tiles_per_seg;             // unit tiles (up) / row tiles (down) per segment
     int max_tokens;                // most pairs an expert can have in this call (the LDS is laid out for it)
-    int planes;                    // every 16-row tile is stored in planes (REG only)
 };
 constexpr int kWalkWaves = 4;          // waves per workgroup: two workgroups share a CU
 constexpr int kWalkMaxRowTiles = 16;   // row tiles per segment: one row record per thread
 
 struct WalkRow { int64_t bit0; int flags; float ts, mn; int nat; };       // flags = width | usable << 8 | sliced << 9; nat = place before the sort
 
-template <int T, bool DOWN, bool XC, bool TWO, bool REG>
+template <int T, bool DOWN, bool XC, bool TWO, MoeStored ST>
 __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
+    constexpr bool REG = ST != kAnyhow, PL = ST == kInPlanes;       // (as in moe_one_kernel)
     using F = Fmt<false>;
     using XI = XIn<false, XC>;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -783,8 +804,7 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
     // REG (one width, rows at regular places, see moe_one_kernel): the stack's width, first bit, bits between experts
     const int reg_nb = REG ? (int)a.nbits[0] : 0;
     int64_t reg_base = REG ? a.bit_off[0] : 0, reg_stride = REG ? a.bit_off[a.E > 1 ? a.Q : 0] : 0;
-    if (REG) regular_places(a.planes != 0, reg_base, reg_stride);
-    const bool planes = REG && a.planes != 0;                 // already in operand order: lane l asks for entry l of its tile
+    if constexpr (REG) regular_places<PL>(reg_base, reg_stride);
     const int n_active = a.plan.n_bad[1];
     const int per_expert = max(1, (int)gridDim.x / max(1, n_active));
     const int sl = (int)blockIdx.x / per_expert;
@@ -817,7 +837,7 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
         int nb; int64_t bit0;
         if constexpr (REG) {
             nb = reg_nb;
-            bit0 = reg_base + (int64_t)(e_ok ? e : 0) * reg_stride + (int64_t)row_in_expert * a.P * reg_nb;
+            bit0 = reg_base + (int64_t)(e_ok ? e : 0) * reg_stride + (int64_t)(PL ? row_in_expert & ~15 : row_in_expert) * a.P * reg_nb;     // PL: the tile's
         } else {
             nb = a.nbits[mi];
             bit0 = a.bit_off[mi];
@@ -833,10 +853,9 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
         }
         bool row_usable = false;
         if (tid < n_rows) {
-            const int64_t end_row = planes ? (int64_t)(16 - (row_in_expert & 15)) : 1;      // (in planes a row ends with its tile)
-            bool ok = e_ok && nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + end_row * nb * a.P + 7) >> 3) + 8 <= a.ids_bytes;
+            bool ok = e_ok && nb >= 1 && nb <= 14 && bit0 >= 0 && ((bit0 + (int64_t)nb * a.P * (PL ? 16 : 1) + 7) >> 3) + 8 <= a.ids_bytes;
             const bool sliced = ok && nb >= 4 && nb <= 8 && (bit0 & 31) == 0;
-            if (planes) ok = sliced;
+            if constexpr (PL) ok = sliced;
             row_usable = ok;
             // REG: the record is complete without anything read from memory; tau_s and min_s go to LDS further down,
             // behind the first requests for ids
@@ -876,26 +895,38 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
             const WalkRow rec = s_row[i * 16 + r];
             // REG: the lane asks for chunk lane % 4 of row lane / 4 of the tile (neighbouring lanes, neighbouring bytes: far
             // fewer L1 accesses per request than a row per lane); to_operand brings the registers into operand order
-            const WalkRow ask = REG ? s_row[i * 16 + (planes ? 0 : lane >> 2)] : rec;
+            if constexpr (PL) {
+                // one run a request, the tile's place the same for all lanes
+                const uint32_t flags = (uint32_t)__builtin_amdgcn_readfirstlane(rec.flags), nbr = flags & 255u;
+                const uint64_t bit0 = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(rec.bit0 >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)rec.bit0);
+                const bool sliced = (flags & 512u) != 0;
+                const uint32_t to_lo = (uint32_t)lane * 16u, to_hi = 1008u + (uint32_t)(lane + 1) * (4u * (nbr - 4u));
+#pragma unroll
+                for (int it = 0; it < T; ++it) {
+                    const bool use = sliced && (step0 + it) < n_steps;         // (else the buffer's first bytes)
+                    const uint8_t* step = a.ids + (use ? (bit0 >> 3) + (uint64_t)(uint32_t)(step0 + it) * (256u * nbr) : 0u);
+                    lo[it] = *reinterpret_cast<const uint4*>(step + (use ? to_lo : 0u));
+                    hi[it] = *reinterpret_cast<const uint4*>(step + (use ? to_hi : 16u));
+                }
+                return rec;
+            }
+            const WalkRow ask = REG ? s_row[i * 16 + (lane >> 2)] : rec;
             const int ask_chunk = REG ? (lane & 3) : kg;
             const uint32_t nbr = (uint32_t)ask.flags & 255u;
             const bool sliced = (ask.flags & 512) != 0;
-            const uint32_t per_step = planes ? 256u * nbr : 16u * nbr;
-            const uint64_t row_off = (uint64_t)(ask.bit0 >> 3) + (planes ? (uint64_t)step0 * per_step + 16u * (uint32_t)lane : (uint64_t)(step0 * 4 + ask_chunk) * (4u * nbr));
-            const uint32_t to_hi = planes ? 1008u + (uint32_t)(lane + 1) * (4u * (nbr - 4u)) - 16u * (uint32_t)lane : 4u * (nbr - 4u);
+            const uint64_t row_off = (uint64_t)(ask.bit0 >> 3) + (uint64_t)(step0 * 4 + ask_chunk) * (4u * nbr);
 #pragma unroll
             for (int it = 0; it < T; ++it) {
                 const bool use = sliced && (step0 + it) < n_steps;
-                const uint64_t off = use ? row_off + (uint64_t)it * per_step : 0;
+                const uint64_t off = use ? row_off + (uint64_t)it * (16u * nbr) : 0;
                 lo[it] = *reinterpret_cast<const uint4*>(a.ids + off);
-                hi[it] = *reinterpret_cast<const uint4*>(a.ids + off + (use ? to_hi : 16u));
+                hi[it] = *reinterpret_cast<const uint4*>(a.ids + off + (use ? 4u * (nbr - 4u) : 16u));
             }
             return rec;
         };
         const int pull = 4 * (4 * r + kg);
         auto to_operand = [&](const uint4& v) __attribute__((always_inline)) -> uint4 {
-            if constexpr (!REG) return v;
-            if (planes) return v;
+            if constexpr (!REG || PL) return v;
             return uint4{(uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.x), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.y),
                          (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.z), (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.w)};
         };
@@ -932,7 +963,7 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
             // REG: one width for the whole stack (rows that cannot be read decode what was loaded and end as NaN)
             const uint32_t info0 = REG ? ((uint32_t)reg_nb | ((reg_nb >= 4 && reg_nb <= 8) ? 256u : 0u)) : (uint32_t)__builtin_amdgcn_readfirstlane((int)info);
             // (usable rows of a regular stack that do not start on dword boundaries are not sliced: zero here, redone below)
-            const bool uniform = REG ? ((info0 >> 8) == 1u && __builtin_amdgcn_ballot_w64((rec.flags & 256) != 0 && !sliced) == 0)
+            const bool uniform = REG ? ((info0 >> 8) == 1u && (PL || __builtin_amdgcn_ballot_w64((rec.flags & 256) != 0 && !sliced) == 0))
                                      : (__builtin_amdgcn_ballot_w64(info != info0) == 0 && (info0 >> 8) == 1u);
 #pragma unroll
             for (int it = 0; it < T; ++it) {
@@ -969,7 +1000,7 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
                 }
                 if constexpr (!REG) { if (kg == 0 && wc == 0) s_fin[i * 16 + r] = float2{(rec.flags & 256) ? rec.ts : __builtin_nanf(""), rec.mn}; }
                 // rows the slicing cannot read: element by element over this wave's columns, token by token
-                uint64_t odd = __builtin_amdgcn_ballot_w64(kg == 0 && !sliced);
+                uint64_t odd = PL ? 0 : __builtin_amdgcn_ballot_w64(kg == 0 && !sliced);
                 while (odd) {
                     const int rr = __builtin_ctzll(odd);
                     odd &= odd - 1;
@@ -1042,14 +1073,14 @@ __device__ __forceinline__ void moe_walk_body(const MoeWalkArgs& a) {
 }
 
 // rows of up to 2048 columns: within 256 registers, two workgroups per CU (one starts while the other walks)
-template <int T, bool DOWN, bool XC, bool TWO, bool REG>
+template <int T, bool DOWN, bool XC, bool TWO, MoeStored ST>
 __global__ void __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) moe_walk_kernel(MoeWalkArgs a) {
-    moe_walk_body<T, DOWN, XC, TWO, REG>(a);
+    moe_walk_body<T, DOWN, XC, TWO, ST>(a);
 }
 // longer rows: eight steps of activations per wave need more registers, one workgroup per CU
-template <bool DOWN, bool XC, bool REG>
+template <bool DOWN, bool XC, MoeStored ST>
 __global__ void __launch_bounds__(64 * kWalkWaves) moe_walk_wide_kernel(MoeWalkArgs a) {
-    moe_walk_body<8, DOWN, XC, false, REG>(a);
+    moe_walk_body<8, DOWN, XC, false, ST>(a);
 }
 
 template <int DT>
@@ -1120,23 +1151,24 @@ bool moe_group_ok(int64_t tokens, int64_t topk, int x_dtype, int64_t P_up, int64
     return moe_walk_shapes_ok(topk, x_dtype, P_up, Q_dn, P_dn) && host::env_int("QVB8_MOE_GROUPED", 1) != 0;
 }
 
-template <bool DOWN, bool XC, int DT, bool REG>
+template <bool DOWN, bool XC, int DT, MoeStored ST>
 int launch_moe_one_as(const MoeOneArgs& a, unsigned blocks, unsigned tokens, hipStream_t s) {
     const int n_steps = a.P / kStepCols;
     // six steps per wave only for the down kernel (one round in flight): a whole row of up to 768 columns per wave, so
     // that eight slots are one round
     if constexpr (DOWN) {
         if (n_steps <= 6) {
-            hipLaunchKernelGGL((moe_one_kernel<6, DOWN, XC, DT, REG>), dim3(blocks, tokens), dim3(64 * kOneWaves), 0, s, a);
+            hipLaunchKernelGGL((moe_one_kernel<6, DOWN, XC, DT, ST>), dim3(blocks, tokens), dim3(64 * kOneWaves), 0, s, a);
             return host::check_launch("qvb8_moe_experts");
         }
     }
-    hipLaunchKernelGGL((moe_one_kernel<4, DOWN, XC, DT, REG>), dim3(blocks, tokens), dim3(64 * kOneWaves), 0, s, a);
+    hipLaunchKernelGGL((moe_one_kernel<4, DOWN, XC, DT, ST>), dim3(blocks, tokens), dim3(64 * kOneWaves), 0, s, a);
     return host::check_launch("qvb8_moe_experts");
 }
 template <bool DOWN, bool XC, int DT>
-int launch_moe_one(const MoeOneArgs& a, bool regular, unsigned blocks, unsigned tokens, hipStream_t s) {
-    return regular ? launch_moe_one_as<DOWN, XC, DT, true>(a, blocks, tokens, s) : launch_moe_one_as<DOWN, XC, DT, false>(a, blocks, tokens, s);
+int launch_moe_one(const MoeOneArgs& a, MoeStored stored, unsigned blocks, unsigned tokens, hipStream_t s) {
+    if (stored == kInPlanes) return launch_moe_one_as<DOWN, XC, DT, kInPlanes>(a, blocks, tokens, s);
+    return stored == kRegular ? launch_moe_one_as<DOWN, XC, DT, kRegular>(a, blocks, tokens, s) : launch_moe_one_as<DOWN, XC, DT, kAnyhow>(a, blocks, tokens, s);
 }
 
 size_t moe_walk_lds(int64_t row_tiles, int W, int max_tokens) {
@@ -1145,7 +1177,7 @@ size_t moe_walk_lds(int64_t row_tiles, int W, int max_tokens) {
 }
 
 // `slots`: the plan's slots (experts that can be in use)
-template <bool DOWN, bool XC, bool REG>
+template <bool DOWN, bool XC, MoeStored ST>
 int launch_moe_walk_as(MoeWalkArgs a, int64_t slots, int64_t max_tokens, hipStream_t s) {
     const int n_steps = a.P / kStepCols;
     // steps per wave: four, with the next tile's ids in flight; a short down row (up to 768 columns) is one wave's; rows
@@ -1167,17 +1199,18 @@ int launch_moe_walk_as(MoeWalkArgs a, int64_t slots, int64_t max_tokens, hipStre
     dim3 grid((unsigned)wgs), block(64 * kWalkWaves);
     if constexpr (DOWN) {
         if (T == 6) {
-            hipLaunchKernelGGL((moe_walk_kernel<6, true, XC, false, REG>), grid, block, lds, s, a);
+            hipLaunchKernelGGL((moe_walk_kernel<6, true, XC, false, ST>), grid, block, lds, s, a);
             return host::check_launch("qvb8_moe_experts");
         }
     }
-    if (T == 4) hipLaunchKernelGGL((moe_walk_kernel<4, DOWN, XC, true, REG>), grid, block, lds, s, a);
-    else hipLaunchKernelGGL((moe_walk_wide_kernel<DOWN, XC, REG>), grid, block, lds, s, a);
+    if (T == 4) hipLaunchKernelGGL((moe_walk_kernel<4, DOWN, XC, true, ST>), grid, block, lds, s, a);
+    else hipLaunchKernelGGL((moe_walk_wide_kernel<DOWN, XC, ST>), grid, block, lds, s, a);
     return host::check_launch("qvb8_moe_experts");
 }
 template <bool DOWN, bool XC>
-int launch_moe_walk(const MoeWalkArgs& a, bool regular, int64_t slots, int64_t max_tokens, hipStream_t s) {
-    return regular ? launch_moe_walk_as<DOWN, XC, true>(a, slots, max_tokens, s) : launch_moe_walk_as<DOWN, XC, false>(a, slots, max_tokens, s);
+int launch_moe_walk(const MoeWalkArgs& a, MoeStored stored, int64_t slots, int64_t max_tokens, hipStream_t s) {
+    if (stored == kInPlanes) return launch_moe_walk_as<DOWN, XC, kInPlanes>(a, slots, max_tokens, s);
+    return stored == kRegular ? launch_moe_walk_as<DOWN, XC, kRegular>(a, slots, max_tokens, s) : launch_moe_walk_as<DOWN, XC, kAnyhow>(a, slots, max_tokens, s);
 }
 }  // namespace
 
@@ -1205,6 +1238,7 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
         || (up_planes && (act & 0xFF) == 0 && P_dn % 16))
         return host::fail(QVB8_ERR_ARG, "moe: tiles in planes need a regular stack, whole 128-column steps and whole 16-row tiles");
     act &= 0xFF;
+    const MoeStored up_stored = moe_stored(up_regular, up_planes), dn_stored = moe_stored(dn_regular, dn_planes);
     if (Q_up <= 0 || P_up <= 0 || Q_dn <= 0 || P_dn <= 0 || Q_up > 0x7fffffff || P_up > 0x7fffffff || Q_dn > 0x7fffffff || P_dn > 0x7fffffff)
         return host::fail(QVB8_ERR_ARG, "qvb8_moe_experts: bad shape");
     if (act == 0 ? (Q_up % 2 != 0 || Q_up / 2 != P_dn) : (Q_up != P_dn)) return host::fail(QVB8_ERR_ARG, "moe: gate_up/down shapes disagree");
@@ -1243,17 +1277,17 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
         const int64_t cap = kOneMaxTiles / RT;
         if (per_wg > cap) per_wg = cap;
         if (per_wg < 1) per_wg = 1;
-        o.tiles_per_wg = (int)per_wg; o.planes = up_planes ? 1 : 0;
+        o.tiles_per_wg = (int)per_wg;
         const unsigned up_blocks = (unsigned)((total_ut + per_wg - 1) / per_wg);
         const unsigned tk = (unsigned)tokens;
-        if (int rc = x_dtype == QVB8_BF16 ? launch_moe_one<false, true, 0>(o, up_regular, up_blocks, tk, s) : launch_moe_one<false, false, 0>(o, up_regular, up_blocks, tk, s)) return rc;
+        if (int rc = x_dtype == QVB8_BF16 ? launch_moe_one<false, true, 0>(o, up_stored, up_blocks, tk, s) : launch_moe_one<false, false, 0>(o, up_stored, up_blocks, tk, s)) return rc;
         o.X = reinterpret_cast<const uint16_t*>(H); o.ids = dn_ids; o.ids_bytes = dn_ids_bytes;
         o.min_s = dn_min; o.tau_s = dn_tau; o.nbits = dn_nb; o.bit_off = dn_off; o.out = out;
-        o.Q = (int)Q_dn; o.P = (int)P_dn; o.units = (int)Q_dn; o.gated = 0; o.tiles_per_wg = 0; o.planes = dn_planes ? 1 : 0;
+        o.Q = (int)Q_dn; o.P = (int)P_dn; o.units = (int)Q_dn; o.gated = 0; o.tiles_per_wg = 0;
         const unsigned dn_blocks = (unsigned)(Q_dn / 16);
-        if (out_dtype == QVB8_F32) return launch_moe_one<true, false, 0>(o, dn_regular, dn_blocks, tk, s);
-        if (out_dtype == QVB8_F16) return launch_moe_one<true, false, 1>(o, dn_regular, dn_blocks, tk, s);
-        return launch_moe_one<true, false, 2>(o, dn_regular, dn_blocks, tk, s);
+        if (out_dtype == QVB8_F32) return launch_moe_one<true, false, 0>(o, dn_stored, dn_blocks, tk, s);
+        if (out_dtype == QVB8_F16) return launch_moe_one<true, false, 1>(o, dn_stored, dn_blocks, tk, s);
+        return launch_moe_one<true, false, 2>(o, dn_stored, dn_blocks, tk, s);
     }
 
     // a thread per pair (or per expert, when they are more) up to the most a workgroup has
@@ -1268,12 +1302,12 @@ int moe_experts(const void* X, int x_dtype, int64_t tokens, const int64_t* idx, 
         wa.X = reinterpret_cast<const uint16_t*>(X); wa.plan = pl; wa.ids = up_ids; wa.ids_bytes = up_ids_bytes;
         wa.min_s = up_min; wa.tau_s = up_tau; wa.nbits = up_nb; wa.bit_off = up_off; wa.out = H;                // H as fp16 (pairs, P_dn)
         wa.E = (int)n_experts; wa.Q = (int)Q_up; wa.P = (int)P_up; wa.topk = (int)topk; wa.units = (int)P_dn; wa.gated = act == 0 ? 1 : 0;
-        wa.tiles_per_seg = 1; wa.max_tokens = 1; wa.planes = up_planes ? 1 : 0;
-        if (int rc = x_dtype == QVB8_BF16 ? launch_moe_walk<false, true>(wa, up_regular, slots, tokens, s) : launch_moe_walk<false, false>(wa, up_regular, slots, tokens, s)) return rc;
+        wa.tiles_per_seg = 1; wa.max_tokens = 1;
+        if (int rc = x_dtype == QVB8_BF16 ? launch_moe_walk<false, true>(wa, up_stored, slots, tokens, s) : launch_moe_walk<false, false>(wa, up_stored, slots, tokens, s)) return rc;
         wa.X = reinterpret_cast<const uint16_t*>(H); wa.ids = dn_ids; wa.ids_bytes = dn_ids_bytes;
         wa.min_s = dn_min; wa.tau_s = dn_tau; wa.nbits = dn_nb; wa.bit_off = dn_off; wa.out = Yd;
-        wa.Q = (int)Q_dn; wa.P = (int)P_dn; wa.units = (int)Q_dn; wa.gated = 0; wa.planes = dn_planes ? 1 : 0;
-        if (int rc = launch_moe_walk<true, false>(wa, dn_regular, slots, tokens, s)) return rc;
+        wa.Q = (int)Q_dn; wa.P = (int)P_dn; wa.units = (int)Q_dn; wa.gated = 0;
+        if (int rc = launch_moe_walk<true, false>(wa, dn_stored, slots, tokens, s)) return rc;
         return launch_moe_combine(Yd, w, out, out_dtype, topk, Q_dn, tokens, pl, s);
     }
     if (tokens > 16 && (reinterpret_cast<uintptr_t>(X) & 15u) == 0 && moe_group_shapes_ok(P_up, Q_dn, P_dn)) {
