@@ -167,7 +167,11 @@ class QVBandExpertsV8(nn.Module):
             gu, dn = list(self.gate_up_experts), list(self.down_experts)
             ok = (self._act_code() is not None and _stackable(gu) and _stackable(dn)
                   and gu[0].out_features == 2 * dn[0].in_features and gu[0].in_features == dn[0].out_features)
-            self._stk = (stack_projection(gu, 2, planes=True), stack_projection(dn, planes=True)) if ok else False
+            # planes for both projections or for neither: the matrix-core kernels want whole steps of both, and the general kernel, which
+            # then takes every call, gains nothing by them (32 experts of 2048/736, us a call, neither / up alone in planes: 1 token
+            # 31.2 / 32.7, 8 tokens 109 / 109, 40 tokens 326 / 333)
+            whole = ok and self._whole_steps()
+            self._stk = (stack_projection(gu, 2, planes=whole), stack_projection(dn, planes=whole)) if ok else False
         return self._stk is not False
 
     def _whole_steps(self) -> bool:

@@ -124,6 +124,15 @@ def test_a_stack_is_back_to_back_unless_planes_are_asked_for(monkeypatch):
         assert not s["planes"] and not ext.rows_in_planes(s["bit_off"])
 
 
+@pytest.mark.parametrize("hidden,inter", [(256, 96), (96, 256), (256, 128)])
+def test_planes_are_for_stacks_of_whole_steps(hidden, inter, monkeypatch):
+    monkeypatch.setattr(BE, "PLANES_FROM_BYTES", 0)
+    monkeypatch.setenv("QVB8_MOE_ONE_WIDTH_GROWTH", "0.25")
+    gu, dn = _experts(2, hidden, inter, 2e-3)
+    mod = BE.QVBandExpertsV8(gu, dn, num_experts=2).prepare()
+    assert [s["planes"] for s in mod._stk] == [hidden % 128 == 0 and inter % 128 == 0] * 2
+
+
 def test_planes_without_what_they_need_are_refused():
     E, hidden, inter = 2, 256, 128
     gu, dn = _experts(E, hidden, inter, 2e-3)
