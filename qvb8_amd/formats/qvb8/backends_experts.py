@@ -91,9 +91,11 @@ def stack_projection(mods, halves: int = 1, planes: bool = False) -> dict:
               and bool((table["bit_off"][:, 0] % 128 == 0).all()) and os.environ.get("QVB8_PLANES", "1") != "0")
     if planes:
         table["bit_off"] = ext.stack_in_planes(shared, table["bit_off"], P, int(table["nbits"][0, 0]))
+        # an expert's rows in row order, for all of them: what a dense restore needs to take whole tiles (the loop, from 257 rows on)
+        in_order = ext.mma_prepare(*(table[name][0] for name in ("nbits", "bit_off", "tau_s", "min_s")), P, shared.numel())
         for m, off in zip(mods, table["bit_off"]):           # the modules' own offsets say where their rows are now
             m.bit_off = off.clone()
-            m._planes = True
+            m._planes, m._rows_in_order = True, in_order
     return dict(ids=shared, Q=Q, P=P, regular=regular, sliced=sliced, planes=planes, **table)
 
 

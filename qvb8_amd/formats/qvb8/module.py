@@ -361,9 +361,14 @@ class QVBandLinearV8(nn.Module):
             y = ext.gemv_multi(xk, self.ids, self.min_s, self.nbits, self.bit_off, self.in_features, self.tau_s,
                                self.esc_idx, self.esc_vals)
             return self._finish(y, orig, out_dtype)
-        # a weight whose rows lie in planes is restored tile by tile, in the order of the row records built with them
+        # a weight whose rows lie in planes is restored tile by tile, in the order of its row records or, an expert of a stack that has
+        # not built any, of its rows
         built = self.__dict__.get("_mma_cache")
-        rowinfo = built[1] if built and self._planes else None
+        rowinfo = None
+        if self._planes:
+            rowinfo = built[1] if built else self.__dict__.get("_rows_in_order")
+            if rowinfo is not None and rowinfo.device != self.ids.device:
+                rowinfo = None
         if xk.dtype == torch.bfloat16 and self.bf16_gemm and self.bf16_certified:
             W = ext.decode_bf16(self.ids, self.min_s, self.nbits, self.bit_off, self.in_features, self.tau_s,
                                 self.esc_idx_bf16, self.esc_vals_bf16, rowinfo)

@@ -133,6 +133,26 @@ def test_planes_are_for_stacks_of_whole_steps(hidden, inter, monkeypatch):
     assert [s["planes"] for s in mod._stk] == [hidden % 128 == 0 and inter % 128 == 0] * 2
 
 
+def test_an_expert_in_planes_is_restored_tile_by_tile(monkeypatch):
+    """More than 256 rows, the first call of a module that has no row records of its own: by the tiles' order, the values of rows back to back."""
+    x = torch.randn(300, 256, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1))
+    out, orders = [], []
+    for name in ("decode", "decode_bf16"):
+        real = getattr(ext, name)
+        monkeypatch.setattr(ext, name, lambda *a, real=real: (orders.append(a[8] if len(a) > 8 else None), real(*a))[1])
+    for least in (1 << 40, 0):
+        monkeypatch.setattr(BE, "PLANES_FROM_BYTES", least)
+        gu, dn = _experts(3, 256, 128, 2e-3)
+        BE.QVBandExpertsV8(gu, dn, num_experts=3).prepare()
+        for dtype in (torch.float32, torch.float16, torch.bfloat16):
+            orders.clear()
+            out.append(gu[1](x.to(dtype)))
+            assert len(orders) == 1 and (orders[0] is not None) == (least == 0)
+        assert gu[1].__dict__.get("_mma_cache") is None
+    for a, b in zip(out[:3], out[3:]):
+        assert torch.equal(a, b)
+
+
 def test_planes_without_what_they_need_are_refused():
     E, hidden, inter = 2, 256, 128
     gu, dn = _experts(E, hidden, inter, 2e-3)
