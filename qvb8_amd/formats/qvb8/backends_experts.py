@@ -122,7 +122,9 @@ class QVBandExpertsV8(nn.Module):
     # us, routed / loop).  8 experts of 4096/14336 (176 M weights): 256 pairs 2239 / 2855, 512 pairs 3591 / 3583, 1024 pairs
     # 6609 / 4886, 2048 pairs 12697 / 8312.  50 M weights: 512 pairs 2137 / 2897 (16 experts of 4096/4096) and 653 / 883 (4 of
     # 2048/8192), 1024 pairs 3874 / 3826 and 1157 / 1182, 2048 pairs 7558 / 5945 and 2082 / 1716.  2048/768 (4.7 M weights): 8192 pairs
-    # 3531 / 4634 (16 experts), 512 pairs 1996 / 19906 (128 experts).
+    # 3531 / 4634 (16 experts), 512 pairs 1996 / 19906 (128 experts).  That was with rows back to back.  Stacks in planes would have the
+    # line at about 1e11 products: 8 experts of 4096/14336, 512 pairs 2700 / 3125, 768 pairs 3850 / 3805, 1024 pairs 5325 / 4520; 16 of
+    # 4096/4096, 1024 pairs 3005 / 3590, 2048 pairs 6020 / 5740; 4 of 2048/8192, 1024 pairs 880 / 1075, 2048 pairs 1620 / 1605.
     LOOP_FROM_PAIRS, LOOP_FROM_PRODUCTS = 512, 5e10
     # Rows the kernels read id by id (width outside 4..8 or off a dword): for each pair again, while the loop restores them once
     # from 97 rows of activations on and is slow below that only where experts are small.  32 experts of 2048/768, a third of
