@@ -9,13 +9,12 @@ constexpr int kColumnsMaxM = 64;
 
 struct ColumnsArgs {
     const uint16_t* X16;           // activations in operand order, kStepCols columns a step, one step of zeros behind the last
-    const float* sx;               // [splits][M] sums of the rows of X over each column range
+    const float* sx;               // sums of the rows of X
     const uint8_t* ids;
     const uint4* fin;
-    float* out;                    // Y (one column range) or the partial results [splits][M][Q]
+    float* out;                    // Y
     int M, Q, P;
     int out_dt;                    // what `out` holds: 0 fp32, 1 fp16, 2 bf16
-    int steps_per_split;
     int planes;                    // whole tiles are stored in planes (see qvb8_device.h)
     int first1, first2;            // positions where the second and the third width start (Q when there is none)
     int units1, units2, units3;    // units before the second, the third width, and behind its whole tiles
@@ -24,10 +23,10 @@ struct ColumnsArgs {
 
 struct ColumnsPlan {
     int MT, G;                     // token tiles, row tiles per workgroup
-    int units, splits, steps_per_split;
+    int units;
     bool taken;                    // whether this kernel is the one for the sizes
     bool by_tile;                  // tiles of one width in planes at multiples of 16
-    int64_t x16_at, sx_at, part_at, bytes;      // workspace layout, bytes from its start (after the row records' place)
+    int64_t x16_at, sx_at, bytes;  // workspace layout, bytes from its start (after the row records' place)
 };
 
 ColumnsPlan plan_columns(int64_t M, int64_t Q, int64_t P);

@@ -30,16 +30,15 @@
 namespace qvb8 {
 namespace {
 
-// One workgroup per row of X (rows M.. of the last token tile: zeros) and column range.
+// One workgroup per row of X (rows M.. of the last token tile: zeros).
 // X16[step][token tile][j][lane = token + 16 kg][8]: columns 128 step + 32 kg + 8 j .. + 7 of the token, what the lane feeds MFMA j.
 template <bool XC>
-__global__ void __launch_bounds__(256) columns_prep_kernel(const uint16_t* __restrict__ X, int M, int P, int steps_per_split, int MT, uint16_t* __restrict__ X16, float* __restrict__ sx) {
+__global__ void __launch_bounds__(256) columns_prep_kernel(const uint16_t* __restrict__ X, int M, int P, int MT, uint16_t* __restrict__ X16, float* __restrict__ sx) {
     __shared__ float red[4];
-    const int m = blockIdx.x, z = blockIdx.y, tid = threadIdx.x, n_steps = P / kStepCols;
-    const int p0 = z * steps_per_split * 16, p1 = min(n_steps, (z + 1) * steps_per_split) * 16;      // 8-column pieces
+    const int m = blockIdx.x, tid = threadIdx.x, n_steps = P / kStepCols;
     uint4* const to = reinterpret_cast<uint4*>(X16) + (m >> 4) * 256 + (m & 15);
     float part = 0.f;
-    for (int p = p0 + tid; p < p1; p += 256) {
+    for (int p = tid; p < n_steps * 16; p += 256) {                                       // 8-column pieces
         uint32_t w[4] = {0u, 0u, 0u, 0u};
         if (m < M) {
             const uint4 v = *reinterpret_cast<const uint4*>(X + (size_t)m * P + 8 * p);
@@ -52,11 +51,11 @@ __global__ void __launch_bounds__(256) columns_prep_kernel(const uint16_t* __res
         }
         to[(size_t)(p >> 4) * MT * 256 + (p & 3) * 64 + ((p >> 2) & 3) * 16] = uint4{w[0], w[1], w[2], w[3]};
     }
-    if (z == 0 && tid < 16) to[(size_t)n_steps * MT * 256 + (tid & 3) * 64 + (tid >> 2) * 16] = uint4{0u, 0u, 0u, 0u};
+    if (tid < 16) to[(size_t)n_steps * MT * 256 + (tid & 3) * 64 + (tid >> 2) * 16] = uint4{0u, 0u, 0u, 0u};
     part = wave_sum(part);
     if ((tid & 63) == 0) red[tid >> 6] = part;
     __syncthreads();
-    if (tid == 0 && m < M) sx[(size_t)z * M + m] = (red[0] + red[1]) + (red[2] + red[3]);
+    if (tid == 0 && m < M) sx[m] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // a lane's slice of one tile and step: the first four dwords and the NB - 4 others
@@ -123,18 +122,17 @@ __device__ __forceinline__ void columns_run(const ColumnsArgs& a, const uint16_t
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kg = lane >> 4;
     const int n_steps = a.P / kStepCols;
-    const int s_begin = (int)blockIdx.y * a.steps_per_split, s_end = min(n_steps, s_begin + a.steps_per_split);
     const uint32_t row_bytes = (uint32_t)a.P / 8u * NB;
     const uint8_t* const tiles = ids_base + u.byte0 + (uint64_t)(uint32_t)(u.pos0 - u.first) * row_bytes;
     const int n_tiles = (u.end - u.pos0 + 15) / 16;
-    // the lane's slice of tile t, step s (past the range: the last one again; past the last tile or row: the last one, not stored)
+    // the lane's slice of tile t, step s (past the end: the last one again; past the last tile or row: the last one, not stored)
     auto request = [&](int t, int s, Slice<NB>& to) __attribute__((always_inline)) {
-        [[maybe_unused]] const uint8_t* at = tiles + ((uint64_t)(uint32_t)min(t, n_tiles - 1) * (16u * row_bytes) + (uint64_t)(uint32_t)min(s, s_end - 1) * (PL ? 256u * NB : 16u * NB));
+        [[maybe_unused]] const uint8_t* at = tiles + ((uint64_t)(uint32_t)min(t, n_tiles - 1) * (16u * row_bytes) + (uint64_t)(uint32_t)min(s, n_steps - 1) * (PL ? 256u * NB : 16u * NB));
         if constexpr (PL) load_slice_at<NB>(at + (uint32_t)lane * 16u, at + 1024u + (uint32_t)lane * (4u * (NB - 4u)), to);
         else {
             const int ln = lane_now(), pos = min(u.pos0 + 16 * min(t, n_tiles - 1) + (ln & 15), u.end - 1), t0 = pos & ~15;
             const bool whole = a.planes && t0 >= u.first && t0 + 16 <= u.run_end;
-            const uint32_t slot = (uint32_t)(pos & 15) + (uint32_t)(ln & 48), g = (uint32_t)(ln >> 4), sc = (uint32_t)min(s, s_end - 1);
+            const uint32_t slot = (uint32_t)(pos & 15) + (uint32_t)(ln & 48), g = (uint32_t)(ln >> 4), sc = (uint32_t)min(s, n_steps - 1);
             const uint8_t* lo = ids_base + u.byte0 + (uint64_t)(uint32_t)((whole ? t0 : pos) - u.first) * row_bytes + (whole ? sc * (256u * NB) + slot * 16u : sc * (16u * NB) + g * (4u * NB));
             load_slice_at<NB>(lo, lo + (whole ? 1024u - slot * 16u + slot * (4u * (NB - 4u)) : 16u), to);
         }
@@ -148,8 +146,8 @@ __device__ __forceinline__ void columns_run(const ColumnsArgs& a, const uint16_t
     // X a quarter of a step at a time (what the MFMAs j take), three quarters ahead
     v4u_t x[4][MT];
     auto request_x = [&](int s, int j) __attribute__((always_inline)) {
-        // past the range: the step of zeros
-        const uint8_t* at = reinterpret_cast<const uint8_t*>(X16) + ((uint64_t)(uint32_t)(s < s_end ? s : n_steps) * (MT * 4096) + (uint32_t)j * 1024u);
+        // past the end: the step of zeros
+        const uint8_t* at = reinterpret_cast<const uint8_t*>(X16) + ((uint64_t)(uint32_t)min(s, n_steps) * (MT * 4096) + (uint32_t)j * 1024u);
 #pragma unroll
         for (int m = 0; m < MT; ++m) x[j][m] = *reinterpret_cast<const v4u_t*>(at + m * 4096 + (uint32_t)lane * 16u);
     };
@@ -166,9 +164,9 @@ __device__ __forceinline__ void columns_run(const ColumnsArgs& a, const uint16_t
     uint4* const s_fin = reinterpret_cast<uint4*>(smem + W * CT * MT * 1024);
     float* const s_sx = reinterpret_cast<float*>(s_fin + 16 * G);
     const uint4 my_fin = a.fin[min(u.pos0 + min(tid, 16 * G - 1), u.end - 1)];
-    const float my_sx = a.sx[(size_t)blockIdx.y * (size_t)a.M + min(lane, a.M - 1)];
+    const float my_sx = a.sx[min(lane, a.M - 1)];
     __builtin_amdgcn_sched_barrier(0);
-    const int s0 = s_begin + wave, n_it = (s_end - s_begin + W - 1) / W;
+    const int s0 = wave, n_it = (n_steps + W - 1) / W;
     request_x(s0, 0);
     request_x(s0, 1);
     request_x(s0, 2);
@@ -204,7 +202,6 @@ __device__ __forceinline__ void columns_run(const ColumnsArgs& a, const uint16_t
         if constexpr (RB == 2) step(s0 + W * (i + 1), raw[RB - 1]);       // (an odd number of steps: the step of zeros)
     }
     // ---- the waves' columns meet ----
-    float* const out = a.out + (size_t)blockIdx.y * (size_t)a.M * (size_t)a.Q;
 #pragma unroll
     for (int t0 = 0; t0 < G; t0 += CT) {
         if (t0 > 0) __syncthreads();
@@ -226,7 +223,7 @@ __device__ __forceinline__ void columns_run(const ColumnsArgs& a, const uint16_t
             for (int k = 0; k < 4; ++k) {
                 const int tok = m * 16 + kg * 4 + k;
                 if (tok < a.M) {
-                    store_y(out, a.out_dt, (int64_t)tok * a.Q + f.z, (float)(ts * (double)sum[k] + mid * (double)s_sx[tok]));
+                    store_y(a.out, a.out_dt, (int64_t)tok * a.Q + f.z, (float)(ts * (double)sum[k] + mid * (double)s_sx[tok]));
                 }
             }
         }
@@ -272,7 +269,7 @@ __global__ void __launch_bounds__(64 * kColumnsWaves, kColumnsWaves / 4) columns
 template <int MT, int G>
 int launch_as(const ColumnsPlan& p, const ColumnsArgs& a, hipStream_t s) {
     constexpr size_t lds = (size_t)kColumnsWaves * columns_tiles_at_once(MT, G) * MT * 1024 + 16 * G * 16 + 64 * 4;
-    const dim3 grid((unsigned)p.units, (unsigned)p.splits), block(64 * kColumnsWaves);
+    const dim3 grid((unsigned)p.units), block(64 * kColumnsWaves);
     if (int rc = p.by_tile ? host::raise_lds_limit<columns_kernel<true, MT, G>>(lds, "qvb8_mma") : host::raise_lds_limit<columns_kernel<false, MT, G>>(lds, "qvb8_mma")) return rc;
     if (p.by_tile) hipLaunchKernelGGL((columns_kernel<true, MT, G>), grid, block, lds, s, a.X16, a.ids, a);
     else hipLaunchKernelGGL((columns_kernel<false, MT, G>), grid, block, lds, s, a.X16, a.ids, a);
@@ -296,48 +293,46 @@ int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 }  // namespace
 
 namespace {
-constexpr int kMostSplits = 4;
+constexpr int kMostRanges = 4;
 constexpr int kGroups[] = {1, 2, 3, 4, 6, 8};                      // row tiles a unit may have
 constexpr int most_tiles(int MT) { return MT == 2 ? 8 : 6; }       // ... as the registers hold
 // What a call takes, in 1/100 us: rounds of units (start and end of each, then its wave's steps -- bound by the ids' share of memory, by the
-// activations' share of L2 or by decode and products), the joining of column ranges.
-int64_t columns_cost(int64_t units, int MT, int G, int64_t M, int64_t Q, int64_t n_steps, int splits) {
-    const int64_t cus = host::device_cus(), rounds = (units * splits + cus - 1) / cus;
-    const int64_t steps = ((n_steps + splits - 1) / splits + kColumnsWaves - 1) / kColumnsWaves;
-    const int64_t memory = 68 * G * std::min<int64_t>(units * splits, rounds * cus) / (rounds * cus);
+// activations' share of L2 or by decode and products).  `ranges`: as if the columns were cut into so many, joined by another launch; with
+// more than one the kernel is not taken.
+int64_t columns_cost(int64_t units, int MT, int G, int64_t M, int64_t Q, int64_t n_steps, int ranges = 1) {
+    const int64_t cus = host::device_cus(), rounds = (units * ranges + cus - 1) / cus;
+    const int64_t steps = ((n_steps + ranges - 1) / ranges + kColumnsWaves - 1) / kColumnsWaves;
+    const int64_t memory = 68 * G * std::min<int64_t>(units * ranges, rounds * cus) / (rounds * cus);
     const int64_t step = std::max<int64_t>({memory, 62 * MT, 22 * G + 6 * G * MT});
-    return rounds * (700 + steps * step) + (splits > 1 ? 500 + 100 * splits + splits * M * Q / 5000 : 0);
+    return rounds * (700 + steps * step) + (ranges > 1 ? 500 + 100 * ranges + ranges * M * Q / 5000 : 0);
 }
 }  // namespace
 
 static ColumnsPlan make_plan(int64_t M, int64_t Q, int64_t P) {
     ColumnsPlan p = {};
     p.MT = M <= 32 ? 2 : M <= 48 ? 3 : 4;
-    // Column ranges by the weight's size alone, not by how its rows are stored: a row's products are then the same bit for bit.
+    // By the weight's size alone, not by how its rows are stored: a row's products are then the same bit for bit.
     const int64_t n_steps = P / kStepCols, tiles = (Q + 15) / 16;
     const int64_t cus = host::device_cus();
     int64_t best = INT64_MAX, units_best = 0;
-    int splits = 1;
-    for (int z = 1; z <= kMostSplits && (z == 1 || n_steps / z >= kColumnsWaves); ++z)
+    int ranges = 1;
+    for (int z = 1; z <= kMostRanges && (z == 1 || n_steps / z >= kColumnsWaves); ++z)
         for (int g : kGroups) {
             if (g > most_tiles(p.MT)) break;
             const int64_t units = (tiles + g - 1) / g, cost = columns_cost(units, p.MT, g, M, Q, n_steps, z);
-            if (cost < best) { best = cost; splits = z; units_best = units * z; }
+            if (cost < best) { best = cost; ranges = z; units_best = units; }
         }
     // The kernels that stage X in LDS (gemm_kernel) keep: up to 32 rows, weights of more than a round of units (34816 x 5120, 20 rows, 40.8 us
     // against 45.7) or of more than 8192 columns (20000 x 9984, 20 rows, 35.9 / 42.0); few rows of W and long ones, whose columns they split over the chip (5120 x 17408, 24 rows 23.8 / 36.5, 64 rows 33.3 / 37).
-    p.taken = splits > 1 ? M > 32 && tiles >= 1024 : (M > 32 || (units_best <= cus && n_steps <= 8 * kColumnsWaves)) && (10 * units_best >= 7 * cus || n_steps <= 4 * kColumnsWaves);
+    p.taken = ranges == 1 && (M > 32 || (units_best <= cus && n_steps <= 8 * kColumnsWaves)) && (10 * units_best >= 7 * cus || n_steps <= 4 * kColumnsWaves);
     // ... and, where they can read the weight (P a multiple of 256), long rows with any number of rows of X (us them / here: 26675 x 8960, 33
-    // rows 64.6 / 70.1, 64 rows 67.7 / 79.3; up to 32 rows from 48 steps on: 12290 x 7936, 17 rows 27.5 / 29.4, 40 rows 36.6 / 33.5) and large weights whose waves would have a single step each (32603 x 1024, 17 rows 14.9 / 18.5,
+    // rows 64.6 / 70.1, 64 rows 67.7 / 79.3; up to 32 rows those of more than 48 steps: 12290 x 7936, 17 rows 27.5 / 29.4, 40 rows 36.6 / 33.5) and large weights whose waves would have a single step each (32603 x 1024, 17 rows 14.9 / 18.5,
     // 64 rows 24.2 / 24.6; of ten steps, 15339 x 1280, 19.4 / 16.6 and 30.3 / 22.6).  The tile kernel, which takes the others, is behind (29291 x 8320,
     // 40 rows, 136 / 80).
     if (P % 256 == 0 && (n_steps > (M <= 32 ? 6 : 8) * kColumnsWaves || (n_steps <= kColumnsWaves && tiles >= 1024))) p.taken = false;
-    p.steps_per_split = (int)((n_steps + splits - 1) / splits);
-    p.splits = (int)((n_steps + p.steps_per_split - 1) / p.steps_per_split);
     p.x16_at = align256(qvb8_mma_rowinfo_bytes(Q));
     p.sx_at = p.x16_at + (n_steps + 1) * p.MT * 4096;
-    p.part_at = p.sx_at + align256((int64_t)p.splits * M * 4);
-    p.bytes = p.part_at + (p.splits > 1 ? (int64_t)p.splits * M * Q * 4 : 0);
+    p.bytes = p.sx_at + align256(M * 4);
     return p;
 }
 
@@ -361,17 +356,17 @@ int launch_columns(ColumnsPlan p, ColumnsArgs a, const uint16_t* X, int mode, ui
         int units[3];
         for (int c = 0; c < 3; ++c) units[c] = ((planes ? rows[c] / 16 : (rows[c] + 15) / 16) + g - 1) / g;
         const int whole = units[0] + units[1] + units[2], all = whole + (planes && a.Q % 16 != 0 ? 1 : 0);
-        const int64_t cost = columns_cost(all, p.MT, g, a.M, a.Q, a.P / kStepCols, p.splits);
+        const int64_t cost = columns_cost(all, p.MT, g, a.M, a.Q, a.P / kStepCols);
         if (cost >= best) continue;
         best = cost;
         p.G = g; p.units = all;
         a.units1 = units[0]; a.units2 = units[0] + units[1]; a.units3 = whole;
     }
-    const dim3 grid((unsigned)(16 * p.MT), (unsigned)p.splits);
-    if (mode == 1) hipLaunchKernelGGL((columns_prep_kernel<true>), grid, dim3(256), 0, s, X, a.M, a.P, p.steps_per_split, p.MT, x16, sx);
-    else hipLaunchKernelGGL((columns_prep_kernel<false>), grid, dim3(256), 0, s, X, a.M, a.P, p.steps_per_split, p.MT, x16, sx);
+    const dim3 grid((unsigned)(16 * p.MT));
+    if (mode == 1) hipLaunchKernelGGL((columns_prep_kernel<true>), grid, dim3(256), 0, s, X, a.M, a.P, p.MT, x16, sx);
+    else hipLaunchKernelGGL((columns_prep_kernel<false>), grid, dim3(256), 0, s, X, a.M, a.P, p.MT, x16, sx);
     if (int rc = host::check_launch("qvb8_mma activations")) return rc;
-    a.X16 = x16; a.sx = sx; a.steps_per_split = p.steps_per_split;
+    a.X16 = x16; a.sx = sx;
     if (p.MT == 2) return launch_rows<2>(p, a, s);
     if (p.MT == 3) return launch_rows<3>(p, a, s);
     return launch_rows<4>(p, a, s);

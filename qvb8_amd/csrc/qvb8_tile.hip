@@ -1578,8 +1578,13 @@ GemmPlan plan_gemm_for(int64_t M, int64_t Q, int64_t P) { return M >= gemm2_from
 // projections, 8 layers: M = 17 0.641 ms against 0.721 for the tile kernel with two token tiles, M = 32 0.70 / 0.87)
 int gemm_from() { const int v = host::env_int("QVB8_MMA_GEMM_FROM", 17); return v < 17 ? 17 : (v > 49 ? 49 : v); }
 
-// (the sizes first: a call of a few rows, bound by the host, does not look at the environment for it)
-bool columns_take(int64_t M) { return M >= 17 && M <= kColumnsMaxM && M >= gemm_from() && host::env_int("QVB8_COLUMNS", 1) != 0; }
+// The kernel whose waves take columns of their own, where its plan says so (the sizes first: a call of a few rows, bound by the host, does not
+// look at the environment for it).
+bool columns_take(int64_t M, int64_t Q, int64_t P, ColumnsPlan& plan) {
+    if (M < 17 || M > kColumnsMaxM || M < gemm_from() || P % kStepCols || (M > 48 && P % (2 * kGemmStageCols)) || host::env_int("QVB8_COLUMNS", 1) == 0) return false;
+    plan = plan_columns(M, Q, P);
+    return plan.taken;
+}
 
 template <int MT, bool BF, bool XC, int RT>
 int launch_gemm_as(const GemmArgs& a, const GemmPlan& g, int row_blocks, hipStream_t s) {
@@ -1677,7 +1682,7 @@ extern "C" int64_t qvb8_mma_workspace_bytes(int64_t M, int64_t Q, int64_t P) {
     int64_t need = qvb8_mma_rowinfo_bytes(Q);
     if (M < gemm_from() || M > 256 || Q < 1 || P < 1) return need;
     if (P % (2 * kGemmStageCols) == 0) need = std::max(need, plan_gemm_for(M, Q, P).bytes);
-    if (columns_take(M) && P % kStepCols == 0) need = std::max(need, plan_columns(M, Q, P).bytes);
+    if (ColumnsPlan cp; columns_take(M, Q, P, cp)) need = std::max(need, cp.bytes);
     return need;
 }
 
@@ -1755,14 +1760,9 @@ extern "C" int qvb8_mma(const void* X, int x_dtype, int64_t M,
     // mode 0: fp16 X, fp16 operands; 1: bf16 X narrowed to saturated fp16 on the way in, fp16 operands; 2: bf16 operands
     const int mode = x_dtype == QVB8_F16 ? 0 : (flags & QVB8_MMA_SATURATE_X) ? 1 : 2;
     int rc;
-    bool columns = columns_take(M) && layout && mode != 2 && (M <= 48 || P % (2 * kGemmStageCols) == 0) && workspace
-                   && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
     ColumnsPlan cp = {};
-    if (columns) {
-        for (int c = 0; c < a.n_classes; ++c) columns = columns && a.nb[c] >= 4 && a.nb[c] <= 8;
-        cp = plan_columns(M, Q, P);
-        columns = columns && cp.taken && workspace_bytes >= cp.bytes;
-    }
+    bool columns = layout && mode != 2 && workspace && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 && columns_take(M, Q, P, cp) && workspace_bytes >= cp.bytes;
+    for (int c = 0; c < a.n_classes; ++c) columns = columns && a.nb[c] >= 4 && a.nb[c] <= 8;
     // Many rows of X: the workgroup-tiled kernel.  It addresses rows arithmetically and decodes whole slices only; from 17
     // rows on it is also the faster one (the tile kernel then keeps too few bytes in flight), so it is taken whenever it
     // can read the weight and the caller brought its workspace.
@@ -1776,17 +1776,11 @@ extern "C" int qvb8_mma(const void* X, int x_dtype, int64_t M,
         unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
         ColumnsArgs ca = {};
         ca.ids = ids; ca.fin = a.fin; ca.M = (int)M; ca.Q = (int)Q; ca.P = (int)P;
-        ca.out = cp.splits > 1 ? reinterpret_cast<float*>(ws + cp.part_at) : Y;
-        ca.out_dt = cp.splits > 1 ? 0 : out_dt;
+        ca.out = Y; ca.out_dt = out_dt;
         ca.planes = a.planes;
         ca.first1 = a.first1; ca.first2 = a.first2;
         ca.widths = (uint32_t)a.nb[0] | ((uint32_t)a.nb[1] << 8) | ((uint32_t)a.nb[2] << 16);
         if ((rc = launch_columns(cp, ca, a.X, mode, reinterpret_cast<uint16_t*>(ws + cp.x16_at), reinterpret_cast<float*>(ws + cp.sx_at), s))) return rc;
-        if (cp.splits > 1) {
-            const int64_t n = M * Q;
-            hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ca.out, Y, n, cp.splits, out_dt);
-            if (int rc2 = host::check_launch("qvb8_mma reduce")) return rc2;
-        }
     } else if (tiled) {
         if (!layout) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_mma: M > 48 needs rows stored in width order (a row layout)");
         if ((P % (2 * kGemmStageCols)) != 0) return host::fail(QVB8_ERR_UNSUPPORTED, "qvb8_mma: M > 48 needs P %% 256 == 0");
