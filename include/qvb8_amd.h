@@ -404,7 +404,8 @@ int qvb8r_gemv_as(const void* X, int x_dtype, int64_t M, const qvb8r_core* core,
 
 /* Measurement aid: the launch of qvb8r_gemv for one row of X with the activations not read and the two multiply-adds per
  * symbol pair replaced by an exclusive-or of the symbols -- the rANS walk alone (slot lookups, 64-bit state updates, word
- * hand-out, ring reads), the ceiling of the fused kernel on this hardware.  Y (f32, Q) receives values without meaning.
+ * hand-out, ring reads), what the fused kernel of fp32 rows cannot be faster than.  (Of 16-bit rows of large weights the
+ * kernel takes symbols that fit a byte without the mask that is part of this: two instructions of a pair's 34.)  Y (f32, Q) receives values without meaning.
  * No counterpart in the reference. */
 int qvb8r_walk_probe(const qvb8r_core* core, int64_t max_tile_rows, float* Y, void* stream);
 

@@ -257,7 +257,8 @@ __device__ __forceinline__ void store_y(void* Y, int y_dt, int64_t i, float v) {
 
 // ---- fused decode + product, one row of X ------------------------------------------------------------------------------
 // WALK_ONLY (a measurement aid, qvb8r_walk_probe): the same launch with the activations not read and the two multiply-adds
-// per pair replaced by an exclusive-or that keeps the symbols alive -- what the walk alone costs, the ceiling of this path.
+// per pair replaced by an exclusive-or that keeps the symbols alive -- what the walk alone costs, with whole symbols (BYTES saves two of a
+// pair's instructions that are counted here).
 // From as many weights per CU (rows of 1024 columns and more) the kernel looks for symbols that fit a byte: below, a launch is bound by the walk's
 // chain of lookups, not by its instructions, and the two barriers that takes show (us without / with: 1000 x 5120 16.6 / 16.8, 4096 x
 // 4096 16.0 / 16.1, 8192 x 2048 16.4 / 16.6, 17000 x 512 18.2 / 18.7; 8192 x 5120 27.2 / 26.4, 12288 x 4096 30.5 / 29.6, 5120 x 17408 66.5 / 62.1).

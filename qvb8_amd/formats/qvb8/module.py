@@ -39,7 +39,8 @@ _MMA_SPLIT_MAX = 2 * _MMA_MAX_M
 def _run_multiple(rows: int) -> int:
     """Rows that a run of one width is stored in multiples of: a 16-row tile, or the tiles one workgroup of the kernels for 17..64 rows
     of X takes (2, 3, 4 or 6 of one width, by the weight's size), so that a run's last ones are no workgroup more: 24576 rows are 256
-    workgroups, one per compute unit, and one more would be a second round (64 rows of X 31 -> 47 us).  Less than 0.3 % more bytes."""
+    workgroups, one per compute unit, and one more would be a second round (64 rows of X 31 -> 47 us).  At most one row less than that moves up
+    at each boundary between widths: 0.44 % more bytes at 12288 rows of 6, 7 and 8 bits, more where widths present are not neighbours."""
     return 192 if rows >= 12288 else 32 if rows >= 8192 else 16
 
 
@@ -250,7 +251,7 @@ class QVBandLinearV8(nn.Module):
                     planes = self.plane_tiles and os.environ.get("QVB8_PLANES", "1") != "0"
                     ids, nbits, bit_off, order = self.ids, self.nbits, self.bit_off, perm
                     # whole tiles only: a tile across two widths is read row by row, and a launch waits for its slowest
-                    # workgroup -- so up to 15 rows per width are stored one width up (their values do not change)
+                    # workgroup -- so a few rows per width are stored one width up (their values do not change)
                     wide = ext.widen_rows_to_whole_tiles(ids, nbits, bit_off, self.in_features, _run_multiple(self.out_features)) if planes else None
                     if wide is not None:
                         ids, nbits, bit_off = wide
