@@ -17,11 +17,25 @@ def _experts(E, hidden, inter, tau):
     return [pack(2 * inter, hidden) for _ in range(E)], [pack(hidden, inter) for _ in range(E)]
 
 
+ROUTED = [(1, 2, torch.bfloat16), (5, 2, torch.float16), (8, 2, torch.bfloat16), (16, 3, torch.float16), (3, 2, torch.float32),
+          (17, 2, torch.float32), (40, 3, torch.bfloat16), (150, 4, torch.bfloat16)]
+
+
 @pytest.mark.parametrize("tau,growth", [(2e-3, 0.25), (1e-3, 0.25), (4e-4, 0.25)])            # 6, 7 and 8 bits a weight
-@pytest.mark.parametrize("T,k,dtype", [(1, 2, torch.bfloat16), (5, 2, torch.float16), (8, 2, torch.bfloat16), (16, 3, torch.float16), (3, 2, torch.float32),
-                                       (17, 2, torch.float32), (40, 3, torch.bfloat16), (150, 4, torch.bfloat16)])
+@pytest.mark.parametrize("T,k,dtype", ROUTED)
 def test_planes_change_no_result(T, k, dtype, tau, growth, monkeypatch):
-    E, hidden, inter = 5, 384, 128
+    _same_in_planes(T, k, dtype, 384, 128, tau, growth, monkeypatch)
+
+
+# one dword in the second plane and none (rows long enough that their ranges, and so their widths, differ little); rows of more than 2048 columns
+@pytest.mark.parametrize("hidden,inter,tau,bits", [(512, 512, 3e-3, 5), (512, 512, 5.6e-3, 4), (2304, 256, 2e-3, 6), (256, 2176, 2e-3, 6)])
+@pytest.mark.parametrize("T,k,dtype", ROUTED)
+def test_planes_of_narrow_and_of_long_rows_change_no_result(T, k, dtype, hidden, inter, tau, bits, monkeypatch):
+    _same_in_planes(T, k, dtype, hidden, inter, tau, 0.25, monkeypatch, bits)
+
+
+def _same_in_planes(T, k, dtype, hidden, inter, tau, growth, monkeypatch, bits=None):
+    E = 5
     monkeypatch.setenv("QVB8_MOE_ONE_WIDTH_GROWTH", str(growth))
     g = torch.Generator(device=DEV).manual_seed(T)
     x = torch.randn(T, hidden, device=DEV, generator=g).to(dtype)
@@ -31,7 +45,7 @@ def test_planes_change_no_result(T, k, dtype, tau, growth, monkeypatch):
         monkeypatch.setattr(BE, "PLANES_FROM_BYTES", least)
         gu, dn = _experts(E, hidden, inter, tau)
         mod = BE.QVBandExpertsV8(gu, dn, num_experts=E).prepare()
-        assert [s["planes"] for s in mod._stk] == [least == 0] * 2
+        assert [s["planes"] for s in mod._stk] == [least == 0] * 2 and bits in (None, int(mod._stk[0]["nbits"][0, 0]))
         out.append(mod(x, idx, w))
         one += [ext.decode_f32(m.ids, m.min_s, m.nbits, m.bit_off, m.in_features, m.tau_s, m.esc_idx, m.esc_vals) for m in (gu[3], dn[1])]
         one[-2:] = [*one[-2:], gu[2](x), dn[4](gu[0](x)[:, :inter])]
