@@ -58,7 +58,8 @@ def stack_projection(mods, halves: int = 1, planes: bool = False) -> dict:
             one_width = hi
     for m, wider in zip(mods, targets):                  # the routed kernels read rows stored back to back only
         if m._planes or ext.rows_in_planes(m.bit_off):
-            m.ids, m.bit_off = ext.rows_back_to_back(m.ids, m.nbits, m.bit_off, m.in_features)
+            # (the module's own rows alone: an expert of an earlier stack in planes reads a buffer that holds all of them)
+            m.ids, m.bit_off = ext.repack_rows(m.ids, m.nbits, m.bit_off, m.in_features, m.nbits)
             m._planes = False
             m.__dict__.pop("_mma_cache", None)
         if one_width is not None:

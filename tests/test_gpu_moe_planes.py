@@ -167,6 +167,20 @@ def test_an_expert_in_planes_is_restored_tile_by_tile(monkeypatch):
         assert torch.equal(a, b)
 
 
+def test_a_second_stack_of_the_same_experts(monkeypatch):
+    """Built from modules that lie in the planes of an earlier one: as large, and the same results."""
+    monkeypatch.setattr(BE, "PLANES_FROM_BYTES", 0)
+    gu, dn = _experts(4, 256, 384, 2e-3)
+    x, idx, w = torch.randn(9, 256, device=DEV).half(), torch.arange(18, device=DEV).view(9, 2) % 4, torch.full((9, 2), 0.5, device=DEV)
+    out, size = [], []
+    for _ in range(2):
+        mod = BE.QVBandExpertsV8(gu, dn, num_experts=4).prepare()
+        assert all(s["planes"] for s in mod._stk)
+        out.append(mod(x, idx, w))
+        size.append([s["ids"].numel() for s in mod._stk])
+    assert torch.equal(*out) and size[0] == size[1]
+
+
 def test_planes_without_what_they_need_are_refused():
     E, hidden, inter = 2, 256, 128
     gu, dn = _experts(E, hidden, inter, 2e-3)
