@@ -284,7 +284,7 @@ def bench_moe(args, dev):
                          "kernel": ("qvb8::moe_one_kernel<4,false,..> + moe_one_kernel<6,true,..> (one layer = 2 launches)" if T <= 6 else
                                     "qvb8::moe_plan_kernel + moe_walk_kernel<4,false,..> + moe_walk_kernel<6,true,..> + "
                                     "moe_combine_kernel (one layer = 4 launches)" if T <= 16 else
-                                    "qvb8::moe_plan_kernel + moe_gemv_kernel<0> + moe_gemv_kernel<1> + moe_combine_kernel "
+                                    "qvb8::moe_plan_kernel + moe_group_kernel<false,..> + moe_group_kernel<true,..> + moe_combine_kernel "
                                     "(one layer = 4 launches)"),
                          "bytes_per_launch": step_bytes // n_calls, "launch_us": round(per_layer_us, 3)},
             "cpu_baseline": None}
